@@ -190,9 +190,9 @@ __device__ void settle(const EditArgs &a, int slot, int n, int m, int64_t found)
     // The narrowest band the strict certificate proves at the found cost: it holds every optimal path.
     const int end = m - n;
     const int64_t target = found + 1;
-    int h = end > 0 ? end : 0, l = end < 0 ? end : 0;
-    while (h < m && off_band(s.costs, h + 1, end) < target) ++h;
-    while (l > -n && off_band(s.costs, l - 1, end) < target) --l;
+    const auto off_at = [&](int64_t k) { return off_band(s.costs, k, end); };
+    const int h = furthest(end > 0 ? end : 0, 1, m, target, off_at);
+    const int l = furthest(end < 0 ? end : 0, -1, -n, target, off_at);
     const int bin = edit_bin_for(h - l + 1, 0);
     const int low = edit_place(l, h, edit_width(bin), n, m);
     s.walk_low[slot] = low;
