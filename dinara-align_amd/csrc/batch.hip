@@ -220,11 +220,7 @@ struct dinara_batch {
     ~dinara_batch() {
         for (DeviceBuffer *buffer : arenas) delete buffer;
         if (edit_graph) (void)hipGraphExecDestroy(edit_graph);
-        if (pinned_counts) (void)hipHostFree(pinned_counts);
     }
-    // Alignments launched one by one: the queue counts a run reads back while its last walk runs (pinned, made at
-    // the first such run).
-    int32_t *pinned_counts = nullptr;
     // the last run's results, by slot
     std::vector<int32_t> cost_h, status_h, cigar_length_h;
     std::vector<int64_t> cigar_offset_h;
@@ -240,7 +236,8 @@ struct dinara_batch {
     bool use_graph = true;                // replay the run's launches as one captured hipGraph
     bool persistent = true;               // pair groups refill from their queue; else one pair a group
     bool keep_first = false;              // alignments: every sweep keeps its decisions (one pass when proven)
-    bool side_by_side_bins = true;        // the bins' first queues (and tracing sweeps) on streams of their own
+    bool side_by_side_bins = true;        // every one-word bin in one launch, the wider ones on streams of their own
+    bool one_stream = false;              // no side streams: the wider bins' launches follow on the main stream
     bool timed = true;                    // launches made one by one record an event pair each
     int grid_per_cu = 8;                  // persistent workgroups a compute unit
     int start_bin[EDIT_LENGTH_CLASSES] = {};  // the least first bin, by the pair's longer side
@@ -791,9 +788,7 @@ int long_walks(const dinara_batch *b) {
 
 // The walk of every slot ready for it: the long slots on `aside` and the others on `stream` at once (forked and joined
 // by marks `mark` and `mark` + 1; `mark` + 2 marks both ended; one after the other when `aside` is `stream`), then
-// the CIGAR text on `stream`. `aside` is the
-// narrowest bin's stream, which no retry uses (retries go to wider bins): a stream of its own would be one more than
-// the hardware queues bench.py asks for, and a stream sharing a queue runs after the other's work.
+// the CIGAR text on `stream`.
 void walk_slots(dinara_batch *b, const EditArgs &a, hipStream_t stream, hipStream_t aside, int mark, bool early) {
     DeviceContext *ctx = b->ctx;
     const int slots = (int)b->slot_pair.size(), longs = long_walks(b);
@@ -839,154 +834,133 @@ size_t arena_bytes(const dinara_batch *b) {
 }
 
 // Timing events of a run launched kernel by kernel: a pair for each bin's first sweep, retry sweep and tracing
-// sweep, and for the walk.
-constexpr int EV_FIRST = 0, EV_RETRY = 2 * EDIT_BINS, EV_TRACE = 4 * EDIT_BINS, EV_WALK = 6 * EDIT_BINS,
-              EV_LATER = 6 * EDIT_BINS + 2;
-// Marks (untimed events) of the early walk's fork and join; the bins side by side use marks 0 .. 4 * EDIT_BINS + 2.
-constexpr int EARLY_WALK = 5 * EDIT_BINS;
-// Marks of the walks' forks and joins (the long slots' launch beside the others'): the early walk's three, the last
-// walk's three; then the queue counts' read-back.
-constexpr int WALK_MARKS = 5 * EDIT_BINS + 2;
-constexpr int COUNTS_MARK = WALK_MARKS + 6;
+// sweep (the bins that share a launch share bin 0's pair), and for the walk.
+constexpr int EV_FIRST = 0, EV_RETRY = 2 * EDIT_BINS, EV_TRACE = 4 * EDIT_BINS, EV_WALK = 6 * EDIT_BINS;
+// Marks (untimed events) that order the streams: a pass's fork and its wide bins' ends (each pass WIDE_BINS + 1), the
+// fork and join of what runs beside the retries, and the walks' (the early walk's three, the last walk's three).
+constexpr int WIDE_BINS = EDIT_BINS - EDIT_NARROW;
+constexpr int FIRST_MARKS = 0, RETRY_MARKS = FIRST_MARKS + WIDE_BINS + 1, TRACE_MARKS = RETRY_MARKS + WIDE_BINS + 1,
+              BESIDE_MARKS = TRACE_MARKS + WIDE_BINS + 1, WALK_MARKS = BESIDE_MARKS + 2;
+// The side streams: one a wide bin (the first walks the long pairs once the sweeps are done), one for what runs beside
+// the retries. With the main stream they are four, as many as HIP's hardware queues by default: streams sharing a queue
+// run one after the other.
+constexpr int SIDE_WIDE = 0, SIDE_BESIDE = WIDE_BINS;
 
-// Runs `launch(bin, stream)` for each bin `use(bin)` picks, every one on a stream of its own forked from the main
-// stream and joined back to it (`mark_base` picks the ordering events), each between timing events EV + 2 bin and
-// EV + 2 bin + 1 when `timed`. Side by side, the widest bin is launched first: its long pairs are the run's
-// longest chains, and the hardware queues take the streams in order.
-template <typename Use, typename Launch>
-void side_by_side(DeviceContext *ctx, int mark_base, bool timed, int ev, bool apart, Use use, Launch launch) {
-    if (apart) (void)hipEventRecord(ctx->mark(mark_base), ctx->stream);
-    for (int k = 0; k < EDIT_BINS; ++k) {
-        const int bin = apart ? EDIT_BINS - 1 - k : k;
-        if (!use(bin)) continue;
-        if (!apart) {  // one after another on the main stream
-            if (timed) (void)hipEventRecord(ctx->event(ev + 2 * bin), ctx->stream);
-            launch(bin, ctx->stream);
-            if (timed) (void)hipEventRecord(ctx->event(ev + 2 * bin + 1), ctx->stream);
-            continue;
-        }
-        hipStream_t side = ctx->side(bin);
-        (void)hipStreamWaitEvent(side, ctx->mark(mark_base), 0);
-        if (timed) (void)hipEventRecord(ctx->event(ev + 2 * bin), side);
-        launch(bin, side);
-        if (timed) (void)hipEventRecord(ctx->event(ev + 2 * bin + 1), side);
-        (void)hipEventRecord(ctx->mark(mark_base + 1 + bin), side);
-        (void)hipStreamWaitEvent(ctx->stream, ctx->mark(mark_base + 1 + bin), 0);
+int timing_pair(const dinara_batch *b, int bin) { return b->side_by_side_bins && bin < EDIT_NARROW ? 0 : 2 * bin; }
+
+// One sweep of every bin's queue (`reach`: the pairs each may hold) on `stream`: the one-word bins in one launch, the
+// wider ones beside it, widest first (their pairs are the longest chains); or, not side by side, the bins one after
+// another. `mark` is the first of the pass's marks; `timed` records the pairs of events from `ev`.
+void sweep_bins(dinara_batch *b, const EditArgs &a, bool trace, const int64_t (&reach)[EDIT_BINS], hipStream_t stream,
+                int mark, bool timed, int ev) {
+    DeviceContext *ctx = b->ctx;
+    const auto around = [&](int pair, hipStream_t on, auto launch) {
+        if (timed) (void)hipEventRecord(ctx->event(ev + pair), on);
+        launch();
+        if (timed) (void)hipEventRecord(ctx->event(ev + pair + 1), on);
+        b->launches += 1;
+    };
+    int grid[EDIT_BINS], narrow = 0;
+    for (int bin = 0; bin < EDIT_BINS; ++bin) {
+        grid[bin] = edit_grid(b, bin, reach[bin]);
+        if (bin < EDIT_NARROW) narrow += grid[bin];
     }
+    if (!b->side_by_side_bins) {
+        for (int bin = 0; bin < EDIT_BINS; ++bin) {
+            if (!grid[bin]) continue;
+            int only[EDIT_BINS] = {};
+            only[bin] = grid[bin];
+            around(2 * bin, stream, [&] {
+                if (bin < EDIT_NARROW) launch_edit_sweep(a, trace, only, stream);
+                else launch_edit_sweep_wide(a, bin, trace, grid[bin], stream);
+            });
+        }
+        return;
+    }
+    bool forked = false;
+    for (int bin = EDIT_BINS - 1; bin >= EDIT_NARROW; --bin) {
+        if (!grid[bin]) continue;
+        hipStream_t side = stream;
+        if (!b->one_stream) {
+            if (!forked) (void)hipEventRecord(ctx->mark(mark), stream);
+            forked = true;
+            side = ctx->side(SIDE_WIDE + bin - EDIT_NARROW);
+            (void)hipStreamWaitEvent(side, ctx->mark(mark), 0);
+        }
+        around(2 * bin, side, [&] { launch_edit_sweep_wide(a, bin, trace, grid[bin], side); });
+        if (!b->one_stream) (void)hipEventRecord(ctx->mark(mark + 1 + bin - EDIT_NARROW), side);
+    }
+    if (narrow) around(0, stream, [&] { launch_edit_sweep(a, trace, grid, stream); });
+    for (int bin = EDIT_NARROW; bin < EDIT_BINS; ++bin)
+        if (grid[bin] && !b->one_stream) (void)hipStreamWaitEvent(stream, ctx->mark(mark + 1 + bin - EDIT_NARROW), 0);
 }
 
-// The run's launches: reset; every bin's first queue, the bins side by side; the retry queues, narrowest bin
-// first; then (alignments) every bin's tracing sweep side by side, and the walk. `timed` records an event pair
-// around each launch (not under capture); `may_wait` lets the host read queue counts back between launches.
-int64_t enqueue_unit(dinara_batch *b, const EditArgs &a, bool timed, bool trace, bool may_wait) {
+// The run's launches: reset; every bin's first queue; the retry queues; then (alignments) the tracing sweep, and the
+// walk. `timed` records an event pair around each launch (not under capture).
+//
+// Under the certified policy a retry always proves its pair: its band holds every diagonal a path cheaper than the
+// first band's cost could visit, its own cost is no higher, so no path outside it is cheaper (certify). So there are no
+// later retries, and an alignment's retries keep their decisions (a band traced again would cost a long pair's chain
+// twice), while the pairs the first pass proved are traced beside them. 4,000 uneven pairs, one call, the tracing pass
+// after the retries: 42.3 ms; beside them and every bin in one launch: 17.1 ms. Plain band doubling files again and
+// again: its later retries go one bin after another, and its tracing sweep follows them.
+//
+// With kept first bands the tracing queues stay empty: a pair whose decisions found no room is deferred (the arena's
+// used count has then passed its capacity for the whole run), not queued.
+int64_t enqueue_unit(dinara_batch *b, const EditArgs &a, bool timed, bool trace) {
     DeviceContext *ctx = b->ctx;
     const int slots = (int)b->slot_pair.size();
     launch_edit_reset(a, slots, ctx->stream);
-    side_by_side(ctx, 0, timed, EV_FIRST, b->side_by_side_bins, [&](int bin) { return b->first_count[bin] > 0; },
-                 [&](int bin, hipStream_t st) {
-                     launch_edit_sweep(a, bin, false, edit_grid(b, bin, b->first_count[bin]), st);
-                 });
+    sweep_bins(b, a, false, b->first_count, ctx->stream, FIRST_MARKS, timed, EV_FIRST);
     // Kept decisions: the pairs the first pass proved are walked on a stream of their own while the retries sweep.
     const bool early = trace && b->keep_first;
+    const bool beside = trace && !b->keep_first && !b->doubling;
     if (early) {
         launch_edit_snapshot(a, slots, ctx->stream);
-        (void)hipEventRecord(ctx->mark(EARLY_WALK), ctx->stream);
-        hipStream_t walker = ctx->side(EDIT_BINS);
-        (void)hipStreamWaitEvent(walker, ctx->mark(EARLY_WALK), 0);
+        (void)hipEventRecord(ctx->mark(BESIDE_MARKS), ctx->stream);
+        hipStream_t walker = ctx->side(SIDE_BESIDE);
+        (void)hipStreamWaitEvent(walker, ctx->mark(BESIDE_MARKS), 0);
         // The early walk's two launches one after the other: side by side they slow the retries beside them,
         // whose long pairs are the run's tail.
         walk_slots(b, a, walker, walker, WALK_MARKS, true);
-        (void)hipEventRecord(ctx->mark(EARLY_WALK + 1), walker);
+        (void)hipEventRecord(ctx->mark(BESIDE_MARKS + 1), walker);
     }
-    // The first retries side by side, filing into the later set; the later retries one bin after another.
     EditArgs retry = a;
     retry.lists = a.file_lists;
     retry.counts = a.file_counts;
     retry.file_lists = static_cast<int32_t *>(b->edit_later_lists.ptr);
     retry.file_counts = static_cast<int32_t *>(b->edit_later_counts.ptr);
-    side_by_side(ctx, 3 * EDIT_BINS + 2, timed, EV_RETRY, b->side_by_side_bins,
-                 [&](int bin) { return b->retry_reach[bin] > 0; },
-                 [&](int bin, hipStream_t st) {
-                     launch_edit_sweep(retry, bin, false, edit_grid(b, bin, b->retry_reach[bin]), st);
-                 });
-    EditArgs later = retry;
-    later.lists = retry.file_lists;
-    later.counts = retry.file_counts;
-    // Launched one by one (`may_wait`, not captured): the later retries begin at the narrowest bin whose queue holds
-    // a pair once the retries have ended (a later retry files only into wider bins), and a tracing sweep is made only
-    // for a queue that holds a pair; the counts are read back, the main stream waiting (the early walk goes on). An
-    // empty launch costs about 0.08 ms of the main stream. A launch not made has its timing events back to back.
-    // Launched one by one (`may_wait`, not captured), the later retries begin at the narrowest bin whose queue holds
-    // a pair once the retries have ended (a later retry files only into wider bins), and a tracing sweep is made only
-    // for a queue that holds a pair: one read brings both sets of counts, the tracing queues' copied beside the
-    // later retries' first (the later-retry counts' buffer has room past its lengths and heads). An empty launch
-    // costs about 0.08 ms of the main stream. A launch not made has its timing events back to back.
-    //
-    // Alignments launched one by one walk the pairs ready once the retries end at once, while the counts come back
-    // (pinned, waited for on an event): the host's round trip, about 0.6 ms, is then hidden under that walk. Only
-    // when a later retry or a tracing sweep runs does a second walk follow them.
-    int32_t pending[3 * EDIT_BINS] = {};
-    int32_t *const trace_pending = pending + 2 * EDIT_BINS;
-    int from = 0;
-    bool walked = false;
-    if (may_wait) {
-        int32_t *later_counts = static_cast<int32_t *>(b->edit_later_counts.ptr);
-        if (trace && hipMemcpyAsync(later_counts + 2 * EDIT_BINS, b->trace_counts.ptr, EDIT_BINS * 4,
-                                    hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
-            return DINARA_OUT_OF_MEMORY;
-        if (trace && !b->pinned_counts &&
-            hipHostMalloc(reinterpret_cast<void **>(&b->pinned_counts), sizeof(pending)) != hipSuccess)
-            b->pinned_counts = nullptr;
-        if (trace && b->pinned_counts) {
-            if (hipMemcpyAsync(b->pinned_counts, later_counts, sizeof(pending), hipMemcpyDeviceToHost, ctx->stream) !=
-                    hipSuccess ||
-                hipEventRecord(ctx->mark(COUNTS_MARK), ctx->stream) != hipSuccess)
-                return DINARA_OUT_OF_MEMORY;
-            if (early) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(WALK_MARKS + 2), 0);
-            if (timed) (void)hipEventRecord(ctx->event(EV_WALK), ctx->stream);
-            walk_slots(b, a, ctx->stream, ctx->side(0), WALK_MARKS + 3, false);
-            walked = true;
-            if (hipEventSynchronize(ctx->mark(COUNTS_MARK)) != hipSuccess) return DINARA_OUT_OF_MEMORY;
-            std::memcpy(pending, b->pinned_counts, sizeof(pending));
-        } else if (!b->edit_later_counts.read(ctx, pending, sizeof(pending))) {
-            return DINARA_OUT_OF_MEMORY;
-        }
-        while (from < EDIT_BINS && pending[from] == 0) ++from;
+    if (beside) {
+        retry.keep_first = 1;
+        (void)hipEventRecord(ctx->mark(BESIDE_MARKS), ctx->stream);
+        hipStream_t tracer = ctx->side(SIDE_BESIDE);
+        (void)hipStreamWaitEvent(tracer, ctx->mark(BESIDE_MARKS), 0);
+        sweep_bins(b, a, true, b->trace_reach, tracer, TRACE_MARKS, timed, EV_TRACE);
+        (void)hipEventRecord(ctx->mark(BESIDE_MARKS + 1), tracer);
     }
-    for (int bin = 0; bin < EDIT_BINS; ++bin) {
-        const int grid = edit_grid(b, bin, b->retry_reach[bin]);
-        if (!grid) continue;
-        if (timed) (void)hipEventRecord(ctx->event(EV_LATER + 2 * bin), ctx->stream);
-        if (bin >= from) launch_edit_sweep(later, bin, false, grid, ctx->stream);
-        if (timed) (void)hipEventRecord(ctx->event(EV_LATER + 2 * bin + 1), ctx->stream);
+    sweep_bins(b, retry, false, b->retry_reach, ctx->stream, RETRY_MARKS, timed, EV_RETRY);
+    if (b->doubling) {
+        EditArgs later = retry;
+        later.lists = retry.file_lists;
+        later.counts = retry.file_counts;
+        for (int bin = 0; bin < EDIT_BINS; ++bin) {
+            if (!edit_power_bin(bin)) continue;
+            int64_t only[EDIT_BINS] = {};
+            only[bin] = b->retry_reach[bin];
+            sweep_bins(b, later, false, only, ctx->stream, RETRY_MARKS, false, 0);
+        }
     }
     if (trace) {
-        if (may_wait && from < EDIT_BINS && !b->trace_counts.read(ctx, trace_pending, EDIT_BINS * 4))
-            return DINARA_OUT_OF_MEMORY;
-        const auto traced = [&](int bin) { return b->trace_reach[bin] > 0 && (!may_wait || trace_pending[bin] > 0); };
-        bool any_traced = false;
-        for (int bin = 0; bin < EDIT_BINS; ++bin) any_traced = any_traced || traced(bin);
-        if (timed)
-            for (int bin = 0; bin < EDIT_BINS; ++bin)
-                if (b->trace_reach[bin] > 0 && !traced(bin)) {
-                    (void)hipEventRecord(ctx->event(EV_TRACE + 2 * bin), ctx->stream);
-                    (void)hipEventRecord(ctx->event(EV_TRACE + 2 * bin + 1), ctx->stream);
-                }
-        side_by_side(ctx, EDIT_BINS + 1, timed, EV_TRACE, b->side_by_side_bins, traced,
-                     [&](int bin, hipStream_t st) {
-                         launch_edit_sweep(a, bin, true, edit_grid(b, bin, b->trace_reach[bin]), st);
-                     });
+        if (!b->keep_first && b->doubling)
+            sweep_bins(b, a, true, b->trace_reach, ctx->stream, TRACE_MARKS, timed, EV_TRACE);
+        if (beside) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(BESIDE_MARKS + 1), 0);
         // The last walk follows the early walk's kernels (it writes moves of slots the early walk marked unwalked)
-        // and runs while the early walk's text is made; the run ends when both texts are made. After a walk already
-        // made, a second one only for what later retries and tracing sweeps proved (it marks the first's slots
-        // unwalked, whose text the first made before it on this stream).
-        if (!walked || from < EDIT_BINS || any_traced) {
-            if (early && !walked) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(WALK_MARKS + 2), 0);
-            if (timed && !walked) (void)hipEventRecord(ctx->event(EV_WALK), ctx->stream);
-            walk_slots(b, a, ctx->stream, ctx->side(0), WALK_MARKS + 3, false);
-        }
+        // and runs while the early walk's text is made; the run ends when both texts are made.
+        if (early) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(WALK_MARKS + 2), 0);
+        if (timed) (void)hipEventRecord(ctx->event(EV_WALK), ctx->stream);
+        walk_slots(b, a, ctx->stream, ctx->side(SIDE_WIDE), WALK_MARKS + 3, false);
         if (timed) (void)hipEventRecord(ctx->event(EV_WALK + 1), ctx->stream);
-        if (early) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(EARLY_WALK + 1), 0);
+        if (early) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(BESIDE_MARKS + 1), 0);
     }
     return hipPeekAtLastError() == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
 }
@@ -1030,7 +1004,7 @@ int64_t run_unit(dinara_batch *b, bool trace) {
             hipGraph_t captured = nullptr;
             if (hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
                 return DINARA_OUT_OF_MEMORY;
-            const int64_t code = enqueue_unit(b, a, false, trace, false);
+            const int64_t code = enqueue_unit(b, a, false, trace);
             const hipError_t ended = hipStreamEndCapture(ctx->stream, &captured);
             if (code || ended != hipSuccess) return DINARA_OUT_OF_MEMORY;
             const hipError_t made = hipGraphInstantiate(&b->edit_graph, captured, nullptr, nullptr, 0);
@@ -1046,7 +1020,7 @@ int64_t run_unit(dinara_batch *b, bool trace) {
         b->graph_used = 1;
     } else {
         if (hipEventRecord(ctx->start, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
-        if (const int64_t code = enqueue_unit(b, a, b->timed, trace, true)) return code;
+        if (const int64_t code = enqueue_unit(b, a, b->timed, trace)) return code;
     }
     if (hipEventRecord(ctx->sweep_stop, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
     // Pairs whose decisions found no room: trace them in further passes, the arena emptied each time.
@@ -1059,10 +1033,8 @@ int64_t run_unit(dinara_batch *b, bool trace) {
                                ctx->stream) != hipSuccess)
                 return DINARA_OUT_OF_MEMORY;
             launch_edit_requeue(a, static_cast<const int32_t *>(b->deferred_held.ptr), deferred, ctx->stream);
-            for (int bin = 0; bin < EDIT_BINS; ++bin)
-                if (const int grid = edit_grid(b, bin, b->trace_reach[bin]))
-                    launch_edit_sweep(a, bin, true, grid, ctx->stream);
-            walk_slots(b, a, ctx->stream, ctx->side(0), WALK_MARKS + 3, false);
+            sweep_bins(b, a, true, b->trace_reach, ctx->stream, TRACE_MARKS, false, 0);
+            walk_slots(b, a, ctx->stream, ctx->side(SIDE_WIDE), WALK_MARKS + 3, false);
             int32_t left = 0;
             if (hipPeekAtLastError() != hipSuccess || !b->deferred_count.read(ctx, &left, 4)) return DINARA_OUT_OF_MEMORY;
             if (left >= deferred) return DINARA_OUT_OF_MEMORY;  // a pair larger than the whole arena
@@ -1080,21 +1052,17 @@ int64_t run_unit(dinara_batch *b, bool trace) {
     // short batch's run is then one graph launch and one wait.
     b->stats_pending = true;
     b->stats_slots = slots;
-    for (int bin = 0; bin < EDIT_BINS; ++bin) {
-        if (!graph && b->timed) {
+    if (!graph && b->timed) {
+        const auto spent = [&](int ev, int bin) {
             float ms = 0;
-            if (b->first_count[bin] > 0 &&
-                hipEventElapsedTime(&ms, ctx->event(EV_FIRST + 2 * bin), ctx->event(EV_FIRST + 2 * bin + 1)) == hipSuccess)
-                b->edit_ms[bin] += ms;
-            if (b->retry_reach[bin] > 0 &&
-                hipEventElapsedTime(&ms, ctx->event(EV_RETRY + 2 * bin), ctx->event(EV_RETRY + 2 * bin + 1)) == hipSuccess)
-                b->edit_ms[bin] += ms;
-            if (b->retry_reach[bin] > 0 &&
-                hipEventElapsedTime(&ms, ctx->event(EV_LATER + 2 * bin), ctx->event(EV_LATER + 2 * bin + 1)) == hipSuccess)
-                b->edit_ms[bin] += ms;
-            if (trace && b->trace_reach[bin] > 0 &&
-                hipEventElapsedTime(&ms, ctx->event(EV_TRACE + 2 * bin), ctx->event(EV_TRACE + 2 * bin + 1)) == hipSuccess)
-                b->trace_ms[bin] = ms;
+            const int pair = ev + timing_pair(b, bin);
+            return hipEventElapsedTime(&ms, ctx->event(pair), ctx->event(pair + 1)) == hipSuccess ? (double)ms : 0.0;
+        };
+        const bool traced = trace && !b->keep_first;
+        for (int bin = 0; bin < EDIT_BINS; ++bin) {
+            if (b->first_count[bin] > 0) b->edit_ms[bin] += spent(EV_FIRST, bin);
+            if (b->retry_reach[bin] > 0) b->edit_ms[bin] += spent(EV_RETRY, bin);
+            if (traced && b->trace_reach[bin] > 0) b->trace_ms[bin] = spent(EV_TRACE, bin);
         }
     }
     if (!graph && trace && b->timed) {
@@ -1102,7 +1070,7 @@ int64_t run_unit(dinara_batch *b, bool trace) {
         (void)hipEventElapsedTime(&ms, ctx->event(EV_WALK), ctx->event(EV_WALK + 1));
         b->walk_ms = ms;
     }
-    b->launches = graph ? 1 : 1 + EDIT_BINS * (trace ? 2 : 1) + (trace ? 1 : 0);
+    if (graph) b->launches = 1;
     b->ran = true;
     return 0;
 }
@@ -2204,7 +2172,7 @@ int64_t carved_unit_distances(Carve *carve, int64_t gpu, int64_t pairs, const ch
     } else {
         // One stream, launches one by one: no graph to instantiate, no side streams or timing events to make.
         b->use_graph = false;
-        b->side_by_side_bins = false;
+        b->one_stream = true;
         b->timed = false;
         code = run(b);
         if (code == 0) code = dinara_batch_distances(b, results);

@@ -154,9 +154,20 @@ struct EditStart {
     uint32_t bins;
 };
 
-// Host-side entry points of edit.hip. `grid` is the workgroups of each persistent launch (256 threads each).
+// The workgroups of a sweep over every one-word bin, where each bin's end: bin EDIT_NARROW - 1 - k's first EDIT_LEAD at
+// end[k], its others at end[EDIT_NARROW + k]. The lead comes first of every bin, so that each bin's longest pairs (its
+// queue's first) start at once; eleven bins' leads fit the compute units together.
+constexpr int EDIT_NARROW = 11;
+constexpr int EDIT_LEAD = 64;
+struct EditGrid {
+    int end[2 * EDIT_NARROW];
+};
+
+// Host-side entry points of edit.hip. `grid` is each bin's persistent workgroups (256 threads each): launch_edit_sweep
+// sweeps the queues of every one-word bin in one launch, launch_edit_sweep_wide those of a bin of more words a lane.
 void launch_edit_reset(const EditArgs &a, int slots, hipStream_t stream);
-void launch_edit_sweep(const EditArgs &a, int bin, bool trace, int grid, hipStream_t stream);
+void launch_edit_sweep(const EditArgs &a, bool trace, const int (&grid)[EDIT_BINS], hipStream_t stream);
+void launch_edit_sweep_wide(const EditArgs &a, int bin, bool trace, int grid, hipStream_t stream);
 // The walk, in two launches that may run at once: the first `long_slots` slots (those whose longer side is at least
 // EDIT_WALK_LONG letters: slots are longest first) a wave a pair, and slots `first` .. `slots` - 1 a lane a pair.
 // `early`: walk the slots ready at the first pass's end (copied by launch_edit_snapshot), while the retries sweep on

@@ -7,6 +7,7 @@
 // letter alone, else a query letter alone, and two equal letters only when no edit is; Ties.LEFT walks both
 // sequences reversed (edit_distance.mojo:295-297). At unit costs that rule and the reference's DP-flag rule
 // (lanes.mojo:905-923) give the same CIGAR.
+#include <algorithm>
 #include <type_traits>
 
 #include "bands.h"
@@ -251,8 +252,9 @@ typedef u64x2 __attribute__((address_space(1))) global_decisions;
 
 __device__ __forceinline__ u64x2 planes_of(ulonglong2 v) { return u64x2{v.x, v.y}; }
 
+// `places`: the wave's staging rows (one-word lanes keeping decisions).
 template <int L, int K, int BITS, int MODE>
-__global__ __launch_bounds__(256) void edit_sweep(EditArgs a, int bin) {
+__device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglong2 (*places)[64]) {
     constexpr bool TRACE = MODE == 1;          // sweeps settled pairs' traced bands again
     constexpr bool RECORD = MODE != 0;         // keeps decisions
     constexpr int W = 64 * L * K;
@@ -293,8 +295,6 @@ __global__ __launch_bounds__(256) void edit_sweep(EditArgs a, int bin) {
     // the wave's line reads (eight lanes a line, one place each) fall in different banks with no padding: 32 KB a
     // workgroup, five to a compute unit.
     constexpr bool STAGED = RECORD && K == 1;
-    __shared__ ulonglong2 stage[STAGED ? 4 : 1][STAGED ? 8 : 1][STAGED ? 64 : 1];
-    ulonglong2 (*const places)[STAGED ? 64 : 1] = stage[STAGED ? threadIdx.x >> 6 : 0];
     int t = 0;       // the wave's column steps so far (the same in every lane)
     int t0 = 0;      // the step count when the lane's pair was claimed
     // More words a lane: the last HOLD columns' decision planes in registers, oldest first.
@@ -683,6 +683,44 @@ __global__ __launch_bounds__(256) void edit_sweep(EditArgs a, int bin) {
         top += (int)((uint32_t)pv[0] & 1u) + __builtin_amdgcn_sbfe((int)(uint32_t)mv[0], 0, 1);
         }
     }
+}
+
+// Every one-word bin in one launch: a workgroup finds its bin from its place in the grid (EditGrid: every bin's first
+// workgroups, widest bin first, then the rest of each) and sweeps that bin's queue. What bounds a batch of a few
+// thousand uneven pairs is its longest pairs' chains, column after column, one in each bin: launches of their own, a
+// bin a stream, ran four at a time on HIP's four hardware queues, each as long as its longest pair. 4,000 pairs
+// (1.5 kbp median, up to 20 kbp): the retries of ten bins took 14.0 ms so and their traces 19.2; the retries keeping
+// their decisions take 6.3 ms in one launch. 20,000 seeded pairs: 36.6 ms of sweeps and walks, 15.2 in one launch.
+template <int BITS, int MODE>
+__global__ __launch_bounds__(256) void edit_sweep(EditArgs a, EditGrid grid) {
+    constexpr bool STAGED = MODE != 0;
+    __shared__ ulonglong2 stage[STAGED ? 4 : 1][STAGED ? 8 : 1][64];
+    ulonglong2 (*const places)[64] = stage[STAGED ? threadIdx.x >> 6 : 0];
+    const int at = (int)blockIdx.x;
+    int bin = -1;
+#pragma unroll
+    for (int k = 2 * EDIT_NARROW - 1; k >= 0; --k)
+        if (at < grid.end[k]) bin = EDIT_NARROW - 1 - k % EDIT_NARROW;
+    switch (bin) {
+        case 0: sweep_queue<1, 1, BITS, MODE>(a, bin, places); break;
+        case 1: sweep_queue<2, 1, BITS, MODE>(a, bin, places); break;
+        case 2: sweep_queue<3, 1, BITS, MODE>(a, bin, places); break;
+        case 3: sweep_queue<4, 1, BITS, MODE>(a, bin, places); break;
+        case 4: sweep_queue<6, 1, BITS, MODE>(a, bin, places); break;
+        case 5: sweep_queue<8, 1, BITS, MODE>(a, bin, places); break;
+        case 6: sweep_queue<12, 1, BITS, MODE>(a, bin, places); break;
+        case 7: sweep_queue<16, 1, BITS, MODE>(a, bin, places); break;
+        case 8: sweep_queue<21, 1, BITS, MODE>(a, bin, places); break;
+        case 9: sweep_queue<32, 1, BITS, MODE>(a, bin, places); break;
+        case 10: sweep_queue<64, 1, BITS, MODE>(a, bin, places); break;
+        default: break;
+    }
+}
+
+// The bins of 64 lanes of two and four words, a launch each: their registers (and few pairs) stay out of the others'.
+template <int K, int BITS, int MODE>
+__global__ __launch_bounds__(256) void edit_sweep_wide(EditArgs a, int bin) {
+    sweep_queue<64, K, BITS, MODE>(a, bin, nullptr);
 }
 
 // ------------------------------------------------------------------ the walk
@@ -1191,31 +1229,29 @@ __global__ void edit_seed_clear(int32_t *counts) {
     if (threadIdx.x < EDIT_BINS) counts[threadIdx.x] = 0;
 }
 
-template <int L, int K, int MODE>
-void sweep_bits(const EditArgs &a, int bin, int grid, hipStream_t stream) {
-    if (a.s.tape.bits == 2)
-        hipLaunchKernelGGL((edit_sweep<L, K, 2, MODE>), dim3(grid), dim3(256), 0, stream, a, bin);
-    else
-        hipLaunchKernelGGL((edit_sweep<L, K, 8, MODE>), dim3(grid), dim3(256), 0, stream, a, bin);
+template <int BITS, int MODE>
+void sweep_narrow(const EditArgs &a, const EditGrid &grid, hipStream_t stream) {
+    hipLaunchKernelGGL((edit_sweep<BITS, MODE>), dim3(grid.end[2 * EDIT_NARROW - 1]), dim3(256), 0, stream, a, grid);
 }
 
-template <int MODE>
-void sweep_bin(const EditArgs &a, int bin, int grid, hipStream_t stream) {
-    switch (bin) {
-        case 0: sweep_bits<1, 1, MODE>(a, bin, grid, stream); break;
-        case 1: sweep_bits<2, 1, MODE>(a, bin, grid, stream); break;
-        case 2: sweep_bits<3, 1, MODE>(a, bin, grid, stream); break;
-        case 3: sweep_bits<4, 1, MODE>(a, bin, grid, stream); break;
-        case 4: sweep_bits<6, 1, MODE>(a, bin, grid, stream); break;
-        case 5: sweep_bits<8, 1, MODE>(a, bin, grid, stream); break;
-        case 6: sweep_bits<12, 1, MODE>(a, bin, grid, stream); break;
-        case 7: sweep_bits<16, 1, MODE>(a, bin, grid, stream); break;
-        case 8: sweep_bits<21, 1, MODE>(a, bin, grid, stream); break;
-        case 9: sweep_bits<32, 1, MODE>(a, bin, grid, stream); break;
-        case 10: sweep_bits<64, 1, MODE>(a, bin, grid, stream); break;
-        case 11: sweep_bits<64, 2, MODE>(a, bin, grid, stream); break;
-        default: sweep_bits<64, 4, MODE>(a, bin, grid, stream); break;
-    }
+template <int BITS, int MODE>
+void sweep_wide(const EditArgs &a, int bin, int grid, hipStream_t stream) {
+    if (edit_words(bin) == 2)
+        hipLaunchKernelGGL((edit_sweep_wide<2, BITS, MODE>), dim3(grid), dim3(256), 0, stream, a, bin);
+    else
+        hipLaunchKernelGGL((edit_sweep_wide<4, BITS, MODE>), dim3(grid), dim3(256), 0, stream, a, bin);
+}
+
+// Calls `launch(bits, mode)` with the batch's letters and the sweep's use as compile-time constants.
+template <typename Launch>
+void for_sweep(const EditArgs &a, bool trace, Launch launch) {
+    const auto as = [&](auto bits) {
+        if (trace) launch(bits, std::integral_constant<int, TRACE>());
+        else if (a.keep_first) launch(bits, std::integral_constant<int, SWEEP_TRACED>());
+        else launch(bits, std::integral_constant<int, SWEEP>());
+    };
+    if (a.s.tape.bits == 2) as(std::integral_constant<int, 2>());
+    else as(std::integral_constant<int, 8>());
 }
 
 }  // namespace
@@ -1229,13 +1265,19 @@ void launch_edit_reset(const EditArgs &a, int slots, hipStream_t stream) {
     hipLaunchKernelGGL(edit_reset, dim3((threads + 255) / 256), dim3(256), 0, stream, a, slots);
 }
 
-void launch_edit_sweep(const EditArgs &a, int bin, bool trace, int grid, hipStream_t stream) {
-    if (trace)
-        sweep_bin<TRACE>(a, bin, grid, stream);
-    else if (a.keep_first)
-        sweep_bin<SWEEP_TRACED>(a, bin, grid, stream);
-    else
-        sweep_bin<SWEEP>(a, bin, grid, stream);
+void launch_edit_sweep(const EditArgs &a, bool trace, const int (&grid)[EDIT_BINS], hipStream_t stream) {
+    EditGrid g{};
+    int end = 0;
+    for (int k = 0; k < EDIT_NARROW; ++k) g.end[k] = end += std::min(grid[EDIT_NARROW - 1 - k], EDIT_LEAD);
+    for (int k = 0; k < EDIT_NARROW; ++k)
+        g.end[EDIT_NARROW + k] = end += std::max(grid[EDIT_NARROW - 1 - k] - EDIT_LEAD, 0);
+    if (end == 0) return;
+    for_sweep(a, trace, [&](auto bits, auto mode) { sweep_narrow<bits.value, mode.value>(a, g, stream); });
+}
+
+void launch_edit_sweep_wide(const EditArgs &a, int bin, bool trace, int grid, hipStream_t stream) {
+    if (grid > 0)
+        for_sweep(a, trace, [&](auto bits, auto mode) { sweep_wide<bits.value, mode.value>(a, bin, grid, stream); });
 }
 
 void launch_edit_seed(const EditArgs &a, const float *prediction, double margin, double slope, const EditStart &start,

@@ -231,7 +231,7 @@ void dinara_batch_free(dinara_batch *batch);
  * bins, 13 the first pass's bin set (dinara_batch_set_bins); 14 above zero when the gap-cost group sweeps hold
  * packed 16-bit cells (shifted costs, mismatch at most two extensions, pairs short enough), 0 for 32-bit ones; for
  * bin b (widths 64, 128, 192, 256, 384, 512, 768, 1024, 1344, 2048, 4096, 8192, 16384 diagonals) 1200+b
- * its width, 600+b its sweep's time (ms, runs without the graph), 700+b the sweeps it began, 800+b its tracing
+ * its width, 600+b its sweep's time (ms, runs without the graph; bins swept by one launch share its time), 700+b the sweeps it began, 800+b its tracing
  * sweep's time, 900+b the traces it began, 1000+b and 1100+b the word-columns (a pair's columns times its band's
  * 64-bit words) its sweeps and traces covered. Every
  * batch: 10 the pairs no band settled that the whole-matrix path swept after the run, 11 that path's time (ms,
@@ -305,7 +305,7 @@ int64_t dinara_batch_set_tuning(dinara_batch *batch, int64_t grid_per_cu, const 
  * band doubling keeps to the powers of two. DINARA_INVALID_MODE for an empty set or bits past bin 12. Results do
  * not change, only the work. */
 int64_t dinara_batch_set_bins(dinara_batch *batch, int64_t bins);
-/* Each bin's first queue, and each bin's tracing sweep, on a stream of its own so the bins run side by side (1, the
+/* Every bin of one word a lane swept by one launch, the wider ones beside it on streams of their own (1, the
  * default), or the bins one after another (0). */
 int64_t dinara_batch_set_side_by_side(dinara_batch *batch, int64_t on);
 /* Chooses that shape by timing the batch's own first pass (workgroups a compute unit, side by side or not, then
