@@ -255,7 +255,7 @@ struct dinara_batch {
         arena_used, edit_stats, edit_work;
     size_t arena_capacity = 0;            // the bytes of the context's arena this batch's runs use
     const void *arena_ptr = nullptr;      // where that arena was when the captured graph was made
-    size_t arena_want = 0;                // the bytes it asks for (0: not worked out yet)
+    size_t arena_ask = 0, arena_bound = 0;  // the bytes it asks for and the most it may use (0: not worked out yet)
     hipGraphExec_t edit_graph = nullptr;
     double edit_ms[EDIT_BINS] = {}, trace_ms[EDIT_BINS] = {}, edit_sweeps[EDIT_BINS] = {},
            trace_sweeps[EDIT_BINS] = {}, graph_used = 0, trace_passes = 0, walked_first = 0;
@@ -815,22 +815,34 @@ int edit_grid(const dinara_batch *b, int bin, int64_t reach) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(every, (int64_t)b->ctx->compute_units * b->grid_per_cu));
 }
 
-// The arena the traced bands' decisions take: the batch's bound (no traced band is wider than its whole matrix),
-// at most 0.6 of the free memory, at least 1 MiB. DINARA_TRACE_ARENA sets it in bytes.
-size_t arena_bytes(const dinara_batch *b) {
-    if (const char *env = std::getenv("DINARA_TRACE_ARENA")) return std::max<size_t>(std::strtoull(env, nullptr, 10), 4096);
-    size_t bound = 0;
+// The arena the kept bands' decisions may take (`bound`: no band is wider than its whole matrix) and what the batch is
+// likely to need (`ask`: bands a quarter of the pairs' longer side). Mapping device memory takes about 30 ms a GB, and
+// 20,000 uneven pairs are bound by the 0.6 of the card's memory a run may take: a process's first run on such a batch
+// spent 5.1 s there, and so did every later batch whose bound came out a little larger. So the arena is made for what
+// is likely, kept, and doubled when a run has left pairs without room (they are traced in further passes). At most 0.6
+// of the free memory, at least 1 MiB; DINARA_TRACE_ARENA sets it in bytes.
+struct ArenaNeed {
+    size_t ask, bound;
+};
+ArenaNeed arena_need(const dinara_batch *b) {
+    if (const char *env = std::getenv("DINARA_TRACE_ARENA")) {
+        const size_t set = std::max<size_t>(std::strtoull(env, nullptr, 10), 4096);
+        return {set, set};
+    }
+    size_t bound = 0, likely = 0;
     for (size_t s = 0; s < b->slot_pair.size(); ++s) {
-        const int n = b->rows[s], m = b->cols[s];
-        const int bin = edit_widest(n + m);
-        bound += (size_t)edit_trace_bytes(m, bin);
+        const int n = b->rows[s], m = b->cols[s], widest = edit_widest(n + m);
+        const int usual = edit_bin_for(std::abs(m - n) + std::max(n, m) / 4 + 64, 0);
+        bound += (size_t)edit_trace_bytes(m, widest);
+        likely += (size_t)edit_trace_bytes(m, usual < 0 ? widest : std::min(usual, widest));
     }
     size_t free_bytes = 0, total = 0;
     (void)hipMemGetInfo(&free_bytes, &total);
     if (b->ctx->edit_arena) free_bytes += b->ctx->edit_arena->size;  // the arena itself is there to be used
-    const size_t most = free_bytes / 10 * 6;
+    const size_t most = std::max<size_t>(free_bytes / 10 * 6, size_t(1) << 20);
     if (b->keep_first) bound *= 3;  // every attempt keeps its decisions
-    return std::max<size_t>(std::min(bound, most), size_t(1) << 20);
+    bound = std::min(std::max<size_t>(bound, size_t(1) << 20), most);
+    return {std::min(bound, std::max<size_t>(likely, size_t(1) << 31)), bound};
 }
 
 // Timing events of a run launched kernel by kernel: a pair for each bin's first sweep, retry sweep and tracing
@@ -979,15 +991,23 @@ int64_t run_unit(dinara_batch *b, bool trace) {
         return 0;
     }
     if (b->kind == DINARA_BATCH_ALIGNMENTS) {
-        // The context's arena, grown when this batch wants more than it holds; the graph is made again when the
-        // arena it was captured with moved or this batch's share of it changed.
+        // The context's arena, grown when this batch is likely to need more than it holds (by half at least, so that
+        // a run of ever larger batches maps it a few times only) or the last run had too little; the graph is made
+        // again when the arena it was captured with moved or this batch's share of it changed.
         if (!ctx->edit_arena) ctx->edit_arena = new DeviceBuffer();
-        if (!b->arena_want) b->arena_want = arena_bytes(b);
-        const size_t bytes = b->arena_want;
-        if (ctx->edit_arena->size < bytes) {
-            ctx->edit_arena->release();
-            if (!ctx->edit_arena->reserve(bytes)) return DINARA_OUT_OF_MEMORY;
+        if (!b->arena_bound) {
+            const ArenaNeed need = arena_need(b);
+            b->arena_ask = need.ask;
+            b->arena_bound = need.bound;
         }
+        const size_t held = ctx->edit_arena->size, ask = std::min(std::max(b->arena_ask, ctx->arena_wanted), b->arena_bound);
+        if (held < ask) {
+            ctx->edit_arena->release();
+            if (!ctx->edit_arena->reserve(std::min(std::max(ask, held + held / 2), b->arena_bound)) &&
+                !ctx->edit_arena->reserve(ask))
+                return DINARA_OUT_OF_MEMORY;
+        }
+        const size_t bytes = std::min(ctx->edit_arena->size, b->arena_bound);
         if (b->arena_ptr != ctx->edit_arena->ptr || b->arena_capacity != bytes) {
             b->arena_ptr = ctx->edit_arena->ptr;
             b->arena_capacity = bytes;
@@ -1027,6 +1047,7 @@ int64_t run_unit(dinara_batch *b, bool trace) {
     int32_t deferred = 0;
     if (trace) {
         if (!b->deferred_count.read(ctx, &deferred, 4)) return DINARA_OUT_OF_MEMORY;
+        if (deferred > 0) ctx->arena_wanted = 2 * b->arena_capacity;
         while (deferred > 0) {
             b->trace_passes += 1;
             if (hipMemcpyAsync(b->deferred_held.ptr, b->deferred.ptr, (size_t)deferred * 4, hipMemcpyDeviceToDevice,
@@ -1954,7 +1975,7 @@ int64_t dinara_batch_set_keep_first(dinara_batch *b, int64_t on) {
     if (!b) return DINARA_INVALID_MODE;
     b->keep_first = on != 0;
     drop_graph(b);
-    b->arena_want = 0;  // the arena it asks for follows the setting: worked out again at the next run
+    b->arena_bound = 0;  // the arena it asks for follows the setting: worked out again at the next run
     return 0;
 }
 
