@@ -6,11 +6,15 @@
 // The network: 288 inputs (258 features and zero padding) -> 256 -> 256 -> 1, ReLU, bf16 weights and activations,
 // fp32 accumulation and fp32 master weights updated by Adam. It predicts log(1 + cost).
 //
-// GEMM: one wave a 32 x 32 tile of C, v_mfma_f32_32x32x8_bf16 over K in steps of 8. Operands as the instruction
-// reads them: lane l holds A[l % 32][4(l / 32) .. 4(l / 32) + 3] and B[4(l / 32) .. + 3][l % 32]; the 16 results
-// of lane l are C[8(r / 4) + 4(l / 32) + r % 4][l % 32], r = 0..15. Either operand may be read transposed, so the
-// backward products (X^T dZ, dZ W^T) use the same kernel. The products are small (256 wide); their tiles are read
-// straight from global memory, which the caches serve.
+// Products: v_mfma_f32_32x32x8_bf16 over K in steps of 8. Operands as the instruction reads them: lane l holds
+// A[l % 32][4(l / 32) .. 4(l / 32) + 3] and B[4(l / 32) .. + 3][l % 32]; the 16 results of lane l are C[8(r / 4) +
+// 4(l / 32) + r % 4][l % 32], r = 0..15. So an operand is kept as quads: four consecutive K of one row (or column) in
+// 8 bytes, the quads of one K side by side, and a lane reads its operand with one 8-byte load, 32 lanes 256 bytes in a
+// row; and a lane's results are quads of four consecutive rows, which is how the products over rows (the weights'
+// gradients) read them. A training step is two launches: one takes 32 rows a workgroup through both layers, the output
+// and back to the first layer's gradients (everything that stays within a row), the other makes every sum over rows and
+// updates the weights with it. Every sum is taken in one fixed order (products by K, the others row by row), so a
+// network's numbers do not depend on how the work is split.
 
 #include <stdint.h>
 
@@ -18,6 +22,7 @@
 #include <cmath>
 #include <cstring>
 #include <random>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/dinara.h"
@@ -130,184 +135,328 @@ __device__ inline float from_bf16(uint16_t h) { return __uint_as_float((uint32_t
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// C (M x N) = A (M x K) . B (K x N) + bias, in 32 x 32 tiles; A read as A[i][k] = a[i * lda + k] (or a[k * lda + i]
-// transposed), B as B[k][j] = b[k * ldb + j] (or b[j * ldb + k]). Writes the fp32 product to `c` when non-null and
-// its bf16 to `cb` when non-null: after ReLU when `relu`, zeroed where mask[i][j] <= 0 when `mask` is non-null.
-template <bool TA, bool TB>
-__global__ __launch_bounds__(64) void gemm_bf16(const uint16_t *a, int lda, const uint16_t *b, int ldb, int K,
-                                                const float *bias, int relu, const float *mask, int ldm, float *c,
-                                                int ldc, uint16_t *cb, int ldcb) {
-    const int lane = threadIdx.x;
-    const int i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
-    const int row = lane & 31, kq = (lane >> 5) * 4;
+constexpr int HIDDEN = 256;
+constexpr int IN_QUADS = FEATURE_STRIDE / 4, HIDDEN_QUADS = HIDDEN / 4;
+// The flat weights (as the C ABI gives them) and their bf16 copies: w1 and w2 as quads along their rows (the forward
+// products' K), w2 again as quads along its columns (the backward product's K), w3 as it is.
+constexpr int W1 = 0, B1 = W1 + FEATURE_STRIDE * HIDDEN, W2 = B1 + HIDDEN, B2 = W2 + HIDDEN * HIDDEN,
+              W3 = B2 + HIDDEN, B3 = W3 + HIDDEN, WEIGHTS = B3 + 1;
+constexpr int W1_QUADS = 0, W2_QUADS = W1_QUADS + FEATURE_STRIDE * HIDDEN, W2T_QUADS = W2_QUADS + HIDDEN * HIDDEN,
+              W3_COPY = W2T_QUADS + HIDDEN * HIDDEN, COPIES = W3_COPY + HIDDEN;
+
+// Where w[k][j] of a `HIDDEN`-column matrix is among its quads along k.
+__host__ __device__ constexpr int quad_place(int k, int j) { return ((k >> 2) * HIDDEN + j) * 4 + (k & 3); }
+
+// What a training step reads and leaves. `x` (rows x FEATURE_STRIDE fp32) and `targets` are read at `index` (null: in
+// order); the first `count` of the step's rows are real. For the sums over rows: x, both layers' activations and their
+// gradients as bf16 quads of four rows, and per row the output's gradient and squared error.
+struct StepArgs {
+    const float *x, *targets;
+    const int32_t *index;
+    int count, rows;
+    const float *weights;
+    const uint16_t *copies;
+    bf16x4 *x_quads, *a1_quads, *a2_quads, *dz1_quads, *dz2_quads;
+    float *dy, *sq, *y;
+};
+
+// Quads of a 32-row block in LDS, K quad q of row i at [q][i]: a row of 33, so that the lanes that write a column's
+// quads fall in different banks.
+constexpr int LDS_ROW = 33;
+
+// One wave's 32 x 32 tile of A (32 rows, quads in LDS) . B (columns `column`, quads of HIDDEN columns in global
+// memory), K = 8 STEPS: B's operands are loaded GROUP steps at once.
+template <int STEPS, int GROUP>
+__device__ __forceinline__ f32x16 block_product(const bf16x4 *a, const bf16x4 *b, int column, int lane) {
+    static_assert(STEPS % GROUP == 0, "whole groups");
+    const int half = lane >> 5, row = lane & 31;
     f32x16 acc = {};
-    for (int k0 = 0; k0 < K; k0 += 8) {
-        bf16x4 va, vb;
+    for (int s0 = 0; s0 < STEPS; s0 += GROUP) {
+        bf16x4 vb[GROUP];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k = k0 + kq + j;
-            va[j] = (short)(TA ? a[(size_t)k * lda + i0 + row] : a[(size_t)(i0 + row) * lda + k]);
-            vb[j] = (short)(TB ? b[(size_t)(j0 + row) * ldb + k] : b[(size_t)k * ldb + j0 + row]);
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va, vb, acc, 0, 0, 0);
-    }
-    const int j = j0 + row;
+        for (int u = 0; u < GROUP; ++u) vb[u] = b[(size_t)(2 * (s0 + u) + half) * HIDDEN + column];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int i = i0 + 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-        float v = acc[r] + (bias ? bias[j] : 0.0f);
-        if (c) c[(size_t)i * ldc + j] = v;
-        if (cb) {
-            if (relu) v = v > 0.0f ? v : 0.0f;
-            if (mask && mask[(size_t)i * ldm + j] <= 0.0f) v = 0.0f;
-            cb[(size_t)i * ldcb + j] = to_bf16(v);
-        }
+        for (int u = 0; u < GROUP; ++u)
+            acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a[(2 * (s0 + u) + half) * LDS_ROW + row], vb[u], acc, 0, 0, 0);
     }
+    return acc;
 }
 
-template <bool TA, bool TB>
-static void gemm(hipStream_t stream, const uint16_t *a, int lda, const uint16_t *b, int ldb, int M, int N, int K,
-                 const float *bias, int relu, const float *mask, int ldm, float *c, int ldc, uint16_t *cb,
-                 int ldcb) {
-    hipLaunchKernelGGL((gemm_bf16<TA, TB>), dim3(M / 32, N / 32), dim3(64), 0, stream, a, lda, b, ldb, K, bias,
-                       relu, mask, ldm, c, ldc, cb, ldcb);
+// A lane's value of row i, column j as an element of the next product's A quads.
+__device__ __forceinline__ void put_quad(bf16x4 *quads, int i, int j, uint16_t v) {
+    reinterpret_cast<uint16_t *>(quads)[((j >> 2) * LDS_ROW + i) * 4 + (j & 3)] = v;
 }
 
-// ------------------------------------------------------------------ prediction in one pass
-
-// (rows x cols) bf16 into (cols x rows).
-__global__ void transpose_bf16(const uint16_t *in, int rows, int cols, uint16_t *out) {
-    const int at = blockIdx.x * blockDim.x + threadIdx.x;
-    if (at >= rows * cols) return;
-    out[(size_t)(at % cols) * rows + at / cols] = in[at];
-}
-
-constexpr int PREDICT_HIDDEN = 256;
-
-// The network's prediction for 32 rows a wave, both hidden layers and the output in one pass: the fp32 features
-// are rounded to bf16 as they are read, each layer is 8 MFMA tiles of 32 x 32 (the weights read transposed, 4
-// bf16 a lane), and a layer's activations go through LDS to become the next product's left operand. The products
-// take their K steps in the order `gemm_bf16` takes them, so the prediction is the same as the layer-by-layer one.
-__global__ __launch_bounds__(64) void predict_rows(const float *features, int rows, const uint16_t *w1t,
-                                                   const float *b1, const uint16_t *w2t, const float *b2,
-                                                   const uint16_t *w3, const float *b3, float *y) {
-    __shared__ uint16_t act[32 * PREDICT_HIDDEN];
-    const int lane = threadIdx.x, row = lane & 31, kq = (lane >> 5) * 4;
-    const int i0 = blockIdx.x * 32;
-    f32x16 acc[8];
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) acc[nt] = f32x16{};
-    const bool real = i0 + row < rows;
-    const float *x = features + (size_t)(real ? i0 + row : 0) * FEATURE_STRIDE;
-    for (int k0 = 0; k0 < FEATURE_STRIDE; k0 += 8) {
-        const float4 f = real ? *reinterpret_cast<const float4 *>(x + k0 + kq) : make_float4(0.f, 0.f, 0.f, 0.f);
-        bf16x4 va;
-        va[0] = (short)to_bf16(f.x);
-        va[1] = (short)to_bf16(f.y);
-        va[2] = (short)to_bf16(f.z);
-        va[3] = (short)to_bf16(f.w);
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const bf16x4 vb = *reinterpret_cast<const bf16x4 *>(w1t + (size_t)(nt * 32 + row) * FEATURE_STRIDE + k0 + kq);
-            acc[nt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va, vb, acc[nt], 0, 0, 0);
+// 32 rows a workgroup, a wave a 32-column tile: the forward pass and the output, and (TRAIN) the loss's gradient back
+// to the first layer. Bounded by its chains (36 and 32 matrix steps of 64 cycles, the output's 256 additions a row):
+// 4,096 rows took 15 us a product and 150 for the output as kernels of their own, each activation out to memory and
+// back; here the activations pass through LDS, 25 us for all of it.
+template <bool TRAIN>
+__global__ __launch_bounds__(512) void network_rows(StepArgs a) {
+    __shared__ bf16x4 in_quads[IN_QUADS * LDS_ROW], act[HIDDEN_QUADS * LDS_ROW];
+    __shared__ float slope[32];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int i0 = blockIdx.x * 32, j = wave * 32 + (lane & 31), half = lane >> 5;
+    for (int at = t; at < 32 * IN_QUADS; at += 512) {
+        const int i = at / IN_QUADS, q = at % IN_QUADS, r = i0 + i;
+        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r < a.count)
+            f = *reinterpret_cast<const float4 *>(a.x + (size_t)(a.index ? a.index[r] : r) * FEATURE_STRIDE + 4 * q);
+        in_quads[q * LDS_ROW + i] =
+            bf16x4{(short)to_bf16(f.x), (short)to_bf16(f.y), (short)to_bf16(f.z), (short)to_bf16(f.w)};
+    }
+    __syncthreads();
+    if (TRAIN) {
+        const short *x = reinterpret_cast<const short *>(in_quads);
+        for (int at = t; at < 8 * FEATURE_STRIDE; at += 512) {
+            const int i = 4 * (at / FEATURE_STRIDE), k = at % FEATURE_STRIDE;
+            const short *from = x + ((k >> 2) * LDS_ROW + i) * 4 + (k & 3);
+            a.x_quads[(size_t)((i0 + i) >> 2) * FEATURE_STRIDE + k] = bf16x4{from[0], from[4], from[8], from[12]};
         }
     }
-    // Bias, ReLU and bf16 into LDS, row-major: MFMA result r of lane l is row 8(r/4) + 4(l/32) + r%4, column l%32.
-    auto keep = [&](const float *bias) {
+    const bf16x4 *const copies = reinterpret_cast<const bf16x4 *>(a.copies);
+    // A layer's bias and ReLU: bf16 activations into `to`, and (TRAIN) four rows at a time into `rows_to`.
+    const auto activate = [&](f32x16 &z, const float *bias, bf16x4 *to, bf16x4 *rows_to) __attribute__((always_inline)) {
+        const float b = bias[j];
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const int j = nt * 32 + row;
+        for (int q = 0; q < 4; ++q) {
+            bf16x4 four;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int i = 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
-                const float v = acc[nt][r] + bias[j];
-                act[i * PREDICT_HIDDEN + j] = to_bf16(v > 0.0f ? v : 0.0f);
+            for (int e = 0; e < 4; ++e) {
+                const float v = z[4 * q + e] + b;
+                z[4 * q + e] = v;
+                four[e] = (short)to_bf16(v > 0.0f ? v : 0.0f);
+                put_quad(to, 8 * q + 4 * half + e, j, (uint16_t)four[e]);
             }
-            acc[nt] = f32x16{};
+            if (TRAIN) rows_to[(size_t)((i0 + 8 * q + 4 * half) >> 2) * HIDDEN + j] = four;
         }
     };
-    keep(b1);
-    __syncthreads();
-    for (int k0 = 0; k0 < PREDICT_HIDDEN; k0 += 8) {
-        const bf16x4 va = *reinterpret_cast<const bf16x4 *>(act + row * PREDICT_HIDDEN + k0 + kq);
+    f32x16 z1 = block_product<IN_QUADS / 2, 12>(in_quads, copies + W1_QUADS / 4, j, lane);
+    activate(z1, a.weights + B1, act, a.a1_quads);
+    uint32_t live1 = 0;  // the first layer's units the gradient passes
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const bf16x4 vb = *reinterpret_cast<const bf16x4 *>(w2t + (size_t)(nt * 32 + row) * PREDICT_HIDDEN + k0 + kq);
-            acc[nt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va, vb, acc[nt], 0, 0, 0);
+    for (int r = 0; r < 16; ++r) live1 |= (z1[r] <= 0.0f ? 0u : 1u) << r;
+    __syncthreads();
+    f32x16 z2 = block_product<HIDDEN_QUADS / 2, 16>(act, copies + W2_QUADS / 4, j, lane);
+    __syncthreads();
+    activate(z2, a.weights + B2, act, a.a2_quads);
+    __syncthreads();
+    // The output: a lane a row, summed in column order.
+    const uint16_t *const w3 = a.copies + W3_COPY;
+    if (t < 32) {
+        const int r = i0 + t;
+        float s = a.weights[B3];
+#pragma unroll 16
+        for (int q = 0; q < HIDDEN_QUADS; ++q) {
+            const bf16x4 four = act[q * LDS_ROW + t];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s += from_bf16((uint16_t)four[e]) * from_bf16(w3[4 * q + e]);
+        }
+        if (!TRAIN) {
+            if (r < a.count) a.y[r] = s;
+        } else {
+            const float target = r < a.count ? a.targets[a.index ? a.index[r] : r] : 0.0f;
+            const float d = r < a.count ? 2.0f * (s - target) / (float)a.count : 0.0f;
+            a.dy[r] = slope[t] = d;
+            a.sq[r] = r < a.count ? (s - target) * (s - target) : 0.0f;
         }
     }
-    __syncthreads();
-    keep(b2);
-    __syncthreads();
-    // The output: one lane a row, summed in column order like `head`.
-    if (lane < 32 && real) {
-        float sum = b3[0];
-        for (int k = 0; k < PREDICT_HIDDEN; ++k) sum += from_bf16(act[row * PREDICT_HIDDEN + k]) * from_bf16(w3[k]);
-        y[i0 + row] = sum;
+    if constexpr (TRAIN) {
+        __syncthreads();
+        // dZ2 = dy w3 where Z2 > 0, dZ1 = dZ2 W2^T where Z1 > 0.
+        const float w = from_bf16(w3[j]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bf16x4 four;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = 8 * q + 4 * half + e;
+                four[e] = (short)to_bf16(z2[4 * q + e] > 0.0f ? slope[i] * w : 0.0f);
+                put_quad(act, i, j, (uint16_t)four[e]);
+            }
+            a.dz2_quads[(size_t)((i0 + 8 * q + 4 * half) >> 2) * HIDDEN + j] = four;
+        }
+        __syncthreads();
+        const f32x16 dz1 = block_product<HIDDEN_QUADS / 2, 16>(act, copies + W2T_QUADS / 4, j, lane);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bf16x4 four;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                four[e] = (short)to_bf16((live1 >> (4 * q + e)) & 1u ? dz1[4 * q + e] : 0.0f);
+            a.dz1_quads[(size_t)((i0 + 8 * q + 4 * half) >> 2) * HIDDEN + j] = four;
+        }
     }
 }
 
-// ------------------------------------------------------------------ the network's small kernels
-
-__global__ void to_bf16_kernel(const float *in, uint16_t *out, int64_t count) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) out[i] = to_bf16(in[i]);
+// One Adam step on a parameter: m, v the moments, `scale` = lr * sqrt(1 - b2^t) / (1 - b1^t).
+struct AdamArgs {
+    float *w, *m, *v;
+    uint16_t *copies;
+    float b1, b2, scale, eps;
+};
+__device__ __forceinline__ float adam(const AdamArgs &p, int at, float gi) {
+    const float mi = p.b1 * p.m[at] + (1.0f - p.b1) * gi;
+    const float vi = p.b2 * p.v[at] + (1.0f - p.b2) * gi * gi;
+    p.m[at] = mi;
+    p.v[at] = vi;
+    const float wi = p.w[at] - p.scale * mi / (sqrtf(vi) + p.eps);
+    p.w[at] = wi;
+    return wi;
 }
 
-// Rows `index[r]` of `in` (FEATURE_STRIDE floats each) as bf16 rows of `out`; rows past `count` zero.
-__global__ void gather_rows(const float *in, const int32_t *index, int count, uint16_t *out, int rows) {
-    const int r = blockIdx.x, k = threadIdx.x;
-    if (r >= rows || k >= FEATURE_STRIDE) return;
-    const float v = r < count ? in[(size_t)index[r] * FEATURE_STRIDE + k] : 0.0f;
-    out[(size_t)r * FEATURE_STRIDE + k] = to_bf16(v);
+// A chain of `steps` in order, `load(bank, place, step)` AHEAD steps before `use(bank, place)`: two banks of registers
+// take turns, the loads of one all made before the other is used (the fence keeps them there: left to itself the
+// compiler moved each load behind its bank's last use, and every bank waited for memory). Loads past the end read the
+// last step again.
+constexpr int AHEAD = 16;
+template <typename Load, typename Use>
+__device__ __forceinline__ void ahead(int steps, Load load, Use use) {
+    const auto fill = [&](auto bank, int from) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) load(bank, u, from + u < steps ? from + u : steps - 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto drain = [&](auto bank, int left) __attribute__((always_inline)) {
+        if (left >= AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) use(bank, u);
+        } else {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+                if (u < left) use(bank, u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const std::integral_constant<int, 0> one;
+    const std::integral_constant<int, 1> other;
+    fill(one, 0);
+    for (int step = 0; step < steps; step += 2 * AHEAD) {
+        fill(other, step + AHEAD);
+        drain(one, steps - step);
+        fill(one, step + 2 * AHEAD);
+        drain(other, steps - step - AHEAD);
+    }
 }
 
-// The output layer and the loss: y = A2 . w3 + b3 per row; with targets, dy = 2 (y - t) / count (zero past
-// `count`), the row's squared error into `sq`, and dZ2 = dy w3 where Z2 > 0, as bf16.
-__global__ void head(const uint16_t *a2, const uint16_t *w3, const float *b3, int hidden, int rows, int count,
-                     const float *targets, float *y, float *dy, float *sq, const float *z2, uint16_t *dz2) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    float s = b3[0];
-    for (int k = 0; k < hidden; ++k) s += from_bf16(a2[(size_t)r * hidden + k]) * from_bf16(w3[k]);
-    if (y) y[r] = s;
-    if (!targets) return;
-    const float d = r < count ? 2.0f * (s - targets[r]) / (float)count : 0.0f;
-    dy[r] = d;
-    sq[r] = r < count ? (s - targets[r]) * (s - targets[r]) : 0.0f;
-    for (int k = 0; k < hidden; ++k)
-        dz2[(size_t)r * hidden + k] = to_bf16(z2[(size_t)r * hidden + k] > 0.0f ? d * from_bf16(w3[k]) : 0.0f);
-}
-
-// Column sums: out[j] = sum over rows of x[r][j] (bf16 x, or fp32 v[r] * bf16 x when `weights`).
-__global__ void column_sums(const uint16_t *x, int rows, int cols, const float *weights, float *out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) return;
+// One column's sum over `quads` quads of rows, each row times its weight or as it is, row by row.
+template <bool WEIGHTED>
+__device__ __forceinline__ float column_sum(const bf16x4 *from, const float *weights, int quads) {
+    const float4 *by = reinterpret_cast<const float4 *>(weights);
     float s = 0.0f;
-    for (int r = 0; r < rows; ++r) s += (weights ? weights[r] : 1.0f) * from_bf16(x[(size_t)r * cols + j]);
-    out[j] = s;
+    bf16x4 v[2][AHEAD];
+    float4 w[2][AHEAD];
+    ahead(quads,
+          [&](auto bank, int u, int q) __attribute__((always_inline)) {
+              v[bank.value][u] = from[(size_t)q * HIDDEN];
+              if (WEIGHTED) w[bank.value][u] = by[q];
+          },
+          [&](auto bank, int u) __attribute__((always_inline)) {
+              const bf16x4 four = v[bank.value][u];
+              const float4 f = WEIGHTED ? w[bank.value][u] : make_float4(1.f, 1.f, 1.f, 1.f);
+              s += f.x * from_bf16((uint16_t)four[0]);
+              s += f.y * from_bf16((uint16_t)four[1]);
+              s += f.z * from_bf16((uint16_t)four[2]);
+              s += f.w * from_bf16((uint16_t)four[3]);
+          });
+    return s;
 }
 
-__global__ void sum_kernel(const float *x, int count, float *out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Every sum over a step's rows, a wave each: the 32 x 32 tiles of dW1 = X^T dZ1 and dW2 = A1^T dZ2, 64 columns of db1,
+// db2 or dw3 = A2^T dy, and db3 with the loss. UPDATE takes an Adam step with each sum, else it is left in `grad`.
+// Each sum is one chain over the rows (a matrix step of 64 cycles every 8, an addition each), so the launch takes what
+// its longest chain does: at 4,096 rows the products took 279 us each, a column's sums 633 and a row's 149, loading one
+// value at a time where the chain waited for it; with quads loaded AHEAD steps before, 39 us for all of them together.
+constexpr int TILES1 = FEATURE_STRIDE / 32 * (HIDDEN / 32), TILES2 = HIDDEN / 32 * (HIDDEN / 32),
+              COLUMN_WAVES = HIDDEN / 64;
+template <bool UPDATE>
+__global__ __launch_bounds__(64) void network_sums(StepArgs a, float *grad, float *loss, AdamArgs p) {
+    const int lane = threadIdx.x, quads = a.rows >> 2;
+    int at = (int)blockIdx.x;
+    if (at < TILES1 + TILES2) {
+        const bool first = at < TILES1;
+        if (!first) at -= TILES1;
+        const int i0 = at / (HIDDEN / 32) * 32, j0 = at % (HIDDEN / 32) * 32, half = lane >> 5, place = lane & 31;
+        const int width = first ? FEATURE_STRIDE : HIDDEN;
+        const bf16x4 *left = (first ? a.x_quads : a.a1_quads) + (size_t)half * width + i0 + place;
+        const bf16x4 *right = (first ? a.dz1_quads : a.dz2_quads) + (size_t)half * HIDDEN + j0 + place;
+        f32x16 acc = {};
+        const int steps = quads >> 1;  // a multiple of 4
+        bf16x4 va[2][AHEAD], vb[2][AHEAD];
+        ahead(steps,
+              [&](auto bank, int u, int step) __attribute__((always_inline)) {
+                  va[bank.value][u] = left[(size_t)step * 2 * width];
+                  vb[bank.value][u] = right[(size_t)step * 2 * HIDDEN];
+              },
+              [&](auto bank, int u) __attribute__((always_inline)) {
+                  acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(va[bank.value][u], vb[bank.value][u], acc, 0, 0, 0);
+              });
+        const int j = j0 + place, base = first ? W1 : W2;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = i0 + 8 * q + 4 * half;
+            bf16x4 four;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int place_of = base + (i + e) * HIDDEN + j;
+                if (UPDATE) {
+                    four[e] = (short)to_bf16(adam(p, place_of, acc[4 * q + e]));
+                    if (!first) p.copies[W2T_QUADS + quad_place(j, i + e)] = (uint16_t)four[e];
+                } else {
+                    grad[place_of] = acc[4 * q + e];
+                }
+            }
+            if (UPDATE)
+                *reinterpret_cast<bf16x4 *>(p.copies + (first ? W1_QUADS : W2_QUADS) + quad_place(i, j)) = four;
+        }
+        return;
+    }
+    at -= TILES1 + TILES2;
+    if (at < 3 * COLUMN_WAVES) {
+        // 64 columns of db1, db2 or dw3, the last with each row's dy.
+        const int which = at / COLUMN_WAVES, j = at % COLUMN_WAVES * 64 + lane;
+        const bf16x4 *from = (which == 0 ? a.dz1_quads : which == 1 ? a.dz2_quads : a.a2_quads) + j;
+        const float s = which == 2 ? column_sum<true>(from, a.dy, quads) : column_sum<false>(from, a.dy, quads);
+        const int place_of = (which == 0 ? B1 : which == 1 ? B2 : W3) + j;
+        if (UPDATE) {
+            const float wi = adam(p, place_of, s);
+            if (which == 2) p.copies[W3_COPY + j] = to_bf16(wi);
+        } else {
+            grad[place_of] = s;
+        }
+        return;
+    }
+    // The output's gradient (lane 0) and the squared errors (lane 1), row by row.
+    if (lane > 1) return;
+    const float4 *from = reinterpret_cast<const float4 *>(lane == 0 ? a.dy : a.sq);
     float s = 0.0f;
-    for (int i = 0; i < count; ++i) s += x[i];
-    out[0] = s;
+    float4 v[2][AHEAD];
+    ahead(quads, [&](auto bank, int u, int q) __attribute__((always_inline)) { v[bank.value][u] = from[q]; },
+          [&](auto bank, int u) __attribute__((always_inline)) {
+              s += v[bank.value][u].x;
+              s += v[bank.value][u].y;
+              s += v[bank.value][u].z;
+              s += v[bank.value][u].w;
+          });
+    if (lane == 1)
+        *loss = s;
+    else if (UPDATE)
+        adam(p, B3, s);
+    else
+        grad[B3] = s;
 }
 
-// One Adam step on `count` parameters: m, v the moments, `scale` = lr * sqrt(1 - b2^t) / (1 - b1^t).
-__global__ void adam(float *w, const float *g, float *m, float *v, int64_t count, float b1, float b2, float scale,
-                     float eps, uint16_t *wb) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - scale * mi / (sqrtf(vi) + eps);
-    w[i] = wi;
-    if (wb) wb[i] = to_bf16(wi);
+// The bf16 copies of the fp32 weights.
+__global__ void copy_weights(const float *w, uint16_t *copies) {
+    const int at = blockIdx.x * 256 + threadIdx.x;
+    if (at < B1) {
+        copies[W1_QUADS + quad_place(at / HIDDEN, at % HIDDEN)] = to_bf16(w[W1 + at]);
+    } else if (at >= W2 && at < B2) {
+        const int i = (at - W2) / HIDDEN, j = (at - W2) % HIDDEN;
+        copies[W2_QUADS + quad_place(i, j)] = copies[W2T_QUADS + quad_place(j, i)] = to_bf16(w[at]);
+    } else if (at >= W3 && at < B3) {
+        copies[W3_COPY + at - W3] = to_bf16(w[at]);
+    }
 }
 
 }  // namespace dinara
@@ -318,18 +467,14 @@ using namespace dinara;
 
 struct dinara_mlp {
     DeviceContext *ctx = nullptr;
-    int hidden = 256;
     int rows_cap = 0;   // rows the work buffers hold
     int64_t step = 0;   // Adam's step count
-    // fp32 master weights, their bf16 copies, gradients, Adam moments (one flat buffer each: w1, b1, w2, b2, w3, b3)
-    DeviceBuffer master, bf, grad, m1, m2;
+    // fp32 master weights, gradients and Adam moments (flat: w1, b1, w2, b2, w3, b3), and the weights' bf16 copies
+    DeviceBuffer master, copies, grad, m1, m2;
     // per-step work
-    DeviceBuffer x, z1, a1, z2, a2, y, dy, sq, dz2, dz1, targets, index, loss, features;
-    DeviceBuffer identity;  // 0, 1, 2, ... for gathers of consecutive rows
-    DeviceBuffer transposed;  // w1 and w2 as bf16, transposed, for the one-pass prediction
-    DeviceBuffer predicted;   // the one-pass prediction's output for `dinara_mlp_predict`
-    int identity_rows = 0;
-    size_t off_w1, off_b1, off_w2, off_b2, off_w3, off_b3, total;
+    DeviceBuffer x_quads, a1_quads, a2_quads, dz1_quads, dz2_quads, dy, sq;
+    DeviceBuffer features, targets, index, loss;
+    DeviceBuffer predicted;   // the prediction's output for `dinara_mlp_predict`
 };
 
 namespace {
@@ -337,141 +482,71 @@ namespace {
 using Net = dinara_mlp;
 
 float *f32(DeviceBuffer &b, size_t offset = 0) { return static_cast<float *>(b.ptr) + offset; }
-uint16_t *h16(DeviceBuffer &b, size_t offset = 0) { return static_cast<uint16_t *>(b.ptr) + offset; }
 
 bool reserve_rows(Net *net, int rows) {
     if (rows <= net->rows_cap) return true;
-    const size_t r = (size_t)rows, h = (size_t)net->hidden;
-    if (!net->x.reserve(r * FEATURE_STRIDE * 2) || !net->z1.reserve(r * h * 4) || !net->a1.reserve(r * h * 2) ||
-        !net->z2.reserve(r * h * 4) || !net->a2.reserve(r * h * 2) || !net->y.reserve(r * 4) ||
-        !net->dy.reserve(r * 4) || !net->sq.reserve(r * 4) || !net->dz2.reserve(r * h * 2) ||
-        !net->dz1.reserve(r * h * 2) || !net->targets.reserve(r * 4) || !net->loss.reserve(16))
-        return false;
+    const size_t r = (size_t)rows;
+    for (DeviceBuffer *b : {&net->a1_quads, &net->a2_quads, &net->dz1_quads, &net->dz2_quads})
+        if (!b->reserve(r * HIDDEN * 2)) return false;
+    if (!net->x_quads.reserve(r * FEATURE_STRIDE * 2) || !net->dy.reserve(r * 4) || !net->sq.reserve(r * 4)) return false;
     net->rows_cap = rows;
     return true;
 }
 
-// Forward over `rows` rows of bf16 inputs in net->x: Z1, A1, Z2, A2 and y.
-void forward(Net *net, int rows, hipStream_t s) {
-    const int h = net->hidden;
-    gemm<false, false>(s, h16(net->x), FEATURE_STRIDE, h16(net->bf, net->off_w1), h, rows, h, FEATURE_STRIDE,
-                       f32(net->master, net->off_b1), 1, nullptr, 0, f32(net->z1), h, h16(net->a1), h);
-    gemm<false, false>(s, h16(net->a1), h, h16(net->bf, net->off_w2), h, rows, h, h, f32(net->master, net->off_b2),
-                       1, nullptr, 0, f32(net->z2), h, h16(net->a2), h);
+StepArgs step_args(Net *net, const float *x, int count, int rows) {
+    StepArgs a{};
+    a.x = x;
+    a.count = count;
+    a.rows = rows;
+    a.weights = f32(net->master);
+    a.copies = static_cast<const uint16_t *>(net->copies.ptr);
+    const auto quads = [](DeviceBuffer &b) { return static_cast<bf16x4 *>(b.ptr); };
+    a.x_quads = quads(net->x_quads);
+    a.a1_quads = quads(net->a1_quads);
+    a.a2_quads = quads(net->a2_quads);
+    a.dz1_quads = quads(net->dz1_quads);
+    a.dz2_quads = quads(net->dz2_quads);
+    a.dy = f32(net->dy);
+    a.sq = f32(net->sq);
+    return a;
 }
 
-// Forward and backward over `rows` rows (the first `count` real), targets in net->targets: the gradients into
-// net->grad and the summed squared error into net->loss[0].
-void forward_backward(Net *net, int rows, int count, hipStream_t s) {
-    const int h = net->hidden;
-    forward(net, rows, s);
-    hipLaunchKernelGGL(head, dim3((rows + 255) / 256), dim3(256), 0, s, h16(net->a2), h16(net->bf, net->off_w3),
-                       f32(net->master, net->off_b3), h, rows, count, f32(net->targets), f32(net->y), f32(net->dy),
-                       f32(net->sq), f32(net->z2), h16(net->dz2));
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(1), 0, s, f32(net->sq), rows, f32(net->loss));
-    // Output layer: dw3 = A2^T dy, db3 = sum dy.
-    hipLaunchKernelGGL(column_sums, dim3((h + 255) / 256), dim3(256), 0, s, h16(net->a2), rows, h, f32(net->dy),
-                       f32(net->grad, net->off_w3));
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(1), 0, s, f32(net->dy), rows, f32(net->grad, net->off_b3));
-    // Second layer: dW2 = A1^T dZ2, db2 = sum dZ2, dZ1 = (dZ2 W2^T) where Z1 > 0.
-    gemm<true, false>(s, h16(net->a1), h, h16(net->dz2), h, h, h, rows, nullptr, 0, nullptr, 0,
-                      f32(net->grad, net->off_w2), h, nullptr, 0);
-    hipLaunchKernelGGL(column_sums, dim3((h + 255) / 256), dim3(256), 0, s, h16(net->dz2), rows, h, nullptr,
-                       f32(net->grad, net->off_b2));
-    gemm<false, true>(s, h16(net->dz2), h, h16(net->bf, net->off_w2), h, rows, h, h, nullptr, 0, f32(net->z1), h,
-                      nullptr, 0, h16(net->dz1), h);
-    // First layer: dW1 = X^T dZ1, db1 = sum dZ1.
-    gemm<true, false>(s, h16(net->x), FEATURE_STRIDE, h16(net->dz1), h, FEATURE_STRIDE, h, rows, nullptr, 0,
-                      nullptr, 0, f32(net->grad, net->off_w1), h, nullptr, 0);
-    hipLaunchKernelGGL(column_sums, dim3((h + 255) / 256), dim3(256), 0, s, h16(net->dz1), rows, h, nullptr,
-                       f32(net->grad, net->off_b1));
+// A step's two launches over `a.rows` rows (a multiple of 32); its summed squared error into *loss.
+template <bool UPDATE>
+void launch_step(Net *net, const StepArgs &a, float *loss, const AdamArgs &p) {
+    hipStream_t s = net->ctx->stream;
+    hipLaunchKernelGGL((network_rows<true>), dim3(a.rows / 32), dim3(512), 0, s, a);
+    hipLaunchKernelGGL((network_sums<UPDATE>), dim3(TILES1 + TILES2 + 3 * COLUMN_WAVES + 1), dim3(64), 0, s, a,
+                       f32(net->grad), loss, p);
 }
 
-void refresh_bf16(Net *net, hipStream_t s) {
-    hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)((net->total + 255) / 256)), dim3(256), 0, s,
-                       f32(net->master), h16(net->bf), (int64_t)net->total);
-}
-
-// Uploads `rows` fp32 feature rows (FEATURE_STRIDE each) as bf16 into net->x, padded to a multiple of 32.
-bool upload_rows(Net *net, int64_t rows, const float *features, int *padded) {
-    const int p = (int)((rows + 31) / 32 * 32);
-    if (!reserve_rows(net, std::max(p, 32))) return false;
-    if (!net->features.reserve((size_t)std::max<int64_t>(rows, 1) * FEATURE_STRIDE * 4)) return false;
-    if (rows > 0 && !net->features.write(net->ctx, features, (size_t)rows * FEATURE_STRIDE * 4)) return false;
-    std::vector<int32_t> idx((size_t)std::max<int64_t>(rows, 1));
-    for (int64_t i = 0; i < rows; ++i) idx[i] = (int32_t)i;
-    if (!net->index.upload(net->ctx, idx.data(), idx.size() * 4)) return false;
-    hipLaunchKernelGGL(gather_rows, dim3(p), dim3(FEATURE_STRIDE), 0, net->ctx->stream, f32(net->features),
-                       static_cast<const int32_t *>(net->index.ptr), (int)rows, h16(net->x), p);
-    *padded = p;
-    return true;
+void refresh_copies(Net *net) {
+    hipLaunchKernelGGL(copy_weights, dim3((WEIGHTS + 255) / 256), dim3(256), 0, net->ctx->stream, f32(net->master),
+                       static_cast<uint16_t *>(net->copies.ptr));
 }
 
 }  // namespace
+
+int64_t mlp_predict_into(dinara_mlp *net, const float *features, int64_t rows, float *out) {
+    if (!net) return DINARA_INVALID_MODE;
+    DeviceGuard guard(net->ctx);
+    constexpr int64_t most = int64_t(1) << 22;  // rows a launch: row numbers times the stride stay in 32 bits
+    for (int64_t first = 0; first < rows; first += most) {
+        const int count = (int)std::min(most, rows - first);
+        StepArgs a = step_args(net, features + first * FEATURE_STRIDE, count, count);
+        a.y = out + first;
+        hipLaunchKernelGGL((network_rows<false>), dim3((count + 31) / 32), dim3(512), 0, net->ctx->stream, a);
+    }
+    return hipPeekAtLastError() == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
+}
 
 int64_t mlp_predict_device(dinara_mlp *net, const float *features, int64_t rows, float *out) {
     if (!net) return DINARA_INVALID_MODE;
     if (rows <= 0) return 0;
     DeviceGuard guard(net->ctx);
-    hipStream_t s = net->ctx->stream;
-    const int64_t chunk = 1 << 16;
-    if (!reserve_rows(net, (int)chunk) || !net->index.reserve((size_t)chunk * 4)) return DINARA_OUT_OF_MEMORY;
-    std::vector<int32_t> idx((size_t)chunk);
-    for (int64_t first = 0; first < rows; first += chunk) {
-        const int64_t count = std::min(chunk, rows - first);
-        const int padded = (int)((count + 31) / 32 * 32);
-        for (int64_t i = 0; i < count; ++i) idx[i] = (int32_t)(first + i);
-        if (!net->index.write(net->ctx, idx.data(), (size_t)count * 4)) return DINARA_OUT_OF_MEMORY;
-        hipLaunchKernelGGL(gather_rows, dim3(padded), dim3(FEATURE_STRIDE), 0, s, features,
-                           static_cast<const int32_t *>(net->index.ptr), (int)count, h16(net->x), padded);
-        forward(net, padded, s);
-        hipLaunchKernelGGL(head, dim3((padded + 255) / 256), dim3(256), 0, s, h16(net->a2), h16(net->bf, net->off_w3),
-                           f32(net->master, net->off_b3), net->hidden, padded, (int)count, nullptr, f32(net->y),
-                           nullptr, nullptr, nullptr, nullptr);
-        if (!net->y.read(net->ctx, out + first, (size_t)count * 4)) return DINARA_OUT_OF_MEMORY;
-    }
-    return 0;
-}
-
-int64_t mlp_predict_into(dinara_mlp *net, const float *features, int64_t rows, float *out) {
-    if (!net) return DINARA_INVALID_MODE;
-    if (rows <= 0) return 0;
-    DeviceGuard guard(net->ctx);
-    hipStream_t s = net->ctx->stream;
-    if (net->hidden == PREDICT_HIDDEN && rows <= INT32_MAX / FEATURE_STRIDE) {
-        const size_t w1 = (size_t)FEATURE_STRIDE * PREDICT_HIDDEN, w2 = (size_t)PREDICT_HIDDEN * PREDICT_HIDDEN;
-        if (!net->transposed.reserve((w1 + w2) * 2)) return DINARA_OUT_OF_MEMORY;
-        uint16_t *w1t = h16(net->transposed), *w2t = w1t + w1;
-        hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)((w1 + 255) / 256)), dim3(256), 0, s,
-                           h16(net->bf, net->off_w1), FEATURE_STRIDE, PREDICT_HIDDEN, w1t);
-        hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)((w2 + 255) / 256)), dim3(256), 0, s,
-                           h16(net->bf, net->off_w2), PREDICT_HIDDEN, PREDICT_HIDDEN, w2t);
-        hipLaunchKernelGGL(predict_rows, dim3((unsigned)((rows + 31) / 32)), dim3(64), 0, s, features, (int)rows, w1t,
-                           f32(net->master, net->off_b1), w2t, f32(net->master, net->off_b2),
-                           h16(net->bf, net->off_w3), f32(net->master, net->off_b3), out);
-        return hipPeekAtLastError() == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
-    }
-    const int chunk = 1 << 16;
-    if (!reserve_rows(net, chunk)) return DINARA_OUT_OF_MEMORY;
-    if (net->identity_rows < chunk) {
-        std::vector<int32_t> idx((size_t)chunk);
-        for (int i = 0; i < chunk; ++i) idx[i] = i;
-        if (!net->identity.upload(net->ctx, idx.data(), idx.size() * 4)) return DINARA_OUT_OF_MEMORY;
-        net->identity_rows = chunk;
-    }
-    for (int64_t first = 0; first < rows; first += chunk) {
-        const int count = (int)std::min<int64_t>(chunk, rows - first);
-        const int padded = (count + 31) / 32 * 32;
-        hipLaunchKernelGGL(gather_rows, dim3(padded), dim3(FEATURE_STRIDE), 0, s, features + first * FEATURE_STRIDE,
-                           static_cast<const int32_t *>(net->identity.ptr), count, h16(net->x), padded);
-        forward(net, padded, s);
-        hipLaunchKernelGGL(head, dim3((padded + 255) / 256), dim3(256), 0, s, h16(net->a2), h16(net->bf, net->off_w3),
-                           f32(net->master, net->off_b3), net->hidden, padded, count, nullptr, f32(net->y),
-                           nullptr, nullptr, nullptr, nullptr);
-        if (hipMemcpyAsync(out + first, net->y.ptr, (size_t)count * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
-            return DINARA_OUT_OF_MEMORY;
-    }
-    return hipPeekAtLastError() == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
+    if (!net->predicted.reserve((size_t)rows * 4)) return DINARA_OUT_OF_MEMORY;
+    if (const int64_t code = mlp_predict_into(net, features, rows, f32(net->predicted))) return code;
+    return net->predicted.read(net->ctx, out, (size_t)rows * 4) ? 0 : DINARA_OUT_OF_MEMORY;
 }
 
 extern "C" {
@@ -482,32 +557,24 @@ dinara_mlp *dinara_mlp_new(int64_t gpu, uint64_t seed) {
     DeviceGuard guard(ctx);
     auto *net = new Net();
     net->ctx = ctx;
-    const size_t h = (size_t)net->hidden;
-    net->off_w1 = 0;
-    net->off_b1 = net->off_w1 + (size_t)FEATURE_STRIDE * h;
-    net->off_w2 = net->off_b1 + h;
-    net->off_b2 = net->off_w2 + h * h;
-    net->off_w3 = net->off_b2 + h;
-    net->off_b3 = net->off_w3 + h;
-    net->total = net->off_b3 + 1;
     // He-normal weights for the ReLU layers (the padding inputs' rows zero), a small output layer, zero biases.
-    std::vector<float> w(net->total, 0.0f);
+    std::vector<float> w(WEIGHTS, 0.0f);
     std::mt19937_64 rng(seed);
-    std::normal_distribution<float> n1(0.0f, std::sqrt(2.0f / FEATURES)), n2(0.0f, std::sqrt(2.0f / (float)h)),
-        n3(0.0f, std::sqrt(1.0f / (float)h));
-    for (size_t k = 0; k < (size_t)FEATURES; ++k)
-        for (size_t j = 0; j < h; ++j) w[net->off_w1 + k * h + j] = n1(rng);
-    for (size_t k = 0; k < h * h; ++k) w[net->off_w2 + k] = n2(rng);
-    for (size_t k = 0; k < h; ++k) w[net->off_w3 + k] = n3(rng);
-    w[net->off_b3] = 7.0f;  // log(1 + cost) of a typical pair, where training starts
-    const size_t bytes = net->total * 4;
-    std::vector<float> zero(net->total, 0.0f);
-    if (!net->master.upload(ctx, w.data(), bytes) || !net->bf.reserve(net->total * 2) || !net->grad.reserve(bytes) ||
-        !net->m1.upload(ctx, zero.data(), bytes) || !net->m2.upload(ctx, zero.data(), bytes)) {
+    std::normal_distribution<float> n1(0.0f, std::sqrt(2.0f / FEATURES)), n2(0.0f, std::sqrt(2.0f / (float)HIDDEN)),
+        n3(0.0f, std::sqrt(1.0f / (float)HIDDEN));
+    for (size_t k = 0; k < (size_t)FEATURES * HIDDEN; ++k) w[W1 + k] = n1(rng);
+    for (size_t k = 0; k < (size_t)HIDDEN * HIDDEN; ++k) w[W2 + k] = n2(rng);
+    for (size_t k = 0; k < (size_t)HIDDEN; ++k) w[W3 + k] = n3(rng);
+    w[B3] = 7.0f;  // log(1 + cost) of a typical pair, where training starts
+    const size_t bytes = (size_t)WEIGHTS * 4;
+    std::vector<float> zero(WEIGHTS, 0.0f);
+    if (!net->master.upload(ctx, w.data(), bytes) || !net->copies.reserve((size_t)COPIES * 2) ||
+        !net->grad.reserve(bytes) || !net->m1.upload(ctx, zero.data(), bytes) ||
+        !net->m2.upload(ctx, zero.data(), bytes)) {
         delete net;
         return nullptr;
     }
-    refresh_bf16(net, ctx->stream);
+    refresh_copies(net);
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) {
         delete net;
         return nullptr;
@@ -521,20 +588,20 @@ void dinara_mlp_free(dinara_mlp *net) {
     delete net;
 }
 
-int64_t dinara_mlp_parameter_count(dinara_mlp *net) { return net ? (int64_t)net->total : 0; }
+int64_t dinara_mlp_parameter_count(dinara_mlp *net) { return net ? (int64_t)WEIGHTS : 0; }
 
 // The fp32 master weights, flat: w1 (288 x 256, row k input k), b1 (256), w2 (256 x 256), b2, w3 (256), b3 (1).
 int64_t dinara_mlp_get_weights(dinara_mlp *net, float *out) {
     if (!net) return DINARA_INVALID_MODE;
     DeviceGuard guard(net->ctx);
-    return net->master.read(net->ctx, out, net->total * 4) ? 0 : DINARA_OUT_OF_MEMORY;
+    return net->master.read(net->ctx, out, (size_t)WEIGHTS * 4) ? 0 : DINARA_OUT_OF_MEMORY;
 }
 
 int64_t dinara_mlp_set_weights(dinara_mlp *net, const float *in) {
     if (!net) return DINARA_INVALID_MODE;
     DeviceGuard guard(net->ctx);
-    if (!net->master.write(net->ctx, in, net->total * 4)) return DINARA_OUT_OF_MEMORY;
-    refresh_bf16(net, net->ctx->stream);
+    if (!net->master.write(net->ctx, in, (size_t)WEIGHTS * 4)) return DINARA_OUT_OF_MEMORY;
+    refresh_copies(net);
     return hipStreamSynchronize(net->ctx->stream) == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
 }
 
@@ -544,14 +611,17 @@ int64_t dinara_mlp_gradients(dinara_mlp *net, int64_t rows, const float *feature
                              float *gradients, double *loss) {
     if (!net || rows <= 0) return DINARA_INVALID_MODE;
     DeviceGuard guard(net->ctx);
-    int padded = 0;
-    if (!upload_rows(net, rows, features, &padded)) return DINARA_OUT_OF_MEMORY;
-    std::vector<float> t((size_t)padded, 0.0f);
-    std::memcpy(t.data(), targets, (size_t)rows * 4);
-    if (!net->targets.write(net->ctx, t.data(), t.size() * 4)) return DINARA_OUT_OF_MEMORY;
-    forward_backward(net, padded, (int)rows, net->ctx->stream);
+    const int64_t padded = (rows + 31) / 32 * 32;
+    if (padded > INT32_MAX / FEATURE_STRIDE || !reserve_rows(net, (int)padded) || !net->loss.reserve(4) ||
+        !net->features.upload(net->ctx, features, (size_t)rows * FEATURE_STRIDE * 4) ||
+        !net->targets.upload(net->ctx, targets, (size_t)rows * 4))
+        return DINARA_OUT_OF_MEMORY;
+    StepArgs a = step_args(net, f32(net->features), (int)rows, (int)padded);
+    a.targets = f32(net->targets);
+    launch_step<false>(net, a, f32(net->loss), AdamArgs{});
     float sq = 0;
-    if (!net->grad.read(net->ctx, gradients, net->total * 4) || !net->loss.read(net->ctx, &sq, 4))
+    if (hipPeekAtLastError() != hipSuccess || !net->grad.read(net->ctx, gradients, (size_t)WEIGHTS * 4) ||
+        !net->loss.read(net->ctx, &sq, 4))
         return DINARA_OUT_OF_MEMORY;
     if (loss) *loss = sq / (double)rows;
     return 0;
@@ -562,82 +632,58 @@ int64_t dinara_mlp_predict(dinara_mlp *net, int64_t rows, const float *features,
     if (!net) return DINARA_INVALID_MODE;
     if (rows <= 0) return 0;
     DeviceGuard guard(net->ctx);
-    if (net->hidden == PREDICT_HIDDEN && rows <= INT32_MAX / FEATURE_STRIDE) {  // the one-pass prediction
-        const size_t bytes = (size_t)rows * FEATURE_STRIDE * 4;
-        if (!net->features.reserve(bytes) || !net->features.write(net->ctx, features, bytes) ||
-            !net->predicted.reserve((size_t)rows * 4))
-            return DINARA_OUT_OF_MEMORY;
-        if (const int64_t code = mlp_predict_into(net, f32(net->features), rows, f32(net->predicted))) return code;
-        return net->predicted.read(net->ctx, out, (size_t)rows * 4) ? 0 : DINARA_OUT_OF_MEMORY;
-    }
-    const int64_t chunk = 1 << 16;
-    for (int64_t first = 0; first < rows; first += chunk) {
-        const int64_t count = std::min(chunk, rows - first);
-        int padded = 0;
-        if (!upload_rows(net, count, features + first * FEATURE_STRIDE, &padded)) return DINARA_OUT_OF_MEMORY;
-        forward(net, padded, net->ctx->stream);
-        hipLaunchKernelGGL(head, dim3((padded + 255) / 256), dim3(256), 0, net->ctx->stream, h16(net->a2),
-                           h16(net->bf, net->off_w3), f32(net->master, net->off_b3), net->hidden, padded, count,
-                           nullptr, f32(net->y), nullptr, nullptr, nullptr, nullptr);
-        if (!net->y.read(net->ctx, out + first, (size_t)count * 4)) return DINARA_OUT_OF_MEMORY;
-    }
-    return 0;
+    if (!net->features.upload(net->ctx, features, (size_t)rows * FEATURE_STRIDE * 4)) return DINARA_OUT_OF_MEMORY;
+    return mlp_predict_device(net, f32(net->features), rows, out);
 }
 
 // Trains on `rows` rows for `epochs` passes in shuffled batches of `batch` rows (a multiple of 32) by Adam at
-// learning rate `lr`: every step's forward, backward and update on the device. Writes the last epoch's mean loss.
+// learning rate `lr`: every step's forward, backward and update on the device, the host waiting once an epoch (for the
+// steps' losses). Writes the last epoch's mean loss.
 int64_t dinara_mlp_train(dinara_mlp *net, int64_t rows, const float *features, const float *targets, int64_t epochs,
                          int64_t batch, double lr, uint64_t seed, double *final_loss) {
     if (!net || rows <= 0 || batch <= 0 || batch % 32 != 0) return DINARA_INVALID_MODE;
     DeviceContext *ctx = net->ctx;
     DeviceGuard guard(ctx);
-    hipStream_t s = ctx->stream;
-    if (!reserve_rows(net, (int)batch)) return DINARA_OUT_OF_MEMORY;
-    DeviceBuffer all_targets;
-    if (!net->features.upload(ctx, features, (size_t)rows * FEATURE_STRIDE * 4) ||
-        !all_targets.upload(ctx, targets, (size_t)rows * 4) || !net->index.reserve((size_t)rows * 4))
+    const int64_t steps = (rows + batch - 1) / batch;
+    if (batch > INT32_MAX / FEATURE_STRIDE || !reserve_rows(net, (int)batch) || !net->loss.reserve((size_t)steps * 4) ||
+        !net->features.upload(ctx, features, (size_t)rows * FEATURE_STRIDE * 4) ||
+        !net->targets.upload(ctx, targets, (size_t)rows * 4) || !net->index.reserve((size_t)rows * 4))
         return DINARA_OUT_OF_MEMORY;
     std::vector<int32_t> order((size_t)rows);
     for (int64_t i = 0; i < rows; ++i) order[i] = (int32_t)i;
     std::mt19937_64 rng(seed);
-    std::vector<float> batch_targets((size_t)batch);
+    std::vector<float> losses((size_t)steps);
     double epoch_loss = 0;
-    const float b1 = 0.9f, b2 = 0.999f;
+    AdamArgs p{};
+    p.w = f32(net->master);
+    p.m = f32(net->m1);
+    p.v = f32(net->m2);
+    p.copies = static_cast<uint16_t *>(net->copies.ptr);
+    p.b1 = 0.9f;
+    p.b2 = 0.999f;
+    p.eps = 1e-8f;
     for (int64_t e = 0; e < epochs; ++e) {
         std::shuffle(order.begin(), order.end(), rng);
         if (!net->index.write(ctx, order.data(), order.size() * 4)) return DINARA_OUT_OF_MEMORY;
-        std::vector<float> shuffled((size_t)rows);
-        for (int64_t i = 0; i < rows; ++i) shuffled[i] = targets[order[i]];
-        DeviceBuffer shuffled_targets;
-        if (!shuffled_targets.upload(ctx, shuffled.data(), shuffled.size() * 4)) return DINARA_OUT_OF_MEMORY;
-        double sum = 0;
-        int64_t seen = 0;
-        for (int64_t first = 0; first < rows; first += batch) {
-            const int count = (int)std::min<int64_t>(batch, rows - first);
-            hipLaunchKernelGGL(gather_rows, dim3((unsigned)batch), dim3(FEATURE_STRIDE), 0, s, f32(net->features),
-                               static_cast<const int32_t *>(net->index.ptr) + first, count, h16(net->x), (int)batch);
-            if (hipMemcpyAsync(net->targets.ptr, f32(shuffled_targets) + first, (size_t)count * 4,
-                               hipMemcpyDeviceToDevice, s) != hipSuccess)
-                return DINARA_OUT_OF_MEMORY;
-            if (count < batch && hipMemsetAsync(f32(net->targets) + count, 0, (size_t)(batch - count) * 4, s) != hipSuccess)
-                return DINARA_OUT_OF_MEMORY;
-            forward_backward(net, (int)batch, count, s);
+        for (int64_t at = 0; at < steps; ++at) {
+            const int64_t first = at * batch;
+            StepArgs a = step_args(net, f32(net->features), (int)std::min<int64_t>(batch, rows - first), (int)batch);
+            a.targets = f32(net->targets);
+            a.index = static_cast<const int32_t *>(net->index.ptr) + first;
             ++net->step;
-            const double bias1 = 1.0 - std::pow((double)b1, (double)net->step);
-            const double bias2 = 1.0 - std::pow((double)b2, (double)net->step);
-            const float scale = (float)(lr * std::sqrt(bias2) / bias1);
-            hipLaunchKernelGGL(adam, dim3((unsigned)((net->total + 255) / 256)), dim3(256), 0, s, f32(net->master),
-                               f32(net->grad), f32(net->m1), f32(net->m2), (int64_t)net->total, b1, b2, scale, 1e-8f,
-                               h16(net->bf));
-            float sq = 0;
-            if (!net->loss.read(ctx, &sq, 4)) return DINARA_OUT_OF_MEMORY;
-            sum += sq;
-            seen += count;
+            const double bias1 = 1.0 - std::pow((double)p.b1, (double)net->step);
+            const double bias2 = 1.0 - std::pow((double)p.b2, (double)net->step);
+            p.scale = (float)(lr * std::sqrt(bias2) / bias1);
+            launch_step<true>(net, a, f32(net->loss) + at, p);
         }
-        epoch_loss = sum / (double)seen;
+        if (hipPeekAtLastError() != hipSuccess || !net->loss.read(ctx, losses.data(), losses.size() * 4))
+            return DINARA_OUT_OF_MEMORY;
+        double sum = 0;
+        for (float sq : losses) sum += sq;
+        epoch_loss = sum / (double)rows;
     }
     if (final_loss) *final_loss = epoch_loss;
-    return hipStreamSynchronize(s) == hipSuccess ? 0 : DINARA_OUT_OF_MEMORY;
+    return 0;
 }
 
 }  // extern "C"

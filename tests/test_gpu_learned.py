@@ -111,6 +111,39 @@ def test_gradients_match_numpy():
         net.free()
 
 
+@pytest.mark.parametrize("rows", [1, 32, 95, 512, 544, 1100])
+def test_gradients_of_small_integers_are_exact(rows):
+    # One block of 32 rows, part of one, whole and part register banks of the sums over rows (16 steps of 8 rows, two
+    # banks). Weights and inputs are small integers and the targets make each row's output gradient one too, so every
+    # product, activation and sum is a whole number bf16 (256) and fp32 (2^24) hold: no order of the sums rounds, and the
+    # gradients equal the oracle's. The loss, a sum of larger squares, is within one rounding an addition.
+    rng = np.random.default_rng(rows)
+    weights = np.zeros(288 * 256 + 256 + 256 * 256 + 256 + 256 + 1, dtype=np.float32)
+    w1, b1, w2, b2, w3, b3 = mlp.split(weights)
+    for j in range(256):
+        w1[rng.choice(mlp.FEATURES, 4, replace=False), j] = rng.choice([-1, 1], 4)
+        w2[rng.choice(256, 4, replace=False), j] = rng.choice([-1, 1], 4)
+    b1[:], b2[:] = rng.integers(-1, 2, 256), rng.integers(-1, 2, 256)
+    w3[rng.choice(256, 4, replace=False)] = (1, -1, 1, -1)
+    b3[0] = 7
+    weights = np.concatenate([v.reshape(-1) for v in (w1, b1, w2, b2, w3, b3)]).astype(np.float32)
+    x = np.zeros((rows, F), dtype=np.float32)
+    x[:, :mlp.FEATURES] = rng.integers(0, 3, (rows, mlp.FEATURES))
+    out = mlp.forward(weights, x)[0]
+    t = (out - rng.integers(-2, 3, rows) * rows / 2).astype(np.float32)
+    net = Net(1)
+    try:
+        assert net.h.dinara_mlp_set_weights(net.ptr, weights.ctypes.data) == 0
+        assert np.array_equal(net.predict(x), out)
+        got, loss = net.gradients(x, t)
+        want, want_loss = mlp.gradients(weights, x, t)
+        for name, a, b in zip(("w1", "b1", "w2", "b2", "w3", "b3"), mlp.split(got), mlp.split(want)):
+            assert np.array_equal(a, b), name
+        assert abs(loss - want_loss) <= 2 * rows * 2.0 ** -24 * want_loss
+    finally:
+        net.free()
+
+
 def test_forward_matches_numpy():
     net = Net(4)
     try:
