@@ -120,34 +120,21 @@ __device__ __forceinline__ bool certify_ends(const SweepArgs &a, int rows, int c
     return false;
 }
 
-// The class of band a pair of `letters` letters needing `need` diagonals takes next: the narrowest that holds them.
-// A group or block band is placed on an even diagonal, so it holds one diagonal fewer than its width. Pairs under a
-// user band take the wave bands, which bar diagonals outside it; pairs longer than a group launch stages take
-// blocks.
-__device__ __forceinline__ int class_for(int need, int letters, const SweepArgs &a) {
-    if (!a.user_band && a.groups_fit && letters <= a.group_max_letters) {
-        for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
-            if (need < band_width(cls)) return cls;
-    }
-    if (!a.user_band) {
-        for (int cls = CLASS_BLOCK_FIRST; cls < CLASSES; ++cls)
-            if (((a.block_mask >> (cls - CLASS_BLOCK_FIRST)) & 1) && need < band_width(cls)) return cls;
-    }
-    for (int cls = CLASS_WAVE_FIRST; cls <= CLASS_WAVE_LAST; ++cls)
-        if (need <= band_width(cls)) return cls;
-    return CLASS_TOO_WIDE;
-}
-
 __device__ __forceinline__ void file_retry(const SweepArgs &a, int slot, int letters, int want_low, int want_high) {
     a.want_low[slot] = want_low;
     a.want_high[slot] = want_high;
-    const int cls = class_for(want_high - want_low + 1, letters, a);
+    const int cls = band_class(want_high - want_low + 1, letters, a.user_band != 0, a.group_max_letters, a.strip_letters,
+                               a.strip_widest);
     // A wave sweep stages both sequences in LDS: a pair they overflow has no class to go to.
     if (cls == CLASS_TOO_WIDE || (band_is_wave(cls) && letters > a.lds_limit)) {
         a.status[slot] = 2;
         return;
     }
     a.status[slot] = 1;
+    if (band_is_strip(cls)) {
+        a.strip_retries[atomicAdd(&a.retry_counts[CLASS_STRIP_FIRST], 1)] = make_int4(slot, want_low, want_high, 0);
+        return;
+    }
     const int at = atomicAdd(&a.retry_counts[cls], 1);
     a.retry_lists[(size_t)cls * a.retry_capacity + at] = slot;
 }

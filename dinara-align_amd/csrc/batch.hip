@@ -22,9 +22,9 @@
 #include "common.h"
 #include "device.h"
 #include "edit.h"
-#include "full.h"
 #include "host.h"
 #include "learned.h"
+#include "strip.h"
 
 using namespace dinara;
 
@@ -146,25 +146,6 @@ int64_t pair_code(const char *ref, int64_t n, const char *qry, int64_t m) {
     return 0;
 }
 
-// The class a pair's first band takes: the narrowest group band holding `need` diagonals (one fewer than its width:
-// a group band starts on an even diagonal), else the narrowest block band, else the narrowest wave band (as the
-// device's class_for).
-int first_class_for(int need, bool groups, int block_mask, bool user_band) {
-    if (groups && !user_band)
-        for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
-            if (need < class_width(cls)) return cls;
-    if (!user_band)
-        for (int cls = CLASS_BLOCK_FIRST; cls < CLASSES; ++cls)
-            if (((block_mask >> (cls - CLASS_BLOCK_FIRST)) & 1) && need < class_width(cls)) return cls;
-    for (int cls = CLASS_WAVE_FIRST; cls <= CLASS_WAVE_LAST; ++cls)
-        if (need <= class_width(cls)) return cls;
-    return CLASS_TOO_WIDE;
-}
-
-// LDS bytes one block of class `cls` stages: four pairs' letters for a group, one pair's and the reads past it
-// for a block.
-size_t block_letters(int max_letters, int cls) { return ((size_t)max_letters + class_width(cls) / 2 + 16 + 3) & ~size_t(3); }
-
 }  // namespace
 
 // ------------------------------------------------------------------ the batch
@@ -195,10 +176,9 @@ struct dinara_batch {
     int max_letters = 0;                  // the most letters of a pair, both sequences
     int32_t max_rows = 0;
     int group_letters = 4;                // LDS bytes a pair takes in a group launch
-    int group_max_letters = 0;            // the longest pair a group launch stages
-    bool groups_fit = false;              // four pairs' letters fit one block's LDS, their costs the tags
+    int group_max_letters = 0;            // the longest pair a group launch stages (0: no groups)
     int group16_top = 0;                  // > 0: packed 16-bit group cells, this the unreachable value
-    int block_mask = 0;                   // the block classes whose letters and tags fit
+    int strip_letters = 0, strip_widest = 0;  // the pairs and bands the strips take (SweepArgs)
     int64_t dearest = 1;                  // the dearest single step: a substitution or a gap's first letter
     // Free ends (wave sweeps): the letters each end of each sequence may leave out (reference start, end, query
     // start, end), the phase a run is in (1 the forward phase finding cost and end, 2 the anchored phase keeping
@@ -262,13 +242,15 @@ struct dinara_batch {
     double sweep_work[EDIT_BINS] = {}, trace_work[EDIT_BINS] = {};  // word-columns swept by each bin
     bool stats_pending = false;  // the unit path's device counters of the last run, read when first asked for
     int64_t stats_slots = 0;
-    // The whole-matrix path (full.hip) for pairs the band sweeps leave unsettled: whether any pair is long enough
+    // The whole-matrix path (strip.hip) for pairs the band sweeps leave unsettled: whether any pair is long enough
     // to need it (-1 not worked out yet), and the last run's count and time.
     int may_need_full = -1;
     bool whole = false;  // every pair takes the whole-matrix path, no band sweep (for checking and comparison)
     double full_pairs = 0, full_ms = 0;
-    DeviceBuffer full_list, full_count, full_decisions, full_carry, full_claim, full_slots, full_strips,
-        full_decision_at, full_carry_at;
+    DeviceBuffer full_list, full_count;
+    // The strip launches' plan (pairs, then the order their strips are claimed in) and memory, and the slots filed for
+    // strip bands (two sets taking turns, as the retry lists).
+    DeviceBuffer strip_plan, strip_counts, strip_best, strip_carry, strip_decisions, strip_retries;
 };
 
 namespace {
@@ -276,6 +258,12 @@ namespace {
 int64_t unit_lists(dinara_batch *b);
 int64_t unit_buffers(dinara_batch *b, const std::vector<int32_t> &lists, const std::vector<int32_t> &counts,
                      size_t cap);
+
+// The class of a slot's first band of `need` diagonals.
+int first_class(const dinara_batch *b, int64_t s, int need) {
+    return band_class(need, (int64_t)b->rows[s] + b->cols[s], b->user_band, b->group_max_letters, b->strip_letters,
+                      b->strip_widest);
+}
 
 // Builds the tape: pairs by length, longest first, 64 to a group, each group's words transposed.
 int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qrys) {
@@ -436,10 +424,14 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
             b->group_max_letters = std::max(b->group_max_letters, b->rows[s] + b->cols[s]);
     b->group_letters = (b->group_max_letters + 128 + 16 + 3) & ~3;
     // The group sweep holds costs times 16 with a tag (group.hip) and runs up to half its widest band past the
-    // corner: every value it makes stays under 2^30.
-    // The group and block sweeps hold one gap piece: two-piece batches take the wave sweeps alone.
-    b->groups_fit = !b->parsed.two_piece && !b->free_ends && group_cap > 0 && (size_t)4 * b->group_letters <= b->lds_limit &&
-                    ((int64_t)b->group_max_letters + 2 * 256 + 8) * b->dearest < REAL_LIMIT;
+    // corner: every value it makes stays under 2^30. It holds one gap piece and no free ends.
+    if (b->parsed.two_piece || b->free_ends || group_cap <= 0 || (size_t)4 * b->group_letters > b->lds_limit ||
+        ((int64_t)b->group_max_letters + 2 * 256 + 8) * b->dearest >= REAL_LIMIT)
+        b->group_max_letters = 0;
+    // The strips take bands of pairs up to 65,536 letters, free ends' up to 2,048 diagonals; longer pairs and wider
+    // bands are swept whole after the run.
+    b->strip_letters = 65536;
+    b->strip_widest = b->free_ends ? 2048 : band_width(CLASSES - 1);
     // Packed 16-bit group cells (group.hip) for shifted costs (equal extensions e) whose mismatch is no dearer than
     // two extension letters: a tagged value then lies in [-16 e (n + m), 32 opening + 15] and a cell no path
     // reaches stays above `top` - 16 e (n + m), so both fit 16 bits, apart, while 16 e (n + m) + 32 opening + 15
@@ -450,17 +442,11 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         const CostParams &k = b->costs;
         const int64_t e = k.del_ext, opening = std::max(k.del_open, k.ins_open);
         const int64_t top = (32767 - 16 * opening - 32) & ~int64_t(15);
-        if (b->groups_fit && !std::getenv("DINARA_GROUP_CELLS32") && k.pieces != 2 && k.del_ext == k.ins_ext &&
+        if (b->group_max_letters > 0 && !std::getenv("DINARA_GROUP_CELLS32") && k.pieces != 2 && k.del_ext == k.ins_ext &&
             e >= 0 && k.mismatch >= 0 && k.mismatch <= 2 * e && std::min(k.del_open, k.ins_open) >= 0 &&
             16 * e * b->group_max_letters + 32 * opening + 15 < top - 64 && (size_t)8 * b->group_letters <= b->lds_limit)
             b->group16_top = (int)top;
     }
-    b->block_mask = 0;
-    for (int cls = CLASS_BLOCK_FIRST; cls < CLASSES && !b->parsed.two_piece && !b->free_ends; ++cls)
-        if (block_letters(b->max_letters, cls) <= b->lds_limit &&
-            ((int64_t)b->max_letters + class_width(cls) + 8) * b->dearest < REAL_LIMIT &&
-            !(block_s(cls) > 8 && b->kind == DINARA_BATCH_ALIGNMENTS))  // the widest keep no decisions
-            b->block_mask |= 1 << (cls - CLASS_BLOCK_FIRST);
     // The first band: the lanes' start and end diagonals and one either side (lanes.mojo:1207-1215), within the
     // user band; swept at no less than the initial width, centred.
     b->first_low.resize(slots);
@@ -492,11 +478,9 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         }
         b->first_low[s] = lo;
         b->first_high[s] = hi;
-        const int need = std::max(hi - lo + 1, b->initial_width);
-        const int cls = first_class_for(need, b->groups_fit && n + m <= b->group_max_letters, b->block_mask,
-                                        b->user_band);
-        // A pair whose start and end diagonals lie further apart than the widest band is left unswept: its
-        // status stays unsettled and it reports DINARA_OUT_OF_MEMORY.
+        // A pair whose start and end diagonals lie further apart than the widest band is left unswept (its status
+        // stays unsettled).
+        const int cls = first_class(b, s, std::max(hi - lo + 1, b->initial_width));
         if (cls != CLASS_TOO_WIDE) b->first_lists[cls].push_back((int32_t)s);
         // A walk's moves, 2 bits each in 64-bit words; the CIGAR text, at most two bytes a move.
         b->scratch_base[s] = scratch;
@@ -545,6 +529,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         !b->walk_class.reserve(std::max<int64_t>(slots, 1) * 4) ||
         !b->retry_lists.reserve((size_t)2 * CLASSES * std::max<int64_t>(slots, 1) * 4) ||
         !b->retry_counts.reserve(2 * CLASSES * 4) ||
+        !b->strip_retries.reserve((size_t)2 * std::max<int64_t>(slots, 1) * sizeof(int4)) ||
         !b->first_lists_d.upload(ctx, first_all.data(), std::max<size_t>(first_all.size(), 1) * 4) ||
         !b->walk_flags.reserve(std::max<int64_t>(slots, 1) * 8))
         return DINARA_OUT_OF_MEMORY;
@@ -589,10 +574,10 @@ SweepArgs sweep_args(dinara_batch *b) {
     a.walk_flags = static_cast<uint64_t *>(b->walk_flags.ptr);
     a.group_letters = b->group_letters;
     a.doubling = b->doubling ? 1 : 0;
-    a.groups_fit = b->groups_fit;
     a.group_max_letters = b->group_max_letters;
     a.group16_top = b->group16_top;
-    a.block_mask = b->block_mask;
+    a.strip_letters = b->strip_letters;
+    a.strip_widest = b->strip_widest;
     a.cigar_scratch = static_cast<char *>(b->cigar_scratch.ptr);
     a.cigar_scratch_base = static_cast<const int64_t *>(b->cigar_scratch_base.ptr);
     a.cigars = static_cast<char *>(b->cigars.ptr);
@@ -620,20 +605,16 @@ SweepArgs sweep_args(dinara_batch *b) {
 }
 
 
-// Launches class `cls` over `count` slots listed at `list` (device memory), filing retries into `retry_lists` /
-// `retry_counts`. Each launch keeps its decisions in an arena of its own, a fixed stride a listed pair, until the
+// Launches class `cls` over `count` slots listed at `list` (device memory), filing retries where `round` says. Each
+// launch keeps its decisions in an arena of its own, a fixed stride a listed pair, until the
 // walk; a launch whose arena would pass the budget is cut in pieces. `arena_index` counts the run's arenas.
-int64_t launch_class(dinara_batch *b, int cls, const int32_t *list, int64_t count, int32_t *retry_lists,
-                     int32_t *retry_counts, size_t &arena_index) {
-    DeviceContext *ctx = b->ctx;
-    SweepArgs a = sweep_args(b);
+int64_t launch_class(dinara_batch *b, const SweepArgs &round, int cls, const int32_t *list, int64_t count,
+                     size_t &arena_index, hipStream_t stream) {
+    SweepArgs a = round;
     a.cls = cls;
-    a.retry_lists = retry_lists;
-    a.retry_counts = retry_counts;
     const bool wave = class_is_wave(cls);
-    const size_t lds = wave                     ? (size_t)std::min<int>(std::max(b->max_letters, 4), (int)b->lds_limit)
-                       : band_is_block(cls) ? block_letters(b->max_letters, cls)
-                                            : (size_t)(b->group16_top > 0 && cls >= 1 ? 8 : 4) * b->group_letters;
+    const size_t lds = wave ? (size_t)std::min<int>(std::max(b->max_letters, 4), (int)b->lds_limit)
+                            : (size_t)(b->group16_top > 0 && cls >= 1 ? 8 : 4) * b->group_letters;
     int64_t chunk = count;
     size_t stride = 0;
     if (a.record) {
@@ -654,11 +635,129 @@ int64_t launch_class(dinara_batch *b, int cls, const int32_t *list, int64_t coun
             a.arena = static_cast<uint8_t *>(arena->ptr);
             a.arena_stride = (int64_t)stride;
         }
-        launch_sweep(a, lds, ctx->stream);
+        launch_sweep(a, lds, stream);
         if (hipGetLastError() != hipSuccess) return DINARA_OUT_OF_MEMORY;
         b->launches += 1;
         b->class_launches[cls] += 1;
         b->class_pairs[cls] += a.count;
+    }
+    return 0;
+}
+
+// The columns a lane of a pair's strips holds: the fewest that take its columns in one strip, for a short query; for
+// a longer one, eight (half the strips and pipeline starts of four, and less of a row step spent outside the cells).
+int strip_c(int64_t m) { return m <= strip_columns(2) ? 2 : m <= strip_columns(4) ? 4 : 8; }
+
+// A strip launch's parts: consecutive pairs of the plan whose decisions fit the budget together.
+struct StripPart {
+    size_t pair, pairs, strip, strips;
+    size_t decision_bytes, carry_words;
+};
+struct StripPlan {
+    std::vector<StripPair> pairs;
+    std::vector<int2> order;
+    std::vector<StripPart> parts;
+    size_t decision_bytes = 0, carry_words = 0;  // the largest part's
+};
+
+// The plan of the pairs listed in `bands` (slot, low, high): each pair's strips, where its records lie, and the order
+// its strips are claimed in: the strips furthest from their pair's end first, so that the longest pipelines start first
+// and a strip always follows the one to its left.
+StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bool record) {
+    StripPlan plan;
+    const int pieces = b->costs.pieces == 2 ? 2 : 1;
+    const bool views = b->free_ends;
+    std::vector<size_t> at;
+    for (size_t next = 0; next < bands.size();) {
+        StripPart part{plan.pairs.size(), 0, plan.order.size(), 0, 0, 0};
+        int most = 0;
+        for (; next < bands.size(); ++next) {
+            const int4 &band = bands[next];
+            const int64_t n = views && b->phase == 2 ? b->b_rows_h[band.x] : b->rows[band.x];
+            const int64_t m = views && b->phase == 2 ? b->b_cols_h[band.x] : b->cols[band.x];
+            StripPair p{};
+            p.slot = band.x;
+            p.lo = band.y;
+            p.hi = band.z;
+            p.c = strip_c(m);
+            p.strips = (int)std::max<int64_t>(1, (m + strip_columns(p.c) - 1) / strip_columns(p.c));
+            p.rows = (int)std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)p.hi - p.lo + strip_columns(p.c)));
+            const size_t records = (size_t)p.strips * p.rows * 64;
+            const size_t bytes = record ? (records * strip_record_bytes(p.c, pieces) + 255) & ~size_t(255) : 0;
+            if (part.pairs > 0 && part.decision_bytes + bytes > ARENA_BUDGET) break;
+            p.decision_at = (int64_t)part.decision_bytes;
+            p.carry_at = (int64_t)part.carry_words;
+            part.decision_bytes += bytes;
+            part.carry_words += p.strips > 1 ? (size_t)p.strips * p.rows * pieces : 0;
+            part.strips += p.strips;
+            ++part.pairs;
+            most = std::max(most, p.strips);
+            plan.pairs.push_back(p);
+        }
+        // By strips left to the pair's end, most first.
+        at.assign((size_t)most + 1, 0);
+        for (size_t i = 0; i < part.pairs; ++i)
+            for (int left = 1; left <= plan.pairs[part.pair + i].strips; ++left) ++at[most - left];
+        for (size_t k = 0, sum = 0; k < at.size(); ++k) {
+            const size_t here = at[k];
+            at[k] = sum;
+            sum += here;
+        }
+        plan.order.resize(part.strip + part.strips);
+        for (size_t i = 0; i < part.pairs; ++i) {
+            const int strips = plan.pairs[part.pair + i].strips;
+            for (int strip = 0; strip < strips; ++strip)
+                plan.order[part.strip + at[most - (strips - strip)]++] = make_int2((int)i, strip);
+        }
+        plan.decision_bytes = std::max(plan.decision_bytes, part.decision_bytes);
+        plan.carry_words = std::max(plan.carry_words, part.carry_words);
+        plan.parts.push_back(part);
+    }
+    return plan;
+}
+
+// The plan onto the device, and room for its launches. Waits for the main stream.
+int64_t upload_strips(dinara_batch *b, const StripPlan &plan) {
+    const size_t pairs = plan.pairs.size() * sizeof(StripPair), order = plan.order.size() * sizeof(int2);
+    std::vector<uint8_t> host(pairs + order);
+    std::memcpy(host.data(), plan.pairs.data(), pairs);
+    std::memcpy(host.data() + pairs, plan.order.data(), order);
+    size_t most = 0;
+    for (const StripPart &part : plan.parts) most = std::max(most, part.pairs);
+    if (!b->strip_plan.upload(b->ctx, host.data(), host.size()) || !b->strip_counts.reserve((2 * most + 1) * 4) ||
+        !b->strip_best.reserve(most * 8) || !b->strip_carry.reserve(std::max<size_t>(plan.carry_words, 1) * 8) ||
+        (plan.decision_bytes && !b->strip_decisions.reserve(plan.decision_bytes)))
+        return DINARA_OUT_OF_MEMORY;
+    return 0;
+}
+
+// The plan's launches on `stream`, each part's sweep and (when decisions are kept) its walks, filing unproven pairs
+// where `round` says; `whole`: the bands are whole matrices.
+int64_t launch_strips(dinara_batch *b, const SweepArgs &round, const StripPlan &plan, bool whole, hipStream_t stream) {
+    for (const StripPart &part : plan.parts) {
+        StripArgs a{};
+        a.s = round;
+        a.pairs = static_cast<const StripPair *>(b->strip_plan.ptr) + part.pair;
+        a.order = reinterpret_cast<const int2 *>(static_cast<const StripPair *>(b->strip_plan.ptr) + plan.pairs.size()) +
+                  part.strip;
+        a.count = (int)part.pairs;
+        a.strips = (int)part.strips;
+        a.whole = whole ? 1 : 0;
+        a.decisions = part.decision_bytes ? static_cast<uint8_t *>(b->strip_decisions.ptr) : nullptr;
+        a.carry = static_cast<unsigned long long *>(b->strip_carry.ptr);
+        a.claim = static_cast<int *>(b->strip_counts.ptr);
+        a.failed = a.claim + 1;
+        a.done = a.failed + part.pairs;
+        a.best = static_cast<unsigned long long *>(b->strip_best.ptr);
+        if (hipMemsetAsync(b->strip_counts.ptr, 0, (2 * part.pairs + 1) * 4, stream) != hipSuccess ||
+            (part.carry_words &&
+             hipMemsetAsync(b->strip_carry.ptr, 0, part.carry_words * 8, stream) != hipSuccess) ||
+            (b->free_ends && hipMemsetAsync(b->strip_best.ptr, 0xFF, part.pairs * 8, stream) != hipSuccess))
+            return DINARA_OUT_OF_MEMORY;
+        launch_strip_sweep(a, stream);
+        if (a.decisions) launch_strip_walk(a, stream);
+        if (hipPeekAtLastError() != hipSuccess) return DINARA_OUT_OF_MEMORY;
+        b->launches += 1;
     }
     return 0;
 }
@@ -844,6 +943,9 @@ ArenaNeed arena_need(const dinara_batch *b) {
     bound = std::min(std::max<size_t>(bound, size_t(1) << 20), most);
     return {std::min(bound, std::max<size_t>(likely, size_t(1) << 31)), bound};
 }
+
+// The streams a round of band sweeps runs on: the main one and three at its side, HIP's hardware queues by default.
+constexpr int SWEEP_STREAMS = 4;
 
 // Timing events of a run launched kernel by kernel: a pair for each bin's first sweep, retry sweep and tracing
 // sweep (the bins that share a launch share bin 0's pair), and for the walk.
@@ -1096,9 +1198,24 @@ int64_t run_unit(dinara_batch *b, bool trace) {
     return 0;
 }
 
+// A slot's first strip band: its start and end diagonals', widened to a strip's columns (a strip's rows are the band's
+// and its columns', so up to there a band is cheap), inside the matrix.
+int4 first_strip_band(const dinara_batch *b, int32_t s) {
+    const int n = b->rows[s], m = b->cols[s];
+    int lo = b->first_low[s], hi = b->first_high[s];
+    const int more = strip_columns(strip_c(m)) - (hi - lo + 1);
+    if (more > 0 && !b->free_ends) {
+        lo = std::max(lo - more / 2, -n);
+        hi = std::min(hi + more / 2, m);
+    }
+    return make_int4(s, lo, hi, 0);
+}
+
 // Sweeps every slot of the first lists until each is settled or left unsettled: want bands from first_low_d /
 // first_high_d, round 0 the first lists, each later round the lists the round before filed, kept on the device,
-// two sets taking turns. Only the counts come back to the host. Caller holds the device lock.
+// two sets taking turns. Only the counts come back to the host, and the pairs filed for strips, which the host plans.
+// A round's launches (the strips' and each other class's) run side by side: each lasts as long as its longest pair, and
+// one after another the classes of 2,000 uneven pairs took 149 ms. Caller holds the device lock.
 int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
     DeviceContext *ctx = b->ctx;
     const int64_t slots = (int64_t)b->slot_pair.size();
@@ -1110,46 +1227,99 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         hipMemsetAsync(b->status.ptr, 0xFF, slots * 4, ctx->stream) != hipSuccess)
         return DINARA_OUT_OF_MEMORY;
     int64_t counts[CLASSES] = {};
-    for (int c = 0; c < CLASSES; ++c) counts[c] = b->first_offset[c + 1] - b->first_offset[c];
+    for (int c = 0; c < CLASS_STRIP_FIRST; ++c) counts[c] = b->first_offset[c + 1] - b->first_offset[c];
+    std::vector<int4> strips;
+    for (int c = CLASS_STRIP_FIRST; c < CLASSES; ++c)
+        for (int32_t s : b->first_lists[c]) strips.push_back(first_strip_band(b, s));
     int32_t *lists = static_cast<int32_t *>(b->retry_lists.ptr);
     int32_t *count_d = static_cast<int32_t *>(b->retry_counts.ptr);
     const size_t capacity = (size_t)std::max<int64_t>(slots, 1);
+    const SweepArgs args = sweep_args(b);
     for (int round = 0; round < 64; ++round) {
-        int64_t pending = 0;
-        for (int c = 0; c < CLASSES; ++c) pending += counts[c];
+        int64_t pending = (int64_t)strips.size();
+        for (int c = 0; c < CLASS_STRIP_FIRST; ++c) pending += counts[c];
         if (pending == 0) break;
-        int32_t *out_lists = lists + (size_t)(round % 2) * CLASSES * capacity;
-        int32_t *out_counts = count_d + (round % 2) * CLASSES;
+        SweepArgs a = args;
+        a.retry_lists = lists + (size_t)(round % 2) * CLASSES * capacity;
+        a.retry_counts = count_d + (round % 2) * CLASSES;
+        a.strip_retries = static_cast<int4 *>(b->strip_retries.ptr) + (size_t)(round % 2) * capacity;
         const int32_t *in_lists = lists + (size_t)((round + 1) % 2) * CLASSES * capacity;
-        if (hipMemsetAsync(out_counts, 0, CLASSES * 4, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
+        StripPlan plan;
+        if (!strips.empty()) {
+            plan = plan_strips(b, strips, a.record != 0);
+            if (const int64_t code = upload_strips(b, plan)) return code;
+        }
+        if (hipMemsetAsync(a.retry_counts, 0, CLASSES * 4, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
         (void)hipEventRecord(ctx->sweep_start, ctx->stream);
-        for (int c = 0; c < CLASSES; ++c) {
+        // The launches in turn on the main stream and the side streams, the strips first.
+        (void)hipEventRecord(ctx->mark(0), ctx->stream);
+        int turn = 0;
+        bool forked[SWEEP_STREAMS] = {};
+        const auto next_stream = [&]() {
+            const int k = turn++ % SWEEP_STREAMS;
+            if (k == 0) return ctx->stream;
+            if (!forked[k]) (void)hipStreamWaitEvent(ctx->side(k - 1), ctx->mark(0), 0);
+            forked[k] = true;
+            return ctx->side(k - 1);
+        };
+        const auto timed = [&](int c, auto launch) -> int64_t {
+            hipStream_t stream = next_stream();
+            (void)hipEventRecord(ctx->event(2 * c), stream);
+            if (const int64_t code = launch(stream)) return code;
+            (void)hipEventRecord(ctx->event(2 * c + 1), stream);
+            return 0;
+        };
+        if (!strips.empty()) {
+            for (const int4 &band : strips) {
+                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, 0, 1, 1 << 20));
+                b->class_pairs[cls] += 1;
+            }
+            b->class_launches[CLASS_STRIP_FIRST] += 1;
+            if (const int64_t code = timed(CLASS_STRIP_FIRST, [&](hipStream_t stream) {
+                    return launch_strips(b, a, plan, false, stream);
+                }))
+                return code;
+        }
+        for (int c = CLASS_STRIP_FIRST - 1; c >= 0; --c) {
             if (counts[c] == 0) continue;
             const int32_t *list = round == 0 ? static_cast<const int32_t *>(b->first_lists_d.ptr) + b->first_offset[c]
                                              : in_lists + (size_t)c * capacity;
-            // Each class's launches between two events of their own, for the per-kernel time.
-            (void)hipEventRecord(ctx->event(2 * c), ctx->stream);
-            if (const int64_t code = launch_class(b, c, list, counts[c], out_lists, out_counts, arena_index))
+            if (const int64_t code = timed(c, [&](hipStream_t stream) {
+                    return launch_class(b, a, c, list, counts[c], arena_index, stream);
+                }))
                 return code;
-            (void)hipEventRecord(ctx->event(2 * c + 1), ctx->stream);
+        }
+        for (int k = 1; k < SWEEP_STREAMS; ++k) {
+            if (!forked[k]) continue;
+            (void)hipEventRecord(ctx->mark(k), ctx->side(k - 1));
+            (void)hipStreamWaitEvent(ctx->stream, ctx->mark(k), 0);
         }
         (void)hipEventRecord(ctx->sweep_stop, ctx->stream);
         int32_t filed[CLASSES];
-        if (hipMemcpyAsync(filed, out_counts, sizeof(filed), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+        if (hipMemcpyAsync(filed, a.retry_counts, sizeof(filed), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess)
             return DINARA_OUT_OF_MEMORY;
         float ms = 0;
         (void)hipEventElapsedTime(&ms, ctx->sweep_start, ctx->sweep_stop);
         b->sweep_ms += ms;
         int64_t retried = 0;
-        for (int c = 0; c < CLASSES; ++c) {
-            if (counts[c] > 0) {
+        for (int c = 0; c <= CLASS_STRIP_FIRST; ++c) {
+            if (c == CLASS_STRIP_FIRST ? !strips.empty() : counts[c] > 0) {
                 float class_ms = 0;
                 (void)hipEventElapsedTime(&class_ms, ctx->event(2 * c), ctx->event(2 * c + 1));
                 b->class_ms[c] += class_ms;
             }
             counts[c] = filed[c];
             retried += filed[c];
+        }
+        strips.resize((size_t)filed[CLASS_STRIP_FIRST]);
+        if (!strips.empty()) {
+            if (hipMemcpyAsync(strips.data(), a.strip_retries, strips.size() * sizeof(int4), hipMemcpyDeviceToHost,
+                               ctx->stream) != hipSuccess ||
+                hipStreamSynchronize(ctx->stream) != hipSuccess)
+                return DINARA_OUT_OF_MEMORY;
+            // Longest first (slots are): the launch's longest pipelines claim their strips first.
+            std::sort(strips.begin(), strips.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
         }
         if (round == 0 && b->phase <= 1) b->first_proven = (double)(slots - retried);
     }
@@ -1163,6 +1333,11 @@ int64_t free_phase_a(dinara_batch *b) {
     if (slots == 0) return 0;
     b->phase = 1;
     b->first_offset = b->a_first_offset;
+    b->first_low = b->a_first_low;
+    b->first_high = b->a_first_high;
+    for (int c = 0; c < CLASSES; ++c)
+        b->first_lists[c].assign(b->a_first_all.begin() + b->a_first_offset[c],
+                                 b->a_first_all.begin() + b->a_first_offset[c + 1]);
     if (!b->view_rows_d.write(ctx, b->a_rows.data(), slots * 4) || !b->view_cols_d.write(ctx, b->a_cols.data(), slots * 4) ||
         !b->view_ref_at_d.write(ctx, b->a_at.data(), slots * 4) || !b->view_qry_at_d.write(ctx, b->a_at.data(), slots * 4) ||
         !b->free_d.write(ctx, b->a_free.data(), slots * 16) ||
@@ -1229,7 +1404,7 @@ int64_t free_phase_b(dinara_batch *b) {
         while (l > -re && off(l - 1) < target) --l;
         b->first_low[s] = (int32_t)l;
         b->first_high[s] = (int32_t)h;
-        const int cls = first_class_for((int)(h - l + 1), false, 0, false);
+        const int cls = first_class(b, s, (int)(h - l + 1));
         if (cls != CLASS_TOO_WIDE) b->first_lists[cls].push_back((int32_t)s);
     }
     std::vector<int32_t> first_all;
@@ -1253,8 +1428,8 @@ int64_t free_phase_b(dinara_batch *b) {
 // The decision bytes one pair may take on the whole-matrix path: past it the pair stays unsettled.
 constexpr size_t FULL_BUDGET = size_t(16) << 30;
 
-// After a run, every pair the band sweeps left unsettled (wider than the widest band, or too many letters for the
-// kernels that stage them in LDS) is swept whole, one pair after another, and walked (full.hip); a pair under free
+// After a run, every pair the band sweeps left unsettled (wider than the widest band, or more letters than the strips
+// take in bands) is swept whole and walked (strip.hip); a pair under free
 // ends or a user band, or whose decisions pass FULL_BUDGET, stays unsettled. A batch none of
 // whose pairs could need it skips the pass; otherwise the unsettled slots are listed on the device and only their
 // count (and list) come back. Caller holds the device lock.
@@ -1272,12 +1447,12 @@ int64_t full_pass(dinara_batch *b) {
     }
     if (!b->may_need_full && !b->whole) return 0;
     const auto began = std::chrono::steady_clock::now();
-    if (!b->full_list.reserve((size_t)slots * 4) || !b->full_count.reserve(4) || !b->full_claim.reserve(8) ||
+    if (!b->full_list.reserve((size_t)slots * 4) || !b->full_count.reserve(4) ||
         hipMemsetAsync(b->full_count.ptr, 0, 4, ctx->stream) != hipSuccess)
         return DINARA_OUT_OF_MEMORY;
-    launch_full_collect(static_cast<const int32_t *>(b->status.ptr), (int)slots,
-                        static_cast<int32_t *>(b->full_list.ptr), static_cast<int32_t *>(b->full_count.ptr),
-                        ctx->stream);
+    launch_collect_unsettled(static_cast<const int32_t *>(b->status.ptr), (int)slots,
+                             static_cast<int32_t *>(b->full_list.ptr), static_cast<int32_t *>(b->full_count.ptr),
+                             ctx->stream);
     int32_t count = 0;
     if (hipPeekAtLastError() != hipSuccess || !b->full_count.read(ctx, &count, 4)) return DINARA_OUT_OF_MEMORY;
     if (count == 0) return 0;
@@ -1285,63 +1460,21 @@ int64_t full_pass(dinara_batch *b) {
     if (!b->full_list.read(ctx, list.data(), (size_t)count * 4)) return DINARA_OUT_OF_MEMORY;
     std::sort(list.begin(), list.end());
     const bool record = b->kind == DINARA_BATCH_ALIGNMENTS;
-    const int pieces = b->costs.pieces == 2 ? 2 : 1;
-    const size_t record_bytes = pieces == 2 ? 8 : 4;
-    // The listed pairs in launches of as many as fit FULL_BUDGET together (a pair past it alone stays unsettled).
-    size_t next = 0;
-    bool launched = false;
-    while (next < list.size()) {
-        // The buffers below are refilled (and may move) for each launch: the one before must be done with them.
-        if (launched && hipStreamSynchronize(ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
-        std::vector<int32_t> pair_slot, strip_first;
-        std::vector<int64_t> decision_at, carry_at;
-        int64_t strips = 0, records = 0, carry_words = 0;
-        for (; next < list.size(); ++next) {
-            const int32_t slot = list[next];
-            if (slot < 0 || slot >= slots) continue;
-            const int64_t n = b->rows[slot], m = b->cols[slot];
-            const int64_t own = std::max<int64_t>(1, (m + FULL_STRIP - 1) / FULL_STRIP);
-            const int64_t own_records = record ? own * n * 64 : 0;
-            if ((size_t)own_records * record_bytes > FULL_BUDGET) continue;
-            if (!pair_slot.empty() && (size_t)(records + own_records) * record_bytes > FULL_BUDGET) break;
-            pair_slot.push_back(slot);
-            strip_first.push_back((int32_t)strips);
-            decision_at.push_back(records);
-            carry_at.push_back(carry_words);
-            strips += own;
-            records += own_records;
-            carry_words += own * (n + 1) * pieces;
-        }
-        if (pair_slot.empty()) continue;
-        strip_first.push_back((int32_t)strips);
-        const int64_t count = (int64_t)pair_slot.size();
-        if ((record && !b->full_decisions.reserve((size_t)records * record_bytes)) ||
-            !b->full_carry.reserve((size_t)carry_words * 8) || !b->full_claim.reserve((size_t)(count + 1) * 4) ||
-            !b->full_slots.upload(ctx, pair_slot.data(), (size_t)count * 4) ||
-            !b->full_strips.upload(ctx, strip_first.data(), (size_t)(count + 1) * 4) ||
-            !b->full_decision_at.upload(ctx, decision_at.data(), (size_t)count * 8) ||
-            !b->full_carry_at.upload(ctx, carry_at.data(), (size_t)count * 8) ||
-            hipMemsetAsync(b->full_carry.ptr, 0, (size_t)carry_words * 8, ctx->stream) != hipSuccess ||
-            hipMemsetAsync(b->full_claim.ptr, 0, (size_t)(count + 1) * 4, ctx->stream) != hipSuccess)
-            return DINARA_OUT_OF_MEMORY;
-        FullArgs fa{};
-        fa.s = sweep_args(b);
-        fa.pairs = (int)count;
-        fa.pair_slot = static_cast<const int32_t *>(b->full_slots.ptr);
-        fa.strip_first = static_cast<const int32_t *>(b->full_strips.ptr);
-        fa.decision_at = static_cast<const int64_t *>(b->full_decision_at.ptr);
-        fa.carry_at = static_cast<const int64_t *>(b->full_carry_at.ptr);
-        fa.record = record ? 1 : 0;
-        fa.decisions = record ? b->full_decisions.ptr : nullptr;
-        fa.carry = static_cast<unsigned long long *>(b->full_carry.ptr);
-        fa.claim = static_cast<int *>(b->full_claim.ptr);
-        fa.failed = static_cast<int *>(b->full_claim.ptr) + 1;
-        launch_full_sweep(fa, (int)strips, ctx->stream);
-        if (record) launch_full_walk(fa, ctx->stream);
-        if (hipPeekAtLastError() != hipSuccess) return DINARA_OUT_OF_MEMORY;
-        b->full_pairs += (double)count;
-        launched = true;
+    const size_t record_bytes = b->costs.pieces == 2 ? 8 : 4;
+    std::vector<int4> bands;
+    for (const int32_t slot : list) {
+        if (slot < 0 || slot >= slots) continue;
+        const int64_t n = b->rows[slot], m = b->cols[slot];
+        const int64_t strips = std::max<int64_t>(1, (m + strip_columns(8) - 1) / strip_columns(8));
+        if (record && (size_t)(strips * n * 64) * record_bytes > FULL_BUDGET) continue;
+        bands.push_back(make_int4(slot, (int)-n, (int)m, 0));
     }
+    if (!bands.empty()) {
+        const StripPlan plan = plan_strips(b, bands, record);
+        if (const int64_t code = upload_strips(b, plan)) return code;
+        if (const int64_t code = launch_strips(b, sweep_args(b), plan, true, ctx->stream)) return code;
+    }
+    b->full_pairs = (double)bands.size();
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
     b->full_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - began).count();
     return 0;
@@ -1741,9 +1874,7 @@ int64_t seed_slots(dinara_batch *b, GuessOf guess_of) {
         }
         b->first_low[s] = lo;
         b->first_high[s] = hi;
-        const int need = std::max(hi - lo + 1, 32);
-        const int cls = first_class_for(need, b->groups_fit && n + m <= b->group_max_letters, b->block_mask,
-                                        b->user_band);
+        const int cls = first_class(b, s, std::max(hi - lo + 1, 32));
         if (cls != CLASS_TOO_WIDE) b->first_lists[cls].push_back((int32_t)s);
     }
     std::vector<int32_t> first_all;

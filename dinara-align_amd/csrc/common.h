@@ -42,44 +42,48 @@ struct Tape {
 };
 
 // The sweep classes: four sixteen-lane-group bands (32, 64, 128, 256 diagonals, group.hip); wave-per-pair bands of
-// 64Q (Q = 1..32, sweep.hip), which also take every pair under a user band; and block bands, one pair a block of G
-// waves with S diagonal pairs a lane, 128SG diagonals (group.hip): 512 to 16384, in steps of at most a third.
+// 64Q (Q = 1..32, sweep.hip) for every pair under a user band; and strip bands (strip.hip), 512 to 16384 diagonals by
+// width, which one launch a round takes together.
 constexpr int CLASS_GROUP32 = 0;
 constexpr int CLASS_GROUP256 = 3;
 constexpr int CLASS_WAVE_FIRST = 4;  // Q = 1, 2, 4, 8, 16, 32 for classes 4..9
 constexpr int CLASS_WAVE_LAST = 9;
-constexpr int CLASS_BLOCK_FIRST = 10;
-constexpr int BLOCK_CLASSES = 12;
-constexpr int CLASSES = CLASS_BLOCK_FIRST + BLOCK_CLASSES;
+constexpr int CLASS_STRIP_FIRST = 10;
+constexpr int STRIP_CLASSES = 12;
+constexpr int CLASSES = CLASS_STRIP_FIRST + STRIP_CLASSES;
 constexpr int CLASS_TOO_WIDE = -1;
 
-// A block class's diagonal pairs a lane (S) and waves (G), block class b = cls - CLASS_BLOCK_FIRST: 512 (4 x 1),
-// 1024 (8 x 1), 1536 (4 x 3), 2048 (8 x 2), 3072 (8 x 3), then 8 x 4..8 (4096..8192), 12288 (12 x 8), 16384 (16 x 8).
-__host__ __device__ constexpr int block_s(int cls) {
-    return (cls - CLASS_BLOCK_FIRST == 0 || cls - CLASS_BLOCK_FIRST == 2) ? 4
-           : cls - CLASS_BLOCK_FIRST == 10                              ? 12
-           : cls - CLASS_BLOCK_FIRST == 11                              ? 16
-                                                                        : 8;
-}
-__host__ __device__ constexpr int block_waves(int cls) {
-    return cls - CLASS_BLOCK_FIRST == 0   ? 1
-           : cls - CLASS_BLOCK_FIRST == 1 ? 1
-           : cls - CLASS_BLOCK_FIRST == 2 ? 3
-           : cls - CLASS_BLOCK_FIRST == 3 ? 2
-           : cls - CLASS_BLOCK_FIRST == 4 ? 3
-           : cls - CLASS_BLOCK_FIRST <= 9 ? cls - CLASS_BLOCK_FIRST - 1
-                                          : 8;
-}
-
-// The diagonals a class's band holds.
+// The diagonals a class's band holds (a strip class's at most: 512, 1024, 1536, 2048, 3072, 4096 .. 8192 in steps of
+// 1024, 12288, 16384).
 __host__ __device__ constexpr int band_width(int cls) {
-    return cls <= CLASS_GROUP256    ? 32 << cls
-           : cls <= CLASS_WAVE_LAST ? 64 << (cls - CLASS_WAVE_FIRST)
-                                    : 128 * block_s(cls) * block_waves(cls);
+    return cls <= CLASS_GROUP256      ? 32 << cls
+           : cls <= CLASS_WAVE_LAST   ? 64 << (cls - CLASS_WAVE_FIRST)
+           : cls < CLASS_STRIP_FIRST + 4 ? 512 * (cls - CLASS_STRIP_FIRST + 1)
+           : cls < CLASS_STRIP_FIRST + 10 ? 1024 * (cls - CLASS_STRIP_FIRST - 1)
+                                          : 4096 * (cls - CLASS_STRIP_FIRST - 7);
 }
 __host__ __device__ constexpr bool band_is_wave(int cls) { return cls >= CLASS_WAVE_FIRST && cls <= CLASS_WAVE_LAST; }
-__host__ __device__ constexpr bool band_is_block(int cls) { return cls >= CLASS_BLOCK_FIRST; }
+__host__ __device__ constexpr bool band_is_strip(int cls) { return cls >= CLASS_STRIP_FIRST; }
 
+// The class of band a pair of `letters` letters needing `need` diagonals takes: the narrowest that holds them. A group
+// band is placed on an even diagonal, so it holds one diagonal fewer than its width. Pairs under a user band take the
+// wave bands, which bar diagonals outside it; pairs longer than a group launch stages (`group_letters`, 0 where no
+// group takes the batch) the strips, up to `strip_letters` letters and bands `strip_widest` wide.
+__host__ __device__ inline int band_class(int need, int64_t letters, bool user_band, int group_letters,
+                                          int strip_letters, int strip_widest) {
+    if (user_band) {
+        for (int cls = CLASS_WAVE_FIRST; cls <= CLASS_WAVE_LAST; ++cls)
+            if (need <= band_width(cls)) return cls;
+        return CLASS_TOO_WIDE;
+    }
+    if (group_letters > 0 && letters <= group_letters)
+        for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
+            if (need < band_width(cls)) return cls;
+    if (letters <= strip_letters)
+        for (int cls = CLASS_STRIP_FIRST; cls < CLASSES; ++cls)
+            if (need <= band_width(cls) && band_width(cls) <= strip_widest) return cls;
+    return CLASS_TOO_WIDE;
+}
 
 // Everything a sweep launch reads and writes.
 struct SweepArgs {
@@ -111,11 +115,11 @@ struct SweepArgs {
     int64_t arena_stride;
     uint64_t *walk_flags;    // per slot: the address of its settled band's decisions
     int group_letters;       // LDS bytes a pair takes in a group launch (four pairs a block)
-    int groups_fit;          // 1 when four pairs' letters fit one block's LDS
-    int group_max_letters;   // the longest pair (both sequences) a group launch stages; longer pairs take blocks
+    int group_max_letters;   // the longest pair (both sequences) a group launch stages (0: none); longer take strips
     int group16_top;         // > 0: group launches of two slots a lane and more hold their steady cells as 16-bit
                              // halves, `group16_top` the unreachable value (letters then take 2 bytes each in LDS)
-    int block_mask;          // bit c - CLASS_BLOCK_FIRST: block class c's letters fit its LDS and its costs its tags
+    int strip_letters;       // the most letters (both sequences) of a pair the strips take in bands
+    int strip_widest;        // and the widest of those bands
     // CIGARs: each slot's scratch run of 2(n+m)+2 bytes from cigar_scratch_base, compacted into `cigars` at an
     // offset taken from `cigar_used`
     char *cigar_scratch;
@@ -128,7 +132,8 @@ struct SweepArgs {
     int32_t *retry_lists;  // CLASSES lists of `retry_capacity` slots each
     int32_t *retry_counts;
     int retry_capacity;
-    // Free ends (wave sweeps only). Each slot sweeps a view of its pair: view_rows reference letters from
+    int4 *strip_retries;   // the slots filed for strip bands (counted at CLASS_STRIP_FIRST): slot, low, high, 0
+    // Free ends (strip sweeps only). Each slot sweeps a view of its pair: view_rows reference letters from
     // view_ref_at and view_cols query letters from view_qry_at, read back to front when `view_reversed`; free[4 s ..
     // 4 s + 3] the letters it may leave out for nothing at the start and end of the view's reference, then at those
     // of its query. A settled slot's end cell (the least cost; ties to the highest diagonal, or the lowest with
@@ -147,6 +152,5 @@ bool class_is_wave(int cls);
 void launch_sweep(const SweepArgs &a, size_t lds, hipStream_t stream);
 void launch_walk(const SweepArgs &a, hipStream_t stream);
 void launch_group(int s, const SweepArgs &a, size_t lds, hipStream_t stream);
-void launch_block(int s, int waves, const SweepArgs &a, size_t lds, hipStream_t stream);
 
 }  // namespace dinara
