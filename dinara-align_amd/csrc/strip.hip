@@ -14,14 +14,16 @@
 // A strip's lane 0 takes its left neighbours from the last column of the strip to its left, which that strip's lane 63
 // writes to a carry record a row, with a relaxed agent-scope atomic store: the record's own nonzero value says it is
 // there, so no fence or flag is needed, and agent scope keeps it coherent across the XCDs' L2s. The reading wave
-// fetches 64 rows' records at once (lane i row s + i) every 64 steps, and lane 0 takes row s's with a readlane. So a
+// fetches 64 rows' records at once (lane i row s + i) every 64 steps, and lane 0 takes row s's with a readlane; column
+// 0's borders are made the same way. So a
 // pair's strips run as a pipeline over the whole chip, each 64 C + 128 rows or so behind the one to its left, and one
 // launch takes every pair of a round, whatever its band. Waves claim strips in the host's order, in which a strip
 // always follows the one to its left (which is then held by a running wave), the pairs with the most strips first (their
 // pipelines are the launch's longest chains); every wait gives up after STRIP_POLL_LIMIT polls.
 //
-// The reference's letters pass through a ring of four 256-letter chunks in LDS, as the Scoring sweep's long references
-// do; the lane's query letters sit in registers.
+// The reference's letters pass through a ring in LDS, 64 written every 64 steps and loaded 64 steps before that; the
+// lane's query letters sit in registers. Between refills a step is the cells, two DPP moves, the letter's read and the
+// stores: a pair of 20,000 letters is a chain of 25,000 steps, whose every instruction counts.
 //
 // One gap piece (ONE): values and decisions as the group sweep's (group.hip): with decisions kept, cost * 16 + a tag
 // whose minimum breaks ties the reference's way, a cell's nibble bits 3:2 (source + 3) mod 4 (source 0 two unequal
@@ -31,6 +33,8 @@
 // + L layer L extends into the cell. A lane's record of a row is its C cells, low first, at the pair's first decision +
 // ((strip * rows + r - the strip's first row) * 64 + lane) * strip_record_bytes.
 
+#include <type_traits>
+
 #include "bands.h"
 #include "strip.h"
 
@@ -38,9 +42,8 @@ namespace dinara {
 
 namespace {
 
-constexpr int RING_CHUNK = 256;  // letters a chunk: four a lane
-constexpr int RING_CHUNKS = 4;
-constexpr int RING_MASK = RING_CHUNK * RING_CHUNKS - 1;
+constexpr int SEGMENT = 64;     // steps between refills: of the ring of letters, and of the left neighbours
+constexpr int RING = 4 * SEGMENT;
 constexpr int TAG_INF = 1 << 30;  // unreachable: above every real tagged value, with room to add
 
 __device__ __forceinline__ int from_left_lane(int old, int v) {
@@ -65,28 +68,16 @@ __device__ __forceinline__ unsigned long long carry_record(int h, int i) {
 // The sequence letters a slot (or its view) sweeps.
 struct Letters {
     const uint32_t *ref, *qry;
-    int bits, per, n, m, ref_at, qry_at;
+    int bits, shift, n, m, ref_at, qry_at;  // a tape word holds 1 << shift letters
     uint32_t mask;
     bool back;
 
     __device__ uint32_t at(const uint32_t *words, int x) const {
-        return (words[(size_t)(x / per) * 64] >> (bits * (x % per))) & mask;
+        return (words[(size_t)(x >> shift) * 64] >> (bits * (x & ((1 << shift) - 1)))) & mask;
     }
     __device__ uint32_t query(int i) const { return at(qry, back ? qry_at + m - 1 - i : qry_at + i); }
-    // Four reference letters from `i` (a multiple of 4) on, a byte each (zero past the end).
-    __device__ uint32_t ref4(int i) const {
-        if (i >= n) return 0;
-        if (!back && ref_at == 0) {  // one tape word holds them
-            const uint32_t word = ref[(size_t)(i / per) * 64];
-            if (bits == 8) return word;
-            const uint32_t four = word >> (2 * (i & 15));
-            return (four & 3u) | ((four & 12u) << 6) | ((four & 48u) << 12) | ((four & 192u) << 18);
-        }
-        uint32_t w = 0;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            if (i + t < n) w |= at(ref, back ? ref_at + n - 1 - i - t : ref_at + i + t) << (8 * t);
-        return w;
+    __device__ uint32_t reference(int i) const {  // zero past the end
+        return i < n ? at(ref, back ? ref_at + n - 1 - i : ref_at + i) : 0u;
     }
 };
 
@@ -172,12 +163,11 @@ __device__ __forceinline__ int key_diagonal(unsigned long long key, int lowest_e
 // One strip. Returns false when a wait for the left strip gave up; else leaves in `ending` what it found.
 template <int C, int P, bool RECORD, bool SH, bool FREE>
 __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair &p, int pair, int strip,
-                                            uint32_t *ring_words, Ending &ending) {
+                                            uint8_t *ring, Ending &ending) {
     constexpr bool ONE = P == 1;
     constexpr bool TAGS = ONE && RECORD;
     constexpr int SCALE = TAGS ? 16 : 1;
     constexpr int FAR = ONE ? TAG_INF : INF;  // unreachable
-    const uint8_t *ring = reinterpret_cast<const uint8_t *>(ring_words);
     const int lane = threadIdx.x;
     const CostParams k = a.s.costs;
     const int slot = p.slot;
@@ -189,7 +179,7 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
         text.ref = a.s.tape.words + a.s.tape.group_base[group] + (slot & 63);
         text.qry = text.ref + (size_t)a.s.tape.group_ref_words[group] * 64;
         text.bits = a.s.tape.bits;
-        text.per = 32 / text.bits;
+        text.shift = text.bits == 2 ? 4 : 2;
         text.mask = (1u << text.bits) - 1;
         text.n = n;
         text.m = m;
@@ -237,36 +227,38 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
     unsigned long long *const carry = a.carry + p.carry_at;
     const unsigned long long *const left_carry = strip > 0 ? carry + (size_t)(strip - 1) * p.rows * P : nullptr;
     unsigned long long *const own_carry = last_strip ? nullptr : carry + (size_t)strip * p.rows * P;
-    unsigned long long fetched = 0, fetched2 = 0;  // lane i: the left strip's record, 64 rows at a time
-    // Waits for the left strip's records of row `row` (this lane's; none for a lane that wants none).
+    // The left neighbours of the segment's rows, lane t's that of its row t: H, and I as column c0 + 1 takes it.
+    int left_h = FAR, left_i = FAR, left_i2 = FAR;
+    // Those of row `row` (this lane's) from the left strip's records, waited for; unreachable where `want` is not set.
     const auto fetch = [&](int row, bool want) __attribute__((always_inline)) {
         const unsigned long long *from = left_carry + (size_t)(want ? row - left_first : 0) * P;
+        unsigned long long record = 0, record2 = 0;
         for (int polls = 0;; ++polls) {
             if (want) {
-                fetched = __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (P == 2) fetched2 = __hip_atomic_load(from + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                record = __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (P == 2) record2 = __hip_atomic_load(from + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            const bool missing = want && (fetched == 0 || (P == 2 && fetched2 == 0));
-            if (__ballot(missing) == 0) return true;
+            const bool missing = want && (record == 0 || (P == 2 && record2 == 0));
+            if (__ballot(missing) == 0) break;
             if (polls > STRIP_POLL_LIMIT) return false;
             __builtin_amdgcn_s_sleep(2);
         }
+        left_h = want ? uncarried((uint32_t)(record >> 32)) : FAR;
+        left_i = want ? uncarried((uint32_t)record) : FAR;
+        left_i2 = P == 2 && want ? uncarried((uint32_t)record2) : FAR;
+        return true;
     };
     if (left_carry && first > 1) {  // the cell above-left of the strip's first: on the band's highest diagonal
         if (!fetch(first - 1, true)) return false;
-        if (lane == 0) left_prev = uncarried((uint32_t)(fetched >> 32));
+        if (lane == 0) left_prev = left_h;
     }
 
-    // The ring: chunk x holds letters 256 x .. 256 x + 255 (row r's letter is r - 1). Lane j reads letter base + s - 1
-    // - j at step s; while lane 0 is in chunk x, chunks x - 1, x and x + 1 are held, and x + 2 waits in a register.
-    const int base = first - 1;
+    // The ring holds the letters of the segment's steps and the one before (row r's letter is r - 1; lane j reads letter
+    // first - 1 + s - j at step s = 0, 1, ...) and the next segment's; the one after's wait in a register.
     __syncthreads();
-    {
-        const int x = base / RING_CHUNK;
-        ring_words[(x & (RING_CHUNKS - 1)) * 64 + lane] = text.ref4(x * RING_CHUNK + 4 * lane);
-        ring_words[((x + 1) & (RING_CHUNKS - 1)) * 64 + lane] = text.ref4((x + 1) * RING_CHUNK + 4 * lane);
-    }
-    uint32_t pending = text.ref4((base / RING_CHUNK + 2) * RING_CHUNK + 4 * lane);
+    ring[(first - 1 + lane) & (RING - 1)] = (uint8_t)text.reference(first - 1 + lane);
+    ring[(first - 1 + SEGMENT + lane) & (RING - 1)] = (uint8_t)text.reference(first - 1 + SEGMENT + lane);
+    uint32_t pending = text.reference(first - 1 + 2 * SEGMENT + lane);
     __syncthreads();
 
     // Free ends: the least key of this lane's ends so far. Column m's lane and place, and the rows and columns that
@@ -286,43 +278,25 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
         if (lane == 0 && strip == 0 && end_col_from <= 0) consider(left_border(n), n, 0);
     }
     int corner = FAR;
-    uint8_t *const record_at =
-        RECORD ? a.decisions + p.decision_at +
-                     ((size_t)strip * p.rows * 64 + lane) * strip_record_bytes(C, P)
-               : nullptr;
+    // Decisions: a row's records are 64 lanes', and lane j is j rows behind lane 0: from the place of lane 63's, each
+    // lane's lies a fixed way on.
+    constexpr int BYTES = strip_record_bytes(C, P);
+    uint8_t *record_base =
+        RECORD ? a.decisions + p.decision_at + ((int64_t)strip * p.rows - 63) * (64 * BYTES) : nullptr;
+    const uint32_t record_off = (uint32_t)((63 - lane) * 64 + lane) * BYTES;
 
     const int rows = last - first + 1, steps = rows + 63;
-    uint32_t letter = ring[(base - lane) & RING_MASK];
-    for (int s = 1; s <= steps; ++s) {
-        const int at = base + s - 1;  // lane 0's letter
-        if ((at & (RING_CHUNK - 1)) == 0 && s > 1) {
-            const int x = at / RING_CHUNK;
-            ring_words[((x + 1) & (RING_CHUNKS - 1)) * 64 + lane] = pending;
-            pending = text.ref4((x + 2) * RING_CHUNK + 4 * lane);
-            __syncthreads();
-        }
-        if (left_carry && (s & 63) == 1 && s <= rows) {
-            const int row = first + s - 1 + lane;
-            if (!fetch(row, row <= left_last && row <= last)) return false;
-        }
-        const uint32_t next_letter = ring[(at + 1 - lane) & RING_MASK];
-        const int r = first + s - 1 - lane;
-        // Lane 0's left neighbours: column 0, or row first + s - 1 of the left strip's last column.
-        int lh, li, li2 = FAR;
-        if (left_carry) {
-            const int from = (s - 1) & 63;
-            lh = uncarried(__builtin_amdgcn_readlane((uint32_t)(fetched >> 32), from));
-            li = uncarried(__builtin_amdgcn_readlane((uint32_t)fetched, from));
-            if (P == 2) li2 = uncarried(__builtin_amdgcn_readlane((uint32_t)fetched2, from));
-            if (first + s - 1 > left_last) lh = li = li2 = FAR;
-        } else {
-            lh = left_border(first + s - 1);
-            li = ONE ? lh + open_i + ext_i : FAR;
-        }
-        lh = from_left_lane(lh, out_h);
-        li = from_left_lane(li, out_i);
-        if (P == 2) li2 = from_left_lane(li2, out_i2);
-        if (r >= first && r <= last) {
+    uint32_t letter = ring[(first - 1 - lane) & (RING - 1)];
+    // Step s (lane 0's row is first + s), t its place in the segment. EDGE: lanes may be above the strip's first row or
+    // below its last, and the last row's ends are looked at.
+    const auto step = [&](auto edge, int s, int t) __attribute__((always_inline)) {
+        constexpr bool EDGE = edge.value;
+        const uint32_t next_letter = ring[(first + s - lane) & (RING - 1)];
+        const int r = first + s - lane;
+        const int lh = from_left_lane(__builtin_amdgcn_readlane(left_h, t), out_h);
+        const int li = from_left_lane(__builtin_amdgcn_readlane(left_i, t), out_i);
+        const int li2 = P == 2 ? from_left_lane(__builtin_amdgcn_readlane(left_i2, t), out_i2) : FAR;
+        if (!EDGE || (r >= first && r <= last)) {
             int hl = lh, il = li, il2 = li2, hd = left_prev;
             uint32_t nibbles = 0;
             unsigned long long bytes = 0;
@@ -335,10 +309,10 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
                     const int sub = hd + (eq ? sub_eq : sub_ne);
                     const int dc = TAGS ? (D[i] & ~2) : D[i];
                     const int ic = TAGS ? (il & ~1) : il;
-                    const int t = min(sub, min(dc, ic));
-                    h = TAGS ? (t & ~15) : t;
+                    const int low = min(sub, min(dc, ic));
+                    h = TAGS ? (low & ~15) : low;
                     const int dn = min(h + open_d, dc) + ext_d, in = min(h + open_i, ic) + ext_i;
-                    if (TAGS) nibbles = __builtin_amdgcn_alignbit((uint32_t)((dn ^ in) + t), nibbles, 4);
+                    if (TAGS) nibbles = __builtin_amdgcn_alignbit((uint32_t)((dn ^ in) + low), nibbles, 4);
                     D[i] = dn;
                     il = in;
                 } else {
@@ -376,7 +350,7 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
             out_i2 = il2;
             left_prev = lh;
             if (RECORD) {
-                uint8_t *to = record_at + (size_t)(r - first) * 64 * strip_record_bytes(C, P);
+                uint8_t *to = record_base + record_off;
                 if constexpr (ONE) {
                     if constexpr (C == 8) *reinterpret_cast<uint32_t *>(to) = nibbles;
                     else if constexpr (C == 4) *reinterpret_cast<uint16_t *>(to) = (uint16_t)(nibbles >> 16);
@@ -388,7 +362,7 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
                 }
             }
             if (own_carry && lane == 63) {
-                unsigned long long *to = own_carry + (size_t)(r - first) * P;
+                unsigned long long *to = own_carry + (int64_t)(s - 63) * P;
                 __hip_atomic_store(to, carry_record(out_h, out_i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (P == 2)
                     __hip_atomic_store(to + 1, carry_record(0, out_i2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -400,17 +374,39 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
                     for (int i = 0; i < C; ++i) end = i == end_place ? H[i] : end;
                     if (end_place >= 0 && end_place < C) consider(end, r, m);
                 }
-                if (r == n) {
+                if (EDGE && r == n) {
 #pragma unroll
                     for (int i = 0; i < C; ++i)
                         if (c0 + i + 1 <= m && c0 + i + 1 >= end_col_from) consider(H[i], n, c0 + i + 1);
                 }
-            } else if (last_strip && r == n) {
+            } else if (EDGE && last_strip && r == n) {
 #pragma unroll
                 for (int i = 0; i < C; ++i) corner = i == end_place ? H[i] : corner;
             }
         }
+        if (RECORD) record_base += 64 * BYTES;
         letter = next_letter;
+    };
+    for (int s0 = 0; s0 < steps; s0 += SEGMENT) {
+        if (s0 > 0) {
+            ring[(first - 1 + s0 + SEGMENT + lane) & (RING - 1)] = (uint8_t)pending;
+            pending = text.reference(first - 1 + s0 + 2 * SEGMENT + lane);
+            __syncthreads();
+        }
+        const int row = first + s0 + lane;
+        if (!left_carry) {
+            left_h = left_border(row);
+            left_i = ONE ? left_h + open_i + ext_i : FAR;
+        } else if (!fetch(row, row <= left_last && row <= last)) {
+            return false;
+        }
+        if (s0 > 0 && s0 + SEGMENT < rows) {
+#pragma unroll 2
+            for (int t = 0; t < SEGMENT; ++t) step(std::false_type(), s0 + t, t);
+        } else {
+            const int here = steps - s0 < SEGMENT ? steps - s0 : SEGMENT;
+            for (int t = 0; t < here; ++t) step(std::true_type(), s0 + t, t);
+        }
     }
 
     if (!FREE) {
@@ -442,7 +438,7 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
 
 template <int P, bool RECORD, bool SH, bool FREE>
 __global__ __launch_bounds__(64) void strip_sweep(StripArgs a) {
-    __shared__ uint32_t ring_words[RING_CHUNK * RING_CHUNKS / 4];
+    __shared__ uint8_t ring[RING];
     for (;;) {
         // The wave comes together before it claims. Without this the compiler joined "lane 0 settles the pair", at a
         // strip's end, to "lane 0 claims", here, and sent the other lanes round again without lane 0, to sweep strip 0
@@ -459,9 +455,9 @@ __global__ __launch_bounds__(64) void strip_sweep(StripArgs a) {
         bool swept;
         Ending ending;
         switch (p.c) {
-            case 2: swept = sweep_strip<2, P, RECORD, SH, FREE>(a, p, pair, strip, ring_words, ending); break;
-            case 4: swept = sweep_strip<4, P, RECORD, SH, FREE>(a, p, pair, strip, ring_words, ending); break;
-            default: swept = sweep_strip<8, P, RECORD, SH, FREE>(a, p, pair, strip, ring_words, ending); break;
+            case 2: swept = sweep_strip<2, P, RECORD, SH, FREE>(a, p, pair, strip, ring, ending); break;
+            case 4: swept = sweep_strip<4, P, RECORD, SH, FREE>(a, p, pair, strip, ring, ending); break;
+            default: swept = sweep_strip<8, P, RECORD, SH, FREE>(a, p, pair, strip, ring, ending); break;
         }
         if (!swept) {
             if (threadIdx.x == 0) atomicExch(a.failed + pair, 1);
