@@ -259,6 +259,11 @@ int64_t unit_lists(dinara_batch *b);
 int64_t unit_buffers(dinara_batch *b, const std::vector<int32_t> &lists, const std::vector<int32_t> &counts,
                      size_t cap);
 
+// Which of a batch's pairs take group bands (prepare): those up to GROUP_LETTERS letters, and of a batch of more pairs
+// than a launch needs for a wave on each SIMD (256 compute units of four, four pairs a wave) those no longer than its
+// GROUP_PAIRS-th longest.
+constexpr int64_t GROUP_PAIRS = 4096, GROUP_LETTERS = 4096;
+
 // The class of a slot's first band of `need` diagonals.
 int first_class(const dinara_batch *b, int64_t s, int need) {
     return band_class(need, (int64_t)b->rows[s] + b->cols[s], b->user_band, b->group_max_letters, b->strip_letters,
@@ -416,8 +421,18 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         b->max_letters = std::max<int>(b->max_letters, b->rows[s] + b->cols[s]);
     }
     // A group pair's LDS region: both sequences and room for reads up to half the widest group band (256) past
-    // the query's end (group.hip). Pairs up to a quarter of the LDS take group bands; longer ones take blocks.
-    const int group_cap = (int)(b->lds_limit / 4) - 128 - 16 - 4;
+    // the query's end (group.hip). Pairs up to a quarter of the LDS may take group bands. A group launch is four pairs
+    // a wave, each a chain over its anti-diagonals, so the batch's longest pairs, too few to give every SIMD a wave, are
+    // chains with nothing beside them: those past GROUP_LETTERS letters take the strips, whose chain is a row a step
+    // (361 pairs of up to 16,000 letters in 256 diagonals: 8.9 ms as groups; 2,000 uneven pairs whole: 14.5 ms, 11.1 with
+    // these in strips). Beyond that many pairs the groups' cells cost half as much.
+    int64_t group_cap = (int64_t)(b->lds_limit / 4) - 128 - 16 - 4;
+    {
+        const int64_t last = std::min<int64_t>(slots, GROUP_PAIRS) - 1;
+        group_cap = std::min(group_cap, std::max<int64_t>(GROUP_LETTERS, slots > GROUP_PAIRS
+                                                                             ? (int64_t)b->rows[last] + b->cols[last]
+                                                                             : 0));
+    }
     b->group_max_letters = 0;
     for (int64_t s = 0; s < slots; ++s)
         if (b->rows[s] + b->cols[s] <= group_cap)
