@@ -111,11 +111,12 @@ int64_t gap_run(const ParsedScoring &p, int64_t letters) {
     return letters == 0 ? 0 : p.open + (letters - 1) * (int64_t)p.extend;
 }
 
-// Columns a lane: a strip of at most 512 columns, the strips as even as C allows.
-int lane_columns(int cols) {
-    const int strips = std::max(1, (cols + SCORE_STRIP_MAX - 1) / SCORE_STRIP_MAX);
-    const int per_strip = (cols + strips - 1) / strips;
-    return std::min(SCORE_MAX_C, std::max(1, (per_strip + 63) / 64));
+// Whether a pair of a pass of `pairs` takes a quarter wave: it holds the pair and its staged reference, and the pass is
+// large enough that sharing a wave pays. Whole waves' chains are shorter (148 columns: 3 a lane rather than 10) but
+// there are four times as many. Scores of a pass, quarters against wholes: 256 pairs of 60 letters 14 to 16 us; of 148
+// letters 34 to 31 at 1,000 pairs, 37 to 44 at 1,500; of 240 residues 89 to 71 at 2,000, 89 to 93 at 3,000.
+bool takes_quarter(int64_t pairs, int64_t rows, int64_t cols) {
+    return cols <= SCORE_NARROW_COLS && rows + 4 <= SCORE_RING && cols * cols <= 16 * pairs;
 }
 
 // The last place `needle` occurs in `hay` (reference scoring.mojo:734-735, String.rfind over bytes).
@@ -151,8 +152,8 @@ struct dinara_scoring_batch {
     std::vector<char> cigars_h;
     int64_t max_rows = 0, max_cols = 0;
     // device memory
-    DeviceBuffer codes, ref_at, qry_at, view, list, table, score, end_row, end_col, target, walk_base, arena, carry,
-        op_scratch, op_base, cigars, cigar_used, cigar_offset, cigar_length;
+    DeviceBuffer codes, ref_at, qry_at, view, list, table, score, end_row, end_col, target, walk_base, walk_columns, arena,
+        arena_at, carry, carry_at, op_scratch, op_base, cigars, cigar_used, cigar_offset, cigar_length;
     // timing of the last run
     double run_ms = 0, pass_ms[4] = {0, 0, 0, 0}, walk_ms = 0;
     int launches = 0;
@@ -180,6 +181,7 @@ ScoreArgs score_args(Batch *b, int mode, int reversed) {
     a.end_col = static_cast<int32_t *>(b->end_col.ptr);
     a.target = static_cast<const int32_t *>(b->target.ptr);
     a.walk_base = static_cast<uint64_t *>(b->walk_base.ptr);
+    a.walk_columns = static_cast<int32_t *>(b->walk_columns.ptr);
     a.eqx = b->eqx;
     a.op_scratch = static_cast<char *>(b->op_scratch.ptr);
     a.op_base = static_cast<const int64_t *>(b->op_base.ptr);
@@ -191,15 +193,6 @@ ScoreArgs score_args(Batch *b, int mode, int reversed) {
     return a;
 }
 
-// One pass over the slots whose views are not empty: grouped by the columns a lane takes, each group one launch (or
-// more, when a trace's decisions pass the budget), each trace launch followed by its walk.
-// The reference letters a block can stage whole in LDS beside the profile; a longer reference goes through the
-// ring.
-int64_t lds_room(const Batch *b) {
-    const size_t profile = (size_t)b->scoring.letters * 64 * 8;
-    return b->ctx->lds_limit > profile ? (int64_t)(b->ctx->lds_limit - profile) : 0;
-}
-
 // The table's best score (at least 0).
 int top_score(const Batch *b) {
     int top = 0;
@@ -208,68 +201,100 @@ int top_score(const Batch *b) {
     return top;
 }
 
+// Whether scores may be held less `extend` a row and a column: the raised letters' scores still fit their bytes.
+bool extensions_free(const Batch *b) {
+    int top = -128;
+    for (int x = 0; x < b->scoring.letters; ++x)
+        for (int y = 0; y < b->scoring.letters; ++y) top = std::max<int>(top, b->scoring.table[x * 32 + y]);
+    return top - 2 * (int64_t)b->scoring.extend <= 127;
+}
+
+// One pass over the slots whose views are not empty: the pairs that take a whole wave in one launch, those that take a
+// quarter in another (or more, when a trace's decisions pass the budget), each trace launch followed by its walk.
 int64_t run_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &slots, hipEvent_t start,
                  hipEvent_t stop, double *pass_ms, double *walk_ms) {
     DeviceContext *ctx = b->ctx;
-    // Groups by the columns a lane takes and by whether the reference fits LDS whole (group g = c + ring * G).
-    constexpr int G = SCORE_MAX_C + 1;
-    const int64_t room = lds_room(b);
-    std::vector<int32_t> by_c[2 * G];
-    int64_t rows_max[2 * G] = {0}, cols_max[2 * G] = {0};
+    const int32_t *view = b->view_h.data();
+    const bool shifted = mode != SCORE_LOCAL && extensions_free(b);
+    auto rows_of = [&](int32_t s) { return (int64_t)view[4 * s + 1]; };
+    auto cols_of = [&](int32_t s) { return (int64_t)view[4 * s + 3]; };
+    const bool quarters = shifted && (mode == SCORE_GLOBAL || mode == SCORE_TRACE);
+    std::vector<int32_t> all, narrow;  // the whole-wave pairs, then the quarter-wave pairs
+    all.reserve(slots.size());
     for (int32_t s : slots) {
-        const int32_t rows = b->view_h[4 * s + 1], cols = b->view_h[4 * s + 3];
-        if (rows <= 0 || cols <= 0) continue;
-        const int g = lane_columns(cols) + (rows > room ? G : 0);
-        by_c[g].push_back(s);
-        rows_max[g] = std::max<int64_t>(rows_max[g], rows);
-        cols_max[g] = std::max<int64_t>(cols_max[g], cols);
+        if (rows_of(s) <= 0 || cols_of(s) <= 0) continue;
+        if (quarters && takes_quarter((int64_t)slots.size(), rows_of(s), cols_of(s))) narrow.push_back(s);
+        else all.push_back(s);
     }
-    std::vector<int32_t> all;
-    std::vector<size_t> at(2 * G, 0);
-    for (int g = 0; g < 2 * G; ++g) {
-        at[g] = all.size();
-        all.insert(all.end(), by_c[g].begin(), by_c[g].end());
-    }
+    const int64_t wide = (int64_t)all.size();
+    // Pairs that share a wave are of a size; whole views come sorted.
+    if (b->local)
+        std::stable_sort(narrow.begin(), narrow.end(),
+                         [&](int32_t x, int32_t y) { return rows_of(x) * cols_of(x) > rows_of(y) * cols_of(y); });
+    all.insert(all.end(), narrow.begin(), narrow.end());
     if (all.empty()) return 0;
     if (!b->list.upload(ctx, all.data(), all.size() * 4)) return failed("list upload");
-    const int32_t *list = static_cast<const int32_t *>(b->list.ptr);
     ScoreArgs a = score_args(b, mode, reversed);
+    a.shifted = shifted;
     hipEventRecord(start, ctx->stream);
-    for (int g = 0; g < 2 * G; ++g) {
-        const int64_t count = (int64_t)by_c[g].size();
-        if (count == 0) continue;
-        const int c = g % G;
-        a.c = c;
-        a.ring = g >= G;
-        const int strip_cols = 64 * c;
-        const int64_t strips = (cols_max[g] + strip_cols - 1) / strip_cols;
-        const size_t lds = score_lds(b->scoring.letters, (int)rows_max[g], a.ring != 0);
-        int64_t chunk = count;
-        if (mode == SCORE_TRACE) {
-            a.arena_stride = strips * (rows_max[g] + 1) * 64;
-            chunk = std::max<int64_t>(1, std::min<int64_t>(count, (int64_t)(ARENA_BUDGET / 4 / a.arena_stride)));
+    for (int kind = 0; kind < 2; ++kind) {
+        const int64_t begin = kind == 0 ? 0 : wide, end = kind == 0 ? wide : (int64_t)all.size();
+        if (begin == end) continue;
+        a.lanes = kind == 0 ? 64 : SCORE_NARROW;
+        const int64_t pairs = 64 / a.lanes, waves = (end - begin + pairs - 1) / pairs;
+        int64_t rows_max = 0;
+        for (int64_t i = begin; i < end; ++i) rows_max = std::max(rows_max, rows_of(all[i]));
+        a.ref_room = (int)std::min<int64_t>(SCORE_RING, (rows_max + 4 + 3) & ~int64_t(3));
+        // What the launch stages, and each wave's place among the decisions and the kept columns, by its largest pair.
+        size_t lds = 0;
+        int64_t best = 0, carry = 0, decisions = 0, most_decisions = 0;
+        std::vector<int64_t> carry_at, arena_at;
+        std::vector<int64_t> first_wave{0};  // of each launch
+        for (int64_t w = 0; w < waves; ++w) {
+            int64_t rows = 0, cols = 0;
+            for (int64_t i = begin + w * pairs; i < std::min(end, begin + (w + 1) * pairs); ++i) {
+                rows = std::max(rows, rows_of(all[i]));
+                cols = std::max(cols, cols_of(all[i]));
+                best = std::max(best, std::min(rows_of(all[i]), cols_of(all[i])));
+            }
+            lds = std::max(lds, score_lds(b->scoring.letters, a.lanes, (int)cols, a.ref_room));
+            const int64_t kept = score_carry(a.lanes, rows, cols);
+            if (kept > 0 && carry_at.empty()) carry_at.resize(waves, 0);
+            if (!carry_at.empty()) carry_at[w] = carry;
+            carry += kept;
+            if (mode == SCORE_TRACE) {
+                const int64_t words = score_decisions(a.lanes, rows, cols);
+                if (w > first_wave.back() && (decisions + words) * 4 > (int64_t)ARENA_BUDGET) {
+                    first_wave.push_back(w);
+                    decisions = 0;
+                }
+                arena_at.push_back(decisions);
+                decisions += words;
+                most_decisions = std::max(most_decisions, decisions);
+            }
         }
-        a.carry_stride = strips > 1 ? 2 * (rows_max[g] + 1) : 0;
+        first_wave.push_back(waves);
         // A local end's key: the rows' bits below a score no greater than the table's best times the shorter side.
         a.end_bits = 0;
         if (mode == SCORE_LOCAL) {
             int bits = 1;
-            while (bits < 31 && (int64_t(1) << bits) <= rows_max[g]) ++bits;
-            const int64_t best = (int64_t)top_score(b) * std::min(rows_max[g], cols_max[g]);
-            if (best < (int64_t(1) << (32 - bits))) a.end_bits = bits;
+            while (bits < 31 && (int64_t(1) << bits) <= rows_max) ++bits;
+            if ((int64_t)top_score(b) * best < (int64_t(1) << (32 - bits))) a.end_bits = bits;
         }
-        for (int64_t first = 0; first < count; first += chunk) {
-            a.list = list + at[g] + first;
-            a.count = (int)std::min(chunk, count - first);
-            a.carry = nullptr;
-            if (strips > 1) {
-                if (!b->carry.reserve((size_t)a.count * a.carry_stride * 4)) return failed("carry");
-                a.carry = static_cast<int32_t *>(b->carry.ptr);
-            }
-            if (mode == SCORE_TRACE) {
-                if (!b->arena.reserve((size_t)a.count * a.arena_stride * 4)) return failed("arena");
-                a.arena = static_cast<uint32_t *>(b->arena.ptr);
-            }
+        if (carry > 0 && (!b->carry.reserve((size_t)carry * 4) ||
+                          !b->carry_at.upload(ctx, carry_at.data(), carry_at.size() * 8)))
+            return failed("carry");
+        if (mode == SCORE_TRACE && (!b->arena.reserve((size_t)most_decisions * 4) ||
+                                    !b->arena_at.upload(ctx, arena_at.data(), arena_at.size() * 8)))
+            return failed("arena");
+        for (size_t l = 0; l + 1 < first_wave.size(); ++l) {
+            const int64_t from = begin + first_wave[l] * pairs;
+            a.list = static_cast<const int32_t *>(b->list.ptr) + from;
+            a.count = (int)(std::min(end, begin + first_wave[l + 1] * pairs) - from);
+            a.carry = static_cast<int32_t *>(b->carry.ptr);
+            a.carry_at = carry > 0 ? static_cast<const int64_t *>(b->carry_at.ptr) + first_wave[l] : nullptr;
+            a.arena = static_cast<uint32_t *>(b->arena.ptr);
+            a.arena_at = mode == SCORE_TRACE ? static_cast<const int64_t *>(b->arena_at.ptr) + first_wave[l] : nullptr;
             launch_score(a, lds, ctx->stream);
             if (hipPeekAtLastError() != hipSuccess) return failed("score launch");
             b->launches += 1;
@@ -278,6 +303,10 @@ int64_t run_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &s
                 if (hipPeekAtLastError() != hipSuccess) return failed("walk launch");
             }
         }
+        // The other kind's launch may move the buffers this one reads.
+        if (kind == 0 && wide < (int64_t)all.size() && (carry > 0 || mode == SCORE_TRACE) &&
+            hipStreamSynchronize(ctx->stream) != hipSuccess)
+            return failed("pass");
     }
     hipEventRecord(stop, ctx->stream);
     if (hipEventSynchronize(stop) != hipSuccess) return failed("pass");
@@ -361,7 +390,8 @@ int64_t prepare(Batch *b, const char *const *refs, const int64_t *ref_lens, cons
         !b->score.reserve(n4) || !b->end_row.reserve(n4) || !b->end_col.reserve(n4) || !b->target.reserve(n4))
         return DINARA_OUT_OF_MEMORY;
     if (b->kind == DINARA_BATCH_ALIGNMENTS) {
-        if (!b->walk_base.reserve(n4 * 2) || !b->op_base.upload(ctx, op_base.data(), op_base.size() * 8) ||
+        if (!b->walk_base.reserve(n4 * 2) || !b->walk_columns.reserve(n4) ||
+            !b->op_base.upload(ctx, op_base.data(), op_base.size() * 8) ||
             !b->op_scratch.reserve(std::max<int64_t>(ops, 8)) || !b->cigars.reserve(std::max<int64_t>(text, 1)) ||
             !b->cigar_used.reserve(8) || !b->cigar_offset.reserve(n4 * 2) || !b->cigar_length.reserve(n4))
             return DINARA_OUT_OF_MEMORY;

@@ -237,3 +237,30 @@ def test_tall_references_go_through_the_ring():
     # Local ends are kept as one key a column, score above a row of 17 bits here, while the scores fit the 15 bits
     # left; a match of 120 against a 600-letter query does not, and the ends are kept by compare and select.
     check_local(refs, qrys, da.Scoring.uniform(120, -4, -19, -1))
+
+
+def test_quarter_waves_equal_whole_waves():
+    # Batches of 4,096 pairs and more give all pairs of up to 256 columns and 1,020 rows a quarter of a wave each, where
+    # a letter's score raised by two extensions fits a byte; small batches take whole waves. Every columns-a-lane
+    # count and its edges, the rows' limit, waves whose four pairs differ, and a last wave that is not full.
+    rng = random.Random(53)
+    sizes = [(rng.randint(1, 40), rng.randint(1, 40)) for _ in range(3701)]
+    sizes += [(rng.randint(1, 300), 16 * c + d) for c in range(1, 17) for d in (-1, 0, 1) for _ in range(8)]
+    sizes += [(rows, cols) for rows in (1, 15, 16, 17, 1019, 1020, 1021, 1025) for cols in (1, 16, 255, 256, 257)]
+    for scoring in (DNA, REGIMES[0], da.Scoring.uniform(5, -4, -19, -100)):
+        refs, qrys = [], []
+        for rows, cols in sizes:
+            r = "".join(rng.choice("ACGT") for _ in range(rows))
+            refs.append(r)
+            qrys.append((mutated(r, 0.1, rng, "ACGT") + "".join(rng.choice("ACGT") for _ in range(cols)))[:cols])
+        assert len(refs) % 4 and len(refs) >= 4096
+        scores = da.scores(refs, qrys, scoring)
+        found = da.alignments(refs, qrys, scoring)
+        for at in range(0, len(refs), 50):  # the whole-wave path (past 28 columns), itself checked against the oracle above
+            part = slice(at, at + 50)
+            assert scores[part] == da.scores(refs[part], qrys[part], scoring)
+            assert found[part] == da.alignments(refs[part], qrys[part], scoring)
+        os_ = to_oracle(scoring)
+        for i in range(0, len(refs), 97):
+            want = o.scoring_global_align(refs[i], qrys[i], os_)
+            assert (found[i].score, found[i].cigar) == want and scores[i] == want[0], i
