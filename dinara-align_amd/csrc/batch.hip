@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <numeric>
+#include <optional>
 #include <thread>
 #include <vector>
 
@@ -163,6 +164,7 @@ struct dinara_batch {
     int initial_width = 32;
     std::vector<int64_t> code;            // per pair: 0 on the device, else its own result code
     std::vector<int64_t> reference_length, query_length;
+    std::vector<uint8_t> plain;           // per pair: 1 when its letters are A, C, G and T alone
     std::vector<int32_t> slot_pair;       // slot -> pair
     std::vector<int32_t> rows, cols;      // per slot
     std::vector<int32_t> first_low, first_high;
@@ -197,9 +199,11 @@ struct dinara_batch {
         first_high_d, cost, status, walk_low, walk_class, cigar_scratch, cigar_scratch_base, cigars, cigar_used,
         cigar_offset, cigar_length, retry_lists, retry_counts, first_lists_d, walk_flags, view_rows_d, view_cols_d,
         view_ref_at_d, view_qry_at_d, free_d, end_row_d, end_col_d;
+    Region region;  // what most of the buffers lie in
     ~dinara_batch() {
         for (DeviceBuffer *buffer : arenas) delete buffer;
         if (edit_graph) (void)hipGraphExecDestroy(edit_graph);
+        if (region.base) give_back(ctx, region);
     }
     // the last run's results, by slot
     std::vector<int32_t> cost_h, status_h, cigar_length_h;
@@ -277,10 +281,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     order.reserve(pairs);
     for (int64_t i = 0; i < pairs; ++i)
         if (b->code[i] == 0) order.push_back((int32_t)i);
-    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
-        return std::max(b->reference_length[x], b->query_length[x]) >
-               std::max(b->reference_length[y], b->query_length[y]);
-    });
+    longest_first(order, [&](int32_t p) { return (uint32_t)std::max(b->reference_length[p], b->query_length[p]); });
     const int64_t slots = (int64_t)order.size();
     b->slot_pair = order;
     b->first_offset.assign(CLASSES + 1, 0);
@@ -291,22 +292,14 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         b->rows[s] = (int32_t)b->reference_length[order[s]];
         b->cols[s] = (int32_t)b->query_length[order[s]];
     }
-    // One pass over every pair's letters: which of A, C, G, T it holds and whether it holds any other byte. Two
-    // bits a letter when every pair holds at most four distinct bytes (each pair its own codes: only equality
+    // Two bits a letter when every pair holds at most four distinct bytes (each pair its own codes: only equality
     // counts), else a byte a letter.
-    static const ByteClasses classes;
-    std::vector<uint8_t> plain(slots, 0);  // 1: the pair's letters are A, C, G and T alone
     std::atomic<bool> wide{false};
-    parallel_for(slots, b->threads, [&](int64_t lo, int64_t hi) {
+    const bool all_plain = std::all_of(order.begin(), order.end(), [&](int32_t p) { return b->plain[p] != 0; });
+    parallel_for(all_plain ? 0 : slots, b->threads, [&](int64_t lo, int64_t hi) {
         for (int64_t s = lo; s < hi; ++s) {
             const int32_t p = order[s];
-            const uint32_t seen = classes.seen(refs[p], b->reference_length[p]) |
-                                  classes.seen(qrys[p], b->query_length[p]);
-            if (!(seen & ByteClasses::OTHER)) {
-                plain[s] = 1;
-                continue;
-            }
-            if (wide.load(std::memory_order_relaxed)) continue;
+            if (b->plain[p] || wide.load(std::memory_order_relaxed)) continue;
             bool present[256] = {false};
             int distinct = 0;
             auto scan = [&](const char *text, int64_t len) {
@@ -362,10 +355,10 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
                 }
                 const int32_t p = order[s];
                 const int64_t n = b->reference_length[p], m = b->query_length[p];
-                if (b->bits == 2 && plain[s]) {
+                if (b->bits == 2 && b->plain[p]) {
                     // A, C, G and T are codes 0, 1, 2, 3 in every pair (the k-mer features read them so).
-                    classes.pack2(refs[p], n, reversed, ref_out, gref[g]);
-                    classes.pack2(qrys[p], m, reversed, qry_out, gqry[g]);
+                    Dna::pack2(refs[p], n, reversed, ref_out, gref[g]);
+                    Dna::pack2(qrys[p], m, reversed, qry_out, gqry[g]);
                     continue;
                 }
                 // Two-bit codes for a pair with other bytes: A, C, G and T keep 0, 1, 2, 3, any other byte the
@@ -513,6 +506,21 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     }
     b->first_offset[CLASSES] = (int64_t)first_all.size();
     if (first_all.empty()) first_all.push_back(0);  // every pair too wide: the device list still needs room
+    // The batch's buffers in one block, as far as it goes; what a run grows is allocated apart.
+    DeviceContext *ctx = b->ctx;
+    Carve carve;
+    std::optional<CarveScope> scope;
+    if (!CarveScope::active()) {
+        const size_t slot_bytes = 256 + 8 * CLASSES + (b->unit ? 20 * EDIT_BINS + 64 : 0) + (b->free_ends ? 48 : 0);
+        b->region = ctx->take_region((size_t)padded * 4 + slots * slot_bytes + scratch + text + (64 << 10));
+        if (b->region.base) {
+            carve.base = b->region.base;
+            carve.size = b->region.size;
+            carve.image = b->region.image;
+            carve.strict = false;
+            scope.emplace(&carve);
+        }
+    }
     if (b->free_ends) {
         // The forward phase's lists and bands, uploaded again at each run (the anchored phase writes its own).
         b->a_first_low = b->first_low;
@@ -530,7 +538,6 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     }
 
     // Upload.
-    DeviceContext *ctx = b->ctx;
     if (!b->tape.upload(ctx, tape.get(), (size_t)padded * 4) ||
         !b->group_base.upload(ctx, gbase.data(), gbase.size() * 8) ||
         !b->group_ref_words.upload(ctx, gref.data(), gref.size() * 4) ||
@@ -558,7 +565,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
             !b->cigar_length.reserve(std::max<int64_t>(slots, 1) * 4))
             return DINARA_OUT_OF_MEMORY;
     }
-    return 0;
+    return carve.flush(ctx) ? 0 : DINARA_OUT_OF_MEMORY;
 }
 
 SweepArgs sweep_args(dinara_batch *b) {
@@ -1561,6 +1568,56 @@ int64_t run(dinara_batch *b) {
     return full_pass(b);
 }
 
+// A small batch's results in one copy: everything of the region from the first of them to the last (up to 1 MiB, most
+// of it the CIGARs' room), rather than six copies waited for one after another.
+constexpr int64_t SMALL_FETCH = 256;
+
+int64_t fetch_at_once(dinara_batch *b) {
+    const int64_t slots = (int64_t)b->slot_pair.size();
+    const bool aligned = b->kind == DINARA_BATCH_ALIGNMENTS, ends = aligned && b->free_ends;
+    DeviceBuffer *wanted[] = {&b->cost, &b->status, ends ? &b->end_row_d : nullptr, ends ? &b->end_col_d : nullptr,
+                              aligned ? &b->cigar_used : nullptr, aligned ? &b->cigar_offset : nullptr,
+                              aligned ? &b->cigar_length : nullptr, aligned ? &b->cigars : nullptr};
+    const uint8_t *base = b->region.base;
+    const uint8_t *first = base + b->region.size, *last = base;
+    for (DeviceBuffer *buffer : wanted)
+        if (buffer && b->region.holds(buffer->ptr, buffer->size)) {
+            const uint8_t *at = static_cast<const uint8_t *>(buffer->ptr);
+            first = std::min(first, at);
+            last = std::max(last, at + buffer->size);
+        }
+    if (last > first && (hipMemcpyAsync(b->region.image + (first - base), first, last - first, hipMemcpyDeviceToHost,
+                                        b->ctx->stream) != hipSuccess ||
+                         hipStreamSynchronize(b->ctx->stream) != hipSuccess))
+        return DINARA_OUT_OF_MEMORY;
+    auto read = [&](DeviceBuffer &buffer, void *host, size_t bytes) {
+        if (bytes > buffer.size) return false;
+        if (!b->region.holds(buffer.ptr, buffer.size)) return buffer.read(b->ctx, host, bytes);
+        std::memcpy(host, b->region.image + (static_cast<uint8_t *>(buffer.ptr) - base), bytes);
+        return true;
+    };
+    if (!read(b->cost, b->cost_h.data(), slots * 4) || !read(b->status, b->status_h.data(), slots * 4))
+        return DINARA_OUT_OF_MEMORY;
+    if (ends) {
+        b->b_end_row_h.resize(slots);
+        b->b_end_col_h.resize(slots);
+        if (!read(b->end_row_d, b->b_end_row_h.data(), slots * 4) ||
+            !read(b->end_col_d, b->b_end_col_h.data(), slots * 4))
+            return DINARA_OUT_OF_MEMORY;
+    }
+    if (aligned) {
+        unsigned long long used = 0;
+        b->cigar_offset_h.resize(slots);
+        b->cigar_length_h.resize(slots);
+        if (!read(b->cigar_used, &used, 8) || !read(b->cigar_offset, b->cigar_offset_h.data(), slots * 8) ||
+            !read(b->cigar_length, b->cigar_length_h.data(), slots * 4))
+            return DINARA_OUT_OF_MEMORY;
+        b->cigars_h.resize(std::max<unsigned long long>(used, 1));
+        if (used > 0 && !read(b->cigars, b->cigars_h.data(), used)) return DINARA_OUT_OF_MEMORY;
+    }
+    return 0;
+}
+
 int64_t fetch(dinara_batch *b) {
     DeviceContext *ctx = b->ctx;
     std::lock_guard<std::mutex> serial(ctx->lock);
@@ -1569,6 +1626,7 @@ int64_t fetch(dinara_batch *b) {
     b->cost_h.resize(slots);
     b->status_h.resize(slots);
     if (slots == 0) return 0;
+    if (b->region.image && slots <= SMALL_FETCH) return fetch_at_once(b);
     if (!b->cost.read(ctx, b->cost_h.data(), slots * 4) || !b->status.read(ctx, b->status_h.data(), slots * 4))
         return DINARA_OUT_OF_MEMORY;
     if (b->free_ends && b->kind == DINARA_BATCH_ALIGNMENTS) {
@@ -1671,13 +1729,15 @@ dinara_batch *batch_new(int64_t gpu, int64_t kind, int64_t pairs, const char *co
         dearest = std::max(dearest, std::max(parsed.opening2 + parsed.extension2, parsed.del_opening2 + parsed.del_extension2));
     b->dearest = std::max<int64_t>(dearest, 1);
     b->code.assign(b->pairs, 0);
+    b->plain.assign(b->pairs, 0);
     b->reference_length.assign(b->pairs, 0);
     b->query_length.assign(b->pairs, 0);
     const bool capped = o.max_cost >= 0;
     parallel_for(b->pairs, threads, [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
             const int64_t n = ref_lens[i], m = qry_lens[i];
-            int64_t code = pair_code(refs[i], n, qrys[i], m);
+            b->plain[i] = n >= 0 && m >= 0 && Dna::plain(refs[i], n) && Dna::plain(qrys[i], m);
+            int64_t code = b->plain[i] ? 0 : pair_code(refs[i], n, qrys[i], m);
             if (code == 0) {
                 // Every cost the sweep holds stays well inside 32 bits.
                 if ((n + m + 4) * dearest >= REAL_LIMIT || n >= (int64_t(1) << 28) || m >= (int64_t(1) << 28))

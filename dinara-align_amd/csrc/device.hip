@@ -1,6 +1,8 @@
 // Device contexts and memory (see device.h).
 #include "device.h"
 
+#include <algorithm>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -98,9 +100,96 @@ void *Carve::take(size_t bytes) {
     return base + at;
 }
 
+bool Carve::flush(DeviceContext *ctx) {
+    const size_t bytes = gathered;
+    gathered = 0;
+    return bytes == 0 || hipMemcpyAsync(base, image, bytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess;
+}
+
+Region DeviceContext::take_region(size_t bytes) {
+    const bool small = bytes <= REGION_SMALL;
+    if (bytes > REGION_LARGE) return Region{};
+    {
+        std::lock_guard<std::mutex> hold(regions_lock);
+        std::vector<Region> &kept = small ? regions_small : regions_large;
+        size_t &out = small ? regions_small_out : regions_large_out;
+        if (out >= (small ? REGIONS_SMALL_OUT : REGIONS_LARGE_OUT)) return Region{};
+        ++out;
+        if (!kept.empty()) {
+            const Region region = kept.back();
+            kept.pop_back();
+            return region;
+        }
+    }
+    Region region;
+    region.size = small ? REGION_SMALL : REGION_LARGE;
+    if (hipMalloc(reinterpret_cast<void **>(&region.base), region.size) != hipSuccess) {
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> hold(regions_lock);
+        --(small ? regions_small_out : regions_large_out);
+        return Region{};
+    }
+    if (small && hipHostMalloc(reinterpret_cast<void **>(&region.image), region.size) != hipSuccess) {
+        (void)hipGetLastError();
+        region.image = nullptr;
+    }
+    return region;
+}
+
+static void free_region(const Region &region) {
+    (void)hipFree(region.base);
+    if (region.image) (void)hipHostFree(region.image);
+}
+
+void DeviceContext::give_region(const Region &region) {
+    {
+        std::lock_guard<std::mutex> hold(regions_lock);
+        const bool small = region.size == REGION_SMALL;
+        std::vector<Region> &kept = small ? regions_small : regions_large;
+        --(small ? regions_small_out : regions_large_out);
+        if (kept.size() < (small ? REGIONS_SMALL : REGIONS_LARGE)) {
+            kept.push_back(region);
+            return;
+        }
+    }
+    free_region(region);
+}
+
+void DeviceContext::drop_regions() {
+    std::vector<Region> dropped;
+    {
+        std::lock_guard<std::mutex> hold(regions_lock);
+        dropped.swap(regions_small);
+        dropped.insert(dropped.end(), regions_large.begin(), regions_large.end());
+        regions_large.clear();
+    }
+    for (const Region &region : dropped) free_region(region);
+}
+
+void give_back(DeviceContext *ctx, const Region &region) {
+    std::lock_guard<std::mutex> serial(ctx->lock);
+    DeviceGuard guard(ctx);
+    (void)hipDeviceSynchronize();
+    ctx->give_region(region);
+}
+
+// Frees what the current device's context keeps, for an allocation that found no memory.
+static void drop_kept_regions() {
+    int id = -1;
+    if (hipGetDevice(&id) != hipSuccess) return;
+    DeviceContext *ctx = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(contexts_mutex);
+        if (id >= 0 && id < (int)contexts.size()) ctx = contexts[id];
+    }
+    if (ctx) ctx->drop_regions();
+}
+
 CarveScope::CarveScope(Carve *carve) : previous(active_carve) { active_carve = carve; }
 
 CarveScope::~CarveScope() { active_carve = previous; }
+
+bool CarveScope::active() { return active_carve != nullptr; }
 
 DeviceBuffer::~DeviceBuffer() {
     if (ptr && !carved) (void)hipFree(ptr);
@@ -117,16 +206,21 @@ bool DeviceBuffer::reserve(size_t bytes) {
     if (bytes <= size && ptr) return true;
     release();
     if (Carve *carve = active_carve) {
-        // A call that may not allocate: the bytes come from its region, or the reservation fails.
         ptr = carve->take(bytes);
-        if (!ptr) return false;
-        carved = true;
-        size = bytes;
-        return true;
+        if (!ptr && carve->strict) return false;  // a call that may not allocate
+        if (ptr) {
+            carved = true;
+            size = bytes;
+            return true;
+        }
     }
     if (hipMalloc(&ptr, bytes) != hipSuccess) {
-        ptr = nullptr;
-        return false;
+        drop_kept_regions();
+        if (hipMalloc(&ptr, bytes) != hipSuccess) {
+            ptr = nullptr;
+            return false;
+        }
+        (void)hipGetLastError();  // the first try's
     }
     size = bytes;
     return true;
@@ -135,6 +229,12 @@ bool DeviceBuffer::reserve(size_t bytes) {
 bool DeviceBuffer::upload(DeviceContext *ctx, const void *host, size_t bytes) {
     if (!reserve(bytes < 4 ? 4 : bytes)) return false;
     if (bytes == 0) return true;
+    if (Carve *carve = active_carve; carve && carve->image && carved) {
+        const size_t at = static_cast<uint8_t *>(ptr) - carve->base;
+        std::memcpy(carve->image + at, host, bytes);
+        carve->gathered = std::max(carve->gathered, at + bytes);
+        return true;
+    }
     return hipMemcpyAsync(ptr, host, bytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
            hipStreamSynchronize(ctx->stream) == hipSuccess;
 }

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -120,16 +121,26 @@ bool takes_quarter(int64_t pairs, int64_t rows, int64_t cols) {
 }
 
 // The last place `needle` occurs in `hay` (reference scoring.mojo:734-735, String.rfind over bytes).
+// Eight bytes are compared before the call that compares them all.
 int64_t rfind(const char *hay, int64_t n, const char *needle, int64_t k) {
     if (k == 0) return 0;
-    for (int64_t at = n - k; at >= 0; --at)
-        if (std::memcmp(hay + at, needle, (size_t)k) == 0) return at;
+    uint64_t head = 0, there = 0;
+    if (k >= 8) std::memcpy(&head, needle, 8);
+    for (int64_t at = n - k; at >= 0; --at) {
+        if (k >= 8) std::memcpy(&there, hay + at, 8);
+        if (there == head && std::memcmp(hay + at, needle, (size_t)k) == 0) return at;
+    }
     return -1;
 }
 
 }  // namespace
 
 // ------------------------------------------------------------------ the batch
+
+struct ScoreLaunch {
+    ScoreArgs args;
+    size_t lds;
+};
 
 struct dinara_scoring_batch {
     int gpu = 0;
@@ -155,9 +166,16 @@ struct dinara_scoring_batch {
     DeviceBuffer codes, ref_at, qry_at, view, list, table, score, end_row, end_col, target, walk_base, walk_columns, arena,
         arena_at, carry, carry_at, op_scratch, op_base, cigars, cigar_used, cigar_offset, cigar_length;
     // timing of the last run
-    double run_ms = 0, pass_ms[4] = {0, 0, 0, 0}, walk_ms = 0;
+    double run_ms = 0, pass_ms[4] = {0, 0, 0, 0};
     int launches = 0;
     bool ran = false;
+    // A global batch's one pass, laid out by its first run: its views are its whole pairs, at every run the same.
+    bool planned = false;
+    std::vector<ScoreLaunch> plan;
+    Region region;  // what most of the buffers lie in
+    ~dinara_scoring_batch() {
+        if (region.base) give_back(ctx, region);
+    }
 };
 
 namespace {
@@ -209,15 +227,15 @@ bool extensions_free(const Batch *b) {
     return top - 2 * (int64_t)b->scoring.extend <= 127;
 }
 
-// One pass over the slots whose views are not empty: the pairs that take a whole wave in one launch, those that take a
-// quarter in another (or more, when a trace's decisions pass the budget), each trace launch followed by its walk.
-int64_t run_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &slots, hipEvent_t start,
-                 hipEvent_t stop, double *pass_ms, double *walk_ms) {
+// Lays one pass out over the slots whose views are not empty: the pairs that take a whole wave in one launch, those that
+// take a quarter in another (or more, when a trace's decisions pass the budget).
+int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &slots, std::vector<ScoreLaunch> &out) {
     DeviceContext *ctx = b->ctx;
     const int32_t *view = b->view_h.data();
     const bool shifted = mode != SCORE_LOCAL && extensions_free(b);
     auto rows_of = [&](int32_t s) { return (int64_t)view[4 * s + 1]; };
     auto cols_of = [&](int32_t s) { return (int64_t)view[4 * s + 3]; };
+    out.clear();
     const bool quarters = shifted && (mode == SCORE_GLOBAL || mode == SCORE_TRACE);
     std::vector<int32_t> all, narrow;  // the whole-wave pairs, then the quarter-wave pairs
     all.reserve(slots.size());
@@ -233,87 +251,96 @@ int64_t run_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &s
                          [&](int32_t x, int32_t y) { return rows_of(x) * cols_of(x) > rows_of(y) * cols_of(y); });
     all.insert(all.end(), narrow.begin(), narrow.end());
     if (all.empty()) return 0;
-    if (!b->list.upload(ctx, all.data(), all.size() * 4)) return failed("list upload");
-    ScoreArgs a = score_args(b, mode, reversed);
-    a.shifted = shifted;
-    hipEventRecord(start, ctx->stream);
+    // Each wave's place among the kept columns and its launch's decisions, by its largest pair.
+    std::vector<int64_t> carry_at, arena_at;
+    std::vector<size_t> first_wave;  // of each launch
+    std::vector<int64_t> first_pair;
+    int64_t carry = 0, decisions = 0, most_decisions = 0;
     for (int kind = 0; kind < 2; ++kind) {
         const int64_t begin = kind == 0 ? 0 : wide, end = kind == 0 ? wide : (int64_t)all.size();
         if (begin == end) continue;
+        ScoreArgs a = score_args(b, mode, reversed);
+        a.shifted = shifted;
         a.lanes = kind == 0 ? 64 : SCORE_NARROW;
-        const int64_t pairs = 64 / a.lanes, waves = (end - begin + pairs - 1) / pairs;
-        int64_t rows_max = 0;
-        for (int64_t i = begin; i < end; ++i) rows_max = std::max(rows_max, rows_of(all[i]));
-        a.ref_room = (int)std::min<int64_t>(SCORE_RING, (rows_max + 4 + 3) & ~int64_t(3));
-        // What the launch stages, and each wave's place among the decisions and the kept columns, by its largest pair.
-        size_t lds = 0;
-        int64_t best = 0, carry = 0, decisions = 0, most_decisions = 0;
-        std::vector<int64_t> carry_at, arena_at;
-        std::vector<int64_t> first_wave{0};  // of each launch
-        for (int64_t w = 0; w < waves; ++w) {
-            int64_t rows = 0, cols = 0;
-            for (int64_t i = begin + w * pairs; i < std::min(end, begin + (w + 1) * pairs); ++i) {
-                rows = std::max(rows, rows_of(all[i]));
-                cols = std::max(cols, cols_of(all[i]));
-                best = std::max(best, std::min(rows_of(all[i]), cols_of(all[i])));
-            }
-            lds = std::max(lds, score_lds(b->scoring.letters, a.lanes, (int)cols, a.ref_room));
-            const int64_t kept = score_carry(a.lanes, rows, cols);
-            if (kept > 0 && carry_at.empty()) carry_at.resize(waves, 0);
-            if (!carry_at.empty()) carry_at[w] = carry;
-            carry += kept;
-            if (mode == SCORE_TRACE) {
-                const int64_t words = score_decisions(a.lanes, rows, cols);
-                if (w > first_wave.back() && (decisions + words) * 4 > (int64_t)ARENA_BUDGET) {
-                    first_wave.push_back(w);
-                    decisions = 0;
-                }
-                arena_at.push_back(decisions);
-                decisions += words;
-                most_decisions = std::max(most_decisions, decisions);
-            }
+        const int64_t pairs = 64 / a.lanes;
+        int64_t rows_max = 0, shorter = 0;
+        for (int64_t i = begin; i < end; ++i) {
+            rows_max = std::max(rows_max, rows_of(all[i]));
+            shorter = std::max(shorter, std::min(rows_of(all[i]), cols_of(all[i])));
         }
-        first_wave.push_back(waves);
+        a.ref_room = (int)std::min<int64_t>(SCORE_RING, (rows_max + 4 + 3) & ~int64_t(3));
         // A local end's key: the rows' bits below a score no greater than the table's best times the shorter side.
-        a.end_bits = 0;
         if (mode == SCORE_LOCAL) {
             int bits = 1;
             while (bits < 31 && (int64_t(1) << bits) <= rows_max) ++bits;
-            if ((int64_t)top_score(b) * best < (int64_t(1) << (32 - bits))) a.end_bits = bits;
+            if ((int64_t)top_score(b) * shorter < (int64_t(1) << (32 - bits))) a.end_bits = bits;
         }
-        if (carry > 0 && (!b->carry.reserve((size_t)carry * 4) ||
-                          !b->carry_at.upload(ctx, carry_at.data(), carry_at.size() * 8)))
-            return failed("carry");
-        if (mode == SCORE_TRACE && (!b->arena.reserve((size_t)most_decisions * 4) ||
-                                    !b->arena_at.upload(ctx, arena_at.data(), arena_at.size() * 8)))
-            return failed("arena");
-        for (size_t l = 0; l + 1 < first_wave.size(); ++l) {
-            const int64_t from = begin + first_wave[l] * pairs;
-            a.list = static_cast<const int32_t *>(b->list.ptr) + from;
-            a.count = (int)(std::min(end, begin + first_wave[l + 1] * pairs) - from);
-            a.carry = static_cast<int32_t *>(b->carry.ptr);
-            a.carry_at = carry > 0 ? static_cast<const int64_t *>(b->carry_at.ptr) + first_wave[l] : nullptr;
-            a.arena = static_cast<uint32_t *>(b->arena.ptr);
-            a.arena_at = mode == SCORE_TRACE ? static_cast<const int64_t *>(b->arena_at.ptr) + first_wave[l] : nullptr;
-            launch_score(a, lds, ctx->stream);
-            if (hipPeekAtLastError() != hipSuccess) return failed("score launch");
-            b->launches += 1;
-            if (mode == SCORE_TRACE) {
-                launch_score_walk(a, ctx->stream);
-                if (hipPeekAtLastError() != hipSuccess) return failed("walk launch");
+        const size_t launches = out.size();
+        size_t lds = 0;
+        for (int64_t at = begin; at < end; at += pairs) {
+            int64_t rows = 0, cols = 0;
+            for (int64_t i = at; i < std::min(end, at + pairs); ++i) {
+                rows = std::max(rows, rows_of(all[i]));
+                cols = std::max(cols, cols_of(all[i]));
             }
+            lds = std::max(lds, score_lds(b->scoring.letters, a.lanes, (int)cols, a.ref_room));
+            const int64_t words = mode == SCORE_TRACE ? score_decisions(a.lanes, rows, cols) : 0;
+            if (at == begin || (decisions > 0 && (decisions + words) * 4 > (int64_t)ARENA_BUDGET)) {
+                decisions = 0;
+                out.push_back({a, 0});
+                first_wave.push_back(carry_at.size());
+                first_pair.push_back(at);
+            }
+            out.back().args.count += (int)(std::min(end, at + pairs) - at);
+            carry_at.push_back(carry);
+            carry += score_carry(a.lanes, rows, cols);
+            arena_at.push_back(decisions);
+            decisions += words;
+            most_decisions = std::max(most_decisions, decisions);
         }
-        // The other kind's launch may move the buffers this one reads.
-        if (kind == 0 && wide < (int64_t)all.size() && (carry > 0 || mode == SCORE_TRACE) &&
-            hipStreamSynchronize(ctx->stream) != hipSuccess)
-            return failed("pass");
+        for (size_t l = launches; l < out.size(); ++l) out[l].lds = lds;
+    }
+    if (!b->list.upload(ctx, all.data(), all.size() * 4)) return failed("list upload");
+    if (carry > 0 && (!b->carry.reserve((size_t)carry * 4) ||
+                      !b->carry_at.upload(ctx, carry_at.data(), carry_at.size() * 8)))
+        return failed("carry");
+    if (mode == SCORE_TRACE && (!b->arena.reserve((size_t)most_decisions * 4) ||
+                                !b->arena_at.upload(ctx, arena_at.data(), arena_at.size() * 8)))
+        return failed("arena");
+    for (size_t l = 0; l < out.size(); ++l) {
+        ScoreArgs &a = out[l].args;
+        a.list = static_cast<const int32_t *>(b->list.ptr) + first_pair[l];
+        if (carry > 0) {
+            a.carry = static_cast<int32_t *>(b->carry.ptr);
+            a.carry_at = static_cast<const int64_t *>(b->carry_at.ptr) + first_wave[l];
+        }
+        if (mode == SCORE_TRACE) {
+            a.arena = static_cast<uint32_t *>(b->arena.ptr);
+            a.arena_at = static_cast<const int64_t *>(b->arena_at.ptr) + first_wave[l];
+        }
+    }
+    return 0;
+}
+
+// One pass as planned, each trace launch followed by its walk.
+int64_t run_pass(Batch *b, const std::vector<ScoreLaunch> &plan, hipEvent_t start, hipEvent_t stop, double *pass_ms) {
+    DeviceContext *ctx = b->ctx;
+    if (plan.empty()) return 0;
+    hipEventRecord(start, ctx->stream);
+    for (const ScoreLaunch &launch : plan) {
+        launch_score(launch.args, launch.lds, ctx->stream);
+        if (hipPeekAtLastError() != hipSuccess) return failed("score launch");
+        b->launches += 1;
+        if (launch.args.mode == SCORE_TRACE) {
+            launch_score_walk(launch.args, ctx->stream);
+            if (hipPeekAtLastError() != hipSuccess) return failed("walk launch");
+        }
     }
     hipEventRecord(stop, ctx->stream);
     if (hipEventSynchronize(stop) != hipSuccess) return failed("pass");
     float ms = 0;
     hipEventElapsedTime(&ms, start, stop);
     *pass_ms += ms;
-    (void)walk_ms;
     return 0;
 }
 
@@ -383,6 +410,17 @@ int64_t prepare(Batch *b, const char *const *refs, const int64_t *ref_lens, cons
     });
     b->view_h.assign(4 * std::max<int64_t>(slots, 1), 0);
     const size_t n4 = (size_t)std::max<int64_t>(slots, 1) * 4;
+    // The batch's buffers in one block, as far as it goes; what a run needs besides is allocated apart.
+    Carve carve;
+    b->region = ctx->take_region(codes.size() + 24 * n4 + ops + text + (64 << 10));
+    std::optional<CarveScope> scope;
+    if (b->region.base) {
+        carve.base = b->region.base;
+        carve.size = b->region.size;
+        carve.image = b->region.image;
+        carve.strict = false;
+        scope.emplace(&carve);
+    }
     if (!b->codes.upload(ctx, codes.data(), codes.size()) ||
         !b->ref_at.upload(ctx, ref_at.data(), ref_at.size() * 8) ||
         !b->qry_at.upload(ctx, qry_at.data(), qry_at.size() * 8) ||
@@ -396,7 +434,7 @@ int64_t prepare(Batch *b, const char *const *refs, const int64_t *ref_lens, cons
             !b->cigar_used.reserve(8) || !b->cigar_offset.reserve(n4 * 2) || !b->cigar_length.reserve(n4))
             return DINARA_OUT_OF_MEMORY;
     }
-    return 0;
+    return carve.flush(ctx) ? 0 : DINARA_OUT_OF_MEMORY;
 }
 
 // Sets every slot's view: both sequences whole, forward.
@@ -421,7 +459,7 @@ int64_t run(Batch *b) {
     std::lock_guard<std::mutex> serial(ctx->lock);
     DeviceGuard guard(ctx);
     b->launches = 0;
-    b->run_ms = b->walk_ms = 0;
+    b->run_ms = 0;
     for (double &ms : b->pass_ms) ms = 0;
     const size_t slots = b->slot_pair.size();
     b->ran = true;
@@ -429,18 +467,24 @@ int64_t run(Batch *b) {
     (void)hipGetLastError();  // an earlier, unrelated call's error is not this run's
     hipEvent_t start = ctx->event(0), stop = ctx->event(1), begin = ctx->event(2), end = ctx->event(3);
     hipEventRecord(begin, ctx->stream);
-    std::vector<int32_t> all(slots);
-    for (size_t s = 0; s < slots; ++s) all[s] = (int32_t)s;
-    whole_views(b);
-    if (!b->view.write(ctx, b->view_h.data(), b->view_h.size() * 4)) return failed("views");
+    std::vector<int32_t> all;
+    if (!b->planned) {
+        all.resize(slots);
+        for (size_t s = 0; s < slots; ++s) all[s] = (int32_t)s;
+        whole_views(b);
+        if (!b->view.write(ctx, b->view_h.data(), b->view_h.size() * 4)) return failed("views");
+    }
     const bool align = b->kind == DINARA_BATCH_ALIGNMENTS;
     if (align) hipMemsetAsync(b->cigar_used.ptr, 0, 8, ctx->stream);
     int64_t code = 0;
     if (!b->local) {
-        code = run_pass(b, align ? SCORE_TRACE : SCORE_GLOBAL, 0, all, start, stop, &b->pass_ms[align ? 3 : 0],
-                        &b->walk_ms);
+        if (!b->planned) code = plan_pass(b, align ? SCORE_TRACE : SCORE_GLOBAL, 0, all, b->plan);
+        b->planned = code == 0;
+        if (code == 0) code = run_pass(b, b->plan, start, stop, &b->pass_ms[align ? 3 : 0]);
     } else {
-        code = run_pass(b, SCORE_LOCAL, 0, all, start, stop, &b->pass_ms[1], &b->walk_ms);
+        std::vector<ScoreLaunch> plan;
+        code = plan_pass(b, SCORE_LOCAL, 0, all, plan);
+        if (code == 0) code = run_pass(b, plan, start, stop, &b->pass_ms[1]);
         if (code == 0 && align) {
             // The reach back from every local end above zero, over both prefixes reversed (reference
             // vector_score.mojo:37-162), then the span between start and end aligned globally.
@@ -463,7 +507,8 @@ int64_t run(Batch *b) {
             if (!b->view.write(ctx, b->view_h.data(), b->view_h.size() * 4) ||
                 !b->target.write(ctx, b->score_h.data(), slots * 4))
                 return failed("reach views");
-            code = run_pass(b, SCORE_REACH, 1, reaching, start, stop, &b->pass_ms[2], &b->walk_ms);
+            code = plan_pass(b, SCORE_REACH, 1, reaching, plan);
+            if (code == 0) code = run_pass(b, plan, start, stop, &b->pass_ms[2]);
             if (code == 0) {
                 if (!read_slots(b, b->end_row, b->reach_row_h) || !read_slots(b, b->end_col, b->reach_col_h))
                     return failed("reach starts");
@@ -478,7 +523,8 @@ int64_t run(Batch *b) {
                     v[3] = ec - sc;
                 }
                 if (!b->view.write(ctx, b->view_h.data(), b->view_h.size() * 4)) return failed("trace views");
-                code = run_pass(b, SCORE_TRACE, 0, reaching, start, stop, &b->pass_ms[3], &b->walk_ms);
+                code = plan_pass(b, SCORE_TRACE, 0, reaching, plan);
+                if (code == 0) code = run_pass(b, plan, start, stop, &b->pass_ms[3]);
             }
         }
     }
@@ -541,6 +587,7 @@ Batch *batch_new(int64_t gpu, int64_t kind, int64_t pairs, const char *const *re
     int64_t code;
     {
         DeviceGuard guard(ctx);
+        std::lock_guard<std::mutex> serial(ctx->lock);
         code = prepare(b, refs, ref_lens, qrys, qry_lens);
     }
     if (code) {

@@ -73,3 +73,45 @@ def test_concurrent_calls_from_host_threads_match_calls_alone():
     print(f"[threads] {len(jobs)} batches at once done", flush=True)
     for i, (want, got) in enumerate(zip(alone, together)):
         assert got == want, i
+
+
+def test_batches_held_together_and_freed_out_of_order():
+    # Resident batches whose buffers lie in blocks a context hands out and takes back: more at once than it hands out
+    # (64 small, 4 large), run again, freed out of order, their blocks taken by batches of other sizes and costs, and a
+    # small batch's results in one copy (up to 256 pairs) or several. Each against the same call made alone.
+    h = _lib.lib()
+    affine = _lib.CCosts(4, 6, 2, -1, 0, 0, 0, -1, 0)
+    calls = [(*synthetic.affine_reads(pairs, seed=700 + k, length=length), costs)
+             for k, (pairs, length, costs) in enumerate([(2, 60, None), (256, 90, affine), (257, 60, None),
+                                                         (30, 400, affine), (6000, 100, affine)])]
+    alone = [alignments(refs, qrys, costs, 2)[1] for refs, qrys, costs in calls]
+    texts = [(_lib.Texts(refs), _lib.Texts(qrys)) for refs, qrys, _ in calls]
+
+    def make(k):
+        status = ctypes.c_int64(0)
+        costs = calls[k][2]
+        batch = h.dinara_batch_new(0, _lib.BATCH_ALIGNMENTS, len(calls[k][0]), *texts[k][0].args(),
+                                   *texts[k][1].args(), ctypes.byref(costs) if costs else None, None, None, 2,
+                                   ctypes.byref(status))
+        assert batch, status.value
+        return k, batch
+
+    def check(held):
+        k, batch = held
+        found = (_lib.CAlignment * len(calls[k][0]))()
+        statuses = (ctypes.c_int64 * len(calls[k][0]))()
+        assert h.dinara_batch_run(batch) == 0 and h.dinara_batch_alignments(batch, found, statuses) == 0
+        assert not any(statuses)
+        assert [(f.cost, ctypes.string_at(f.cigar, f.cigar_length)) for f in found] == alone[k], k
+        for f in found:
+            h.dinara_free(f.cigar)
+
+    held = [make(k % 4) for k in range(72)] + [make(4) for _ in range(6)]
+    for batch in held:
+        check(batch)
+    for at in list(range(0, len(held), 2)) + list(range(len(held) - 1, 0, -2)):
+        check(held[at])
+        h.dinara_batch_free(held[at][1])
+        again = make((at + 1) % 5)
+        check(again)
+        h.dinara_batch_free(again[1])
