@@ -263,6 +263,9 @@ int64_t unit_lists(dinara_batch *b);
 int64_t unit_buffers(dinara_batch *b, const std::vector<int32_t> &lists, const std::vector<int32_t> &counts,
                      size_t cap);
 
+// Letters' room a group pair stages besides its own (sweep_group): 132 before, 9 between and 131 past.
+constexpr int GROUP_ROOM = 272;
+
 // Which of a batch's pairs take group bands (prepare): those up to GROUP_LETTERS letters, and of a batch of more pairs
 // than a launch needs for a wave on each SIMD (256 compute units of four, four pairs a wave) those no longer than its
 // GROUP_PAIRS-th longest.
@@ -413,13 +416,13 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         b->max_rows = std::max(b->max_rows, b->rows[s]);
         b->max_letters = std::max<int>(b->max_letters, b->rows[s] + b->cols[s]);
     }
-    // A group pair's LDS region: both sequences and room for reads up to half the widest group band (256) past
-    // the query's end (group.hip). Pairs up to a quarter of the LDS may take group bands. A group launch is four pairs
-    // a wave, each a chain over its anti-diagonals, so the batch's longest pairs, too few to give every SIMD a wave, are
-    // chains with nothing beside them: those past GROUP_LETTERS letters take the strips, whose chain is a row a step
+    // A group pair's LDS region: both sequences, and room for reads up to half the widest group band (256) before the
+    // reference and past the query (group.hip). Pairs up to a quarter of the LDS may take group bands. A group launch
+    // is four pairs a wave, each a chain over its anti-diagonals, so the batch's longest pairs, too few to give every
+    // SIMD a wave, are chains with nothing beside them: those past GROUP_LETTERS letters take the strips, whose chain is a row a step
     // (361 pairs of up to 16,000 letters in 256 diagonals: 8.9 ms as groups; 2,000 uneven pairs whole: 14.5 ms, 11.1 with
     // these in strips). Beyond that many pairs the groups' cells cost half as much.
-    int64_t group_cap = (int64_t)(b->lds_limit / 4) - 128 - 16 - 4;
+    int64_t group_cap = (int64_t)(b->lds_limit / 4) - GROUP_ROOM - 4;
     {
         const int64_t last = std::min<int64_t>(slots, GROUP_PAIRS) - 1;
         group_cap = std::min(group_cap, std::max<int64_t>(GROUP_LETTERS, slots > GROUP_PAIRS
@@ -430,7 +433,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     for (int64_t s = 0; s < slots; ++s)
         if (b->rows[s] + b->cols[s] <= group_cap)
             b->group_max_letters = std::max(b->group_max_letters, b->rows[s] + b->cols[s]);
-    b->group_letters = (b->group_max_letters + 128 + 16 + 3) & ~3;
+    b->group_letters = (b->group_max_letters + GROUP_ROOM + 3) & ~3;
     // The group sweep holds costs times 16 with a tag (group.hip) and runs up to half its widest band past the
     // corner: every value it makes stays under 2^30. It holds one gap piece and no free ends.
     if (b->parsed.two_piece || b->free_ends || group_cap <= 0 || (size_t)4 * b->group_letters > b->lds_limit ||

@@ -54,8 +54,6 @@ struct GroupCosts {
     int sub_eq, sub_ne;  // H(r-1, c-1) to H(r, c): two equal letters (tag 3), two unequal (tag 0)
     int open_d, open_i;  // H to the next gap cell: the opening, tagged D opened / I opened
     int ext_d, ext_i;    // what a gap letter adds after the min (zero when shifted)
-    int row0, col0;      // the borders' step: H(0, c) = ins_open + c * row0, H(r, 0) = del_open + r * col0
-    int ins_open, del_open;
 };
 
 template <bool RECORD, bool SH>
@@ -68,10 +66,6 @@ __device__ __forceinline__ GroupCosts group_costs(const CostParams &k) {
     g.open_i = k.ins_open * 16 + (RECORD ? 9 : 0);
     g.ext_d = SH ? 0 : k.del_ext * 16;
     g.ext_i = SH ? 0 : k.ins_ext * 16;
-    g.row0 = SH ? 0 : k.ins_ext * 16;
-    g.col0 = SH ? 0 : k.del_ext * 16;
-    g.ins_open = k.ins_open * 16;
-    g.del_open = k.del_open * 16;
     return g;
 }
 
@@ -105,29 +99,6 @@ __device__ __forceinline__ void group_cell(const GroupCosts &g, bool eq, int hd,
     group_tail<RECORD, SH>(g, h, hc, dc, ic, dn, in, acc);
 }
 
-// The careful form: row 0 is an insertion of every column before, column 0 a deletion of every row, outside the
-// matrix unreachable; the letters are read clamped inside both sequences, STRIDE bytes apart. Also returns the
-// tagged H in `h`.
-template <bool RECORD, bool SH, int STRIDE = 1>
-__device__ __forceinline__ void careful_cell(const GroupCosts &g, int r, int c, const uint8_t *ref, const uint8_t *qry,
-                                             int last_ref, int last_qry, int hd, int dx, int ix, int &h, int &hc,
-                                             int &dn, int &in, uint32_t &acc) {
-    const int ri = min(max(r - 1, 0), last_ref), ci = min(max(c - 1, 0), last_qry);
-    const bool eq = ref[STRIDE * ri] == qry[STRIDE * ci];
-    const int sub = hd + (eq ? g.sub_eq : g.sub_ne);
-    const int dc = RECORD ? (dx & ~2) : dx;
-    const int ic = RECORD ? (ix & ~1) : ix;
-    h = min(sub, min(dc, ic));
-    if (r <= 0 || c <= 0) {
-        if (r < 0 || c < 0) h = TAG_INF;
-        else if (r == 0) h = c == 0 ? 0 : g.ins_open + c * g.row0;
-        else h = g.del_open + r * g.col0;
-    }
-    hc = RECORD ? (h & ~15) : h;
-    group_tail<RECORD, SH>(g, h, hc, dc, ic, dn, in, acc);
-    if (r < 0 || c < 0) dn = in = TAG_INF;
-}
-
 // A lane's state: per slot the clean H of its last cell (He/Ho), the D it handed the cell below (De/Do) and the
 // I it handed the cell to the right (Ie/Io), for the even and the odd diagonal of each pair; the DPP receivers
 // of the edge slots; the decisions of the current block of 8 anti-diagonals.
@@ -140,26 +111,17 @@ struct GroupState {
 };
 
 // Even anti-diagonal: even slot s's cell takes D from odd slot s (one diagonal up) and I from odd slot s - 1
-// (the lane below's last for slot 0, in from_lower_i, which the caller has shifted in). The careful form captures
-// the corner's tagged H when it is this cell.
-template <int S, bool RECORD, bool SH, bool CAREFUL, int STRIDE = 1>
-__device__ __forceinline__ void even_half(GroupState<S> &st, const GroupCosts &g, int t, int base_k,
-                                          const uint8_t *ref, const uint8_t *qry, int last_ref, int last_qry,
-                                          const uint8_t *rp, const uint8_t *qp, int first_q, int q_end, int tend,
-                                          int &corner) {
+// (the lane below's last for slot 0, in from_lower_i, which the caller has shifted in). `corner_slot` (CORNER): the slot
+// whose cell is the corner on this anti-diagonal, its H kept. Letters lie STRIDE bytes apart.
+template <int S, bool RECORD, bool SH, bool CORNER, int STRIDE = 1>
+__device__ __forceinline__ void even_half(GroupState<S> &st, const GroupCosts &g, const uint8_t *rp, const uint8_t *qp,
+                                          int corner_slot, int &corner) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int ix = s > 0 ? st.Io[s - 1] : st.from_lower_i;
         int hc, dn, in;
-        if (CAREFUL) {
-            const int kk = base_k + 2 * s, r = (t - kk) >> 1;
-            int h;
-            careful_cell<RECORD, SH, STRIDE>(g, r, r + kk, ref, qry, last_ref, last_qry, st.He[s], st.Do[s], ix, h,
-                                             hc, dn, in, st.acc[s]);
-            if (t == tend && first_q + s == q_end) corner = h;
-        } else {
-            group_cell<RECORD, SH>(g, rp[-s] == qp[s], st.He[s], st.Do[s], ix, hc, dn, in, st.acc[s]);
-        }
+        group_cell<RECORD, SH>(g, rp[-s * STRIDE] == qp[s * STRIDE], st.He[s], st.Do[s], ix, hc, dn, in, st.acc[s]);
+        if (CORNER && s == corner_slot) corner = hc;
         st.He[s] = hc;
         st.De[s] = dn;
         st.Ie[s] = in;
@@ -168,24 +130,16 @@ __device__ __forceinline__ void even_half(GroupState<S> &st, const GroupCosts &g
 
 // Odd anti-diagonal: odd slot s's cell takes D from even slot s + 1 (the lane above's first for the last slot, in
 // from_upper_d, which the caller has shifted in) and I from even slot s.
-template <int S, bool RECORD, bool SH, bool CAREFUL, int STRIDE = 1>
-__device__ __forceinline__ void odd_half(GroupState<S> &st, const GroupCosts &g, int t, int base_k,
-                                         const uint8_t *ref, const uint8_t *qry, int last_ref, int last_qry,
-                                         const uint8_t *rp, const uint8_t *qp, int first_q, int q_end, int tend,
-                                         int &corner) {
+template <int S, bool RECORD, bool SH, bool CORNER, int STRIDE = 1>
+__device__ __forceinline__ void odd_half(GroupState<S> &st, const GroupCosts &g, const uint8_t *rp, const uint8_t *qp,
+                                         int corner_slot, int &corner) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int dx = s + 1 < S ? st.De[s + 1] : st.from_upper_d;
         int hc, dn, in;
-        if (CAREFUL) {
-            const int kk = base_k + 2 * s + 1, r = (t - kk) >> 1;
-            int h;
-            careful_cell<RECORD, SH, STRIDE>(g, r, r + kk, ref, qry, last_ref, last_qry, st.Ho[s], dx, st.Ie[s], h,
-                                             hc, dn, in, st.acc[s]);
-            if (t == tend && first_q + s == q_end) corner = h;
-        } else {
-            group_cell<RECORD, SH>(g, rp[-s] == qp[s + 1], st.Ho[s], dx, st.Ie[s], hc, dn, in, st.acc[s]);
-        }
+        group_cell<RECORD, SH>(g, rp[-s * STRIDE] == qp[(s + 1) * STRIDE], st.Ho[s], dx, st.Ie[s], hc, dn, in,
+                               st.acc[s]);
+        if (CORNER && s == corner_slot) corner = hc;
         st.Ho[s] = hc;
         st.Do[s] = dn;
         st.Io[s] = in;
@@ -314,8 +268,8 @@ __device__ __forceinline__ void unpack_state(GroupState<S> &st, const PackedStat
 }
 
 // PACK: the steady anti-diagonals in packed cells (S >= 2, shifted). A pair's letters are then staged as 16-bit
-// positions, the reference's position i holding letters i and i - S/2, the query's i and i + S/2 (the careful
-// cells read the low bytes).
+// positions, the reference's position i holding letters i and i - S/2, the query's i and i + S/2 (32-bit cells read
+// the low bytes).
 template <int S, bool RECORD, bool SH, bool PACK>
 __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
     static_assert(!PACK || (SH && S >= 2 && S % 2 == 0), "packed cells: shifted sweeps of two slots or more");
@@ -336,11 +290,20 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
     const int end = m - n;
     const GroupCosts g = group_costs<RECORD, SH>(a.costs);
 
-    // A pair's region: its reference, its query, and room past the query for the steady state's reads, which run
-    // up to half a band past either sequence's end by the pair's last anti-diagonal. Packed: the reference's S/2
-    // positions past its end hold its last letters' second bytes.
-    uint8_t *ref = letters + (size_t)local * a.group_letters * STRIDE;
-    uint8_t *qry = ref + STRIDE * (n + (PACK ? P : 0));
+    // A pair's region: room before the reference for the cells above row 1 and left of column 1, the reference, the
+    // query, and room past it for reads up to half a band past either sequence's end by the pair's last anti-diagonal.
+    // The letters before each sequence's first differ. Packed: P positions past the reference's end hold its last
+    // letters' second bytes, P more and one the query's first.
+    uint8_t *ref = letters + ((size_t)local * a.group_letters + W / 2 + 4) * STRIDE;
+    uint8_t *qry = ref + STRIDE * (n + 2 * (PACK ? P : 0) + 1);
+    if (lane == 0) {
+        ref[-STRIDE] = 0xFE;
+        qry[-STRIDE] = 0xFF;
+        if (PACK) {
+            ref[STRIDE * (P - 1) + 1] = 0xFE;
+            qry[-STRIDE * (P + 1) + 1] = 0xFF;
+        }
+    }
     {
         const int group = slot >> 6, column = slot & 63;
         const uint32_t *ref_words = a.tape.words + a.tape.group_base[group] + column;
@@ -355,25 +318,19 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
         for (int i = lane; i < m; i += 16) {
             const uint8_t letter = (uint8_t)((qry_words[(size_t)(i / per) * 64] >> (bits * (i % per))) & mask);
             qry[STRIDE * i] = letter;
-            if (PACK && i >= P) qry[STRIDE * (i - P) + 1] = letter;
+            if (PACK) qry[STRIDE * (i - P) + 1] = letter;
         }
     }
     __syncthreads();
 
-    // Steps for the whole wave: to its longest pair's corner, the borders handled until every pair's band has
-    // left row 0 and column 0.
+    // Steps for the whole wave: to its longest pair's corner.
     const int tend = n + m;
     int tmax = tend, tmin = tend;
-    int careful_until = (k0 + W + 1) > (2 - k0) ? (k0 + W + 1) : (2 - k0);
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         tmax = max(tmax, __shfl_xor(tmax, d));
         tmin = min(tmin, __shfl_xor(tmin, d));
-        careful_until = max(careful_until, __shfl_xor(careful_until, d));
     }
-    // The steady loop starts on a block of 8 anti-diagonals once every pair's band has left the borders.
-    careful_until = (careful_until + 7) & ~7;
-    const int last_ref = n > 0 ? n - 1 : 0, last_qry = m > 0 ? m - 1 : 0;
     const int base_k = k0 + 2 * S * lane;  // this lane's lowest diagonal
     const int q_end = (end - k0) >> 1;     // the diagonal pair holding the corner
     const int first_q = S * lane;
@@ -386,6 +343,15 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
     }
     st.from_lower_i = TAG_INF;
     st.from_upper_d = TAG_INF;
+    // The borders take no care: with every value unreachable but the one above-left of (0, 0), which makes that cell 0
+    // (its letters, the ones before the first, differ), row 0 and column 0 come out as the gaps they are and the cells
+    // outside stay unreachable. Every band holds diagonal 0. A lane's border steps were 40 instructions a cell, checked
+    // and their letters clamped, over a band's first W / 2 anti-diagonals and the last few:
+    // 200,000 pairs of 148 letters in 64 diagonals, 0.59 ms so, 0.41 without (14 instructions an anti-diagonal for two
+    // cells a lane, the vector unit's rate).
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (base_k + 2 * s == 0) st.He[s] = -g.sub_ne;
 #pragma unroll
     for (int s = 0; s < S; ++s) st.done[s][0] = st.done[s][1] = st.done[s][2] = 0;
     int corner = TAG_INF;
@@ -415,23 +381,24 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
             }
         }
     };
-    auto careful_pair = [&](int t) __attribute__((always_inline)) {
+    // One even and one odd anti-diagonal in 32-bit cells, the corner kept where it is one of them. A pair past its own
+    // corner sweeps on with its letters' cursors held there; nothing reads what it makes.
+    auto last_pair = [&](int t) __attribute__((always_inline)) {
+        const int r0 = (min(t, tend & ~1) - base_k) >> 1, c0 = r0 + base_k;
+        const uint8_t *rp = ref + (r0 - 1) * STRIDE, *qp = qry + (c0 - 1) * STRIDE;
         st.from_lower_i = shift_from_lower(st.from_lower_i, st.Io[S - 1]);
-        even_half<S, RECORD, SH, true, STRIDE>(st, g, t, base_k, ref, qry, last_ref, last_qry, nullptr, nullptr,
-                                               first_q, q_end, tend, corner);
+        even_half<S, RECORD, SH, true, STRIDE>(st, g, rp, qp, t == tend ? q_end - first_q : -1, corner);
         st.from_upper_d = shift_from_upper(st.from_upper_d, st.De[0]);
-        odd_half<S, RECORD, SH, true, STRIDE>(st, g, t + 1, base_k, ref, qry, last_ref, last_qry, nullptr, nullptr,
-                                              first_q, q_end, tend, corner);
+        odd_half<S, RECORD, SH, true, STRIDE>(st, g, rp, qp, t + 1 == tend ? q_end - first_q : -1, corner);
         if (((t + 1) & 7) == 7) finish_block(t + 1);
     };
     int t = 0;
-    for (; t <= tmax && t < careful_until; t += 2) careful_pair(t);
     // Steady state: until the wave's first corner, blocks of 8 anti-diagonals, the letters from two cursors. On
     // even anti-diagonal t slot s reads reference letter r0 - 1 - s and query letter c0 - 1 + s (odd: c0 + s),
     // r0 and c0 the row and column of slot 0's even cell, both one more each anti-diagonal pair. Whole tiles run
     // four blocks at a time, their blocks' places known.
-    if (t <= tmax) {
-        int r0 = (t - base_k) >> 1, c0 = r0 + base_k;
+    if (tmin > 7) {
+        int r0 = -base_k >> 1, c0 = r0 + base_k;
         PackedState<S> ps;
         PackedCosts pk{};
         if constexpr (PACK) {
@@ -452,20 +419,14 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
                 } else {
                     const uint8_t *rp = ref + r0 - 1, *qp = qry + c0 - 1;
                     st.from_lower_i = shift_from_lower(st.from_lower_i, st.Io[S - 1]);
-                    even_half<S, RECORD, SH, false>(st, g, t, base_k, ref, qry, last_ref, last_qry, rp, qp, first_q,
-                                                    q_end, tend, corner);
+                    even_half<S, RECORD, SH, false>(st, g, rp, qp, -1, corner);
                     st.from_upper_d = shift_from_upper(st.from_upper_d, st.De[0]);
-                    odd_half<S, RECORD, SH, false>(st, g, t, base_k, ref, qry, last_ref, last_qry, rp, qp, first_q,
-                                                   q_end, tend, corner);
+                    odd_half<S, RECORD, SH, false>(st, g, rp, qp, -1, corner);
                 }
                 ++r0;
                 ++c0;
             }
         };
-        for (; t + 7 < tmin && (t & 31) != 0; t += 8) {
-            steady_block();
-            finish_block(t + 7);
-        }
         for (; t + 31 < tmin; t += 32) {
 #pragma unroll
             for (int b = 0; b < 3; ++b) {
@@ -482,8 +443,8 @@ __global__ __launch_bounds__(64) void sweep_group(SweepArgs a) {
         }
         if constexpr (PACK) unpack_state<S>(st, ps);
     }
-    // The tail: every pair's corner, with the borders' care.
-    for (; t <= tmax; t += 2) careful_pair(t);
+    // The tail: every pair's corner.
+    for (; t <= tmax; t += 2) last_pair(t);
     // The corner's tile, unless the wave went past it (then it was stored whole): a part-filled last block's
     // nibbles sit in the word's top, shifted down into place.
     const int last = t - 1, filled = (last & 7) + 1, place = (last >> 3) & 3;
