@@ -153,6 +153,22 @@ template <int BITS>
 using LetterSource = typename std::conditional<BITS == 2, Letters2, Cursor<BITS>>::type;
 
 
+// A function of three 64-bit words, bit by bit (v_bitop3 a half): F is its value over the words' own tables, TABLE_A,
+// TABLE_B and TABLE_C.
+constexpr uint32_t TABLE_A = 0xF0, TABLE_B = 0xCC, TABLE_C = 0xAA;
+template <uint32_t F>
+__device__ __forceinline__ uint64_t of_three(uint64_t a, uint64_t b, uint64_t c) {
+    const uint32_t lo = __builtin_amdgcn_bitop3_b32((uint32_t)a, (uint32_t)b, (uint32_t)c, F & 0xFFu);
+    const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(a >> 32), (uint32_t)(b >> 32), (uint32_t)(c >> 32), F & 0xFFu);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// A word shifted up one bit, its bit 0 taken from bit 31 of `below`.
+__device__ __forceinline__ uint64_t slide_up(uint64_t x, uint32_t below) {
+    const uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
+    return ((uint64_t)__builtin_amdgcn_alignbit(hi, lo, 31) << 32) | __builtin_amdgcn_alignbit(lo, below, 31);
+}
+
 // A plane of K 64-bit words shifted down one bit (bit i takes bit i + 1), each word's bit 63 taken from the next
 // word's bit 0 and the last word's from bit 0 of `incoming`: two alignbits a word.
 template <int K>
@@ -295,6 +311,9 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
     // the wave's line reads (eight lanes a line, one place each) fall in different banks with no padding: 32 KB a
     // workgroup, five to a compute unit.
     constexpr bool STAGED = RECORD && K == 1;
+    // Lines of eight columns unrolled: everywhere without decisions, else where a wave holds few pairs, whose chains are
+    // long (all eleven bins' lines with their stores would pass the instruction cache).
+    constexpr bool WHOLE = MODE == SWEEP || L >= 16;
     int t = 0;       // the wave's column steps so far (the same in every lane)
     int t0 = 0;      // the step count when the lane's pair was claimed
     // More words a lane: the last HOLD columns' decision planes in registers, oldest first.
@@ -352,6 +371,7 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
 #pragma unroll
                         for (int b = 0; b < BITS; ++b) pl[b][kk] = planes[b];
                     }
+                    if (L == 64) t = 0;  // one pair a wave: its lines start with it
                     bottom.begin(ref, -lo, t & 7);
                     query.begin(qry, 0, t & 7);
                     t0 = t;
@@ -497,11 +517,13 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
         // Every lane holds the same count: a scalar loop counter.
         steps = __builtin_amdgcn_readfirstlane(steps);
         const bool active = slot >= 0;
-        for (int step = 0; step < steps; ++step) {
-        // One column. The window moves down a row: each word takes the bit of the word below; the band's bottom
-        // takes +1 under it (Pv), and the new bottom row's letter.
+        // One column, at place PLACE of its line where that is known (below zero: not). The window moves down a row: each
+        // word takes the bit of the word below; the band's bottom takes +1 under it (Pv), and the new bottom row's
+        // letter.
+        auto column = [&](auto known) __attribute__((always_inline)) {
+        constexpr int PLACE = decltype(known)::value;
         ++j;
-        const int place = t & 7;  // this column's place in its line (every lane alike)
+        const int place = PLACE >= 0 ? PLACE : t & 7;  // every lane alike
         ++t;
         if constexpr (BITS == 2) {
             // Each plane slides down a row: its top word's bit 63 comes from bit 0 of the next lane's lowest word (one
@@ -512,12 +534,10 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
             uint32_t ip0 = L > 1 ? wave_neighbour<false>((uint32_t)pl[0][0]) : 0u;
             uint32_t ip1 = L > 1 ? wave_neighbour<false>((uint32_t)pl[1][0]) : 0u;
             const uint32_t code = bottom.next();  // every lane takes it; the band's bottom lane uses it
-            if (last_lane) {
-                ipv = 1u;
-                imv = 0u;
-                ip0 = code;
-                ip1 = code >> 1;
-            }
+            ipv = last_lane ? 1u : ipv;
+            imv = last_lane ? 0u : imv;
+            ip0 = last_lane ? code : ip0;
+            ip1 = last_lane ? code >> 1 : ip1;
             slide_down<K>(pv, ipv);
             slide_down<K>(mv, imv);
             slide_down<K>(pl[0], ip0);
@@ -539,16 +559,16 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
             bottom.refill();
             query.refill();
         }
-        uint64_t eq[K];
+        uint64_t differ[K];
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
-            uint64_t differ = 0;
+            differ[kk] = 0;
 #pragma unroll
             for (int b = 0; b < BITS; ++b) {
-                const uint32_t m = 0u - ((c >> b) & 1u);  // bit b of the letter, in every bit (both halves alike)
-                differ |= pl[b][kk] ^ (((uint64_t)m << 32) | m);
+                const uint32_t bit = 0u - ((c >> b) & 1u);  // bit b of the letter, in every bit (both halves alike)
+                const uint64_t m = ((uint64_t)bit << 32) | bit;
+                differ[kk] = b == 0 ? pl[b][kk] ^ m : of_three<(TABLE_A ^ TABLE_B) | TABLE_C>(pl[b][kk], m, differ[kk]);
             }
-            eq[kk] = ~differ;
         }
         // (Eq & Pv) + Pv over the pair's whole window: carries ripple through a lane's words, and across lanes by
         // generate / propagate ballots (a carry into lane t is bit t of (G + (G | P)) ^ P).
@@ -556,7 +576,7 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
         unsigned long long gen = 0, prop = 0;  // lanes whose words carry out, lanes whose words pass a carry on
         if constexpr (K == 1) {
             // One word: the ballots of the compares themselves, the groups' last lanes masked off in the scalar unit.
-            sum[0] = (eq[0] & pv[0]) + pv[0];
+            sum[0] = of_three<TABLE_A & ~TABLE_B>(pv[0], differ[0], 0) + pv[0];
             // The compares' lane masks (llvm.amdgcn.icmp, predicates 36 unsigned less, 32 equal).
             gen = __builtin_amdgcn_uicmpl(sum[0], pv[0], 36) & inner_lanes;
             prop = __builtin_amdgcn_uicmpl(sum[0], ~0ull, 32) & inner_lanes;
@@ -565,7 +585,7 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
             bool all_ones = true;
 #pragma unroll
             for (int kk = 0; kk < K; ++kk) {
-                const uint64_t x = (eq[kk] & pv[kk]) + pv[kk];
+                const uint64_t x = of_three<TABLE_A & ~TABLE_B>(pv[kk], differ[kk], 0) + pv[kk];
                 const uint32_t c1 = x < pv[kk];
                 sum[kk] = x + carry;
                 carry = c1 | (uint32_t)(carry && x == ~0ull);
@@ -576,38 +596,43 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
         }
         if constexpr (L > 1) {
             const unsigned long long into = (gen + (gen | prop)) ^ prop;
-            if ((into >> lane) & 1ull) {
-                uint32_t up = 1;
+            uint32_t up = __builtin_amdgcn_inverse_ballot_w64(into) ? 1u : 0u;
 #pragma unroll
-                for (int kk = 0; kk < K; ++kk) {
-                    sum[kk] += up;
-                    up = up && sum[kk] == 0;
-                }
+            for (int kk = 0; kk < K; ++kk) {
+                sum[kk] += up;
+                if (kk + 1 < K) up = up && sum[kk] == 0;
             }
         }
         uint64_t ph[K], mh[K], xv[K];
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
-            xv[kk] = eq[kk] | mv[kk];
-            const uint64_t xh = (sum[kk] ^ pv[kk]) | eq[kk];
-            ph[kk] = mv[kk] | ~(xh | pv[kk]);
+            xv[kk] = of_three<TABLE_A | ~TABLE_B>(mv[kk], differ[kk], 0);
+            const uint64_t xh = of_three<(TABLE_A ^ TABLE_B) | ~TABLE_C>(sum[kk], pv[kk], differ[kk]);
+            ph[kk] = of_three<TABLE_A | ~(TABLE_B | TABLE_C)>(mv[kk], xh, pv[kk]);
             mh[kk] = pv[kk] & xh;
         }
         // Horizontal differences one row down: a +1 carries into the band's top (the stand-in above it).
-        uint32_t carried = (uint32_t)(ph[K - 1] >> 63) | ((uint32_t)(mh[K - 1] >> 63) << 1);
-        carried = L > 1 ? wave_neighbour<true>(carried) : 0u;
-        if (first_lane) carried = 1u;
+        uint32_t into_ph = L > 1 ? wave_neighbour<true>((uint32_t)(ph[K - 1] >> 32)) : 0u;
+        uint32_t into_mh = L > 1 ? wave_neighbour<true>((uint32_t)(mh[K - 1] >> 32)) : 0u;
+        into_ph = first_lane ? ~0u : into_ph;
+        into_mh = first_lane ? 0u : into_mh;
 #pragma unroll
         for (int kk = K - 1; kk >= 0; --kk) {
-            const uint64_t phs = (ph[kk] << 1) | (kk ? ph[kk > 0 ? kk - 1 : 0] >> 63 : (uint64_t)(carried & 1));
-            const uint64_t mhs = (mh[kk] << 1) | (kk ? mh[kk > 0 ? kk - 1 : 0] >> 63 : (uint64_t)((carried >> 1) & 1));
-            const uint64_t npv = mhs | ~(xv[kk] | phs);
+            const uint64_t phs = slide_up(ph[kk], kk ? (uint32_t)(ph[kk > 0 ? kk - 1 : 0] >> 32) : into_ph);
+            const uint64_t mhs = slide_up(mh[kk], kk ? (uint32_t)(mh[kk > 0 ? kk - 1 : 0] >> 32) : into_mh);
+            const uint64_t npv = of_three<TABLE_A | ~(TABLE_B | TABLE_C)>(mhs, xv[kk], phs);
             const uint64_t nmv = phs & xv[kk];
+            // Kept decisions. X: unequal letters whose diagonal neighbour is one less (vertical + horizontal difference
+            // 1: one of them +1, neither -1). The planes: X or a reference letter alone; X or a query letter alone.
+            uint64_t plane0 = 0, plane1 = 0;
+            if constexpr (RECORD) {
+                const uint64_t unequal_step =
+                    of_three<TABLE_A & ~TABLE_B & ~TABLE_C>(of_three<(TABLE_A ^ TABLE_B) & TABLE_C>(npv, phs, differ[kk]), nmv, mhs);
+                plane0 = unequal_step | npv;
+                plane1 = of_three<TABLE_A | (TABLE_B & ~TABLE_C)>(unequal_step, ph[kk], npv);
+            }
             if constexpr (STAGED) {
-                // X: unequal letters whose diagonal neighbour is one less (vertical + horizontal difference 1:
-                // one of them +1, neither -1). The planes: X or a reference letter alone; X or a query letter alone.
-                const uint64_t unequal_step = ~eq[kk] & (npv ^ phs) & ~(nmv | mhs);
-                places[place][lane ^ place] = make_ulonglong2(unequal_step | npv, unequal_step | (ph[kk] & ~npv));
+                places[place][lane ^ place] = make_ulonglong2(plane0, plane1);
                 if (place == 7) {
                     // Every lane's line is full: the wave writes them, lanes 8g .. 8g + 7 the eight places of lane
                     // g' = 8i + g's line in instruction i.
@@ -661,17 +686,17 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
                     }
                 }
             } else if constexpr (RECORD) {
-                // X: unequal letters whose diagonal neighbour is one less (vertical + horizontal difference 1:
-                // one of them +1, neither -1).
-                const uint64_t unequal_step = ~eq[kk] & (npv ^ phs) & ~(nmv | mhs);
+                constexpr int AT = PLACE >= 0 ? PLACE % HOLD : HOLD - 1;
+                if constexpr (PLACE < 0) {
 #pragma unroll
-                for (int q = 0; q + 1 < HOLD; ++q) {
-                    held0[q][kk] = held0[q + 1][kk];
-                    held1[q][kk] = held1[q + 1][kk];
+                    for (int q = 0; q + 1 < HOLD; ++q) {
+                        held0[q][kk] = held0[q + 1][kk];
+                        held1[q][kk] = held1[q + 1][kk];
+                    }
                 }
-                held0[HOLD - 1][kk] = unequal_step | npv;
-                held1[HOLD - 1][kk] = unequal_step | (ph[kk] & ~npv);
-                if (active && recording && (j % HOLD) == 0) {
+                held0[AT][kk] = plane0;
+                held1[AT][kk] = plane1;
+                if (PLACE >= 0 ? AT == HOLD - 1 && active && recording : active && recording && (j % HOLD) == 0) {
                     global_decisions *chunk = reinterpret_cast<global_decisions *>((uint64_t)(uintptr_t)trace + held_chunk_at<HOLD>(j / HOLD - 1, WL, k * K + kk));
 #pragma unroll
                     for (int q = 0; q < HOLD; ++q) chunk[q] = u64x2{held0[q][kk], held1[q][kk]};
@@ -681,6 +706,26 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
             mv[kk] = nmv;
         }
         top += (int)((uint32_t)pv[0] & 1u) + __builtin_amdgcn_sbfe((int)(uint32_t)mv[0], 0, 1);
+        };
+        // Whole lines of eight columns where their places are known (WHOLE), their tests, shifts and addresses made once;
+        // the columns up to the next line and the last ones one by one.
+        while (steps > 0) {
+            if constexpr (WHOLE) {
+                if ((t & 7) == 0 && steps >= 8) {
+                    column(std::integral_constant<int, 0>{});
+                    column(std::integral_constant<int, 1>{});
+                    column(std::integral_constant<int, 2>{});
+                    column(std::integral_constant<int, 3>{});
+                    column(std::integral_constant<int, 4>{});
+                    column(std::integral_constant<int, 5>{});
+                    column(std::integral_constant<int, 6>{});
+                    column(std::integral_constant<int, 7>{});
+                    steps -= 8;
+                    continue;
+                }
+            }
+            column(std::integral_constant<int, -1>{});
+            --steps;
         }
     }
 }
@@ -691,8 +736,12 @@ __device__ __forceinline__ void sweep_queue(const EditArgs &a, int bin, ulonglon
 // bin a stream, ran four at a time on HIP's four hardware queues, each as long as its longest pair. 4,000 pairs
 // (1.5 kbp median, up to 20 kbp): the retries of ten bins took 14.0 ms so and their traces 19.2; the retries keeping
 // their decisions take 6.3 ms in one launch. 20,000 seeded pairs: 36.6 ms of sweeps and walks, 15.2 in one launch.
+// A column is one chain of about 60 vector and scalar instructions (100 with its decisions) whatever runs beside it, so
+// the chain's own instructions are the time: three-input bit functions, and lines of eight columns unrolled so that a
+// column's place needs no tests, shifts or addresses. The seeded pairs' run 14.2 -> 12.4 ms, the 4,000 pairs' call 17.4
+// -> 14.9. Four waves a SIMD: five would spill (17 ms), three (no bound) run the same.
 template <int BITS, int MODE>
-__global__ __launch_bounds__(256) void edit_sweep(EditArgs a, EditGrid grid) {
+__global__ __launch_bounds__(256, 4) void edit_sweep(EditArgs a, EditGrid grid) {
     constexpr bool STAGED = MODE != 0;
     __shared__ ulonglong2 stage[STAGED ? 4 : 1][STAGED ? 8 : 1][64];
     ulonglong2 (*const places)[64] = stage[STAGED ? threadIdx.x >> 6 : 0];

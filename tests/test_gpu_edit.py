@@ -231,6 +231,30 @@ def test_words_of_two_and_four_a_lane():
     assert sum(n for w, n in zip(widths, traced) if w > 4096) == 2, traced
 
 
+@pytest.mark.parametrize("guess,rows", [(12, 0), (500, 0), (0, 700), (0, 1500), (0, 3000), (0, 6000)])
+def test_columns_around_whole_lines(guess, rows):
+    # Queries of 1 to 41 columns and of 8k - 1 to 8k + 1, some starting their lines where another pair's ended: whole
+    # lines of eight columns and the columns left over, in bands of one lane up to two words a lane (a reference `rows`
+    # letters longer takes a band as wide), with decisions kept by the proving sweep, by a later one, and without.
+    rng = random.Random(91 + rows + guess)
+    lengths = list(range(1, 42)) + [8 * k + d for k in (16, 31) for d in (-1, 0, 1)]
+    rng.shuffle(lengths)
+    qrys = ["".join(rng.choice("ACGT") for _ in range(m)) for m in lengths]
+    refs = [mutated(q, 0.2, rng) + "".join(rng.choice("ACGT") for _ in range(rows + rng.randint(0, 9))) for q in qrys]
+    want = oracle_alignments(refs, qrys)
+    h = _lib.lib()
+    for kind, keep in ((1, 0), (1, 1), (0, 0)):
+        b = Batch(refs, qrys, kind)
+        try:
+            h.dinara_batch_set_keep_first(b.ptr, keep)
+            if guess:
+                guesses = np.full(len(refs), guess, dtype=np.int64)
+                assert h.dinara_batch_seed(b.ptr, guesses.ctypes.data) == 0
+            assert b.run() == (want if kind else [cost for cost, _ in want])
+        finally:
+            b.free()
+
+
 def test_byte_letters_and_scaled_costs():
     rng = random.Random(41)
     refs, qrys = pairs_of(60, rng, (0, 400), (0.05, 0.3), alphabet="ACDEFGHIKLMNPQRSTVWY")
