@@ -673,6 +673,12 @@ int64_t launch_class(dinara_batch *b, const SweepArgs &round, int cls, const int
 // a longer one, eight (half the strips and pipeline starts of four, and less of a row step spent outside the cells).
 int strip_c(int64_t m) { return m <= strip_columns(2) ? 2 : m <= strip_columns(4) ? 4 : 8; }
 
+// A round of few strips is as long as its longest pair's pipeline, and a strip of four columns a lane hands on sooner
+// than twice the half of one of eight (its step is shorter, and so are its rows): up to this many strips of eight, four.
+// 2,000 uneven pairs (8,192 strips) 11.1 -> 10.5 ms, 1,000 two-piece CIGARs 11.9 -> 9.9; two a lane 11.6 and 10.7. A
+// round that fills the chip pays for its cells: 200,000 uneven pairs 236 ms with eight, 251 with four.
+constexpr int64_t FEW_STRIPS = 16384;
+
 // A strip launch's parts: consecutive pairs of the plan whose decisions fit the budget together.
 struct StripPart {
     size_t pair, pairs, strip, strips;
@@ -687,11 +693,17 @@ struct StripPlan {
 
 // The plan of the pairs listed in `bands` (slot, low, high): each pair's strips, where its records lie, and the order
 // its strips are claimed in: the strips furthest from their pair's end first, so that the longest pipelines start first
-// and a strip always follows the one to its left.
-StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bool record) {
+// and a strip always follows the one to its left. `round`: a round of bands, whose strips may be narrower.
+StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bool record, bool round) {
     StripPlan plan;
     const int pieces = b->costs.pieces == 2 ? 2 : 1;
     const bool views = b->free_ends;
+    int widest_c = 8;
+    if (round) {
+        int64_t strips = 0;
+        for (const int4 &band : bands) strips += b->cols[band.x] / strip_columns(8) + 1;
+        if (strips <= FEW_STRIPS) widest_c = 4;
+    }
     std::vector<size_t> at;
     for (size_t next = 0; next < bands.size();) {
         StripPart part{plan.pairs.size(), 0, plan.order.size(), 0, 0, 0};
@@ -704,7 +716,7 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
             p.slot = band.x;
             p.lo = band.y;
             p.hi = band.z;
-            p.c = strip_c(m);
+            p.c = std::min(strip_c(m), widest_c);
             p.strips = (int)std::max<int64_t>(1, (m + strip_columns(p.c) - 1) / strip_columns(p.c));
             p.rows = (int)std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)p.hi - p.lo + strip_columns(p.c)));
             const size_t records = (size_t)p.strips * p.rows * 64;
@@ -1271,7 +1283,7 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         const int32_t *in_lists = lists + (size_t)((round + 1) % 2) * CLASSES * capacity;
         StripPlan plan;
         if (!strips.empty()) {
-            plan = plan_strips(b, strips, a.record != 0);
+            plan = plan_strips(b, strips, a.record != 0, true);
             if (const int64_t code = upload_strips(b, plan)) return code;
         }
         if (hipMemsetAsync(a.retry_counts, 0, CLASSES * 4, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
@@ -1495,7 +1507,7 @@ int64_t full_pass(dinara_batch *b) {
         bands.push_back(make_int4(slot, (int)-n, (int)m, 0));
     }
     if (!bands.empty()) {
-        const StripPlan plan = plan_strips(b, bands, record);
+        const StripPlan plan = plan_strips(b, bands, record, false);
         if (const int64_t code = upload_strips(b, plan)) return code;
         if (const int64_t code = launch_strips(b, sweep_args(b), plan, true, ctx->stream)) return code;
     }
