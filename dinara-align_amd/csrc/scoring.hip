@@ -255,7 +255,7 @@ int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &
     std::vector<int64_t> carry_at, arena_at;
     std::vector<size_t> first_wave;  // of each launch
     std::vector<int64_t> first_pair;
-    int64_t carry = 0, decisions = 0, most_decisions = 0;
+    int64_t carry = 0, most_carry = 0, decisions = 0, most_decisions = 0;  // of a launch, and the most of one
     for (int kind = 0; kind < 2; ++kind) {
         const int64_t begin = kind == 0 ? 0 : wide, end = kind == 0 ? wide : (int64_t)all.size();
         if (begin == end) continue;
@@ -286,7 +286,7 @@ int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &
             lds = std::max(lds, score_lds(b->scoring.letters, a.lanes, (int)cols, a.ref_room));
             const int64_t words = mode == SCORE_TRACE ? score_decisions(a.lanes, rows, cols) : 0;
             if (at == begin || (decisions > 0 && (decisions + words) * 4 > (int64_t)ARENA_BUDGET)) {
-                decisions = 0;
+                carry = decisions = 0;
                 out.push_back({a, 0});
                 first_wave.push_back(carry_at.size());
                 first_pair.push_back(at);
@@ -294,6 +294,7 @@ int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &
             out.back().args.count += (int)(std::min(end, at + pairs) - at);
             carry_at.push_back(carry);
             carry += score_carry(a.lanes, rows, cols);
+            most_carry = std::max(most_carry, carry);
             arena_at.push_back(decisions);
             decisions += words;
             most_decisions = std::max(most_decisions, decisions);
@@ -301,8 +302,8 @@ int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &
         for (size_t l = launches; l < out.size(); ++l) out[l].lds = lds;
     }
     if (!b->list.upload(ctx, all.data(), all.size() * 4)) return failed("list upload");
-    if (carry > 0 && (!b->carry.reserve((size_t)carry * 4) ||
-                      !b->carry_at.upload(ctx, carry_at.data(), carry_at.size() * 8)))
+    if (most_carry > 0 && (!b->carry.reserve((size_t)most_carry * 4) ||
+                           !b->carry_at.upload(ctx, carry_at.data(), carry_at.size() * 8)))
         return failed("carry");
     if (mode == SCORE_TRACE && (!b->arena.reserve((size_t)most_decisions * 4) ||
                                 !b->arena_at.upload(ctx, arena_at.data(), arena_at.size() * 8)))
@@ -310,7 +311,7 @@ int64_t plan_pass(Batch *b, int mode, int reversed, const std::vector<int32_t> &
     for (size_t l = 0; l < out.size(); ++l) {
         ScoreArgs &a = out[l].args;
         a.list = static_cast<const int32_t *>(b->list.ptr) + first_pair[l];
-        if (carry > 0) {
+        if (most_carry > 0) {
             a.carry = static_cast<int32_t *>(b->carry.ptr);
             a.carry_at = static_cast<const int64_t *>(b->carry_at.ptr) + first_wave[l];
         }

@@ -224,8 +224,8 @@ void dinara_batch_free(dinara_batch *batch);
  * whole run (ms), 1 the banded sweeps (ms), 2 the number of sweep launches, 4 the pairs the first band proved,
  * 5 the walk-back kernel (ms); for band class c 100+c its kernels' time (ms), 200+c its launches, 400+c the pairs
  * it swept. Classes: 0-3 sixteen lanes a pair (32/64/128/256 diagonals), 4-9 one wave a pair (64..2048, every
- * pair under a user band), 10-21 one pair a block of waves (512, 1024, 1536, 2048, 3072, 4096..8192 in steps of
- * 1024, 12288, 16384; the last two distances only). Unit-cost batches (the bit-parallel path): 6 is 1 when the
+ * pair under a user band), 10-21 strips, a pair a pipeline of waves (512, 1024, 1536, 2048, 3072, 4096..8192 in
+ * steps of 1024, 12288, 16384; one launch takes every width, its time at class 10). Unit-cost batches (the bit-parallel path): 6 is 1 when the
  * batch took it, 7 is 1 when the run replayed its captured hipGraph, 8 the further tracing passes the arena
  * needed, 9 the pairs proven by a sweep that kept its decisions (walked without a second sweep), 12 the number of
  * bins, 13 the first pass's bin set (dinara_batch_set_bins); 14 above zero when the gap-cost group sweeps hold
