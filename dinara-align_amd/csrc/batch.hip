@@ -444,10 +444,11 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     b->strip_letters = 65536;
     b->strip_widest = b->free_ends ? 2048 : band_width(CLASSES - 1);
     // Packed 16-bit group cells (group.hip) for shifted costs (equal extensions e) whose mismatch is no dearer than
-    // two extension letters: a tagged value then lies in [-16 e (n + m), 32 opening + 15] and a cell no path
-    // reaches stays above `top` - 16 e (n + m), so both fit 16 bits, apart, while 16 e (n + m) + 32 opening + 15
-    // stays under `top` (less a margin); `top` leaves room for an opening's add. DINARA_GROUP_CELLS32 set keeps
-    // 32-bit cells, for comparison.
+    // two extension letters: a tagged value then lies in [-16 e (n + m), 32 opening + 15]. A cell no path reaches starts
+    // at `top` on the two anti-diagonals before (0, 0)'s and loses at most 32 e a diagonal step: on anti-diagonal t it
+    // stays at or above `top` - 16 e (t + 2). So both fit 16 bits, apart, while 16 e (n + m + 2) + 32 opening + 15 stays
+    // under `top` (less a margin); `top` leaves room for an opening's add, and the seed's 32 e fits with it.
+    // DINARA_GROUP_CELLS32 set keeps 32-bit cells, for comparison.
     b->group16_top = 0;
     {
         const CostParams &k = b->costs;
@@ -455,7 +456,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         const int64_t top = (32767 - 16 * opening - 32) & ~int64_t(15);
         if (b->group_max_letters > 0 && !std::getenv("DINARA_GROUP_CELLS32") && k.pieces != 2 && k.del_ext == k.ins_ext &&
             e >= 0 && k.mismatch >= 0 && k.mismatch <= 2 * e && std::min(k.del_open, k.ins_open) >= 0 &&
-            16 * e * b->group_max_letters + 32 * opening + 15 < top - 64 && (size_t)8 * b->group_letters <= b->lds_limit)
+            16 * e * (b->group_max_letters + 2) + 32 * opening + 15 < top - 64 && (size_t)8 * b->group_letters <= b->lds_limit)
             b->group16_top = (int)top;
     }
     // The first band: the lanes' start and end diagonals and one either side (lanes.mojo:1207-1215), within the

@@ -257,6 +257,38 @@ def test_packed_group_cells(costs, monkeypatch):
     assert top == 0
     assert beyond[:-1] == want and beyond[-1] == o.costs_align(refs[-1], qrys[-1], oc)
 
+@pytest.mark.parametrize("mismatch,opening,extension", [(1, 0, 70), (1, 0, 60), (2, 0, 40), (1, 0, 30), (1, 3, 20),
+                                                        (5, 0, 16), (1, 0, 12), (3, 20, 12)])
+def test_packed_group_cells_at_their_limit_with_an_empty_side(mismatch, opening, extension):
+    # Cells outside the matrix are swept like the others and lose two extensions a diagonal step: at the longest pairs
+    # the packed cells take they must still lie above every cell inside, which a nearly empty side brings closest (its
+    # border is one gap, the dearest shifted values there are). 16-bit values hold 16 a cost unit: `total` is the most
+    # letters whose values fit beside the ones no path reaches, and 2 below it the packed cells are sure to be taken.
+    top = (32767 - 16 * opening - 32) & ~15
+    total = (top - 64 - 32 * opening - 15 - 1) // (16 * extension)
+    costs = da.Costs.affine(mismatch, opening, extension)
+    rng = random.Random(extension * 100 + opening)
+
+    def batch(letters):
+        refs, qrys = [], []
+        for short in (0, 1, 2, 3, letters // 4, letters // 2):
+            for unit in ("A", "ACGT", None):
+                long = "".join(rng.choice("ACGT") for _ in range(letters - short)) if unit is None else (unit * letters)[
+                    :letters - short]
+                side = "".join(rng.choice("ACGT") for _ in range(short)) if unit is None else (unit * letters)[:short]
+                if len(long) - len(side) < 250:
+                    refs += [long, side]
+                    qrys += [side, long]
+        return refs, qrys
+
+    for letters in range(total - 3, total + 2):
+        refs, qrys = batch(letters)
+        want = [o.costs_align(r, q, to_oracle(costs)) for r, q in zip(refs, qrys)]
+        found, packed = resident_alignments(refs, qrys, costs)
+        assert found == want
+        assert packed > 0 or letters > total - 2
+        check_distances(refs, qrys, costs)
+
 
 def test_block_bands_one_and_several_waves():
     # Long, noisy pairs: bands of 512 to 8192 diagonals, one pair a block of one to eight waves.
