@@ -1000,9 +1000,13 @@ constexpr int SIDE_WIDE = 0, SIDE_BESIDE = WIDE_BINS;
 
 int timing_pair(const dinara_batch *b, int bin) { return b->side_by_side_bins && bin < EDIT_NARROW ? 0 : 2 * bin; }
 
-// One sweep of every bin's queue (`reach`: the pairs each may hold) on `stream`: the one-word bins in one launch, the
-// wider ones beside it, widest first (their pairs are the longest chains); or, not side by side, the bins one after
-// another. `mark` is the first of the pass's marks; `timed` records the pairs of events from `ev`.
+// One sweep of every bin's queue (`reach`: the pairs each may hold): the one-word bins in one launch on `stream`, the
+// wider ones beside it on streams forked from the main one, widest first (their pairs are the longest chains); or, not
+// side by side, the bins one after another on `stream`. `mark` is the first of the pass's marks; `timed` records the
+// pairs of events from `ev`. The main stream waits for the wider bins at join_bins, whatever `stream` is: under capture
+// every fork must come from the stream that captures and every join go to it. A stream forked from one stream and
+// joined to another that was itself forked leaves each the other's parent, and with HIP 7.0 (as shipped with PyTorch)
+// ending such a capture, whose streams end their children's first, ended the process.
 void sweep_bins(dinara_batch *b, const EditArgs &a, bool trace, const int64_t (&reach)[EDIT_BINS], hipStream_t stream,
                 int mark, bool timed, int ev) {
     DeviceContext *ctx = b->ctx;
@@ -1034,7 +1038,7 @@ void sweep_bins(dinara_batch *b, const EditArgs &a, bool trace, const int64_t (&
         if (!grid[bin]) continue;
         hipStream_t side = stream;
         if (!b->one_stream) {
-            if (!forked) (void)hipEventRecord(ctx->mark(mark), stream);
+            if (!forked) (void)hipEventRecord(ctx->mark(mark), ctx->stream);
             forked = true;
             side = ctx->side(SIDE_WIDE + bin - EDIT_NARROW);
             (void)hipStreamWaitEvent(side, ctx->mark(mark), 0);
@@ -1043,8 +1047,14 @@ void sweep_bins(dinara_batch *b, const EditArgs &a, bool trace, const int64_t (&
         if (!b->one_stream) (void)hipEventRecord(ctx->mark(mark + 1 + bin - EDIT_NARROW), side);
     }
     if (narrow) around(0, stream, [&] { launch_edit_sweep(a, trace, grid, stream); });
+}
+
+// The main stream waits for the wider bins of the pass whose marks start at `mark`.
+void join_bins(dinara_batch *b, const int64_t (&reach)[EDIT_BINS], int mark) {
+    if (!b->side_by_side_bins || b->one_stream) return;
     for (int bin = EDIT_NARROW; bin < EDIT_BINS; ++bin)
-        if (grid[bin] && !b->one_stream) (void)hipStreamWaitEvent(stream, ctx->mark(mark + 1 + bin - EDIT_NARROW), 0);
+        if (edit_grid(b, bin, reach[bin]))
+            (void)hipStreamWaitEvent(b->ctx->stream, b->ctx->mark(mark + 1 + bin - EDIT_NARROW), 0);
 }
 
 // The run's launches: reset; every bin's first queue; the retry queues; then (alignments) the tracing sweep, and the
@@ -1064,6 +1074,7 @@ int64_t enqueue_unit(dinara_batch *b, const EditArgs &a, bool timed, bool trace)
     const int slots = (int)b->slot_pair.size();
     launch_edit_reset(a, slots, ctx->stream);
     sweep_bins(b, a, false, b->first_count, ctx->stream, FIRST_MARKS, timed, EV_FIRST);
+    join_bins(b, b->first_count, FIRST_MARKS);
     // Kept decisions: the pairs the first pass proved are walked on a stream of their own while the retries sweep.
     const bool early = trace && b->keep_first;
     const bool beside = trace && !b->keep_first && !b->doubling;
@@ -1091,6 +1102,7 @@ int64_t enqueue_unit(dinara_batch *b, const EditArgs &a, bool timed, bool trace)
         (void)hipEventRecord(ctx->mark(BESIDE_MARKS + 1), tracer);
     }
     sweep_bins(b, retry, false, b->retry_reach, ctx->stream, RETRY_MARKS, timed, EV_RETRY);
+    join_bins(b, b->retry_reach, RETRY_MARKS);
     if (b->doubling) {
         EditArgs later = retry;
         later.lists = retry.file_lists;
@@ -1100,11 +1112,13 @@ int64_t enqueue_unit(dinara_batch *b, const EditArgs &a, bool timed, bool trace)
             int64_t only[EDIT_BINS] = {};
             only[bin] = b->retry_reach[bin];
             sweep_bins(b, later, false, only, ctx->stream, RETRY_MARKS, false, 0);
+            join_bins(b, only, RETRY_MARKS);
         }
     }
     if (trace) {
         if (!b->keep_first && b->doubling)
             sweep_bins(b, a, true, b->trace_reach, ctx->stream, TRACE_MARKS, timed, EV_TRACE);
+        if (!b->keep_first) join_bins(b, b->trace_reach, TRACE_MARKS);
         if (beside) (void)hipStreamWaitEvent(ctx->stream, ctx->mark(BESIDE_MARKS + 1), 0);
         // The last walk follows the early walk's kernels (it writes moves of slots the early walk marked unwalked)
         // and runs while the early walk's text is made; the run ends when both texts are made.
@@ -1195,6 +1209,7 @@ int64_t run_unit(dinara_batch *b, bool trace) {
                 return DINARA_OUT_OF_MEMORY;
             launch_edit_requeue(a, static_cast<const int32_t *>(b->deferred_held.ptr), deferred, ctx->stream);
             sweep_bins(b, a, true, b->trace_reach, ctx->stream, TRACE_MARKS, false, 0);
+            join_bins(b, b->trace_reach, TRACE_MARKS);
             walk_slots(b, a, ctx->stream, ctx->side(SIDE_WIDE), WALK_MARKS + 3, false);
             int32_t left = 0;
             if (hipPeekAtLastError() != hipSuccess || !b->deferred_count.read(ctx, &left, 4)) return DINARA_OUT_OF_MEMORY;

@@ -10,6 +10,8 @@ equals its DP-flag rule (lanes.mojo:905-923); the oracle follows the flag rule a
 import ctypes
 import os
 import random
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -253,6 +255,37 @@ def test_columns_around_whole_lines(guess, rows):
             assert b.run() == (want if kind else [cost for cost, _ in want])
         finally:
             b.free()
+
+
+BESIDE_TORCH = """
+import faulthandler, random, sys
+faulthandler.enable()
+import torch  # its HIP runtime is the one this process loads
+import test_gpu_edit as t
+rng = random.Random(97)
+qrys = ["".join(rng.choice("ACGT") for _ in range(m)) for m in (40, 300, 700, 90, 500)]
+refs = [t.mutated(q, 0.1, rng) + "".join(rng.choice("ACGT") for _ in range(rows))
+        for q, rows in zip(qrys, (0, 5, 6000, 4500, 1500))]
+want = t.oracle_alignments(refs, qrys)
+for keep in (0, 1):
+    b = t.Batch(refs, qrys, 1)
+    b.h.dinara_batch_set_keep_first(b.ptr, keep)
+    for replay in range(3):
+        print("keep_first", keep, "run", replay, flush=True)
+        assert b.run() == want
+        assert b.stat(7) == 1, "not replayed as a graph"
+    b.free()
+"""
+
+
+def test_graphs_of_pairs_of_every_bin_beside_torch():
+    # A run of alignments captured as one graph, its streams all forked from the stream that captures and joined to it,
+    # in a process that holds PyTorch and so its own HIP runtime: pairs whose bands need lanes of several words are
+    # traced on streams of their own beside the retries'.
+    ran = subprocess.run([sys.executable, "-u", "-c", BESIDE_TORCH], cwd=os.path.dirname(os.path.abspath(__file__)),
+                         env={**os.environ, "PYTHONPATH": os.pathsep.join(sys.path)}, capture_output=True, text=True,
+                         timeout=600)  # a first import of PyTorch can take a minute or two
+    assert ran.returncode == 0, (ran.returncode, ran.stdout[-500:], ran.stderr[-2000:])
 
 
 def test_byte_letters_and_scaled_costs():
