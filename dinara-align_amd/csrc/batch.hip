@@ -700,7 +700,9 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
     const int pieces = b->costs.pieces == 2 ? 2 : 1;
     const bool views = b->free_ends;
     int widest_c = 8;
-    if (round) {
+    if (const char *set = std::getenv("DINARA_STRIP_COLUMNS")) {  // for checking: 2, 4 or 8 at most
+        widest_c = std::strtol(set, nullptr, 10) <= 2 ? 2 : std::strtol(set, nullptr, 10) <= 4 ? 4 : 8;
+    } else if (round) {
         int64_t strips = 0;
         for (const int4 &band : bands) strips += b->cols[band.x] / strip_columns(8) + 1;
         if (strips <= FEW_STRIPS) widest_c = 4;

@@ -1,0 +1,100 @@
+"""The strip sweep (strip.hip) where a pair takes several strips and lanes hold two, four or eight columns: free ends,
+whose best end is the least over the strips, and banded rounds keeping decisions, against the oracle bit for bit (cost,
+CIGAR and spans; reference tests/test_alignment.mojo:1944-2113 for the free ends' rule, :3715-3989 for the pairs). A
+strip is 64 lanes of 2, 4 or 8 columns: queries lie on both sides of 128, 256 and 512 letters and run to several strips.
+"""
+
+import random
+
+import pytest
+
+import dinara_align as da
+from dinara_align.types import UNBOUNDED
+from oracle import oracle as o
+from test_gpu_costs import mutated
+from test_gpu_whole import to_oracle
+
+pytestmark = pytest.mark.gpu
+
+TWO = da.Costs.two_piece(4, 6, 2, 24, 1)
+COSTS = [da.Costs.affine(4, 6, 2), TWO, da.Costs.affine(4, 2, 1).with_deletions(6, 3)]
+IDS = ["affine", "two-piece", "deletions"]
+QUERIES = (127, 128, 129, 255, 256, 257, 511, 513, 769, 1500)
+
+
+def letters(rng, count, alphabet="ACGT"):
+    return "".join(rng.choice(alphabet) for _ in range(count))
+
+
+def ends_of(mode):
+    return (mode.reference_start, mode.reference_end, mode.query_start, mode.query_end)
+
+
+def free_pairs(rng):
+    """(reference, query, mode) with the best end in the last strip, in an earlier one (free query ends), and equal ends
+    in different strips (repeats)."""
+    found = []
+    for m in QUERIES:
+        q = letters(rng, m)
+        placed = letters(rng, rng.randint(0, 150)) + mutated(q, 0.05, rng) + letters(rng, rng.randint(0, 150))
+        if len(placed) + m < 2040:  # the first band, every diagonal a path may start or end on, is 2,048 at most
+            found.append((placed, q, da.Mode.INFIX))
+        found.append((mutated(q, 0.03, rng) + letters(rng, 90), q, da.Mode.PREFIX))
+        found.append((letters(rng, 90) + mutated(q, 0.03, rng), q, da.Mode.SUFFIX))
+        # The query's first letters, its middle and its last: ends along the last row, in any strip.
+        for low in (0, m // 3, m - m // 4):
+            part = mutated(q[low:low + max(20, m // 4)], 0.04, rng)
+            found.append((part, q, da.Mode.ends_free(0, 0, UNBOUNDED, UNBOUNDED)))
+            found.append((part, q, da.Mode.ends_free(7, 5, UNBOUNDED, UNBOUNDED)))
+        # A repeat as long as the query: as many equal ends as copies.
+        unit = letters(rng, rng.randint(3, 40))
+        found.append(((unit * 8)[:90], (unit * m)[:m], da.Mode.ends_free(0, 0, UNBOUNDED, UNBOUNDED)))
+        found.append(((unit * m)[:m + 100], (unit * m)[:m], da.Mode.ends_free(50, 50, 20, 20)))
+    return found
+
+
+@pytest.mark.parametrize("columns", [None, "2", "8"])
+@pytest.mark.parametrize("costs", COSTS, ids=IDS)
+def test_free_ends_across_strips(costs, columns, monkeypatch):
+    if columns:
+        monkeypatch.setenv("DINARA_STRIP_COLUMNS", columns)
+    rng = random.Random(101 + len(str(costs)))
+    oc = to_oracle(costs)
+    by_mode = {}
+    for r, q, mode in free_pairs(rng):
+        by_mode.setdefault(ends_of(mode), (mode, [], []))
+        by_mode[ends_of(mode)][1].append(r)
+        by_mode[ends_of(mode)][2].append(q)
+    for ends, (mode, refs, qrys) in by_mode.items():
+        for ties in ("left", "right"):
+            got = da.alignments(refs, qrys, costs, mode, ties=ties)
+            for i, (r, q) in enumerate(zip(refs, qrys)):
+                g = got[i]
+                assert g is not None, (i, len(r), len(q), mode, ties)
+                assert (g.cost, g.cigar, (g.reference_start, g.reference_end, g.query_start, g.query_end)) == o.ends_align(
+                    r, q, oc, ends, right_ties=ties == "right"), (i, len(r), len(q), mode, ties)
+        assert da.distances(refs, qrys, costs, mode) == [o.ends_cost(r, q, oc, ends)[0] for r, q in zip(refs, qrys)]
+
+
+@pytest.mark.parametrize("columns", ["2", "4", "8"])
+@pytest.mark.parametrize("costs", COSTS, ids=IDS)
+def test_banded_strips_of_every_width(costs, columns, monkeypatch):
+    # Bands far narrower than the matrix: strips whose rows begin below the first and end above the last, the cell
+    # above-left of a strip's first from the strip to its left, and decisions in the rows between.
+    monkeypatch.setenv("DINARA_STRIP_COLUMNS", columns)
+    rng = random.Random(7)
+    oc = to_oracle(costs)
+    refs, qrys = [], []
+    for n, rate in [(4100, 0.002), (4100, 0.03), (2300, 0.05), (3000, 0.25), (2600, 0.6), (1300, 0.1)]:
+        r = letters(rng, n)
+        refs.append(r)
+        qrys.append(mutated(r, rate, rng))
+    refs += [letters(rng, 3000), letters(rng, 900), "ACG" * 1000]
+    qrys += [refs[-3][400:2500], letters(rng, 300) + refs[-2] + letters(rng, 1400), "ACG" * 600 + "TTAC" * 300]
+    refs += ["", letters(rng, 700)]
+    qrys += [letters(rng, 700), ""]
+    for ties in ("left", "right"):
+        got = da.alignments(refs, qrys, costs, ties=ties)
+        for i, (r, q) in enumerate(zip(refs, qrys)):
+            assert (got[i].cost, got[i].cigar) == o.costs_align(r, q, oc, right_ties=ties == "right"), (i, len(r), len(q))
+    assert da.distances(refs, qrys, costs) == [o.costs_cost(r, q, oc) for r, q in zip(refs, qrys)]
