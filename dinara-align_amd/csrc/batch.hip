@@ -680,7 +680,13 @@ int strip_c(int64_t m) { return m <= strip_columns(2) ? 2 : m <= strip_columns(4
 // round that fills the chip pays for its cells: 200,000 uneven pairs 236 ms with eight, 251 with four.
 constexpr int64_t FEW_STRIPS = 16384;
 
-// A strip launch's parts: consecutive pairs of the plan whose decisions fit the budget together.
+// A strip launch's parts: consecutive pairs of the plan whose decisions and carry records fit ARENA_BUDGET together. A
+// round of costs keeps no decisions, but each pair's carry records (8 bytes a row a strip, 16 under two pieces; 0.8 MB
+// for a pair of 10,000 letters in 4,500 diagonals): it is cut once it passes CARRY_BUDGET with strips enough to fill the
+// persistent grid several times, so that what a batch asks for stays bounded and a part's tail short beside it.
+// DINARA_STRIP_BUDGET sets the bytes a part may take, for checking.
+constexpr size_t CARRY_BUDGET = size_t(1) << 30;
+constexpr size_t FULL_GRIDS = 4;
 struct StripPart {
     size_t pair, pairs, strip, strips;
     size_t decision_bytes, carry_words;
@@ -707,6 +713,8 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
         for (const int4 &band : bands) strips += b->cols[band.x] / strip_columns(8) + 1;
         if (strips <= FEW_STRIPS) widest_c = 4;
     }
+    size_t budget = ARENA_BUDGET;
+    if (const char *set = std::getenv("DINARA_STRIP_BUDGET")) budget = std::strtoull(set, nullptr, 10);
     std::vector<size_t> at;
     for (size_t next = 0; next < bands.size();) {
         StripPart part{plan.pairs.size(), 0, plan.order.size(), 0, 0, 0};
@@ -724,11 +732,15 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
             p.rows = (int)std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)p.hi - p.lo + strip_columns(p.c)));
             const size_t records = (size_t)p.strips * p.rows * 64;
             const size_t bytes = record ? (records * strip_record_bytes(p.c, pieces) + 255) & ~size_t(255) : 0;
-            if (part.pairs > 0 && part.decision_bytes + bytes > ARENA_BUDGET) break;
+            const size_t carried = p.strips > 1 ? (size_t)p.strips * p.rows * pieces : 0;
+            const size_t carry_bytes = 8 * (part.carry_words + carried);
+            if (part.pairs > 0 && (part.decision_bytes + bytes + carry_bytes > budget ||
+                                   (carry_bytes > CARRY_BUDGET && part.strips >= FULL_GRIDS * STRIP_GRID)))
+                break;
             p.decision_at = (int64_t)part.decision_bytes;
             p.carry_at = (int64_t)part.carry_words;
             part.decision_bytes += bytes;
-            part.carry_words += p.strips > 1 ? (size_t)p.strips * p.rows * pieces : 0;
+            part.carry_words += carried;
             part.strips += p.strips;
             ++part.pairs;
             most = std::max(most, p.strips);

@@ -4,11 +4,13 @@ CIGAR and spans; reference tests/test_alignment.mojo:1944-2113 for the free ends
 strip is 64 lanes of 2, 4 or 8 columns: queries lie on both sides of 128, 256 and 512 letters and run to several strips.
 """
 
+import ctypes
 import random
 
 import pytest
 
 import dinara_align as da
+from dinara_align import _lib
 from dinara_align.types import UNBOUNDED
 from oracle import oracle as o
 from test_gpu_costs import mutated
@@ -98,3 +100,59 @@ def test_banded_strips_of_every_width(costs, columns, monkeypatch):
         for i, (r, q) in enumerate(zip(refs, qrys)):
             assert (got[i].cost, got[i].cigar) == o.costs_align(r, q, oc, right_ties=ties == "right"), (i, len(r), len(q))
     assert da.distances(refs, qrys, costs) == [o.costs_cost(r, q, oc) for r, q in zip(refs, qrys)]
+
+
+def resident(refs, qrys, costs, kind, mode=None):
+    """A resident batch's results of two runs through the C ABI, and the launches of a run."""
+    handle = _lib.lib()
+    R, Q = _lib.Texts(refs), _lib.Texts(qrys)
+    c, status = costs.as_c(), ctypes.c_int64(0)
+    as_c = mode.as_c() if mode else None
+    batch = handle.dinara_batch_new(0, kind, len(refs), *R.args(), *Q.args(), ctypes.byref(c),
+                                    ctypes.byref(as_c) if mode else None, None, 4, ctypes.byref(status))
+    assert batch, status.value
+    try:
+        runs = []
+        for _ in range(2):
+            assert handle.dinara_batch_run(batch) == 0
+            if kind == _lib.BATCH_DISTANCES:
+                out = (ctypes.c_int64 * len(refs))()
+                assert handle.dinara_batch_distances(batch, out) == 0
+                runs.append(list(out))
+                continue
+            found, statuses = (_lib.CAlignment * len(refs))(), (ctypes.c_int64 * len(refs))()
+            assert handle.dinara_batch_alignments(batch, found, statuses) == 0
+            assert not any(statuses)
+            runs.append([(a.cost, ctypes.string_at(a.cigar, a.cigar_length).decode()) for a in found])
+            for a in found:
+                handle.dinara_free(a.cigar)
+        assert runs[0] == runs[1]
+        return runs[0], handle.dinara_batch_stat(batch, 2)
+    finally:
+        handle.dinara_batch_free(batch)
+
+
+@pytest.mark.parametrize("costs", COSTS, ids=IDS)
+def test_rounds_cut_into_parts(costs, monkeypatch):
+    # A round whose memory passes its budget runs in parts, each reusing the memory of the one before: costs alone
+    # (whose carry records are all they keep), CIGARs, and the two phases of free ends.
+    rng = random.Random(19)
+    oc = to_oracle(costs)
+    refs = [letters(rng, rng.randint(2200, 2700)) for _ in range(24)]
+    qrys = [mutated(r, rate, rng) for r, rate in zip(refs, [0.01, 0.1, 0.3, 0.5] * 6)]
+    windows = [letters(rng, 60) + q[:600] + letters(rng, 90) for q in qrys]
+    reads = [mutated(q[:600], 0.05, rng) for q in qrys]
+    want = [o.costs_align(r, q, oc) for r, q in zip(refs, qrys)]
+    ends = [o.ends_align(r, q, oc, ends_of(da.Mode.INFIX)) for r, q in zip(windows, reads)]
+    whole = {}
+    for budget in (None, 300_000, 1):
+        if budget:
+            monkeypatch.setenv("DINARA_STRIP_BUDGET", str(budget))
+        for name, got, right in [
+                ("distances", resident(refs, qrys, costs, 0), [cost for cost, _ in want]),
+                ("alignments", resident(refs, qrys, costs, 1), want),
+                ("placed distances", resident(windows, reads, costs, 0, da.Mode.INFIX), [e[0] for e in ends]),
+                ("placed", resident(windows, reads, costs, 1, da.Mode.INFIX), [e[:2] for e in ends])]:
+            assert got[0] == right, (name, budget)
+            launches = whole.setdefault(name, got[1])
+            assert budget is None or got[1] > launches, (name, budget, got[1], launches)
