@@ -1170,10 +1170,25 @@ int64_t run_unit(dinara_batch *b, bool trace) {
         }
         const size_t held = ctx->edit_arena->size, ask = std::min(std::max(b->arena_ask, ctx->arena_wanted), b->arena_bound);
         if (held < ask) {
-            ctx->edit_arena->release();
-            if (!ctx->edit_arena->reserve(std::min(std::max(ask, held + held / 2), b->arena_bound)) &&
-                !ctx->edit_arena->reserve(ask))
-                return DINARA_OUT_OF_MEMORY;
+            // Not past the memory there is now (the bound is the batch's first run's): a smaller arena serves with
+            // more passes, so what cannot be had is not asked for again, and the size held before is taken back.
+            size_t free_bytes = 0, total = 0;
+            (void)hipMemGetInfo(&free_bytes, &total);
+            if (held == 0 || ask - held <= free_bytes) {
+                ctx->edit_arena->release();
+                if (!ctx->edit_arena->reserve(std::min(std::max(ask, held + held / 2), b->arena_bound)) &&
+                    !ctx->edit_arena->reserve(ask)) {
+                    size_t less = std::max(held, ask / 2);
+                    while (!ctx->edit_arena->reserve(less)) {
+                        if (less <= (size_t(1) << 20)) return DINARA_OUT_OF_MEMORY;
+                        less /= 2;
+                    }
+                }
+            }
+            if (ctx->edit_arena->size < ask) {
+                b->arena_ask = std::min(b->arena_ask, ctx->edit_arena->size);
+                ctx->arena_wanted = 0;
+            }
         }
         const size_t bytes = std::min(ctx->edit_arena->size, b->arena_bound);
         if (b->arena_ptr != ctx->edit_arena->ptr || b->arena_capacity != bytes) {

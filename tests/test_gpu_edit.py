@@ -428,6 +428,25 @@ def test_keep_first_with_a_small_arena(monkeypatch):
     assert got == oracle_alignments(refs, qrys)
 
 
+def test_an_arena_that_cannot_be_had_leaves_the_one_held(monkeypatch):
+    # A run that asks for more memory than the device has takes the arena it holds, and later runs as well.
+    refs, qrys = uneven(200, 73)
+    want = oracle_alignments(refs, qrys)
+    for keep in (0, 1):
+        for arena in (None, 1 << 50, None):
+            if arena:
+                monkeypatch.setenv("DINARA_TRACE_ARENA", str(arena))
+            else:
+                monkeypatch.delenv("DINARA_TRACE_ARENA", raising=False)
+            b = Batch(refs, qrys, 1)
+            try:
+                b.h.dinara_batch_set_keep_first(b.ptr, keep)
+                assert b.run() == want
+                assert b.run() == want
+            finally:
+                b.free()
+
+
 def test_small_arena_traces_in_several_passes(monkeypatch):
     refs, qrys = uneven(300, 53)
     want = oracle_alignments(refs, qrys)
