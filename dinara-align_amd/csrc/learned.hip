@@ -612,7 +612,7 @@ int64_t dinara_mlp_gradients(dinara_mlp *net, int64_t rows, const float *feature
     if (!net || rows <= 0) return DINARA_INVALID_MODE;
     DeviceGuard guard(net->ctx);
     const int64_t padded = (rows + 31) / 32 * 32;
-    if (padded > INT32_MAX / FEATURE_STRIDE || !reserve_rows(net, (int)padded) || !net->loss.reserve(4) ||
+    if (padded > INT32_MAX || !reserve_rows(net, (int)padded) || !net->loss.reserve(4) ||
         !net->features.upload(net->ctx, features, (size_t)rows * FEATURE_STRIDE * 4) ||
         !net->targets.upload(net->ctx, targets, (size_t)rows * 4))
         return DINARA_OUT_OF_MEMORY;
@@ -632,8 +632,14 @@ int64_t dinara_mlp_predict(dinara_mlp *net, int64_t rows, const float *features,
     if (!net) return DINARA_INVALID_MODE;
     if (rows <= 0) return 0;
     DeviceGuard guard(net->ctx);
-    if (!net->features.upload(net->ctx, features, (size_t)rows * FEATURE_STRIDE * 4)) return DINARA_OUT_OF_MEMORY;
-    return mlp_predict_device(net, f32(net->features), rows, out);
+    constexpr int64_t most = int64_t(1) << 20;  // rows on the device at once (1.2 GB of features)
+    for (int64_t first = 0; first < rows; first += most) {
+        const int64_t count = std::min(most, rows - first);
+        if (!net->features.upload(net->ctx, features + first * FEATURE_STRIDE, (size_t)count * FEATURE_STRIDE * 4))
+            return DINARA_OUT_OF_MEMORY;
+        if (const int64_t code = mlp_predict_device(net, f32(net->features), count, out + first)) return code;
+    }
+    return 0;
 }
 
 // Trains on `rows` rows for `epochs` passes in shuffled batches of `batch` rows (a multiple of 32) by Adam at
@@ -645,7 +651,7 @@ int64_t dinara_mlp_train(dinara_mlp *net, int64_t rows, const float *features, c
     DeviceContext *ctx = net->ctx;
     DeviceGuard guard(ctx);
     const int64_t steps = (rows + batch - 1) / batch;
-    if (batch > INT32_MAX / FEATURE_STRIDE || !reserve_rows(net, (int)batch) || !net->loss.reserve((size_t)steps * 4) ||
+    if (batch > INT32_MAX || !reserve_rows(net, (int)batch) || !net->loss.reserve((size_t)steps * 4) ||
         !net->features.upload(ctx, features, (size_t)rows * FEATURE_STRIDE * 4) ||
         !net->targets.upload(ctx, targets, (size_t)rows * 4) || !net->index.reserve((size_t)rows * 4))
         return DINARA_OUT_OF_MEMORY;

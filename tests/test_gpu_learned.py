@@ -155,6 +155,29 @@ def test_forward_matches_numpy():
         net.free()
 
 
+def test_rows_past_32_bit_places():
+    # More rows than 2^31 floats hold: a training batch of which 64 rows are real steps as one of 64 does (the others
+    # add zeros), and a prediction taken in several shares gives each row what it gives it alone.
+    x, t = random_inputs(64, 23)
+    small, large = Net(5), Net(5)
+    try:
+        small.train(x, t, epochs=2, batch=64)
+        large.train(x, t, epochs=2, batch=(2**31 // F + 32) // 32 * 32)
+        np.testing.assert_array_equal(large.weights(), small.weights())
+    finally:
+        small.free()
+        large.free()
+    rows, net = 2**20 + 45, Net(6)
+    try:
+        many = np.zeros((rows, F), dtype=np.float32)
+        many[:, :64] = np.arange(rows, dtype=np.float32)[:, None] % 977 / 977 * np.linspace(-1, 1, 64, dtype=np.float32)
+        got = net.predict(many)
+        for low in (0, 2**20 - 40, rows - 32):
+            np.testing.assert_array_equal(got[low:low + 32], net.predict(many[low:low + 32]))
+    finally:
+        net.free()
+
+
 @pytest.mark.parametrize("kind", [0, 1])
 def test_features_match_numpy(kind):
     # kind 1 (alignments, Ties.LEFT) packs the tape reversed: the features must not change.
