@@ -249,6 +249,7 @@ struct dinara_batch {
     // The whole-matrix path (strip.hip) for pairs the band sweeps leave unsettled: whether any pair is long enough
     // to need it (-1 not worked out yet), and the last run's count and time.
     int may_need_full = -1;
+    bool expired = false;  // a strip's wait gave up in the last run: it left pairs to the whole-matrix path
     bool whole = false;  // every pair takes the whole-matrix path, no band sweep (for checking and comparison)
     double full_pairs = 0, full_ms = 0;
     DeviceBuffer full_list, full_count;
@@ -776,11 +777,20 @@ int64_t upload_strips(dinara_batch *b, const StripPlan &plan) {
     std::memcpy(host.data() + pairs, plan.order.data(), order);
     size_t most = 0;
     for (const StripPart &part : plan.parts) most = std::max(most, part.pairs);
-    if (!b->strip_plan.upload(b->ctx, host.data(), host.size()) || !b->strip_counts.reserve((2 * most + 1) * 4) ||
+    if (!b->strip_plan.upload(b->ctx, host.data(), host.size()) || !b->strip_counts.reserve((most + 1) * 4) ||
         !b->strip_best.reserve(most * 8) || !b->strip_carry.reserve(std::max<size_t>(plan.carry_words, 1) * 8) ||
         (plan.decision_bytes && !b->strip_decisions.reserve(plan.decision_bytes)))
         return DINARA_OUT_OF_MEMORY;
     return 0;
+}
+
+// Where among a round's counts its strips' expired waits are (strip classes are counted together at the first).
+constexpr int STRIP_EXPIRED = CLASS_STRIP_FIRST + 1;
+
+// The polls of a round's waits; DINARA_STRIP_POLLS sets them, for checking.
+int strip_polls() {
+    const char *set = std::getenv("DINARA_STRIP_POLLS");
+    return set ? (int)std::strtol(set, nullptr, 10) : STRIP_POLL_LIMIT;
 }
 
 // The plan's launches on `stream`, each part's sweep and (when decisions are kept) its walks, filing unproven pairs
@@ -798,10 +808,11 @@ int64_t launch_strips(dinara_batch *b, const SweepArgs &round, const StripPlan &
         a.decisions = part.decision_bytes ? static_cast<uint8_t *>(b->strip_decisions.ptr) : nullptr;
         a.carry = static_cast<unsigned long long *>(b->strip_carry.ptr);
         a.claim = static_cast<int *>(b->strip_counts.ptr);
-        a.failed = a.claim + 1;
-        a.done = a.failed + part.pairs;
+        a.done = a.claim + 1;
+        a.polls = whole ? STRIP_POLL_LIMIT : strip_polls();
+        a.expired = whole ? nullptr : round.retry_counts + STRIP_EXPIRED;
         a.best = static_cast<unsigned long long *>(b->strip_best.ptr);
-        if (hipMemsetAsync(b->strip_counts.ptr, 0, (2 * part.pairs + 1) * 4, stream) != hipSuccess ||
+        if (hipMemsetAsync(b->strip_counts.ptr, 0, (part.pairs + 1) * 4, stream) != hipSuccess ||
             (part.carry_words &&
              hipMemsetAsync(b->strip_carry.ptr, 0, part.carry_words * 8, stream) != hipSuccess) ||
             (b->free_ends && hipMemsetAsync(b->strip_best.ptr, 0xFF, part.pairs * 8, stream) != hipSuccess))
@@ -1394,6 +1405,7 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             counts[c] = filed[c];
             retried += filed[c];
         }
+        b->expired = b->expired || filed[STRIP_EXPIRED] > 0;
         strips.resize((size_t)filed[CLASS_STRIP_FIRST]);
         if (!strips.empty()) {
             if (hipMemcpyAsync(strips.data(), a.strip_retries, strips.size() * sizeof(int4), hipMemcpyDeviceToHost,
@@ -1510,8 +1522,8 @@ int64_t free_phase_b(dinara_batch *b) {
 // The decision bytes one pair may take on the whole-matrix path: past it the pair stays unsettled.
 constexpr size_t FULL_BUDGET = size_t(16) << 30;
 
-// After a run, every pair the band sweeps left unsettled (wider than the widest band, or more letters than the strips
-// take in bands) is swept whole and walked (strip.hip); a pair under free
+// After a run, every pair the band sweeps left unsettled (wider than the widest band, more letters than the strips
+// take in bands, or left by a strip's expired wait) is swept whole and walked (strip.hip); a pair under free
 // ends or a user band, or whose decisions pass FULL_BUDGET, stays unsettled. A batch none of
 // whose pairs could need it skips the pass; otherwise the unsettled slots are listed on the device and only their
 // count (and list) come back. Caller holds the device lock.
@@ -1527,7 +1539,7 @@ int64_t full_pass(dinara_batch *b) {
         for (int64_t s = 0; s < slots; ++s)
             if ((int64_t)b->rows[s] + b->cols[s] + 3 > 8192) b->may_need_full = 1;
     }
-    if (!b->may_need_full && !b->whole) return 0;
+    if (!b->may_need_full && !b->whole && !b->expired) return 0;
     const auto began = std::chrono::steady_clock::now();
     if (!b->full_list.reserve((size_t)slots * 4) || !b->full_count.reserve(4) ||
         hipMemsetAsync(b->full_count.ptr, 0, 4, ctx->stream) != hipSuccess)
@@ -1587,6 +1599,7 @@ int64_t run(dinara_batch *b) {
     }
     const int64_t slots = (int64_t)b->slot_pair.size();
     b->launches = b->first_proven = 0;
+    b->expired = false;
     b->run_ms = b->sweep_ms = b->walk_ms = 0;
     for (int c = 0; c < CLASSES; ++c) b->class_ms[c] = b->class_launches[c] = b->class_pairs[c] = 0;
     if (hipEventRecord(ctx->start, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;

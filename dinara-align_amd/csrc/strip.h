@@ -10,8 +10,8 @@ namespace dinara {
 __host__ __device__ constexpr int strip_columns(int c) { return 64 * c; }
 // The persistent sweep's workgroups (a wave each): strips beyond them are claimed as waves finish theirs.
 constexpr int STRIP_GRID = 8192;
-// A wave's wait for its left strip's boundary column gives up after this many polls (the sweep then reports the
-// pair unsettled instead of hanging).
+// A wave's wait for its left strip's boundary column gives up after this many polls instead of hanging: its pair stays
+// unsettled, as do the strips right of it and those no wave is left to claim, and `expired` says so.
 constexpr int STRIP_POLL_LIMIT = 1 << 22;
 
 // One pair of a launch: the diagonals lo..hi it sweeps (query letters less reference letters) and its place in the
@@ -48,7 +48,8 @@ struct StripArgs {
     unsigned long long *carry; // per pair and strip, `rows` boundary records (two words with two pieces), zero: not
                                // yet written
     int *claim;                // the strips claimed so far (zero at launch)
-    int *failed;               // per pair: set when a wait gave up (zero at launch)
+    int polls;                 // a wait gives up after this many
+    int *expired;              // the waits that gave up are added here (null: not counted)
     int *done;                 // free ends, per pair: the strips that have ended (zero at launch)
     unsigned long long *best;  // free ends, per pair: the least cost and its diagonal's rank (all ones at launch)
 };

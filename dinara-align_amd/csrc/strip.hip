@@ -18,7 +18,8 @@
 // 0's borders are made the same way. So a pair's strips run as a pipeline over the whole chip, each 64 C + 128 rows or so behind the one to its left, and one
 // launch takes every pair of a round, whatever its band. Waves claim strips in the host's order, in which a strip
 // always follows the one to its left (which is then held by a running wave), the pairs with the most strips first (their
-// pipelines are the launch's longest chains); every wait gives up after STRIP_POLL_LIMIT polls.
+// pipelines are the launch's longest chains); every wait gives up after STRIP_POLL_LIMIT
+// polls, and the host sweeps the pairs that leaves unsettled whole.
 //
 // The reference's letters pass through a ring in LDS, 64 written every 64 steps and loaded 64 steps before that; the
 // lane's query letters sit in registers. Between refills a step is the cells, two DPP moves, the letter's read and the
@@ -241,7 +242,7 @@ __device__ __forceinline__ bool sweep_strip(const StripArgs &a, const StripPair 
             }
             const bool missing = want && (record == 0 || (P == 2 && record2 == 0));
             if (__ballot(missing) == 0) break;
-            if (polls > STRIP_POLL_LIMIT) return false;
+            if (polls > a.polls) return false;
             __builtin_amdgcn_s_sleep(2);
         }
         left_h = want ? uncarried((uint32_t)(record >> 32)) : FAR;
@@ -461,7 +462,7 @@ __global__ __launch_bounds__(64) void strip_sweep(StripArgs a) {
             default: swept = sweep_strip<8, P, RECORD, SH, FREE>(a, p, pair, strip, ring, ending); break;
         }
         if (!swept) {
-            if (threadIdx.x == 0) atomicExch(a.failed + pair, 1);
+            if (threadIdx.x == 0 && a.expired) atomicAdd(a.expired, 1);
             return;
         }
         if (ending.mine) finish_pair<FREE>(a, p, at, ending);

@@ -103,7 +103,7 @@ def test_banded_strips_of_every_width(costs, columns, monkeypatch):
 
 
 def resident(refs, qrys, costs, kind, mode=None):
-    """A resident batch's results of two runs through the C ABI, and the launches of a run."""
+    """A resident batch's results of two runs through the C ABI, the launches of a run and its pairs swept whole."""
     handle = _lib.lib()
     R, Q = _lib.Texts(refs), _lib.Texts(qrys)
     c, status = costs.as_c(), ctypes.c_int64(0)
@@ -127,7 +127,7 @@ def resident(refs, qrys, costs, kind, mode=None):
             for a in found:
                 handle.dinara_free(a.cigar)
         assert runs[0] == runs[1]
-        return runs[0], handle.dinara_batch_stat(batch, 2)
+        return runs[0], handle.dinara_batch_stat(batch, 2), handle.dinara_batch_stat(batch, 10)
     finally:
         handle.dinara_batch_free(batch)
 
@@ -156,3 +156,20 @@ def test_rounds_cut_into_parts(costs, monkeypatch):
             assert got[0] == right, (name, budget)
             launches = whole.setdefault(name, got[1])
             assert budget is None or got[1] > launches, (name, budget, got[1], launches)
+
+
+@pytest.mark.parametrize("costs", COSTS, ids=IDS)
+def test_pairs_of_expired_waits_are_swept_whole(costs, monkeypatch):
+    # Waits that give up at once (as one would after seconds): every kernel ends, and the pairs that leaves unsettled,
+    # all of them short enough for a band to settle, take the whole-matrix path.
+    rng = random.Random(23)
+    oc = to_oracle(costs)
+    refs = [letters(rng, rng.randint(2200, 2700)) for _ in range(12)] + [letters(rng, 90) for _ in range(20)]
+    qrys = [mutated(r, rate, rng) for r, rate in zip(refs, [0.01, 0.1, 0.3, 0.5] * 8)]
+    want = [o.costs_align(r, q, oc) for r, q in zip(refs, qrys)]
+    assert resident(refs, qrys, costs, 1)[2] == 0
+    monkeypatch.setenv("DINARA_STRIP_POLLS", "0")
+    for kind in (0, 1):
+        got, _, whole = resident(refs, qrys, costs, kind)
+        assert got == (want if kind else [cost for cost, _ in want])
+        assert whole > 0
