@@ -123,8 +123,7 @@ __device__ __forceinline__ bool certify_ends(const SweepArgs &a, int rows, int c
 __device__ __forceinline__ void file_retry(const SweepArgs &a, int slot, int letters, int want_low, int want_high) {
     a.want_low[slot] = want_low;
     a.want_high[slot] = want_high;
-    const int cls = band_class(want_high - want_low + 1, letters, a.user_band != 0, a.group_max_letters, a.strip_letters,
-                               a.strip_widest);
+    const int cls = band_class(want_high - want_low + 1, letters, a.user_band != 0, a.limits);
     // A wave sweep stages both sequences in LDS: a pair they overflow has no class to go to.
     if (cls == CLASS_TOO_WIDE || (band_is_wave(cls) && letters > a.lds_limit)) {
         a.status[slot] = 2;

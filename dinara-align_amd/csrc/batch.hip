@@ -177,10 +177,8 @@ struct dinara_batch {
     DeviceContext *ctx = nullptr;
     int max_letters = 0;                  // the most letters of a pair, both sequences
     int32_t max_rows = 0;
-    int group_letters = 4;                // LDS bytes a pair takes in a group launch
-    int group_max_letters = 0;            // the longest pair a group launch stages (0: no groups)
     int group16_top = 0;                  // > 0: packed 16-bit group cells, this the unreachable value
-    int strip_letters = 0, strip_widest = 0;  // the pairs and bands the strips take (SweepArgs)
+    BandLimits limits{};                  // which pairs take which bands
     int64_t dearest = 1;                  // the dearest single step: a substitution or a gap's first letter
     // Free ends (wave sweeps): the letters each end of each sequence may leave out (reference start, end, query
     // start, end), the phase a run is in (1 the forward phase finding cost and end, 2 the anchored phase keeping
@@ -264,18 +262,25 @@ int64_t unit_lists(dinara_batch *b);
 int64_t unit_buffers(dinara_batch *b, const std::vector<int32_t> &lists, const std::vector<int32_t> &counts,
                      size_t cap);
 
-// Letters' room a group pair stages besides its own (sweep_group): 132 before, 9 between and 131 past.
+// Letters' room a group pair stages besides its own (sweep_group): 132 before, 9 between and 131 past; and its LDS bytes
+// (twice as many in packed cells) where the launch's longest pair has `letters`.
 constexpr int GROUP_ROOM = 272;
+constexpr int64_t LDS_BYTES = 160 << 10;  // a compute unit's
+int group_region(int64_t letters) { return (int)((letters + GROUP_ROOM + 3) & ~int64_t(3)); }
 
-// Which of a batch's pairs take group bands (prepare): those up to GROUP_LETTERS letters, and of a batch of more pairs
-// than a launch needs for a wave on each SIMD (256 compute units of four, four pairs a wave) those no longer than its
-// GROUP_PAIRS-th longest.
-constexpr int64_t GROUP_PAIRS = 4096, GROUP_LETTERS = 4096;
+// Which pairs take which bands (prepare).
+//
+// A group launch is four pairs a wave, each a chain over its anti-diagonals: it takes as long as its longest pair, at
+// any number of pairs up to a wave on each SIMD. A strip round takes as long as its strips' cells, as long as a group
+// chain of as many letters as so many pairs' on average (CIGARs, whose strips write more decisions, have their own). So
+// of the pairs past GROUP_LETTERS letters the longest go to the strips, down to the length that makes the two least
+// together. Groups against strips, ms: 500 pairs of 2.5 kbp at 1% 1.2 and 1.2 (CIGARs 4.2 and 4.0), 2,000 of 5 kbp 4.9
+// and 3.1 (13.0 and 9.1), 4,096 of 2.5 kbp 2.0 and 1.9 (6.8 and 7.9), 20,000 of 2.5 kbp 3.1 and 5.5 (12.5 and 21.3).
+constexpr int64_t GROUP_LETTERS = 4096, GROUP_PAIRS_COSTS = 4096, GROUP_PAIRS_CIGARS = 3072;
 
 // The class of a slot's first band of `need` diagonals.
 int first_class(const dinara_batch *b, int64_t s, int need) {
-    return band_class(need, (int64_t)b->rows[s] + b->cols[s], b->user_band, b->group_max_letters, b->strip_letters,
-                      b->strip_widest);
+    return band_class(need, (int64_t)b->rows[s] + b->cols[s], b->user_band, b->limits);
 }
 
 // Builds the tape: pairs by length, longest first, 64 to a group, each group's words transposed.
@@ -418,32 +423,55 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         b->max_letters = std::max<int>(b->max_letters, b->rows[s] + b->cols[s]);
     }
     // A group pair's LDS region: both sequences, and room for reads up to half the widest group band (256) before the
-    // reference and past the query (group.hip). Pairs up to a quarter of the LDS may take group bands. A group launch
-    // is four pairs a wave, each a chain over its anti-diagonals, so the batch's longest pairs, too few to give every
-    // SIMD a wave, are chains with nothing beside them: those past GROUP_LETTERS letters take the strips, whose chain is a row a step
-    // (361 pairs of up to 16,000 letters in 256 diagonals: 8.9 ms as groups; 2,000 uneven pairs whole: 14.5 ms, 11.1 with
-    // these in strips). Beyond that many pairs the groups' cells cost half as much.
-    int64_t group_cap = (int64_t)(b->lds_limit / 4) - GROUP_ROOM - 4;
-    {
-        const int64_t last = std::min<int64_t>(slots, GROUP_PAIRS) - 1;
-        group_cap = std::min(group_cap, std::max<int64_t>(GROUP_LETTERS, slots > GROUP_PAIRS
-                                                                             ? (int64_t)b->rows[last] + b->cols[last]
-                                                                             : 0));
+    // reference and past the query (group.hip). The group sweep holds costs times 16 with a tag and runs up to half its
+    // widest band past the corner: every value it makes stays under 2^30. It holds one gap piece and no free ends.
+    int64_t letters_in_all = 0;
+    for (int64_t s = 0; s < slots; ++s) letters_in_all += (int64_t)b->rows[s] + b->cols[s];
+    const auto longest_up_to = [&](int64_t cap) {
+        int longest = 0;
+        for (int64_t s = 0; s < slots; ++s)
+            if (b->rows[s] + b->cols[s] <= cap) longest = std::max(longest, b->rows[s] + b->cols[s]);
+        return longest;
+    };
+    b->limits = BandLimits{};
+    if (!b->parsed.two_piece && !b->free_ends) {
+        const int64_t staged = (int64_t)(b->lds_limit / 4) - GROUP_ROOM - 4;
+        const bool cigars = b->kind == DINARA_BATCH_ALIGNMENTS;
+        std::vector<int32_t> longs;
+        int64_t strips = 0;  // those pairs' strips of four columns a lane
+        for (int64_t s = 0; s < slots; ++s) {
+            const int32_t letters = b->rows[s] + b->cols[s];
+            if (letters <= GROUP_LETTERS || letters > staged) continue;
+            longs.push_back(letters);
+            strips += b->cols[s] / strip_columns(4) + 1;
+        }
+        // The cap that makes least the group launch's chain and the strips' work beside it.
+        std::sort(longs.begin(), longs.end(), std::greater<int32_t>());
+        int64_t cap = GROUP_LETTERS, in_strips = 0, least = INT64_MAX;
+        for (size_t i = 0; i <= longs.size(); ++i) {
+            const int64_t chain = i < longs.size() ? longs[i] : (int64_t)longs.size() < slots ? GROUP_LETTERS : 0;
+            const int64_t cost = chain + in_strips / (cigars ? GROUP_PAIRS_CIGARS : GROUP_PAIRS_COSTS);
+            if (cost <= least) {
+                least = cost;
+                cap = std::max(chain, GROUP_LETTERS);
+            }
+            if (i < longs.size()) in_strips += longs[i];
+        }
+        const auto tags_fit = [&](int longest) {
+            return ((int64_t)longest + 2 * 256 + 8) * b->dearest < REAL_LIMIT ? longest : 0;
+        };
+        b->limits.group_letters = tags_fit(longest_up_to(std::min(staged, cap)));
+        // The first band is a narrow one: a short chain, which proves a pair of few errors. Few pairs' CIGARs, whose
+        // strips all run at once, go to the strips with it (and are walked a wave a pair): 64 of 2.5 kbp at 1% 3.3 ms as
+        // groups, 1.5 so.
+        b->limits.group_narrow = b->limits.group_letters;
+        if (!cigars || strips > STRIP_GRID / 2)
+            b->limits.group_narrow = std::max(b->limits.group_letters, tags_fit(longest_up_to(staged)));
     }
-    b->group_max_letters = 0;
-    for (int64_t s = 0; s < slots; ++s)
-        if (b->rows[s] + b->cols[s] <= group_cap)
-            b->group_max_letters = std::max(b->group_max_letters, b->rows[s] + b->cols[s]);
-    b->group_letters = (b->group_max_letters + GROUP_ROOM + 3) & ~3;
-    // The group sweep holds costs times 16 with a tag (group.hip) and runs up to half its widest band past the
-    // corner: every value it makes stays under 2^30. It holds one gap piece and no free ends.
-    if (b->parsed.two_piece || b->free_ends || group_cap <= 0 || (size_t)4 * b->group_letters > b->lds_limit ||
-        ((int64_t)b->group_max_letters + 2 * 256 + 8) * b->dearest >= REAL_LIMIT)
-        b->group_max_letters = 0;
     // The strips take bands of pairs up to 65,536 letters, free ends' up to 2,048 diagonals; longer pairs and wider
     // bands are swept whole after the run.
-    b->strip_letters = 65536;
-    b->strip_widest = b->free_ends ? 2048 : band_width(CLASSES - 1);
+    b->limits.strip_letters = 65536;
+    b->limits.strip_widest = b->free_ends ? 2048 : band_width(CLASSES - 1);
     // Packed 16-bit group cells (group.hip) for shifted costs (equal extensions e) whose mismatch is no dearer than
     // two extension letters: a tagged value then lies in [-16 e (n + m), 32 opening + 15]. A cell no path reaches starts
     // at `top` on the two anti-diagonals before (0, 0)'s and loses at most 32 e a diagonal step: on anti-diagonal t it
@@ -455,9 +483,10 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         const CostParams &k = b->costs;
         const int64_t e = k.del_ext, opening = std::max(k.del_open, k.ins_open);
         const int64_t top = (32767 - 16 * opening - 32) & ~int64_t(15);
-        if (b->group_max_letters > 0 && !std::getenv("DINARA_GROUP_CELLS32") && k.pieces != 2 && k.del_ext == k.ins_ext &&
+        const int64_t longest = b->limits.group_letters;
+        if (longest > 0 && !std::getenv("DINARA_GROUP_CELLS32") && k.pieces != 2 && k.del_ext == k.ins_ext &&
             e >= 0 && k.mismatch >= 0 && k.mismatch <= 2 * e && std::min(k.del_open, k.ins_open) >= 0 &&
-            16 * e * (b->group_max_letters + 2) + 32 * opening + 15 < top - 64 && (size_t)8 * b->group_letters <= b->lds_limit)
+            16 * e * (longest + 2) + 32 * opening + 15 < top - 64 && (size_t)8 * group_region(longest) <= b->lds_limit)
             b->group16_top = (int)top;
     }
     // The first band: the lanes' start and end diagonals and one either side (lanes.mojo:1207-1215), within the
@@ -599,12 +628,9 @@ SweepArgs sweep_args(dinara_batch *b) {
     a.walk_low = static_cast<int32_t *>(b->walk_low.ptr);
     a.walk_class = static_cast<int32_t *>(b->walk_class.ptr);
     a.walk_flags = static_cast<uint64_t *>(b->walk_flags.ptr);
-    a.group_letters = b->group_letters;
     a.doubling = b->doubling ? 1 : 0;
-    a.group_max_letters = b->group_max_letters;
     a.group16_top = b->group16_top;
-    a.strip_letters = b->strip_letters;
-    a.strip_widest = b->strip_widest;
+    a.limits = b->limits;
     a.cigar_scratch = static_cast<char *>(b->cigar_scratch.ptr);
     a.cigar_scratch_base = static_cast<const int64_t *>(b->cigar_scratch_base.ptr);
     a.cigars = static_cast<char *>(b->cigars.ptr);
@@ -632,23 +658,25 @@ SweepArgs sweep_args(dinara_batch *b) {
 }
 
 
-// Launches class `cls` over `count` slots listed at `list` (device memory), filing retries where `round` says. Each
-// launch keeps its decisions in an arena of its own, a fixed stride a listed pair, until the
-// walk; a launch whose arena would pass the budget is cut in pieces. `arena_index` counts the run's arenas.
-int64_t launch_class(dinara_batch *b, const SweepArgs &round, int cls, const int32_t *list, int64_t count,
+// Launches class `cls` over `count` slots listed at `list` (device memory), the longest of `longest` letters, filing
+// retries where `round` says. Each launch keeps its decisions in an arena of its own, a fixed stride a listed pair, until
+// the walk; a launch whose arena would pass the budget is cut in pieces. `arena_index` counts the run's arenas.
+int64_t launch_class(dinara_batch *b, const SweepArgs &round, int cls, const int32_t *list, int64_t count, int longest,
                      size_t &arena_index, hipStream_t stream) {
     SweepArgs a = round;
     a.cls = cls;
     const bool wave = class_is_wave(cls);
-    const size_t lds = wave ? (size_t)std::min<int>(std::max(b->max_letters, 4), (int)b->lds_limit)
-                            : (size_t)(b->group16_top > 0 && cls >= 1 ? 8 : 4) * b->group_letters;
+    a.group_letters = group_region(longest);
+    if (longest > b->limits.group_letters) a.group16_top = 0;  // past the packed cells' bound
+    const size_t lds = wave ? (size_t)std::min<int>(std::max(longest, 4), (int)b->lds_limit)
+                            : (size_t)(a.group16_top > 0 && cls >= 1 ? 8 : 4) * a.group_letters;
     int64_t chunk = count;
     size_t stride = 0;
     if (a.record) {
-        // The batch's largest pair bounds every pair's decisions: rows for a wave band, tiles of 32
+        // The launch's longest pair bounds every pair's decisions: rows for a wave band, tiles of 32
         // anti-diagonals (16 bytes a diagonal pair) for a group's.
-        const int64_t bytes = wave ? (int64_t)b->max_rows * class_width(cls)
-                                   : ((int64_t)b->max_letters / 32 + 1) * (class_width(cls) / 2) * 16;
+        const int64_t bytes = wave ? (int64_t)std::min<int>(b->max_rows, longest) * class_width(cls)
+                                   : ((int64_t)longest / 32 + 1) * (class_width(cls) / 2) * 16;
         stride = ((size_t)bytes + 255) & ~size_t(255);
         chunk = std::max<int64_t>(1, (int64_t)std::min<size_t>(count, ARENA_BUDGET / std::max<size_t>(stride, 1)));
     }
@@ -680,6 +708,9 @@ int strip_c(int64_t m) { return m <= strip_columns(2) ? 2 : m <= strip_columns(4
 // 2,000 uneven pairs (8,192 strips) 11.1 -> 10.5 ms, 1,000 two-piece CIGARs 11.9 -> 9.9; two a lane 11.6 and 10.7. A
 // round that fills the chip pays for its cells: 200,000 uneven pairs 236 ms with eight, 251 with four.
 constexpr int64_t FEW_STRIPS = 16384;
+// Whatever their number, strips of four where costs alone are kept and the band is narrower than this: a strip's rows
+// are its band's and its columns'. 4,000 pairs of 3 kbp at 5% 4.4 -> 3.9 ms; their CIGARs 13.1 -> 16.5, so not those.
+constexpr int NARROW_BAND = 512;
 
 // A strip launch's parts: consecutive pairs of the plan whose decisions and carry records fit ARENA_BUDGET together. A
 // round of costs keeps no decisions, but each pair's carry records (8 bytes a row a strip, 16 under two pieces; 0.8 MB
@@ -706,13 +737,13 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
     StripPlan plan;
     const int pieces = b->costs.pieces == 2 ? 2 : 1;
     const bool views = b->free_ends;
-    int widest_c = 8;
+    int widest_c = 8, narrow_c = round && !record ? 4 : 8;
     if (const char *set = std::getenv("DINARA_STRIP_COLUMNS")) {  // for checking: 2, 4 or 8 at most
-        widest_c = std::strtol(set, nullptr, 10) <= 2 ? 2 : std::strtol(set, nullptr, 10) <= 4 ? 4 : 8;
+        widest_c = narrow_c = std::strtol(set, nullptr, 10) <= 2 ? 2 : std::strtol(set, nullptr, 10) <= 4 ? 4 : 8;
     } else if (round) {
         int64_t strips = 0;
         for (const int4 &band : bands) strips += b->cols[band.x] / strip_columns(8) + 1;
-        if (strips <= FEW_STRIPS) widest_c = 4;
+        if (strips <= FEW_STRIPS) widest_c = narrow_c = 4;
     }
     size_t budget = ARENA_BUDGET;
     if (const char *set = std::getenv("DINARA_STRIP_BUDGET")) budget = std::strtoull(set, nullptr, 10);
@@ -728,7 +759,7 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
             p.slot = band.x;
             p.lo = band.y;
             p.hi = band.z;
-            p.c = std::min(strip_c(m), widest_c);
+            p.c = std::min(strip_c(m), p.hi - p.lo + 1 < NARROW_BAND ? narrow_c : widest_c);
             p.strips = (int)std::max<int64_t>(1, (m + strip_columns(p.c) - 1) / strip_columns(p.c));
             p.rows = (int)std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)p.hi - p.lo + strip_columns(p.c)));
             const size_t records = (size_t)p.strips * p.rows * 64;
@@ -1304,6 +1335,9 @@ int4 first_strip_band(const dinara_batch *b, int32_t s) {
     return make_int4(s, lo, hi, 0);
 }
 
+// Where, among the classes' timing events, those of a group class's long pairs are (a strip class's, which has none).
+constexpr int LONG_PART = CLASS_STRIP_FIRST + 1;
+
 // Sweeps every slot of the first lists until each is settled or left unsettled: want bands from first_low_d /
 // first_high_d, round 0 the first lists, each later round the lists the round before filed, kept on the device,
 // two sets taking turns. Only the counts come back to the host, and the pairs filed for strips, which the host plans.
@@ -1355,8 +1389,10 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             forked[k] = true;
             return ctx->side(k - 1);
         };
+        bool was_timed[CLASSES] = {};
         const auto timed = [&](int c, auto launch) -> int64_t {
             hipStream_t stream = next_stream();
+            was_timed[c] = true;
             (void)hipEventRecord(ctx->event(2 * c), stream);
             if (const int64_t code = launch(stream)) return code;
             (void)hipEventRecord(ctx->event(2 * c + 1), stream);
@@ -1364,7 +1400,7 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         };
         if (!strips.empty()) {
             for (const int4 &band : strips) {
-                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, 0, 1, 1 << 20));
+                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, BandLimits{0, 0, 1, 1 << 20}));
                 b->class_pairs[cls] += 1;
             }
             b->class_launches[CLASS_STRIP_FIRST] += 1;
@@ -1377,10 +1413,32 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             if (counts[c] == 0) continue;
             const int32_t *list = round == 0 ? static_cast<const int32_t *>(b->first_lists_d.ptr) + b->first_offset[c]
                                              : in_lists + (size_t)c * capacity;
-            if (const int64_t code = timed(c, [&](hipStream_t stream) {
-                    return launch_class(b, a, c, list, counts[c], arena_index, stream);
-                }))
-                return code;
+            // The narrow group bands' long pairs (the first of their list, longest side first) in a launch of their own
+            // where the list would not all run at once with the LDS they take: the letters a launch stages are its
+            // longest pair's.
+            int64_t longs = 0;
+            if (c <= CLASS_GROUP64 && round == 0 && b->limits.group_narrow > b->limits.group_letters) {
+                for (int64_t i = 0; i < counts[c]; ++i) {
+                    const int32_t s = b->first_lists[c][i];
+                    if (b->rows[s] + b->cols[s] > b->limits.group_letters) longs = i + 1;
+                }
+                const int64_t at_once = LDS_BYTES / (4 * group_region(b->limits.group_narrow)) * ctx->compute_units;
+                if (longs > 0 && (counts[c] + 3) / 4 <= at_once) longs = counts[c];
+            }
+            const int longest = band_is_wave(c) ? b->max_letters
+                                : c <= CLASS_GROUP64 && (longs > 0 || round > 0) ? b->limits.group_narrow
+                                                                                 : b->limits.group_letters;
+            if (longs > 0)
+                if (const int64_t code = timed(LONG_PART + c, [&](hipStream_t stream) {
+                        return launch_class(b, a, c, list, longs, longest, arena_index, stream);
+                    }))
+                    return code;
+            if (counts[c] > longs)
+                if (const int64_t code = timed(c, [&](hipStream_t stream) {
+                        return launch_class(b, a, c, list + longs, counts[c] - longs,
+                                            longs > 0 ? b->limits.group_letters : longest, arena_index, stream);
+                    }))
+                    return code;
         }
         for (int k = 1; k < SWEEP_STREAMS; ++k) {
             if (!forked[k]) continue;
@@ -1396,12 +1454,13 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         (void)hipEventElapsedTime(&ms, ctx->sweep_start, ctx->sweep_stop);
         b->sweep_ms += ms;
         int64_t retried = 0;
+        for (int c = 0; c <= LONG_PART + CLASS_GROUP64; ++c) {
+            if (!was_timed[c]) continue;
+            float class_ms = 0;
+            (void)hipEventElapsedTime(&class_ms, ctx->event(2 * c), ctx->event(2 * c + 1));
+            b->class_ms[c < LONG_PART ? c : c - LONG_PART] += class_ms;
+        }
         for (int c = 0; c <= CLASS_STRIP_FIRST; ++c) {
-            if (c == CLASS_STRIP_FIRST ? !strips.empty() : counts[c] > 0) {
-                float class_ms = 0;
-                (void)hipEventElapsedTime(&class_ms, ctx->event(2 * c), ctx->event(2 * c + 1));
-                b->class_ms[c] += class_ms;
-            }
             counts[c] = filed[c];
             retried += filed[c];
         }

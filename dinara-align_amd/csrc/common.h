@@ -45,6 +45,7 @@ struct Tape {
 // 64Q (Q = 1..32, sweep.hip) for every pair under a user band; and strip bands (strip.hip), 512 to 16384 diagonals by
 // width, which one launch a round takes together.
 constexpr int CLASS_GROUP32 = 0;
+constexpr int CLASS_GROUP64 = 1;
 constexpr int CLASS_GROUP256 = 3;
 constexpr int CLASS_WAVE_FIRST = 4;  // Q = 1, 2, 4, 8, 16, 32 for classes 4..9
 constexpr int CLASS_WAVE_LAST = 9;
@@ -65,23 +66,27 @@ __host__ __device__ constexpr int band_width(int cls) {
 __host__ __device__ constexpr bool band_is_wave(int cls) { return cls >= CLASS_WAVE_FIRST && cls <= CLASS_WAVE_LAST; }
 __host__ __device__ constexpr bool band_is_strip(int cls) { return cls >= CLASS_STRIP_FIRST; }
 
+// Which pairs take which bands, in letters (both sequences): group bands of up to 64 diagonals up to `group_narrow`, every group
+// band up to `group_letters` (0 where no pair takes them), strips up to `strip_letters` and bands `strip_widest` wide.
+struct BandLimits {
+    int group_narrow, group_letters, strip_letters, strip_widest;
+};
+
 // The class of band a pair of `letters` letters needing `need` diagonals takes: the narrowest that holds them. A group
 // band is placed on an even diagonal, so it holds one diagonal fewer than its width. Pairs under a user band take the
-// wave bands, which bar diagonals outside it; pairs longer than a group launch stages (`group_letters`, 0 where no
-// group takes the batch) the strips, up to `strip_letters` letters and bands `strip_widest` wide.
-__host__ __device__ inline int band_class(int need, int64_t letters, bool user_band, int group_letters,
-                                          int strip_letters, int strip_widest) {
+// wave bands, which bar diagonals outside it.
+__host__ __device__ inline int band_class(int need, int64_t letters, bool user_band, const BandLimits &limits) {
     if (user_band) {
         for (int cls = CLASS_WAVE_FIRST; cls <= CLASS_WAVE_LAST; ++cls)
             if (need <= band_width(cls)) return cls;
         return CLASS_TOO_WIDE;
     }
-    if (group_letters > 0 && letters <= group_letters)
-        for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
-            if (need < band_width(cls)) return cls;
-    if (letters <= strip_letters)
+    for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
+        if (letters <= (cls <= CLASS_GROUP64 ? limits.group_narrow : limits.group_letters) && need < band_width(cls))
+            return cls;
+    if (letters <= limits.strip_letters)
         for (int cls = CLASS_STRIP_FIRST; cls < CLASSES; ++cls)
-            if (need <= band_width(cls) && band_width(cls) <= strip_widest) return cls;
+            if (need <= band_width(cls) && band_width(cls) <= limits.strip_widest) return cls;
     return CLASS_TOO_WIDE;
 }
 
@@ -115,11 +120,9 @@ struct SweepArgs {
     int64_t arena_stride;
     uint64_t *walk_flags;    // per slot: the address of its settled band's decisions
     int group_letters;       // LDS bytes a pair takes in a group launch (four pairs a block)
-    int group_max_letters;   // the longest pair (both sequences) a group launch stages (0: none); longer take strips
     int group16_top;         // > 0: group launches of two slots a lane and more hold their steady cells as 16-bit
                              // halves, `group16_top` the unreachable value (letters then take 2 bytes each in LDS)
-    int strip_letters;       // the most letters (both sequences) of a pair the strips take in bands
-    int strip_widest;        // and the widest of those bands
+    BandLimits limits;       // which pairs take which bands
     // CIGARs: each slot's scratch run of 2(n+m)+2 bytes from cigar_scratch_base, compacted into `cigars` at an
     // offset taken from `cigar_used`
     char *cigar_scratch;

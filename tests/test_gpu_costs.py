@@ -311,6 +311,29 @@ def test_block_bands_one_and_several_waves():
     check_distances(refs, qrys, da.Costs.edit())
 
 
+@pytest.mark.parametrize("shorts", [40, 2600])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_long_pairs_beside_short_ones(shorts, kind):
+    # Pairs past 4,096 letters take a narrow group band first (with few of them, costs alone; their CIGARs go to the
+    # strips at once): beside so many short pairs that those would not all run with the letters the long ones stage, in a
+    # launch of their own. Close pairs are settled there, the others in strips.
+    rng = random.Random(53 + shorts)
+    costs = da.Costs.affine(4, 6, 2)
+    refs, qrys = random_pairs(shorts, rng, lengths=(20, 110), rates=(0.0, 0.02, 0.1, 0.3))
+    for n, rate in [(7900, 0.0005), (2300, 0.001), (5200, 0.0005), (2100, 0.03), (4000, 0.02), (2049, 0.0), (2048, 0.0)]:
+        r = "".join(rng.choice("ACGT") for _ in range(n))
+        refs.append(r)
+        qrys.append(mutated(r, rate, rng) if rate else r)
+    swept = class_pairs(refs, qrys, costs, kind)
+    assert swept[1] >= shorts and sum(swept[10:]) > 0
+    assert (swept[1] > shorts + 1) == (kind == 0), swept
+    if kind:
+        check_alignments(refs, qrys, costs)
+        check_alignments(refs, qrys, costs, ties="right")
+    else:
+        check_distances(refs, qrys, costs)
+
+
 def test_widest_band_distances():
     # First bands past 8192 diagonals: the 12288- and 16384-diagonal blocks, distances only.
     rng = random.Random(41)
