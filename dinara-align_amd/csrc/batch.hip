@@ -278,6 +278,13 @@ int group_region(int64_t letters) { return (int)((letters + GROUP_ROOM + 3) & ~i
 // and 3.1 (13.0 and 9.1), 4,096 of 2.5 kbp 2.0 and 1.9 (6.8 and 7.9), 20,000 of 2.5 kbp 3.1 and 5.5 (12.5 and 21.3).
 constexpr int64_t GROUP_LETTERS = 4096, GROUP_PAIRS_COSTS = 4096, GROUP_PAIRS_CIGARS = 3072;
 
+// The narrowest wave band, a row a step of a pair's own wave, against one strip of the whole matrix and its 63 steps of
+// lanes coming in and going out: the pairs whose strips would take longer than the longest pair's rows. Two pieces, wave
+// against strips, ms: 20,000 pairs of 150 bp 0.67 and 1.12, 3,000 of 600 0.97 and 1.10, 5,000 of 1,000 1.7 and 2.6, 1,000
+// of 1,500 at 0.5% 1.6 and 1.3. The next wider one takes the same pairs' retries (5,000 CIGARs of 1,000 4.9 -> 4.5), under
+// free ends, whose first bands are wide, short pairs alone: reads of 100 with a free reference end 0.69 and 1.03.
+constexpr int64_t WAVE_LETTERS = 512, WAVE_LETTERS_MOST = 8192, WAVE_PAIRS = 2560, WAVE128_LETTERS = 320;
+
 // The class of a slot's first band of `need` diagonals.
 int first_class(const dinara_batch *b, int64_t s, int need) {
     return band_class(need, (int64_t)b->rows[s] + b->cols[s], b->user_band, b->limits);
@@ -434,7 +441,12 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         return longest;
     };
     b->limits = BandLimits{};
-    if (!b->parsed.two_piece && !b->free_ends) {
+    if (b->parsed.two_piece || b->free_ends) {
+        const int64_t cap = std::min(std::max(WAVE_LETTERS, letters_in_all / WAVE_PAIRS), WAVE_LETTERS_MOST);
+        b->limits.wave_letters = longest_up_to(std::min(cap, (int64_t)b->lds_limit));
+        b->limits.wave128_letters =
+            b->free_ends ? (int)std::min<int64_t>(b->limits.wave_letters, WAVE128_LETTERS) : b->limits.wave_letters;
+    } else {
         const int64_t staged = (int64_t)(b->lds_limit / 4) - GROUP_ROOM - 4;
         const bool cigars = b->kind == DINARA_BATCH_ALIGNMENTS;
         std::vector<int32_t> longs;
@@ -1400,7 +1412,7 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         };
         if (!strips.empty()) {
             for (const int4 &band : strips) {
-                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, BandLimits{0, 0, 1, 1 << 20}));
+                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, BandLimits{0, 0, 0, 0, 1, 1 << 20}));
                 b->class_pairs[cls] += 1;
             }
             b->class_launches[CLASS_STRIP_FIRST] += 1;
@@ -1425,7 +1437,9 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
                 const int64_t at_once = LDS_BYTES / (4 * group_region(b->limits.group_narrow)) * ctx->compute_units;
                 if (longs > 0 && (counts[c] + 3) / 4 <= at_once) longs = counts[c];
             }
-            const int longest = band_is_wave(c) ? b->max_letters
+            const int longest = band_is_wave(c) ? (b->user_band              ? b->max_letters
+                                                   : c == CLASS_WAVE_FIRST ? b->limits.wave_letters
+                                                                           : b->limits.wave128_letters)
                                 : c <= CLASS_GROUP64 && (longs > 0 || round > 0) ? b->limits.group_narrow
                                                                                  : b->limits.group_letters;
             if (longs > 0)

@@ -67,9 +67,10 @@ __host__ __device__ constexpr bool band_is_wave(int cls) { return cls >= CLASS_W
 __host__ __device__ constexpr bool band_is_strip(int cls) { return cls >= CLASS_STRIP_FIRST; }
 
 // Which pairs take which bands, in letters (both sequences): group bands of up to 64 diagonals up to `group_narrow`, every group
-// band up to `group_letters` (0 where no pair takes them), strips up to `strip_letters` and bands `strip_widest` wide.
+// band up to `group_letters`, the wave band of 64 diagonals up to `wave_letters` and that of 128 up to
+// `wave128_letters` (0 where no pair takes them), strips up to `strip_letters` and bands `strip_widest` wide.
 struct BandLimits {
-    int group_narrow, group_letters, strip_letters, strip_widest;
+    int group_narrow, group_letters, wave_letters, wave128_letters, strip_letters, strip_widest;
 };
 
 // The class of band a pair of `letters` letters needing `need` diagonals takes: the narrowest that holds them. A group
@@ -81,6 +82,9 @@ __host__ __device__ inline int band_class(int need, int64_t letters, bool user_b
             if (need <= band_width(cls)) return cls;
         return CLASS_TOO_WIDE;
     }
+    for (int cls = CLASS_WAVE_FIRST; cls <= CLASS_WAVE_FIRST + 1; ++cls)
+        if (letters <= (cls == CLASS_WAVE_FIRST ? limits.wave_letters : limits.wave128_letters) && need <= band_width(cls))
+            return cls;
     for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
         if (letters <= (cls <= CLASS_GROUP64 ? limits.group_narrow : limits.group_letters) && need < band_width(cls))
             return cls;

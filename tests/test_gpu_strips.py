@@ -102,6 +102,38 @@ def test_banded_strips_of_every_width(costs, columns, monkeypatch):
     assert da.distances(refs, qrys, costs) == [o.costs_cost(r, q, oc) for r, q in zip(refs, qrys)]
 
 
+@pytest.mark.parametrize("free", [None, da.Mode.ends_free(4, 3, 2, 5), da.Mode.PREFIX])
+@pytest.mark.parametrize("costs", COSTS[:2], ids=IDS[:2])
+def test_narrow_wave_bands_and_wider(costs, free):
+    # Under two pieces or free ends short pairs take wave bands of 64 diagonals and 128 (128 under free ends up to 320
+    # letters, the narrower up to the pairs' mean at least), others strips: first bands of 62 to 66 and 126 to 130
+    # diagonals, retries into each, lengths around the limits.
+    rng = random.Random(29)
+    refs, qrys = [], []
+    for difference in (0, 1, 58, 59, 60, 61, 62, 63, 64, 122, 123, 124, 125, 126, 127, 128):
+        for m in (30, 96, 97, 190):
+            q = letters(rng, m)
+            cut = rng.randint(0, m)
+            refs.append(mutated(q[:cut], 0.05, rng) + letters(rng, difference) + q[cut:])
+            qrys.append(q)
+    for n, rate in [(150, 0.02), (150, 0.3), (255, 0.1), (257, 0.1), (257, 0.5), (400, 0.02), (900, 0.01), (2000, 0.002)]:
+        for _ in range(3):
+            r = letters(rng, n)
+            refs.append(r)
+            qrys.append(mutated(r, rate, rng))
+    refs += ["", "ACGT", ""]
+    qrys += ["ACG", "", ""]
+    oc, ends = to_oracle(costs), ends_of(free) if free else (0, 0, 0, 0)
+    for ties in ("left", "right"):
+        got = da.alignments(refs, qrys, costs, *([free] if free else []), ties=ties)
+        for i, (r, q) in enumerate(zip(refs, qrys)):
+            g = got[i]
+            assert (g.cost, g.cigar, (g.reference_start, g.reference_end, g.query_start, g.query_end)) == o.ends_align(
+                r, q, oc, ends, right_ties=ties == "right"), (i, len(r), len(q), ties)
+    assert da.distances(refs, qrys, costs, *([free] if free else [])) == [
+        o.ends_cost(r, q, oc, ends)[0] for r, q in zip(refs, qrys)]
+
+
 def resident(refs, qrys, costs, kind, mode=None):
     """A resident batch's results of two runs through the C ABI, the launches of a run and its pairs swept whole."""
     handle = _lib.lib()
