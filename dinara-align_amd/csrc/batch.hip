@@ -151,6 +151,17 @@ int64_t pair_code(const char *ref, int64_t n, const char *qry, int64_t m) {
 
 // ------------------------------------------------------------------ the batch
 
+// A strip round's parts, one launch each: consecutive pairs of its plan, and the memory the largest takes.
+struct StripPart {
+    size_t pair, pairs, strip, strips;
+    size_t decision_bytes, carry_words;
+};
+struct StripParts {
+    std::vector<StripPart> parts;
+    size_t pairs = 0, decision_bytes = 0, carry_words = 0;
+    int64_t class_pairs[CLASSES] = {};  // by the class of its band's width
+};
+
 struct dinara_batch {
     int gpu = 0;
     int64_t kind = DINARA_BATCH_DISTANCES;
@@ -254,6 +265,10 @@ struct dinara_batch {
     // The strip launches' plan (pairs, then the order their strips are claimed in) and memory, and the slots filed for
     // strip bands (two sets taking turns, as the retry lists).
     DeviceBuffer strip_plan, strip_counts, strip_best, strip_carry, strip_decisions, strip_retries;
+    // The first round's plan, on the device as long as the first bands stand (seeding moves them).
+    DeviceBuffer first_strip_plan;
+    StripParts first_strips;
+    bool first_strips_planned = false;
 };
 
 namespace {
@@ -277,7 +292,6 @@ int group_region(int64_t letters) { return (int)((letters + GROUP_ROOM + 3) & ~i
 // together. Groups against strips, ms: 500 pairs of 2.5 kbp at 1% 1.2 and 1.2 (CIGARs 4.2 and 4.0), 2,000 of 5 kbp 4.9
 // and 3.1 (13.0 and 9.1), 4,096 of 2.5 kbp 2.0 and 1.9 (6.8 and 7.9), 20,000 of 2.5 kbp 3.1 and 5.5 (12.5 and 21.3).
 constexpr int64_t GROUP_LETTERS = 4096, GROUP_PAIRS_COSTS = 4096, GROUP_PAIRS_CIGARS = 3072;
-
 // The narrowest wave band, a row a step of a pair's own wave, against one strip of the whole matrix and its 63 steps of
 // lanes coming in and going out: the pairs whose strips would take longer than the longest pair's rows. Two pieces, wave
 // against strips, ms: 20,000 pairs of 150 bp 0.67 and 1.12, 3,000 of 600 0.97 and 1.10, 5,000 of 1,000 1.7 and 2.6, 1,000
@@ -731,22 +745,32 @@ constexpr int NARROW_BAND = 512;
 // DINARA_STRIP_BUDGET sets the bytes a part may take, for checking.
 constexpr size_t CARRY_BUDGET = size_t(1) << 30;
 constexpr size_t FULL_GRIDS = 4;
-struct StripPart {
-    size_t pair, pairs, strip, strips;
-    size_t decision_bytes, carry_words;
-};
+// A round's plan on the host, the context's: made anew for each round (under its lock), its memory kept while it is small.
 struct StripPlan {
     std::vector<StripPair> pairs;
-    std::vector<int2> order;
-    std::vector<StripPart> parts;
-    size_t decision_bytes = 0, carry_words = 0;  // the largest part's
+    std::vector<int2> order;  // of the parts with a pair of several strips
+    std::vector<size_t> at;
 };
+constexpr size_t PLAN_KEPT = size_t(1) << 18;  // pairs, strips
+
+StripPlan &strip_plan_of(DeviceContext *ctx) {
+    if (!ctx->strip_plan) ctx->strip_plan = new StripPlan();
+    StripPlan &plan = *static_cast<StripPlan *>(ctx->strip_plan);
+    if (plan.pairs.capacity() > PLAN_KEPT) std::vector<StripPair>().swap(plan.pairs);
+    if (plan.order.capacity() > PLAN_KEPT) std::vector<int2>().swap(plan.order);
+    return plan;
+}
 
 // The plan of the pairs listed in `bands` (slot, low, high): each pair's strips, where its records lie, and the order
 // its strips are claimed in: the strips furthest from their pair's end first, so that the longest pipelines start first
 // and a strip always follows the one to its left. `round`: a round of bands, whose strips may be narrower.
-StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bool record, bool round) {
-    StripPlan plan;
+StripParts plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bool record, bool round) {
+    StripPlan &plan = strip_plan_of(b->ctx);
+    StripParts out;
+    plan.pairs.clear();
+    plan.order.clear();
+    plan.pairs.reserve(bands.size());
+    std::vector<size_t> &at = plan.at;
     const int pieces = b->costs.pieces == 2 ? 2 : 1;
     const bool views = b->free_ends;
     int widest_c = 8, narrow_c = round && !record ? 4 : 8;
@@ -759,7 +783,6 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
     }
     size_t budget = ARENA_BUDGET;
     if (const char *set = std::getenv("DINARA_STRIP_BUDGET")) budget = std::strtoull(set, nullptr, 10);
-    std::vector<size_t> at;
     for (size_t next = 0; next < bands.size();) {
         StripPart part{plan.pairs.size(), 0, plan.order.size(), 0, 0, 0};
         int most = 0;
@@ -789,7 +812,13 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
             ++part.pairs;
             most = std::max(most, p.strips);
             plan.pairs.push_back(p);
+            const int cls = band_class(p.hi - p.lo + 1, 1, false, BandLimits{0, 0, 0, 0, 1, 1 << 20});
+            out.class_pairs[std::max(CLASS_STRIP_FIRST, cls)] += 1;
         }
+        out.decision_bytes = std::max(out.decision_bytes, part.decision_bytes);
+        out.carry_words = std::max(out.carry_words, part.carry_words);
+        out.parts.push_back(part);
+        if (most == 1) continue;  // a strip a pair, claimed as they are listed
         // By strips left to the pair's end, most first.
         at.assign((size_t)most + 1, 0);
         for (size_t i = 0; i < part.pairs; ++i)
@@ -805,26 +834,30 @@ StripPlan plan_strips(const dinara_batch *b, const std::vector<int4> &bands, boo
             for (int strip = 0; strip < strips; ++strip)
                 plan.order[part.strip + at[most - (strips - strip)]++] = make_int2((int)i, strip);
         }
-        plan.decision_bytes = std::max(plan.decision_bytes, part.decision_bytes);
-        plan.carry_words = std::max(plan.carry_words, part.carry_words);
-        plan.parts.push_back(part);
     }
-    return plan;
+    out.pairs = plan.pairs.size();
+    return out;
 }
 
-// The plan onto the device, and room for its launches. Waits for the main stream.
-int64_t upload_strips(dinara_batch *b, const StripPlan &plan) {
+// Room for the launches of a plan's parts.
+bool reserve_strips(dinara_batch *b, const StripParts &of) {
+    size_t most = 1;
+    for (const StripPart &part : of.parts) most = std::max(most, part.pairs);
+    return b->strip_counts.reserve((most + 1) * 4) && b->strip_best.reserve(most * 8) &&
+           b->strip_carry.reserve(std::max<size_t>(of.carry_words, 1) * 8) &&
+           (of.decision_bytes == 0 || b->strip_decisions.reserve(of.decision_bytes));
+}
+
+// The plan made last onto the device: its pairs, then its order. Waits for the main stream.
+bool upload_strips(dinara_batch *b, DeviceBuffer &to) {
+    const StripPlan &plan = strip_plan_of(b->ctx);
     const size_t pairs = plan.pairs.size() * sizeof(StripPair), order = plan.order.size() * sizeof(int2);
-    std::vector<uint8_t> host(pairs + order);
-    std::memcpy(host.data(), plan.pairs.data(), pairs);
-    std::memcpy(host.data() + pairs, plan.order.data(), order);
-    size_t most = 0;
-    for (const StripPart &part : plan.parts) most = std::max(most, part.pairs);
-    if (!b->strip_plan.upload(b->ctx, host.data(), host.size()) || !b->strip_counts.reserve((most + 1) * 4) ||
-        !b->strip_best.reserve(most * 8) || !b->strip_carry.reserve(std::max<size_t>(plan.carry_words, 1) * 8) ||
-        (plan.decision_bytes && !b->strip_decisions.reserve(plan.decision_bytes)))
-        return DINARA_OUT_OF_MEMORY;
-    return 0;
+    hipStream_t stream = b->ctx->stream;
+    return to.reserve(pairs + order) &&
+           hipMemcpyAsync(to.ptr, plan.pairs.data(), pairs, hipMemcpyHostToDevice, stream) == hipSuccess &&
+           (order == 0 || hipMemcpyAsync(static_cast<uint8_t *>(to.ptr) + pairs, plan.order.data(), order,
+                                         hipMemcpyHostToDevice, stream) == hipSuccess) &&
+           hipStreamSynchronize(stream) == hipSuccess;
 }
 
 // Where among a round's counts its strips' expired waits are (strip classes are counted together at the first).
@@ -836,15 +869,16 @@ int strip_polls() {
     return set ? (int)std::strtol(set, nullptr, 10) : STRIP_POLL_LIMIT;
 }
 
-// The plan's launches on `stream`, each part's sweep and (when decisions are kept) its walks, filing unproven pairs
-// where `round` says; `whole`: the bands are whole matrices.
-int64_t launch_strips(dinara_batch *b, const SweepArgs &round, const StripPlan &plan, bool whole, hipStream_t stream) {
-    for (const StripPart &part : plan.parts) {
+// The launches of a plan (on the device at `plan`) on `stream`, each part's sweep and (when decisions are kept) its walks,
+// filing unproven pairs where `round` says; `whole`: the bands are whole matrices.
+int64_t launch_strips(dinara_batch *b, const SweepArgs &round, const StripParts &of, const DeviceBuffer &plan, bool whole,
+                      hipStream_t stream) {
+    const StripPair *pairs = static_cast<const StripPair *>(plan.ptr);
+    for (const StripPart &part : of.parts) {
         StripArgs a{};
         a.s = round;
-        a.pairs = static_cast<const StripPair *>(b->strip_plan.ptr) + part.pair;
-        a.order = reinterpret_cast<const int2 *>(static_cast<const StripPair *>(b->strip_plan.ptr) + plan.pairs.size()) +
-                  part.strip;
+        a.pairs = pairs + part.pair;
+        a.order = part.strips == part.pairs ? nullptr : reinterpret_cast<const int2 *>(pairs + of.pairs) + part.strip;
         a.count = (int)part.pairs;
         a.strips = (int)part.strips;
         a.whole = whole ? 1 : 0;
@@ -1367,15 +1401,20 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         return DINARA_OUT_OF_MEMORY;
     int64_t counts[CLASSES] = {};
     for (int c = 0; c < CLASS_STRIP_FIRST; ++c) counts[c] = b->first_offset[c + 1] - b->first_offset[c];
-    std::vector<int4> strips;
-    for (int c = CLASS_STRIP_FIRST; c < CLASSES; ++c)
-        for (int32_t s : b->first_lists[c]) strips.push_back(first_strip_band(b, s));
+    // The strip bands a round plans, and how many there are.
+    std::vector<int4> bands;
+    size_t strips = (size_t)(b->first_offset[CLASSES] - b->first_offset[CLASS_STRIP_FIRST]);
+    const auto list_first_strips = [&]() {
+        bands.reserve(strips);
+        for (int c = CLASS_STRIP_FIRST; c < CLASSES; ++c)
+            for (int32_t s : b->first_lists[c]) bands.push_back(first_strip_band(b, s));
+    };
     int32_t *lists = static_cast<int32_t *>(b->retry_lists.ptr);
     int32_t *count_d = static_cast<int32_t *>(b->retry_counts.ptr);
     const size_t capacity = (size_t)std::max<int64_t>(slots, 1);
     const SweepArgs args = sweep_args(b);
     for (int round = 0; round < 64; ++round) {
-        int64_t pending = (int64_t)strips.size();
+        int64_t pending = (int64_t)strips;
         for (int c = 0; c < CLASS_STRIP_FIRST; ++c) pending += counts[c];
         if (pending == 0) break;
         SweepArgs a = args;
@@ -1383,10 +1422,18 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
         a.retry_counts = count_d + (round % 2) * CLASSES;
         a.strip_retries = static_cast<int4 *>(b->strip_retries.ptr) + (size_t)(round % 2) * capacity;
         const int32_t *in_lists = lists + (size_t)((round + 1) % 2) * CLASSES * capacity;
-        StripPlan plan;
-        if (!strips.empty()) {
-            plan = plan_strips(b, strips, a.record != 0, true);
-            if (const int64_t code = upload_strips(b, plan)) return code;
+        StripParts later;
+        const bool first = round == 0 && b->phase <= 1;
+        StripParts &of = first ? b->first_strips : later;
+        DeviceBuffer &plan = first ? b->first_strip_plan : b->strip_plan;
+        if (strips > 0) {
+            if (!first || !b->first_strips_planned) {
+                if (round == 0) list_first_strips();
+                of = plan_strips(b, bands, a.record != 0, true);
+                if (!upload_strips(b, plan)) return DINARA_OUT_OF_MEMORY;
+                b->first_strips_planned = b->first_strips_planned || first;
+            }
+            if (!reserve_strips(b, of)) return DINARA_OUT_OF_MEMORY;
         }
         if (hipMemsetAsync(a.retry_counts, 0, CLASSES * 4, ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
         (void)hipEventRecord(ctx->sweep_start, ctx->stream);
@@ -1410,14 +1457,11 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             (void)hipEventRecord(ctx->event(2 * c + 1), stream);
             return 0;
         };
-        if (!strips.empty()) {
-            for (const int4 &band : strips) {
-                const int cls = std::max(CLASS_STRIP_FIRST, band_class(band.z - band.y + 1, 1, false, BandLimits{0, 0, 0, 0, 1, 1 << 20}));
-                b->class_pairs[cls] += 1;
-            }
+        if (strips > 0) {
+            for (int c = CLASS_STRIP_FIRST; c < CLASSES; ++c) b->class_pairs[c] += of.class_pairs[c];
             b->class_launches[CLASS_STRIP_FIRST] += 1;
             if (const int64_t code = timed(CLASS_STRIP_FIRST, [&](hipStream_t stream) {
-                    return launch_strips(b, a, plan, false, stream);
+                    return launch_strips(b, a, of, plan, false, stream);
                 }))
                 return code;
         }
@@ -1479,14 +1523,15 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             retried += filed[c];
         }
         b->expired = b->expired || filed[STRIP_EXPIRED] > 0;
-        strips.resize((size_t)filed[CLASS_STRIP_FIRST]);
-        if (!strips.empty()) {
-            if (hipMemcpyAsync(strips.data(), a.strip_retries, strips.size() * sizeof(int4), hipMemcpyDeviceToHost,
-                               ctx->stream) != hipSuccess ||
+        strips = (size_t)filed[CLASS_STRIP_FIRST];
+        bands.resize(strips);
+        if (strips > 0) {
+            if (hipMemcpyAsync(bands.data(), a.strip_retries, strips * sizeof(int4), hipMemcpyDeviceToHost, ctx->stream) !=
+                    hipSuccess ||
                 hipStreamSynchronize(ctx->stream) != hipSuccess)
                 return DINARA_OUT_OF_MEMORY;
             // Longest first (slots are): the launch's longest pipelines claim their strips first.
-            std::sort(strips.begin(), strips.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
+            std::sort(bands.begin(), bands.end(), [](const int4 &x, const int4 &y) { return x.x < y.x; });
         }
         if (round == 0 && b->phase <= 1) b->first_proven = (double)(slots - retried);
     }
@@ -1637,9 +1682,9 @@ int64_t full_pass(dinara_batch *b) {
         bands.push_back(make_int4(slot, (int)-n, (int)m, 0));
     }
     if (!bands.empty()) {
-        const StripPlan plan = plan_strips(b, bands, record, false);
-        if (const int64_t code = upload_strips(b, plan)) return code;
-        if (const int64_t code = launch_strips(b, sweep_args(b), plan, true, ctx->stream)) return code;
+        const StripParts of = plan_strips(b, bands, record, false);
+        if (!upload_strips(b, b->strip_plan) || !reserve_strips(b, of)) return DINARA_OUT_OF_MEMORY;
+        if (const int64_t code = launch_strips(b, sweep_args(b), of, b->strip_plan, true, ctx->stream)) return code;
     }
     b->full_pairs = (double)bands.size();
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return DINARA_OUT_OF_MEMORY;
@@ -2105,6 +2150,7 @@ int64_t seed_slots(dinara_batch *b, GuessOf guess_of) {
         first_all.insert(first_all.end(), b->first_lists[c2].begin(), b->first_lists[c2].end());
     }
     b->first_offset[CLASSES] = (int64_t)first_all.size();
+    b->first_strips_planned = false;
     if (first_all.empty()) first_all.push_back(0);  // every pair too wide: the device list still needs room
     DeviceContext *ctx = b->ctx;
     std::lock_guard<std::mutex> serial(ctx->lock);

@@ -56,6 +56,7 @@ struct DeviceContext {
     // it returns, so no batch holds it between runs): allocated once, grown when a run wants more, kept until the
     // process ends, so a fresh batch does not pay for mapping tens of gigabytes.
     struct DeviceBuffer *edit_arena = nullptr;
+    void *strip_plan = nullptr;  // the strip rounds' plan on the host (batch.hip), used under `lock`
     size_t arena_wanted = 0;  // twice what the last run that left pairs without room had, for runs that may use it
 };
 

@@ -41,7 +41,7 @@ __host__ __device__ constexpr int strip_record_bytes(int c, int pieces) { return
 struct StripArgs {
     SweepArgs s;               // the batch's tape, costs, certificate, results and CIGAR output
     const StripPair *pairs;
-    const int2 *order;         // the launch's strips (pair, strip) as they are claimed
+    const int2 *order;         // the launch's strips (pair, strip) as they are claimed (null: a strip a pair, in turn)
     int count, strips;         // the pairs and strips of the launch
     int whole;                 // the bands hold the whole matrices: every cost found settles its pair
     uint8_t *decisions;        // null: costs alone

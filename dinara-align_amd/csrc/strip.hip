@@ -450,7 +450,7 @@ __global__ __launch_bounds__(64) void strip_sweep(StripArgs a) {
         if (threadIdx.x == 0) claimed = atomicAdd(a.claim, 1);
         claimed = __builtin_amdgcn_readfirstlane(claimed);
         if (claimed >= a.strips) return;
-        const int2 which = a.order[claimed];
+        const int2 which = a.order ? a.order[claimed] : make_int2(claimed, 0);
         const int pair = __builtin_amdgcn_readfirstlane(which.x), strip = __builtin_amdgcn_readfirstlane(which.y);
         const StripPair *at = a.pairs + pair;
         const StripPair p = *at;

@@ -205,3 +205,39 @@ def test_pairs_of_expired_waits_are_swept_whole(costs, monkeypatch):
         got, _, whole = resident(refs, qrys, costs, kind)
         assert got == (want if kind else [cost for cost, _ in want])
         assert whole > 0
+
+
+def test_first_rounds_after_seeds_and_whole_runs():
+    # The first round's strips are planned once while the first bands stand: seeds move them, and a run of whole matrices
+    # between two banded ones uses the same memory.
+    rng = random.Random(31)
+    costs = COSTS[0]
+    refs = [letters(rng, rng.randint(2200, 2700)) for _ in range(10)] + [letters(rng, 3000)]
+    qrys = [mutated(r, rate, rng) for r, rate in zip(refs, [0.01, 0.1, 0.3, 0.5, 0.02] * 2)] + [refs[-1][900:2100]]
+    want = [o.costs_align(r, q, to_oracle(costs)) for r, q in zip(refs, qrys)]
+    handle = _lib.lib()
+    R, Q, c, status = _lib.Texts(refs), _lib.Texts(qrys), costs.as_c(), ctypes.c_int64(0)
+    for kind in (0, 1):
+        batch = handle.dinara_batch_new(0, kind, len(refs), *R.args(), *Q.args(), ctypes.byref(c), None, None, 4,
+                                        ctypes.byref(status))
+        assert batch, status.value
+        try:
+            for guesses, whole in [(None, 0), (None, 1), (0, 0), (None, 0), (700, 0), (4000, 0), (None, 1), (60, 0)]:
+                if guesses is not None:
+                    seeds = (ctypes.c_int64 * len(refs))(*[guesses] * len(refs))
+                    assert handle.dinara_batch_seed(batch, ctypes.addressof(seeds)) == 0
+                assert handle.dinara_batch_set_whole(batch, whole) == 0
+                assert handle.dinara_batch_run(batch) == 0
+                if kind == 0:
+                    out = (ctypes.c_int64 * len(refs))()
+                    assert handle.dinara_batch_distances(batch, out) == 0
+                    assert list(out) == [cost for cost, _ in want], (guesses, whole)
+                    continue
+                found, statuses = (_lib.CAlignment * len(refs))(), (ctypes.c_int64 * len(refs))()
+                assert handle.dinara_batch_alignments(batch, found, statuses) == 0
+                got = [(a.cost, ctypes.string_at(a.cigar, a.cigar_length).decode()) for a in found]
+                for a in found:
+                    handle.dinara_free(a.cigar)
+                assert got == want, (guesses, whole)
+        finally:
+            handle.dinara_batch_free(batch)
