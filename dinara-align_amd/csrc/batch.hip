@@ -611,7 +611,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         !b->walk_class.reserve(std::max<int64_t>(slots, 1) * 4) ||
         !b->retry_lists.reserve((size_t)2 * CLASSES * std::max<int64_t>(slots, 1) * 4) ||
         !b->retry_counts.reserve(2 * CLASSES * 4) ||
-        !b->strip_retries.reserve((size_t)2 * std::max<int64_t>(slots, 1) * sizeof(int4)) ||
+        (!b->unit && !b->strip_retries.reserve((size_t)2 * std::max<int64_t>(slots, 1) * sizeof(int4))) ||
         !b->first_lists_d.upload(ctx, first_all.data(), std::max<size_t>(first_all.size(), 1) * 4) ||
         !b->walk_flags.reserve(std::max<int64_t>(slots, 1) * 8))
         return DINARA_OUT_OF_MEMORY;

@@ -7,6 +7,7 @@ not serve are refused as DINARA_INVALID_MODE.
 """
 
 import ctypes
+import random
 
 import pytest
 
@@ -58,6 +59,17 @@ def test_static_distances_scaled_costs_caps_and_odd_pairs():
     want, found = both(refs, qrys, None, capped)
     assert found == want
     assert _lib.ABOVE_MAX in found
+
+
+@pytest.mark.parametrize("pairs,length", [(124_000, 20), (115_600, 100), (65_200, 1000)])
+def test_static_distances_of_as_many_pairs_as_the_scratch_holds(pairs, length):
+    # What a pair takes besides its letters does not grow: batches close under the scratch's size are served.
+    rng = random.Random(length)
+    few = ["".join(rng.choice("ACGT") for _ in range(length)).encode() for _ in range(64)]
+    refs = [few[i % 64] for i in range(pairs)]
+    print(f"[static] {pairs} pairs of {length}", flush=True)
+    code, found = call("dinara_gpu_distances_static", refs, refs)
+    assert code == 0 and not any(found)
 
 
 def test_static_distances_refusals():
