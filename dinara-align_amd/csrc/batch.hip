@@ -755,10 +755,7 @@ constexpr size_t PLAN_KEPT = size_t(1) << 18;  // pairs, strips
 
 StripPlan &strip_plan_of(DeviceContext *ctx) {
     if (!ctx->strip_plan) ctx->strip_plan = new StripPlan();
-    StripPlan &plan = *static_cast<StripPlan *>(ctx->strip_plan);
-    if (plan.pairs.capacity() > PLAN_KEPT) std::vector<StripPair>().swap(plan.pairs);
-    if (plan.order.capacity() > PLAN_KEPT) std::vector<int2>().swap(plan.order);
-    return plan;
+    return *static_cast<StripPlan *>(ctx->strip_plan);
 }
 
 // The plan of the pairs listed in `bands` (slot, low, high): each pair's strips, where its records lie, and the order
@@ -769,6 +766,9 @@ StripParts plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bo
     StripParts out;
     plan.pairs.clear();
     plan.order.clear();
+    // A large round's memory goes when the next is planned (this one's is read by upload_strips until then).
+    if (plan.pairs.capacity() > PLAN_KEPT) std::vector<StripPair>().swap(plan.pairs);
+    if (plan.order.capacity() > PLAN_KEPT) std::vector<int2>().swap(plan.order);
     plan.pairs.reserve(bands.size());
     std::vector<size_t> &at = plan.at;
     const int pieces = b->costs.pieces == 2 ? 2 : 1;

@@ -241,3 +241,19 @@ def test_first_rounds_after_seeds_and_whole_runs():
                 assert got == want, (guesses, whole)
         finally:
             handle.dinara_batch_free(batch)
+
+
+@pytest.mark.parametrize("pairs,length", [(270_000, 100), (60_000, 300)])
+def test_plans_larger_than_the_memory_kept_for_them(pairs, length, monkeypatch):
+    # Rounds of more than 262,144 pairs, and of more strips (two columns a lane), in one call after another.
+    monkeypatch.setenv("DINARA_STRIP_COLUMNS", "2")
+    rng = random.Random(length)
+    oc = to_oracle(COSTS[0])
+    windows = [letters(rng, length + rng.randint(0, 5)) for _ in range(40)]
+    reads = [mutated(w, 0.05, rng)[2:] + (letters(rng, 600) if length > 100 and i % 2 else "") for i, w in enumerate(windows)]
+    want = [o.ends_align(r, q, oc, ends_of(da.Mode.INFIX)) for r, q in zip(windows, reads)]
+    print(f"[strips] {pairs} pairs", flush=True)
+    refs, qrys = (windows * (pairs // 40 + 1))[:pairs], (reads * (pairs // 40 + 1))[:pairs]
+    assert da.distances(refs, qrys, COSTS[0], da.Mode.INFIX) == ([e[0] for e in want] * (pairs // 40 + 1))[:pairs]
+    found = da.alignments(refs[:1000], qrys[:1000], COSTS[0], da.Mode.INFIX)
+    assert [(a.cost, a.cigar) for a in found] == ([e[:2] for e in want] * 25)[:1000]
