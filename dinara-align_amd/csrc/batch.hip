@@ -289,9 +289,17 @@ int group_region(int64_t letters) { return (int)((letters + GROUP_ROOM + 3) & ~i
 // any number of pairs up to a wave on each SIMD. A strip round takes as long as its strips' cells, as long as a group
 // chain of as many letters as so many pairs' on average (CIGARs, whose strips write more decisions, have their own). So
 // of the pairs past GROUP_LETTERS letters the longest go to the strips, down to the length that makes the two least
-// together. Groups against strips, ms: 500 pairs of 2.5 kbp at 1% 1.2 and 1.2 (CIGARs 4.2 and 4.0), 2,000 of 5 kbp 4.9
-// and 3.1 (13.0 and 9.1), 4,096 of 2.5 kbp 2.0 and 1.9 (6.8 and 7.9), 20,000 of 2.5 kbp 3.1 and 5.5 (12.5 and 21.3).
-constexpr int64_t GROUP_LETTERS = 4096, GROUP_PAIRS_COSTS = 4096, GROUP_PAIRS_CIGARS = 3072;
+// together. Groups against strips, ms: 1,000 pairs of 1.2 kbp at 5% 0.79 and 0.81 (CIGARs 2.8 and 2.8), of 2 kbp 1.5 and
+// 1.2 (5.8 and 3.5); 500 of 2.5 kbp at 1% 1.2 and 1.2 (4.2 and 4.0), 2,000 of 5 kbp 4.9 and 3.1 (13.0 and 9.1), 4,096 of
+// 2.5 kbp 2.0 and 1.9 (6.8 and 7.9), 20,000 of 2.5 kbp 3.1 and 5.5 (12.5 and 21.3).
+// In 128 diagonals the groups' cells are the fewer: 1,000 CIGARs of 1.8 kbp at 1% 3.1 and 3.5.
+constexpr int64_t GROUP_LETTERS = 3072, GROUP128_LETTERS = 4608, GROUP_PAIRS_COSTS = 4096, GROUP_PAIRS_CIGARS = 3072;
+// The first band is a narrow group band, a short chain that proves a pair of few errors; a pair's first strips are wide
+// (first_strip_band), and prove more. What CIGARs take either way, in ns a letter of the longest pair (a group's sweep
+// and its walks, a lane a pair; a strip round's sweep and its walks, a wave a pair) and of all pairs in strips: 64 pairs
+// of 2.5 kbp at 1% 3.3 ms as groups and 1.5 as strips; at 0.1% 300 of 1.8 kbp 2.0 and 1.6, 1,000 of 2.2 kbp 2.8 and 5.1.
+constexpr double GROUP_SWEEP_NS = 86, GROUP_WALK_NS = 350, STRIP_CHAIN_NS = 250, STRIP_WORK_NS = 0.8;
+
 // The narrowest wave band, a row a step of a pair's own wave, against one strip of the whole matrix and its 63 steps of
 // lanes coming in and going out: the pairs whose strips would take longer than the longest pair's rows. Two pieces, wave
 // against strips, ms: 20,000 pairs of 150 bp 0.67 and 1.12, 3,000 of 600 0.97 and 1.10, 5,000 of 1,000 1.7 and 2.6, 1,000
@@ -463,36 +471,50 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     } else {
         const int64_t staged = (int64_t)(b->lds_limit / 4) - GROUP_ROOM - 4;
         const bool cigars = b->kind == DINARA_BATCH_ALIGNMENTS;
-        std::vector<int32_t> longs;
-        int64_t strips = 0;  // those pairs' strips of four columns a lane
+        std::vector<int32_t> longs;  // letters, most first
+        int32_t longest = 0;         // of the others
+        int64_t past = 0, past_longest = 0;  // letters of the pairs no group launch stages
         for (int64_t s = 0; s < slots; ++s) {
             const int32_t letters = b->rows[s] + b->cols[s];
-            if (letters <= GROUP_LETTERS || letters > staged) continue;
-            longs.push_back(letters);
-            strips += b->cols[s] / strip_columns(4) + 1;
+            if (letters <= GROUP_LETTERS) {
+                longest = std::max(longest, letters);
+            } else if (letters <= staged) {
+                longs.push_back(letters);
+            } else {
+                past += letters;
+                past_longest = std::max<int64_t>(past_longest, letters);
+            }
         }
-        // The cap that makes least the group launch's chain and the strips' work beside it.
         std::sort(longs.begin(), longs.end(), std::greater<int32_t>());
-        int64_t cap = GROUP_LETTERS, in_strips = 0, least = INT64_MAX;
+        // Of each length that may be the longest in group bands (all, then ever fewer of the long pairs): the chain of the
+        // wider bands and the strips beside them, and for CIGARs of the first round and its walks.
+        int64_t cap = GROUP_LETTERS, first_cap = staged, in_strips = 0;
+        double least = 0, least_first = 0;
         for (size_t i = 0; i <= longs.size(); ++i) {
-            const int64_t chain = i < longs.size() ? longs[i] : (int64_t)longs.size() < slots ? GROUP_LETTERS : 0;
-            const int64_t cost = chain + in_strips / (cigars ? GROUP_PAIRS_CIGARS : GROUP_PAIRS_COSTS);
-            if (cost <= least) {
+            const int64_t chain = i < longs.size() ? longs[i] : longest;
+            const double cost = (double)chain + (double)in_strips / (cigars ? GROUP_PAIRS_CIGARS : GROUP_PAIRS_COSTS);
+            const int64_t strip_longest = past_longest > 0 ? past_longest : i > 0 ? longs[0] : 0;
+            const double first = std::max(GROUP_SWEEP_NS * chain, STRIP_CHAIN_NS * strip_longest +
+                                                                      STRIP_WORK_NS * (past + in_strips)) +
+                                 GROUP_WALK_NS * chain;
+            if (i == 0 || cost < least) {
                 least = cost;
                 cap = std::max(chain, GROUP_LETTERS);
+            }
+            if (i == 0 || first < least_first) {
+                least_first = first;
+                first_cap = i == 0 ? staged : std::max(chain, GROUP_LETTERS);
             }
             if (i < longs.size()) in_strips += longs[i];
         }
         const auto tags_fit = [&](int longest) {
             return ((int64_t)longest + 2 * 256 + 8) * b->dearest < REAL_LIMIT ? longest : 0;
         };
-        b->limits.group_letters = tags_fit(longest_up_to(std::min(staged, cap)));
-        // The first band is a narrow one: a short chain, which proves a pair of few errors. Few pairs' CIGARs, whose
-        // strips all run at once, go to the strips with it (and are walked a wave a pair): 64 of 2.5 kbp at 1% 3.3 ms as
-        // groups, 1.5 so.
-        b->limits.group_narrow = b->limits.group_letters;
-        if (!cigars || strips > STRIP_GRID / 2)
-            b->limits.group_narrow = std::max(b->limits.group_letters, tags_fit(longest_up_to(staged)));
+        if (!cigars) first_cap = staged;
+        b->limits.group_letters = tags_fit(longest_up_to(std::min(first_cap, cap)));
+        b->limits.group128_letters =
+            std::max(b->limits.group_letters, tags_fit(longest_up_to(std::min(first_cap, GROUP128_LETTERS))));
+        b->limits.group_narrow = std::max(b->limits.group128_letters, tags_fit(longest_up_to(first_cap)));
     }
     // The strips take bands of pairs up to 65,536 letters, free ends' up to 2,048 diagonals; longer pairs and wider
     // bands are swept whole after the run.
@@ -731,9 +753,11 @@ int strip_c(int64_t m) { return m <= strip_columns(2) ? 2 : m <= strip_columns(4
 
 // A round of few strips is as long as its longest pair's pipeline, and a strip of four columns a lane hands on sooner
 // than twice the half of one of eight (its step is shorter, and so are its rows): up to this many strips of eight, four.
-// 2,000 uneven pairs (8,192 strips) 11.1 -> 10.5 ms, 1,000 two-piece CIGARs 11.9 -> 9.9; two a lane 11.6 and 10.7. A
-// round that fills the chip pays for its cells: 200,000 uneven pairs 236 ms with eight, 251 with four.
-constexpr int64_t FEW_STRIPS = 16384;
+// A round that fills the chip pays for its cells. Four against eight, ms: uneven gap-affine pairs (1.5 kbp median, up to
+// 20 kbp) 1,000 9.1 and 10.1, 4,000 12.9 and 13.2, 8,000 18.8 and 19.0, 200,000 251 and 236; two-piece CIGARs (1.5 kbp)
+// 1,000 10.2 and 12.6, 4,000 19.5 and 19.5, 8,000 31 and 29. Gap-affine CIGARs, whose decisions of four columns go out
+// in half lines, turn sooner: 500 21.5 and 22.0, 1,000 24.1 and 23.5, 2,000 29.0 and 26.6, 8,000 67 and 50.
+constexpr int64_t FEW_STRIPS = 16384, FEW_STRIPS_ONE_PIECE_CIGARS = 4096;
 // Whatever their number, strips of four where costs alone are kept and the band is narrower than this: a strip's rows
 // are its band's and its columns'. 4,000 pairs of 3 kbp at 5% 4.4 -> 3.9 ms; their CIGARs 13.1 -> 16.5, so not those.
 constexpr int NARROW_BAND = 512;
@@ -779,7 +803,7 @@ StripParts plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bo
     } else if (round) {
         int64_t strips = 0;
         for (const int4 &band : bands) strips += b->cols[band.x] / strip_columns(8) + 1;
-        if (strips <= FEW_STRIPS) widest_c = narrow_c = 4;
+        if (strips <= (record && pieces == 1 ? FEW_STRIPS_ONE_PIECE_CIGARS : FEW_STRIPS)) widest_c = narrow_c = 4;
     }
     size_t budget = ARENA_BUDGET;
     if (const char *set = std::getenv("DINARA_STRIP_BUDGET")) budget = std::strtoull(set, nullptr, 10);
@@ -812,7 +836,7 @@ StripParts plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bo
             ++part.pairs;
             most = std::max(most, p.strips);
             plan.pairs.push_back(p);
-            const int cls = band_class(p.hi - p.lo + 1, 1, false, BandLimits{0, 0, 0, 0, 1, 1 << 20});
+            const int cls = band_class(p.hi - p.lo + 1, 1, false, BandLimits{0, 0, 0, 0, 0, 1, 1 << 20});
             out.class_pairs[std::max(CLASS_STRIP_FIRST, cls)] += 1;
         }
         out.decision_bytes = std::max(out.decision_bytes, part.decision_bytes);
@@ -1484,8 +1508,8 @@ int64_t sweep_rounds(dinara_batch *b, size_t &arena_index) {
             const int longest = band_is_wave(c) ? (b->user_band              ? b->max_letters
                                                    : c == CLASS_WAVE_FIRST ? b->limits.wave_letters
                                                                            : b->limits.wave128_letters)
-                                : c <= CLASS_GROUP64 && (longs > 0 || round > 0) ? b->limits.group_narrow
-                                                                                 : b->limits.group_letters;
+                                : c <= CLASS_GROUP64 && longs == 0 && round == 0 ? b->limits.group_letters
+                                                                                 : group_limit(b->limits, c);
             if (longs > 0)
                 if (const int64_t code = timed(LONG_PART + c, [&](hipStream_t stream) {
                         return launch_class(b, a, c, list, longs, longest, arena_index, stream);

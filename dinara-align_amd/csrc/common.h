@@ -66,12 +66,17 @@ __host__ __device__ constexpr int band_width(int cls) {
 __host__ __device__ constexpr bool band_is_wave(int cls) { return cls >= CLASS_WAVE_FIRST && cls <= CLASS_WAVE_LAST; }
 __host__ __device__ constexpr bool band_is_strip(int cls) { return cls >= CLASS_STRIP_FIRST; }
 
-// Which pairs take which bands, in letters (both sequences): group bands of up to 64 diagonals up to `group_narrow`, every group
-// band up to `group_letters`, the wave band of 64 diagonals up to `wave_letters` and that of 128 up to
-// `wave128_letters` (0 where no pair takes them), strips up to `strip_letters` and bands `strip_widest` wide.
+// Which pairs take which bands, in letters (both sequences; 0 where no pair takes them): group bands of up to 64
+// diagonals up to `group_narrow`, of 128 up to `group128_letters`, of 256 up to `group_letters`; the wave band of 64
+// diagonals up to `wave_letters` and that of 128 up to `wave128_letters`; strips up to `strip_letters` and bands
+// `strip_widest` wide.
 struct BandLimits {
-    int group_narrow, group_letters, wave_letters, wave128_letters, strip_letters, strip_widest;
+    int group_narrow, group128_letters, group_letters, wave_letters, wave128_letters, strip_letters, strip_widest;
 };
+
+__host__ __device__ inline int group_limit(const BandLimits &limits, int cls) {
+    return cls <= CLASS_GROUP64 ? limits.group_narrow : cls < CLASS_GROUP256 ? limits.group128_letters : limits.group_letters;
+}
 
 // The class of band a pair of `letters` letters needing `need` diagonals takes: the narrowest that holds them. A group
 // band is placed on an even diagonal, so it holds one diagonal fewer than its width. Pairs under a user band take the
@@ -86,8 +91,7 @@ __host__ __device__ inline int band_class(int need, int64_t letters, bool user_b
         if (letters <= (cls == CLASS_WAVE_FIRST ? limits.wave_letters : limits.wave128_letters) && need <= band_width(cls))
             return cls;
     for (int cls = CLASS_GROUP32; cls <= CLASS_GROUP256; ++cls)
-        if (letters <= (cls <= CLASS_GROUP64 ? limits.group_narrow : limits.group_letters) && need < band_width(cls))
-            return cls;
+        if (need < band_width(cls) && letters <= group_limit(limits, cls)) return cls;
     if (letters <= limits.strip_letters)
         for (int cls = CLASS_STRIP_FIRST; cls < CLASSES; ++cls)
             if (need <= band_width(cls) && band_width(cls) <= limits.strip_widest) return cls;

@@ -334,6 +334,29 @@ def test_long_pairs_beside_short_ones(shorts, kind):
         check_distances(refs, qrys, costs)
 
 
+@pytest.mark.parametrize("kind", [0, 1])
+def test_bands_around_their_limits_of_width_and_length(kind):
+    # First bands of a diagonal less and more than the group bands hold, for pairs on both sides of the lengths up to
+    # which bands of 128 and of 256 diagonals are taken in groups, beside pairs that keep them out of the strips.
+    rng = random.Random(59)
+    refs, qrys = random_pairs(30, rng, lengths=(1400, 1520), rates=(0.01, 0.1))
+    for total in (3070, 3072, 3073, 4607, 4608, 4609):
+        for difference in (59, 61, 62, 123, 125, 126, 251, 253, 254, 300):
+            m = (total - difference) // 2
+            q = "".join(rng.choice("ACGT") for _ in range(m))
+            cut = rng.randint(0, m)
+            r = q[:cut] + "".join(rng.choice("ACGT") for _ in range(total - 2 * m)) + q[cut:]
+            refs.append(r)
+            qrys.append(q)
+    swept = class_pairs(refs, qrys, da.Costs.affine(4, 6, 2), kind)
+    assert min(swept[1:4]) > 0 and sum(swept[10:]) > 0, swept
+    for costs in (da.Costs.affine(4, 6, 2), da.Costs.affine(4, 2, 1).with_deletions(6, 3)):
+        if kind:
+            check_alignments(refs, qrys, costs)
+        else:
+            check_distances(refs, qrys, costs)
+
+
 def test_widest_band_distances():
     # First bands past 8192 diagonals: the 12288- and 16384-diagonal blocks, distances only.
     rng = random.Random(41)
