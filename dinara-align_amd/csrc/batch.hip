@@ -304,8 +304,11 @@ constexpr double GROUP_SWEEP_NS = 86, GROUP_WALK_NS = 350, STRIP_CHAIN_NS = 250,
 // lanes coming in and going out: the pairs whose strips would take longer than the longest pair's rows. Two pieces, wave
 // against strips, ms: 20,000 pairs of 150 bp 0.67 and 1.12, 3,000 of 600 0.97 and 1.10, 5,000 of 1,000 1.7 and 2.6, 1,000
 // of 1,500 at 0.5% 1.6 and 1.3. The next wider one takes the same pairs' retries (5,000 CIGARs of 1,000 4.9 -> 4.5), under
-// free ends, whose first bands are wide, short pairs alone: reads of 100 with a free reference end 0.69 and 1.03.
-constexpr int64_t WAVE_LETTERS = 512, WAVE_LETTERS_MOST = 8192, WAVE_PAIRS = 2560, WAVE128_LETTERS = 320;
+// free ends, whose first bands are wide, short pairs alone: reads of 100 with a free reference end 0.69 and 1.03. CIGARs
+// of these bands are walked a lane a pair, a chain of its own at the run's end: they pay where the strips they spare would
+// take as long, from so many pairs on (1,000 two-piece CIGARs of 1.5 kbp, of which a few are short, 10.4 and 10.0).
+constexpr int64_t WAVE_LETTERS = 512, WAVE_LETTERS_MOST = 8192, WAVE_PAIRS = 2560, WAVE128_LETTERS = 320,
+                  WAVE_PAIRS_CIGARS = 450;
 
 // The class of a slot's first band of `need` diagonals.
 int first_class(const dinara_batch *b, int64_t s, int need) {
@@ -465,7 +468,11 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
     b->limits = BandLimits{};
     if (b->parsed.two_piece || b->free_ends) {
         const int64_t cap = std::min(std::max(WAVE_LETTERS, letters_in_all / WAVE_PAIRS), WAVE_LETTERS_MOST);
-        b->limits.wave_letters = longest_up_to(std::min(cap, (int64_t)b->lds_limit));
+        const int longest = longest_up_to(std::min(cap, (int64_t)b->lds_limit));
+        int64_t letters_there = 0;
+        for (int64_t s = 0; s < slots; ++s)
+            if (b->rows[s] + b->cols[s] <= longest) letters_there += b->rows[s] + b->cols[s];
+        if (b->kind != DINARA_BATCH_ALIGNMENTS || letters_there >= WAVE_PAIRS_CIGARS * longest) b->limits.wave_letters = longest;
         b->limits.wave128_letters =
             b->free_ends ? (int)std::min<int64_t>(b->limits.wave_letters, WAVE128_LETTERS) : b->limits.wave_letters;
     } else {
