@@ -771,11 +771,9 @@ constexpr int NARROW_BAND = 512;
 
 // A strip launch's parts: consecutive pairs of the plan whose decisions and carry records fit ARENA_BUDGET together. A
 // round of costs keeps no decisions, but each pair's carry records (8 bytes a row a strip, 16 under two pieces; 0.8 MB
-// for a pair of 10,000 letters in 4,500 diagonals): it is cut once it passes CARRY_BUDGET with strips enough to fill the
-// persistent grid several times, so that what a batch asks for stays bounded and a part's tail short beside it.
-// DINARA_STRIP_BUDGET sets the bytes a part may take, for checking.
-constexpr size_t CARRY_BUDGET = size_t(1) << 30;
-constexpr size_t FULL_GRIDS = 4;
+// for a pair of 10,000 letters in 4,500 diagonals), so what a batch asks for would grow with its pairs. A part costs its
+// longest pair's pipeline once more: 200,000 uneven distances 241 ms in one part of 10 GB, 243 in parts of 4 GB, 269 in
+// parts of 1 GB. DINARA_STRIP_BUDGET sets the bytes a part may take, for checking.
 // A round's plan on the host, the context's: made anew for each round (under its lock), its memory kept while it is small.
 struct StripPlan {
     std::vector<StripPair> pairs;
@@ -832,9 +830,7 @@ StripParts plan_strips(const dinara_batch *b, const std::vector<int4> &bands, bo
             const size_t bytes = record ? (records * strip_record_bytes(p.c, pieces) + 255) & ~size_t(255) : 0;
             const size_t carried = p.strips > 1 ? (size_t)p.strips * p.rows * pieces : 0;
             const size_t carry_bytes = 8 * (part.carry_words + carried);
-            if (part.pairs > 0 && (part.decision_bytes + bytes + carry_bytes > budget ||
-                                   (carry_bytes > CARRY_BUDGET && part.strips >= FULL_GRIDS * STRIP_GRID)))
-                break;
+            if (part.pairs > 0 && part.decision_bytes + bytes + carry_bytes > budget) break;
             p.decision_at = (int64_t)part.decision_bytes;
             p.carry_at = (int64_t)part.carry_words;
             part.decision_bytes += bytes;
