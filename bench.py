@@ -8,7 +8,7 @@ lengths are log-normal around 1.5 kbp (sigma 1, clipped to 100 bp..20 kbp) at a 
 pairs, compared byte for byte:
   plain doubling   every band from 64 diagonals, twice as wide until the certificate proves it, each band keeping
                    its decisions; one pair a lane group, one launch after another;
-  persistent       length-binned persistent launches replayed as one hipGraph (bins side by side on streams), first
+  persistent       length-binned persistent launches replayed as one hipGraph (every one-word bin in one launch), first
                    bands and launch shape autotuned on the batch, then each proven band traced again;
   learned          the same launches with each pair's first band from a network trained (on the GPU) on the
                    aligner's own distances of separate pairs, seeded on the device inside the step, sweeps keeping
@@ -63,10 +63,10 @@ CLASSES = len(CLASS_NAMES)
 # HBM bytes per launch of the dominant kernel, from rocprofv3 FETCH_SIZE and WRITE_SIZE passes, each scaled by what
 # the same counter reads for a plain 1 GiB device copy: FETCH_SIZE x 2.0, WRITE_SIZE x 1.0. The affine step (100,000
 # pairs of 250 bp): profiles/sweep_group_affine_100k_x_250_hbm_counters.md. The learned run of the mixed-length
-# workload (200,000 pairs), every edit_sweep dispatch of one run summed (the bins run side by side):
+# workload (200,000 pairs), every edit_sweep and edit_sweep_wide dispatch of one run summed:
 # profiles/edit_sweep_learned_uneven_200k_hbm_counters.md.
-MEASURED_TRAFFIC = {("affine", 100_000, "sweep_group<2>"): {"read": 119.1e6, "written": 823.3e6},
-                    ("uneven", 200_000, "edit_sweep"): {"read": 2.439e9, "written": 87.46e9}}
+MEASURED_TRAFFIC = {("affine", 100_000, "sweep_group<2>"): {"read": 119.3e6, "written": 823.3e6},
+                    ("uneven", 200_000, "edit_sweep"): {"read": 9.459e9, "written": 87.50e9}}
 
 
 def host_cores() -> int:
@@ -877,7 +877,7 @@ def run_uneven(args) -> int:
     handle.dinara_batch_set_keep_first(plain, 1)
     handle.dinara_batch_set_persistent(plain, 0)
     handle.dinara_batch_set_graph(plain, 0)
-    # Its bins side by side on their streams or one after another: timed, the faster kept (the stronger baseline).
+    # Its one-word bins in one launch or a bin after another: timed, the faster kept (the stronger baseline).
     plain_apart = {}
     for apart in (1, 0):
         handle.dinara_batch_set_side_by_side(plain, apart)
@@ -1191,7 +1191,7 @@ def run_edit(args) -> int:
         return 1
     cores = host_cores()
     D = _lib.BATCH_DISTANCES
-    # The bins side by side on streams of their own, or one after another, chosen on held-out pairs drawn alike:
+    # The one-word bins in one launch with the wider ones beside it, or a bin after another, chosen on held-out pairs:
     # with every pair proven by its first band, the empty retry launches cost least in one stream.
     tune_r, tune_q = synthetic.edit_short(pairs, seed=5)
     tb, tkeep = edit_batch(handle, tune_r, tune_q, D, min(cores, 16))
@@ -1320,7 +1320,7 @@ def train_network(handle, refs, qrys, workers, epochs, net_file=""):
 def run_learned_profile(args) -> int:
     """The learned path's run alone, for profilers: the mixed-length workload's 200,000 pairs seeded by the network
     (trained as the default bench trains it, or loaded from --net-file), sweeps keeping their decisions, launches
-    one by one so each bin's sweeps are kernels of their own in a trace; `--steps` runs after the training. A plain
+    one by one so each pass is a kernel of its own in a trace; `--steps` runs after the training. A plain
     1 GiB device copy (probe/probe.hip) runs first: the copy the HBM byte counters are calibrated against. Prints the
     library's own per-bin times of the last run as one JSON line."""
     pairs = args.pairs or 200_000

@@ -229,7 +229,7 @@ struct dinara_batch {
     bool use_graph = true;                // replay the run's launches as one captured hipGraph
     bool persistent = true;               // pair groups refill from their queue; else one pair a group
     bool keep_first = false;              // alignments: every sweep keeps its decisions (one pass when proven)
-    bool side_by_side_bins = true;        // every one-word bin in one launch, the wider ones on streams of their own
+    bool side_by_side_bins = true;        // every one-word bin in one launch, the wider ones beside it
     bool one_stream = false;              // no side streams: the wider bins' launches follow on the main stream
     bool timed = true;                    // launches made one by one record an event pair each
     int grid_per_cu = 8;                  // persistent workgroups a compute unit
@@ -374,8 +374,7 @@ int64_t prepare(dinara_batch *b, const char *const *refs, const char *const *qry
         words += (int64_t)(rw + qw) * 64;
     }
     // Every word is written below (a pair's words past its letters are zero), so the tape needs no clearing but
-    // its padding: the unit-cost sweeps' letter cursors read up to three words past a sequence's last without a bounds
-    // check (edit.hip), which past the last group's words lands here.
+    // its padding, where the unit-cost sweeps' unchecked letter reads past the last group land (TAPE_PADDING_WORDS).
     const int64_t padded = words + TAPE_PADDING_WORDS;
     std::unique_ptr<uint32_t[]> tape(new (std::nothrow) uint32_t[padded]);
     if (!tape) return DINARA_OUT_OF_MEMORY;

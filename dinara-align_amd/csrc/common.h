@@ -24,8 +24,11 @@ struct CostParams {
     int del_first2, ins_first2;
 };
 
-// Zero words after the tape's last group: a letter cursor may read two words past its sequence (64 words a word
-// index across the transposed groups).
+// Zero words after the tape's last group, 64 a word index across the transposed groups. The unit-cost sweeps' letter
+// cursors (edit.hip) read ahead with no bounds check, at most two word indices past their group's last: a cursor loads
+// no word more than two past the one that holds its last letter; a query's last letter is m - 1, and a band starts no
+// lower than diagonal -n - 1, so its bottom row's letters end at n + m, which the group's query words, lying behind its
+// reference words, hold but for that same margin.
 constexpr int TAPE_PADDING_WORDS = 4 * 64;
 
 // Which pairs a launch takes and where their letters lie. The tape holds every sequence 2 or 8 bits a

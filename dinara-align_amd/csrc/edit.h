@@ -11,10 +11,11 @@
 //
 // Pairs are binned by band width. A wave holds 64 / lanes pairs, each on `lanes` adjacent lanes, and every pair
 // group takes its next pair from its bin's queue the moment it finishes the last one (a persistent launch): pairs of
-// very different lengths share waves without waiting for each other. Every bin's first queue is swept at once, the
-// bins side by side on streams of their own (a long pair's tail in one bin overlaps the others' work); a pair its
-// band does not prove is filed into a retry queue of a wider bin. The retry queues are swept side by side too,
-// filing into a second retry set, which is swept last, narrowest bin first. The launches have a fixed shape, so one
+// very different lengths share waves without waiting for each other. Every one-word bin's first queue is swept by one
+// launch, a workgroup finding its bin by its place in the grid, with the two wide bins' launches beside it (a long
+// pair's tail in one bin overlaps the others' work). A pair its band does not prove is filed into a retry queue of a
+// wider bin, and those are swept the same way. Under the certified policy a retry always proves its pair; plain band
+// doubling files again, into a later set swept bin after bin, narrowest first. The launches have a fixed shape, so one
 // hipGraph replays them.
 #pragma once
 

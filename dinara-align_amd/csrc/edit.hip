@@ -71,7 +71,7 @@ __device__ __forceinline__ void load_planes(const uint32_t *text, int n, int fir
 // word shifted so its next code is in the low bits; the word after it is loaded a word ahead, so a column never waits
 // on its own load. The refill load has no bounds check, so its result lands straight in the register it is kept in
 // (a checked load's result would be copied there at once, the copy waiting for the load): a cursor reads at most two
-// words past its sequence's last, which the tape's padding and the next group's words hold, and letters past the end
+// words past its group's last, which the next group's words or the tape's padding hold, and letters past the end
 // are never used (columns stop at the query's end; rows below the reference's feed no row above them). A lane with
 // no pair is parked: it never loads. All unsigned: no sign fix-ups in the column step.
 template <int BITS>
@@ -151,7 +151,6 @@ struct Letters2 {
 
 template <int BITS>
 using LetterSource = typename std::conditional<BITS == 2, Letters2, Cursor<BITS>>::type;
-
 
 // A function of three 64-bit words, bit by bit (v_bitop3 a half): F is its value over the words' own tables, TABLE_A,
 // TABLE_B and TABLE_C.

@@ -149,9 +149,10 @@ __device__ __forceinline__ void odd_half(GroupState<S> &st, const GroupCosts &g,
 // Packed cells: two slots of a lane in the 16-bit halves of one register, slot q low and slot q + S/2 high, for
 // the steady anti-diagonals of a shifted sweep (both extensions equal). There a tagged value is 16 (H - e(r + c))
 // plus its tag, between -16 e (r + c) and 32 max(opening) + 15, and a cell no path inside the band reaches holds
-// `top` less at most 16 e (r + c + 2), cells outside the matrix from anti-diagonal -2 on among them: the host takes this form only where both fit 16 bits apart (group16_top), so
-// every min picks what the 32-bit form picks and the low nibble of every sum, the decision, is the same. The adds
-// wrap as 16-bit integers and never reach the wrap; the mins are signed.
+// `top` less at most 16 e (r + c + 2), cells outside the matrix from anti-diagonal -2 on among them: the host takes
+// this form only where both fit 16 bits apart (group16_top), so every min picks what the 32-bit form picks and the low
+// nibble of every sum, the decision, is the same. The adds wrap as 16-bit integers and never reach the wrap; the mins
+// are signed.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pk_add(uint32_t a, uint32_t b) {

@@ -161,7 +161,6 @@ struct dinara_scoring_batch {
     std::vector<int32_t> score_h, end_row_h, end_col_h, reach_row_h, reach_col_h, cigar_length_h;
     std::vector<int64_t> cigar_offset_h;
     std::vector<char> cigars_h;
-    int64_t max_rows = 0, max_cols = 0;
     // device memory
     DeviceBuffer codes, ref_at, qry_at, view, list, table, score, end_row, end_col, target, walk_base, walk_columns, arena,
         arena_at, carry, carry_at, op_scratch, op_base, cigars, cigar_used, cigar_offset, cigar_length;
@@ -387,7 +386,6 @@ int64_t prepare(Batch *b, const char *const *refs, const int64_t *ref_lens, cons
     const int64_t slots = (int64_t)b->slot_pair.size();
     std::vector<int64_t> ref_at(std::max<int64_t>(slots, 1)), qry_at(std::max<int64_t>(slots, 1)), op_base(slots + 1);
     int64_t total = 0, ops = 0, text = 0;
-    b->max_rows = b->max_cols = 0;
     for (int64_t s = 0; s < slots; ++s) {
         const int32_t p = b->slot_pair[s];
         ref_at[s] = total;
@@ -397,8 +395,6 @@ int64_t prepare(Batch *b, const char *const *refs, const int64_t *ref_lens, cons
         op_base[s] = ops;
         ops += 8 * ((b->rows[p] + b->cols[p]) / 32 + 1);
         text += 2 * (b->rows[p] + b->cols[p]) + 2;
-        b->max_rows = std::max(b->max_rows, b->rows[p]);
-        b->max_cols = std::max(b->max_cols, b->cols[p]);
     }
     op_base[slots] = ops;
     std::vector<uint8_t> codes((size_t)std::max<int64_t>(total, 1));

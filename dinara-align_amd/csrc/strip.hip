@@ -1,7 +1,7 @@
 // The strip sweep on MI355X (gfx950): Gotoh's recurrence in cost form over a band of diagonals (or the whole matrix),
 // each cell's decision kept under the reference's flag rule, then the walk back (reference lanes.mojo:795-947
 // recurrence, :905-923 flags, :1410-1460 walk). It takes the bands too wide for a group of sixteen lanes, two-piece
-// gaps, free ends, and the pairs no band settles.
+// gaps and free ends but for short pairs in narrow bands (sweep.hip), and the pairs no band settles.
 //
 // Layout. The query's columns are cut into strips of 64 C (C = 2, 4 or 8 a lane); a wave sweeps a strip top to bottom
 // over the rows whose cells there hold the band, lane j holding columns c0 + 1 .. c0 + C (c0 = strip * 64 C + jC) one
@@ -15,11 +15,12 @@
 // writes to a carry record a row, with a relaxed agent-scope atomic store: the record's own nonzero value says it is
 // there, so no fence or flag is needed, and agent scope keeps it coherent across the XCDs' L2s. The reading wave
 // fetches 64 rows' records at once (lane i row s + i) every 64 steps, and lane 0 takes row s's with a readlane; column
-// 0's borders are made the same way. So a pair's strips run as a pipeline over the whole chip, each 64 C + 128 rows or so behind the one to its left, and one
-// launch takes every pair of a round, whatever its band. Waves claim strips in the host's order, in which a strip
-// always follows the one to its left (which is then held by a running wave), the pairs with the most strips first (their
-// pipelines are the launch's longest chains); every wait gives up after STRIP_POLL_LIMIT
-// polls, and the host sweeps the pairs that leaves unsettled whole.
+// 0's borders are made the same way. So a pair's strips run as a pipeline over the whole chip, each 64 C + 128 rows or
+// so behind the one to its left, and one launch takes every pair of a round, whatever its band, or as many of them as
+// its decisions and carry records find room for. Waves claim strips in the host's order, in which a strip always
+// follows the one to its left (which is then held by a running wave), the pairs with the most strips first (their
+// pipelines are the launch's longest chains); every wait gives up after STRIP_POLL_LIMIT polls, and the host sweeps the
+// pairs that leaves unsettled whole.
 //
 // The reference's letters pass through a ring in LDS, 64 written every 64 steps and loaded 64 steps before that; the
 // lane's query letters sit in registers. Between refills a step is the cells, two DPP moves, the letter's read and the
