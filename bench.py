@@ -478,7 +478,7 @@ def run_oversized(args) -> int:
     cpu = None
     exact = None
     if not args.no_cpu:
-        from oracle import oracle  # the checker, on the CPU leg only
+        from oracle import oracle  # on the CPU leg only
 
         oc = oracle.Costs.affine(MISMATCH, OPEN, EXTEND)
         t0 = time.perf_counter()
