@@ -30,6 +30,9 @@ FLAGS = [
     "-Wall",
     "-Wno-unused-function",
     "-I" + os.path.join(ROOT, "include"),
+    # Host functions start on 128 bytes, so that a loop's place in its cache lines is the source's and not the link's:
+    # drawing a network's weights took 9.3 ms with its function 48 bytes past such a place, 5.4 elsewhere (AMD EPYC).
+    "-Xarch_host", "-falign-functions=128",
     # Packed FP32 forms are kept out of every device code object.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
